@@ -22,6 +22,7 @@
 #include "ctx.hpp"
 #include "kernels.hpp"
 #include "kernels_linalg.hpp"
+#include "kernels_sell.hpp"
 #include "mesh.hpp"
 #include "setup.hpp"
 
@@ -127,6 +128,12 @@ cfdg::Csr to_device_rows(const cfdg::Csr& in, const std::vector<i32>& new2old, c
 
 namespace {
 
+// Bytes of one block of the row-major copy (bfloat16 blocks are padded, see BlockLayout).
+std::size_t csr_block_bytes(int storage) {
+    if (storage == cfdg::kStoreBF16) return cfdg::BlockLayout<cfdg::bf16>::block * sizeof(cfdg::bf16);
+    return 25 * (storage == cfdg::kStoreF32 ? sizeof(float) : sizeof(double));
+}
+
 template <typename F>
 int guarded(cfdg_ctx* c, F&& fn) {
     if (!c) return CFDG_ERR_ARG;
@@ -148,21 +155,7 @@ void upload_groups(cfdg_ctx& c, int slot, const std::vector<i32>& label_mesh, i3
     for (std::size_t i = 0; i < rows.size(); ++i) rows[i] = c.old2new[z(g.rows[i])];
     c.h_gofs[slot] = g.off;
     c.grows[slot].upload(rows, c.stream);
-}
-
-// Forward-sweep flags of every block (device order) from the rows' group
-// labels (mesh order): 1 when the column's group precedes the row's; and of
-// every device row: 1 when it lies in the first group (label 0).
-void upload_lower_flags(cfdg_ctx& c, int slot, const std::vector<i32>& label_mesh) {
-    std::vector<std::uint8_t> f(c.h_cols.size(), 0), first(z(c.nc), 0);
-    for (i32 o = 0; o < c.nc; ++o) {
-        first[z(c.old2new[z(o)])] = label_mesh[z(o)] == 0 ? 1 : 0;
-        for (i32 k = c.h_row_ptr[z(o)]; k < c.h_row_ptr[z(o) + 1]; ++k)
-            f[z(c.blk_dev[z(k)])] = label_mesh[z(c.h_cols[z(k)])] < label_mesh[z(o)] ? 1 : 0;
-    }
-    c.blk_lower[slot].upload(f, c.stream);
-    c.row_first[slot].upload(first, c.stream);
-    c.sync();  // f and first are released on return
+    c.sync();  // rows is released on return
 }
 
 void build_seq_groups(cfdg_ctx& c) {
@@ -170,11 +163,75 @@ void build_seq_groups(cfdg_ctx& c) {
     i32 nfw = 0, nbw = 0;
     const auto lf = cfdg::forward_levels(c.ccf_mesh, c.nc, nfw);
     const auto lb = cfdg::backward_levels(c.ccf_mesh, c.nc, nbw);
-    upload_groups(c, 2, lf, nfw, false);
-    upload_groups(c, 3, lb, nbw, false);
-    upload_lower_flags(c, 1, lf);
+    upload_groups(c, 0, lf, nfw, false);
+    upload_groups(c, 1, lb, nbw, false);
+    // forward-sweep flags of every block (device order): 1 when the column's
+    // level precedes the row's; and of every device row: 1 in the first level
+    std::vector<std::uint8_t> f(c.h_cols.size(), 0), first(z(c.nc), 0);
+    std::size_t kd = 0;
+    for (i32 r = 0; r < c.nc; ++r) {
+        const i32 o = c.new2old[z(r)];
+        first[z(r)] = lf[z(o)] == 0 ? 1 : 0;
+        for (i32 k = c.h_row_ptr[z(o)]; k < c.h_row_ptr[z(o) + 1]; ++k)
+            f[kd++] = lf[z(c.h_cols[z(k)])] < lf[z(o)] ? 1 : 0;
+    }
+    c.blk_lower.upload(f, c.stream);
+    c.row_first.upload(first, c.stream);
     c.sync();
     c.have_seq_groups = true;
+}
+
+// Where the blocks of the ABI's pattern are stored.
+std::vector<i32> mesh_block_codes(const cfdg_ctx& c) {
+    return cfdg::sell_block_codes(c.sell, c.h_row_ptr, c.h_cols, c.old2new);
+}
+
+// The row-major copy of the current blocks (device row order, columns
+// ascending in mesh numbering).
+void ensure_csr(cfdg_ctx& c) {
+    if (c.have_csr) return;
+    if (c.csr_code.size() == 0) {
+        const std::vector<i32> mesh_code = mesh_block_codes(c);
+        std::vector<i32> rp(z(c.nc) + 1, 0), cols(c.h_cols.size()), dg(z(c.nc)), code(c.h_cols.size());
+        for (i32 r = 0; r < c.nc; ++r) {
+            const i32 o = c.new2old[z(r)];
+            const i32 k0 = c.h_row_ptr[z(o)];
+            rp[z(r) + 1] = rp[z(r)] + (c.h_row_ptr[z(o) + 1] - k0);
+            for (i32 k = k0; k < c.h_row_ptr[z(o) + 1]; ++k) {
+                cols[z(rp[z(r)] + (k - k0))] = c.old2new[z(c.h_cols[z(k)])];
+                code[z(rp[z(r)] + (k - k0))] = mesh_code[z(k)];
+            }
+            dg[z(r)] = rp[z(r)] + (c.h_diag[z(o)] - k0);
+        }
+        c.row_ptr.upload(rp, c.stream);
+        c.cols.upload(cols, c.stream);
+        c.diag.upload(dg, c.stream);
+        c.csr_code.upload(code, c.stream);
+        c.sync();
+    }
+    const std::size_t nnzb = c.h_cols.size();
+    const std::size_t bytes = nnzb * csr_block_bytes(c.storage);
+    if (c.values.size() != bytes) {
+        c.values.alloc(bytes);
+        c.values.zero(c.stream);  // the padding of bfloat16 rows
+    }
+    const std::size_t lu_bytes = z(c.nc) * 25 * (c.lu_f32 ? sizeof(float) : sizeof(double));
+    if (c.lu_csr.size() != lu_bytes) c.lu_csr.alloc(lu_bytes);
+    if (c.piv.size() != z(c.nc) * 5) c.piv.alloc(z(c.nc) * 5);
+    cfdg::launch_sell_to_csr(c.csr_code.get(), static_cast<long long>(nnzb), c.sellmatrix(), c.values.get(), c.stream);
+    c.check_launch();
+    c.have_csr = true;
+}
+
+// The work vectors in the layout of the next solve; the sliced kernels and
+// reductions rely on zeros past a slice's rows.
+void use_layout(cfdg_ctx& c, bool sliced) {
+    if (sliced && !c.vectors_sliced) {
+        for (DBuf<double>* v : {&c.r, &c.r0, &c.p, &c.v, &c.s, &c.t, &c.ph, &c.sh}) v->zero(c.stream);
+        auto& f = c.f32;
+        for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh}) v->zero(c.stream);
+    }
+    c.vectors_sliced = sliced;
 }
 
 void eval_residual(cfdg_ctx& c) {
@@ -230,8 +287,9 @@ void compute_dt(cfdg_ctx& c) {
 void assemble_jacobian(cfdg_ctx& c) {
     if (!c.have_dt) throw CfdgError(CFDG_ERR_STATE, "assemble_jacobian before compute_dt");
     hip_check(hipEventRecord(c.ev[5], c.stream), "event");
-    cfdg::launch_jacobian(c.margs(), c.fargs(), c.nargs, c.bargs(), c.alpha.get(), c.values.get(), c.storage,
-                          c.stream);
+    cfdg::launch_jacobian(c.margs(), c.fargs(), c.nargs, c.sellargs(), c.alpha.get(), c.sell_off.get(),
+                          c.sell_diag.get(), c.storage, c.stream);
+    c.have_csr = false;
     hip_check(hipEventRecord(c.ev[6], c.stream), "event");
     c.check_launch();
     c.sync();
@@ -253,11 +311,11 @@ void fetch_dots(cfdg_ctx& c, int n) {
 }
 
 template <class T>
-double dot_device(cfdg_ctx& c, const T* a, const T* b) {
+double dot_device(cfdg_ctx& c, long long n, const T* a, const T* b) {
     cfdg::DotPairsT<T> pr{};
     pr.a[0] = a;
     pr.b[0] = b;
-    cfdg::launch_dots(5LL * c.nc, 1, pr, c.partial.get(), c.dots.get(), c.stream);
+    cfdg::launch_dots(n, 1, pr, c.partial.get(), c.dots.get(), c.stream);
     fetch_dots(c, 1);
     return c.h_dots[0];
 }
@@ -265,7 +323,13 @@ double dot_device(cfdg_ctx& c, const T* a, const T* b) {
 struct Precond {
     int kind = CFDG_PRECOND_NONE;
     int order = CFDG_SGS_MULTICOLOUR;
+    // the multicolour sweeps run on the sliced layout; the dependency levels
+    // and the solve without preconditioner on the row-major copy
+    bool sliced() const { return kind == CFDG_PRECOND_SGS && order == CFDG_SGS_MULTICOLOUR; }
 };
+
+// Elements of a solve's vectors.
+long long vector_size(const cfdg_ctx& c, const Precond& P) { return P.sliced() ? c.sliced_size() : 5LL * c.nc; }
 
 // Work vectors of one Krylov precision.
 template <class T>
@@ -281,8 +345,11 @@ KVecs<float> kvecs32(cfdg_ctx& c) {
 }
 
 template <class T>
-void spmv_stored(cfdg_ctx& c, const T* x, T* y, const double* gate = nullptr) {
-    cfdg::launch_spmv<T>(c.bargs(), c.values.get(), c.storage, x, y, c.stream, gate);
+void spmv_stored(cfdg_ctx& c, const Precond& P, const T* x, T* y, const double* gate = nullptr) {
+    if (P.sliced())
+        cfdg::launch_sell_spmv<T>(c.sellargs(), c.sellmatrix(), x, y, c.stream, gate);
+    else
+        cfdg::launch_spmv<T>(c.bargs(), c.values.get(), c.storage, x, y, c.stream, gate);
 }
 
 // z = M^-1 r: z = 0, forward groups, backward groups (preconditioners.cpp:171-194).
@@ -298,23 +365,44 @@ void spmv_stored(cfdg_ctx& c, const T* x, T* y, const double* gate = nullptr) {
 template <class T>
 void precond_apply(cfdg_ctx& c, const Precond& P, const T* r, T* z, const double* gate = nullptr,
                    bool first_done = false) {
-    const long long n5 = 5LL * c.nc;
     if (P.kind == CFDG_PRECOND_NONE) {
-        hip_check(hipMemcpyAsync(z, r, static_cast<std::size_t>(n5) * sizeof(T), hipMemcpyDeviceToDevice, c.stream),
+        hip_check(hipMemcpyAsync(z, r, static_cast<std::size_t>(vector_size(c, P)) * sizeof(T),
+                                 hipMemcpyDeviceToDevice, c.stream),
                   "copy");
         return;
     }
-    const bool seq = P.order == CFDG_SGS_SEQUENTIAL;
-    const int gf = seq ? 2 : 0;
+    if (P.sliced()) {
+        const auto b = c.sellargs();
+        const auto m = c.sellmatrix();
+        const auto& off = c.sell.colour_slice;
+        const int nc = static_cast<int>(off.size()) - 1;
+        const auto sweep = [&](int k, bool all) {
+            cfdg::launch_sell_sweep<T>(b, m, off[cfdg::z(k)], off[cfdg::z(k) + 1] - off[cfdg::z(k)], all, r, z,
+                                       c.stream, gate);
+        };
+        for (int k = first_done ? 1 : 0; k < nc; ++k) sweep(k, false);
+        for (int k = nc - 2; k >= 0; --k) sweep(k, true);
+        return;
+    }
     const auto b = c.bargs();
     for (int sweep = 0; sweep < 2; ++sweep) {
-        const int gi = gf + sweep;
-        const auto& off = c.h_gofs[gi];
-        const std::uint8_t* lower = sweep == 0 ? c.blk_lower[seq ? 1 : 0].get() : nullptr;
+        const auto& off = c.h_gofs[sweep];
+        const std::uint8_t* lower = sweep == 0 ? c.blk_lower.get() : nullptr;
         for (std::size_t k = (sweep == 1 || first_done ? 1 : 0); k + 1 < off.size(); ++k)
-            cfdg::launch_sgs_group<T>(c.grows[gi].get() + off[k], off[k + 1] - off[k], b, c.values.get(), c.storage,
-                                      c.lu.get(), c.piv.get(), lower, r, z, c.stream, gate);
+            cfdg::launch_sgs_group<T>(c.grows[sweep].get() + off[k], off[k + 1] - off[k], b, c.values.get(), c.storage,
+                                      c.lu_csr.get(), c.piv.get(), lower, r, z, c.stream, gate);
     }
+}
+
+// y = p (op 0) or s (op 1) and the first group's z = M^-1 y in one launch.
+template <class T>
+void vec_sgs_first(cfdg_ctx& c, const Precond& P, int op, const double* ks, const T* r, const T* v, T* y, T* z) {
+    if (P.sliced())
+        cfdg::launch_sell_vec_first<T>(op, c.sellargs(), c.sellmatrix(), c.sell.colour_slice[1], ks, r, v, y, z,
+                                       c.stream);
+    else
+        cfdg::launch_vec_sgs_first<T>(op, c.nc, ks, r, v, y, c.row_first.get(), c.storage, c.lu_csr.get(),
+                                      c.piv.get(), z, c.stream);
 }
 
 // Diagonal-block LU of the SGS preconditioner (preconditioners.cpp:62-93).
@@ -322,11 +410,18 @@ void precond_apply(cfdg_ctx& c, const Precond& P, const T* r, T* z, const double
 // a zero pivot makes the solve produce non-finite values, and the error names
 // the row either way.
 void precond_setup(cfdg_ctx& c, const Precond& P) {
+    use_layout(c, P.sliced());
+    if (!P.sliced()) ensure_csr(c);
     if (P.kind != CFDG_PRECOND_SGS) return;
-    if (P.order == CFDG_SGS_SEQUENTIAL) build_seq_groups(c);
     c.singular.zero(c.stream);
-    cfdg::launch_lu_factor(c.nc, c.diag.get(), c.values.get(), c.storage, c.lu.get(), c.lu_f32, c.piv.get(),
-                           c.singular.get(), c.stream);
+    if (P.sliced()) {
+        cfdg::launch_sell_lu(c.sellargs(), c.sellmatrix(), c.lu.get(), c.lu_f32, c.sell_piv.get(), c.singular.get(),
+                             c.stream);
+    } else {
+        build_seq_groups(c);
+        cfdg::launch_lu_factor(c.nc, c.diag.get(), c.values.get(), c.storage, c.lu_csr.get(), c.lu_f32, c.piv.get(),
+                               c.singular.get(), c.stream);
+    }
     c.check_launch();
 }
 
@@ -347,7 +442,7 @@ void precond_check(cfdg_ctx& c, const Precond& P) {
 template <class T>
 cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& P, const KVecs<T>& w, T* x,
                           const T* bvec, bool zero_fallback = false, bool x_zero = false) {
-    const long long N = 5LL * c.nc;
+    const long long N = vector_size(c, P);
     const std::size_t bytes = static_cast<std::size_t>(N) * sizeof(T);
     cfdg_iter_result res{CFDG_MAX_ITERATIONS, 0, 0.0, 0.0};
     // two state blocks: an iteration that ends in launch_xr_next reads one and
@@ -365,7 +460,7 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
         if (x_zero) {
             hip_check(hipMemcpyAsync(w.r, bvec, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
         } else {
-            spmv_stored<T>(c, x, w.v);
+            spmv_stored<T>(c, P, x, w.v);
             cfdg::launch_axpy_copy<T>(N, bvec, -1.0, w.v, w.r, c.stream);
             pr.a[1] = w.r;
             pr.b[1] = w.r;
@@ -386,7 +481,6 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
         const int slot = (sizeof(T) == sizeof(double)) ? 0 : 1;
         int batch = std::max(1, c.last_iters[slot] - 1);
         const bool sgs = P.kind == CFDG_PRECOND_SGS;
-        const std::uint8_t* first = c.row_first[P.order == CFDG_SGS_SEQUENTIAL ? 1 : 0].get();
         long long enq = 0;
         double* rr = c.dots.get() + 5;
         // with SGS, every iteration but the last of a batch (and the ones with
@@ -401,13 +495,12 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
                 if (p_ready) {
                     // formed by the previous iteration's launch_xr_next
                 } else if (sgs) {
-                    cfdg::launch_vec_sgs_first<T>(0, c.nc, ks, w.r, w.v, w.p, first, c.storage, c.lu.get(),
-                                                  c.piv.get(), w.ph, c.stream);
+                    vec_sgs_first<T>(c, P, 0, ks, w.r, w.v, w.p, w.ph);
                 } else {
                     cfdg::launch_update_p_g<T>(N, ks, w.r, w.v, w.p, c.stream);
                 }
                 precond_apply<T>(c, P, w.p, w.ph, ks, sgs);
-                spmv_stored<T>(c, w.ph, w.v, ks);
+                spmv_stored<T>(c, P, w.ph, w.v, ks);
                 {
                     cfdg::DotPairsT<T> pr{};
                     pr.a[0] = w.r0;
@@ -415,13 +508,12 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
                     cfdg::launch_dots_step(N, 1, pr, c.partial.get(), c.dots.get(), ks, cfdg::kStepAlpha, c.stream);
                 }
                 if (sgs) {
-                    cfdg::launch_vec_sgs_first<T>(1, c.nc, ks, w.r, w.v, w.s, first, c.storage, c.lu.get(),
-                                                  c.piv.get(), w.sh, c.stream);
+                    vec_sgs_first<T>(c, P, 1, ks, w.r, w.v, w.s, w.sh);
                 } else {
                     cfdg::launch_axpy_alpha_g<T>(N, ks, w.r, w.v, w.s, c.stream);
                 }
                 precond_apply<T>(c, P, w.s, w.sh, ks, sgs);
-                spmv_stored<T>(c, w.sh, w.t, ks);
+                spmv_stored<T>(c, P, w.sh, w.t, ks);
                 {
                     cfdg::DotPairsT<T> pr{};
                     const T* A[5] = {w.t, w.t, w.r0, w.r0, w.s};
@@ -434,8 +526,12 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
                 }
                 const bool next_in_batch = b + 1 < batch && enq <= lp.max_iter;
                 if (sgs && next_in_batch && enq % 32 != 0) {
-                    cfdg::launch_xr_next<T>(c.nc, ks, kb[1 - cur], w.ph, w.sh, w.s, w.t, x, w.r, w.v, w.p, first,
-                                            c.storage, c.lu.get(), c.piv.get(), c.stream);
+                    if (P.sliced())
+                        cfdg::launch_sell_xr_next<T>(c.sellargs(), c.sellmatrix(), c.sell.colour_slice[1], ks,
+                                                     kb[1 - cur], w.ph, w.sh, w.s, w.t, x, w.r, w.v, w.p, c.stream);
+                    else
+                        cfdg::launch_xr_next<T>(c.nc, ks, kb[1 - cur], w.ph, w.sh, w.s, w.t, x, w.r, w.v, w.p,
+                                                c.row_first.get(), c.storage, c.lu_csr.get(), c.piv.get(), c.stream);
                     cur = 1 - cur;
                     p_ready = true;
                     continue;
@@ -484,12 +580,12 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
 // FP64 arithmetic over the stored blocks and solves A e = r in FP32 from e = 0.
 cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& P, double* x,
                                    const double* bvec, bool zero_fallback = false, bool x_zero = false) {
-    const long long N = 5LL * c.nc;
+    const long long N = vector_size(c, P);
     cfdg_iter_result res{CFDG_MAX_ITERATIONS, 0, 0.0, 0.0};
     const auto outer_residual = [&]() {
-        spmv_stored<double>(c, x, c.v.get());
+        spmv_stored<double>(c, P, x, c.v.get());
         cfdg::launch_axpy_copy<double>(N, bvec, -1.0, c.v.get(), c.r.get(), c.stream);
-        return std::sqrt(dot_device<double>(c, c.r.get(), c.r.get()));
+        return std::sqrt(dot_device<double>(c, N, c.r.get(), c.r.get()));
     };
     // ||b|| and the first outer residual in one reduction (r = b for a zero guess)
     double bnorm = 0.0, rnorm = 0.0;
@@ -501,7 +597,7 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
             hip_check(hipMemcpyAsync(c.r.get(), bvec, static_cast<std::size_t>(N) * sizeof(double),
                                      hipMemcpyDeviceToDevice, c.stream), "copy");
         } else {
-            spmv_stored<double>(c, x, c.v.get());
+            spmv_stored<double>(c, P, x, c.v.get());
             cfdg::launch_axpy_copy<double>(N, bvec, -1.0, c.v.get(), c.r.get(), c.stream);
             pr.a[1] = c.r.get();
             pr.b[1] = c.r.get();
@@ -513,7 +609,7 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
     }
     if (zero_fallback) {
         if (!(rnorm <= bnorm)) {
-            c.x.zero(c.stream);
+            hip_check(hipMemsetAsync(x, 0, static_cast<std::size_t>(N) * sizeof(double), c.stream), "memset");
             hip_check(hipMemcpyAsync(c.r.get(), bvec, static_cast<std::size_t>(N) * sizeof(double),
                                      hipMemcpyDeviceToDevice, c.stream), "copy");
             rnorm = bnorm;
@@ -565,48 +661,81 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
     return res;
 }
 
-void linear_solve(cfdg_ctx& c, const cfdg_linparams& lp, const double* hb, const double* hx0, double* hx,
-                  cfdg_iter_result* out) {
+// Mesh-order vectors of the ABI (5 per cell) into the sliced layout and back.
+void upload_sliced(cfdg_ctx& c, const double* h, double* dst) {
+    const std::size_t n5 = 5ULL * z(c.nc);
+    if (c.stage.size() != n5) c.stage.alloc(n5);
+    c.h2d(c.stage.get(), h, n5);
+    cfdg::launch_sell_gather(c.sellargs(), c.mesh_of_row.get(), c.stage.get(), dst, c.stream);
+    c.sync();
+}
+void download_sliced(cfdg_ctx& c, const double* src, double* h) {
+    const std::size_t n5 = 5ULL * z(c.nc);
+    if (c.stage.size() != n5) c.stage.alloc(n5);
+    cfdg::launch_sell_scatter(c.sellargs(), c.mesh_of_row.get(), src, c.stage.get(), c.stream);
+    c.d2h(h, c.stage.get(), n5);
+    c.sync();
+}
+
+// The solution stays in c.xs (multicolour SGS) or c.x; returns which Krylov
+// layout the solve used.
+Precond linear_solve(cfdg_ctx& c, const cfdg_linparams& lp, const double* hb, const double* hx0, double* hx,
+                     cfdg_iter_result* out) {
     if (lp.preconditioner != CFDG_PRECOND_NONE && lp.preconditioner != CFDG_PRECOND_SGS)
         throw CfdgError(CFDG_ERR_CONFIG, "unknown preconditioner");
     if (lp.sgs_order != CFDG_SGS_MULTICOLOUR && lp.sgs_order != CFDG_SGS_SEQUENTIAL)
         throw CfdgError(CFDG_ERR_CONFIG, "unknown SGS order");
     if (lp.max_iter < 0) throw CfdgError(CFDG_ERR_ARG, "max_iter must be >= 0");
     require_jacobian(c);
-    const std::size_t n5 = 5ULL * static_cast<std::size_t>(c.nc);
-    if (hb) {
-        const auto d = c.vec_to_device(hb);
-        c.h2d(c.b.get(), d.data(), n5);
-        c.sync();
-    } else {
-        if (!c.have_residual) throw CfdgError(CFDG_ERR_STATE, "implicit right-hand side needs a residual");
-        cfdg::launch_rhs(c.nc, c.nc, c.res.get(), c.b.get(), c.stream);
-    }
-    bool learned = false, x_zero = false;
-    if (hx0) {
-        const auto d = c.vec_to_device(hx0);
-        c.h2d(c.x.get(), d.data(), n5);
-        c.sync();
-    } else if (!hb && c.warm) {
-        learned = cfdg::gnn_warm_guess(c, c.x.get());
-    } else {
-        c.x.zero(c.stream);
-        x_zero = true;
-    }
     Precond P;
     P.kind = lp.preconditioner;
     P.order = lp.sgs_order;
+    const bool sliced = P.sliced();
+    double* const b = sliced ? c.bs.get() : c.b.get();
+    double* const x = sliced ? c.xs.get() : c.x.get();
+    const std::size_t n5 = 5ULL * static_cast<std::size_t>(c.nc);
+    const auto upload = [&](const double* h, double* dst) {
+        if (sliced) {
+            upload_sliced(c, h, dst);
+            return;
+        }
+        const auto d = c.vec_to_device(h);
+        c.h2d(dst, d.data(), n5);
+        c.sync();
+    };
+    if (hb) {
+        upload(hb, b);
+    } else {
+        if (!c.have_residual) throw CfdgError(CFDG_ERR_STATE, "implicit right-hand side needs a residual");
+        if (sliced)
+            cfdg::launch_sell_rhs(c.sellargs(), c.nc, c.res.get(), b, c.stream);
+        else
+            cfdg::launch_rhs(c.nc, c.nc, c.res.get(), b, c.stream);
+    }
+    bool learned = false, x_zero = false;
+    if (hx0) {
+        upload(hx0, x);
+    } else if (!hb && c.warm) {
+        learned = cfdg::gnn_warm_guess(c, c.x.get());
+        if (sliced) cfdg::launch_sell_gather(c.sellargs(), nullptr, c.x.get(), x, c.stream);
+    } else {
+        hip_check(hipMemsetAsync(x, 0, static_cast<std::size_t>(vector_size(c, P)) * sizeof(double), c.stream),
+                  "memset");
+        x_zero = true;
+    }
     hip_check(hipEventRecord(c.ev[5], c.stream), "event");
     precond_setup(c, P);
     const cfdg_iter_result r = (c.prec.krylov == CFDG_PREC_FP32)
-                                   ? defect_correction(c, lp, P, c.x.get(), c.b.get(), learned, x_zero)
-                                   : bicgstab<double>(c, lp, P, kvecs64(c), c.x.get(), c.b.get(), learned, x_zero);
+                                   ? defect_correction(c, lp, P, x, b, learned, x_zero)
+                                   : bicgstab<double>(c, lp, P, kvecs64(c), x, b, learned, x_zero);
     hip_check(hipEventRecord(c.ev[6], c.stream), "event");
     c.sync();
     precond_check(c, P);
-    if (hx) {
+    if (hx && sliced) {
+        download_sliced(c, x, hx);
+    } else if (hx) {
         std::vector<double> d(n5);
-        c.d2h(d.data(), c.x.get(), n5);
+        c.d2h(d.data(), x, n5);
         c.sync();
         c.vec_to_mesh(d, hx);
     }
@@ -614,6 +743,7 @@ void linear_solve(cfdg_ctx& c, const cfdg_linparams& lp, const double* hb, const
     hip_check(hipEventElapsedTime(&ms, c.ev[5], c.ev[6]), "elapsed");
     c.stage_ms[5] = ms;
     if (out) *out = r;
+    return P;
 }
 
 void residual_norms(cfdg_ctx& c, double l2[5]) {
@@ -637,6 +767,24 @@ void check_numerics(const cfdg_numerics* num) {
         throw CfdgError(CFDG_ERR_CONFIG, "gamma > 1, gas_constant > 0 and cfl > 0 required");
     if (num->flow_model == CFDG_VISCOUS_FLOW && (!(num->prandtl > 0.0) || !(num->prandtl_turb > 0.0)))
         throw CfdgError(CFDG_ERR_CONFIG, "viscous flow needs prandtl > 0 and prandtl_turb > 0");
+}
+
+// Block arrays and LU factors of the sliced layout.
+void alloc_blocks(cfdg_ctx& c, int storage) {
+    c.sell_off.alloc(0);
+    c.sell_diag.alloc(0);
+    c.sell_off.alloc(z(c.sell.n_slots) * cfdg::sell_slot_bytes(storage));
+    c.sell_diag.alloc(z(c.n_slices()) * cfdg::sell_slot_bytes(storage));
+    c.sell_off.zero(c.stream);
+    c.sell_diag.zero(c.stream);
+    c.have_csr = false;
+    c.values.alloc(0);
+}
+void alloc_lu(cfdg_ctx& c, int lu_f32) {
+    c.lu.alloc(0);
+    c.lu.alloc(z(c.n_slices()) * cfdg::sell_slot_bytes(lu_f32 ? cfdg::kStoreF32 : cfdg::kStoreF64));
+    c.lu_csr.alloc(0);
+    c.have_csr = false;
 }
 
 void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivity* cn, const cfdg_numerics* num,
@@ -750,6 +898,27 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
                 if (o >= tl.tile_off[z(k)] && o < tl.tile_off[z(k) + 1]) fentry[z(f)] = e;
             }
         c.face_entry.upload(fentry, s);
+        // block matrix: multicolour order of the rows, sliced layout
+        i32 ncol = 0;
+        const auto col = cfdg::greedy_colours(c.ccf_mesh, c.nc, ncol);
+        c.sell = cfdg::sell_plan(tl, col, ncol, cf_dev, tf, owner_dev, other_dev, c.ninner);
+        static_assert(sizeof(cfdg::Slice) == sizeof(int4) && cfdg::kSliceRows == cfdg::kSellRows &&
+                          cfdg::kVisitNone == cfdg::kSellVisitNone &&
+                          cfdg::kVisitNeighbour == cfdg::kSellVisitNeighbour,
+                      "the plan's arrays are read by the kernels as they are");
+        c.sell_slice.alloc(c.sell.slices.size());
+        c.h2d(reinterpret_cast<cfdg::Slice*>(c.sell_slice.get()), c.sell.slices.data(), c.sell.slices.size());
+        c.sell_row.upload(c.sell.row, s);
+        c.sell_pos.upload(c.sell.pos, s);
+        c.sell_count.upload(c.sell.count, s);
+        c.sell_cols.upload(c.sell.cols, s);
+        c.sell_tile_pos.upload(c.sell.tile_pos, s);
+        c.sell_visit.upload(c.sell.visit, s);
+        c.sell_visit_base.upload(c.sell.visit_base, s);
+        c.mesh_of_row.upload(c.new2old, s);
+        c.sync();
+        for (auto* v : {&c.sell.row, &c.sell.tile_pos, &c.sell.visit_base}) std::vector<i32>().swap(*v);
+        std::vector<std::uint32_t>().swap(c.sell.visit);
         const cfdg::Csr ccf_dev = to_device_rows(c.ccf_mesh, c.new2old, &c.old2new);
         c.ccf_off.upload(ccf_dev.off, s);
         c.ccf.upload(ccf_dev.idx, s);
@@ -837,7 +1006,7 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
         }
         c.sync();
     }
-    // BSR: the mesh-order pattern (bsr_helpers.hpp:16-59) and its device rows
+    // BSR: the mesh-order pattern (bsr_helpers.hpp:16-59)
     {
         cfdg::BsrPattern bp_own;
         if (!cn) bp_own = cfdg::bsr_pattern(c.ccf_mesh, c.nc);
@@ -845,48 +1014,6 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
         c.h_row_ptr = bp.row_ptr;
         c.h_cols = bp.cols;
         c.h_diag = bp.diag;
-        std::vector<i32> rp(z(c.nc) + 1, 0), cols(bp.cols.size()), dg(z(c.nc));
-        for (int r = 0; r < c.nc; ++r) {
-            const i32 o = c.new2old[z(r)];
-            rp[z(r) + 1] = rp[z(r)] + (bp.row_ptr[z(o) + 1] - bp.row_ptr[z(o)]);
-        }
-        c.blk_dev.assign(bp.cols.size(), 0);
-        for (int r = 0; r < c.nc; ++r) {
-            const i32 o = c.new2old[z(r)];
-            for (i32 k = bp.row_ptr[z(o)]; k < bp.row_ptr[z(o) + 1]; ++k) {
-                const i32 kd = rp[z(r)] + (k - bp.row_ptr[z(o)]);
-                cols[z(kd)] = c.old2new[z(bp.cols[z(k)])];
-                c.blk_dev[z(k)] = kd;
-            }
-            dg[z(r)] = rp[z(r)] + (bp.diag[z(o)] - bp.row_ptr[z(o)]);
-        }
-        c.row_ptr.upload(rp, s);
-        c.cols.upload(cols, s);
-        c.diag.upload(dg, s);
-        // off-diagonal block of every interior cell face, in the device cell ->
-        // face lists (the Jacobian kernel's store positions)
-        {
-            const cfdg::Csr cf_dev = to_device_rows(cf_mesh, c.new2old, nullptr);
-            std::vector<i32> blk(cf_dev.idx.size(), -1);
-            for (int r = 0; r < c.nc; ++r)
-                for (i32 e = cf_dev.off[z(r)]; e < cf_dev.off[z(r) + 1]; ++e) {
-                    const i32 f = cf_dev.idx[z(e)];
-                    if (f >= c.ninner) continue;
-                    const i32 o = owner_dev[z(f)] == r ? other_dev[z(f)] : owner_dev[z(f)];
-                    i32 k = rp[z(r)];
-                    while (k < rp[z(r) + 1] && cols[z(k)] != o) ++k;
-                    if (k == rp[z(r) + 1]) throw CfdgError(CFDG_ERR_MESH, "face neighbour missing from the BSR row");
-                    blk[z(e)] = k;
-                }
-            c.cf_blk.upload(blk, s);
-            c.sync();  // blk is released at the end of this block
-        }
-        i32 ncol = 0;
-        const auto col = cfdg::greedy_colours(c.ccf_mesh, c.nc, ncol);
-        upload_groups(c, 0, col, ncol, false);
-        upload_groups(c, 1, col, ncol, true);
-        upload_lower_flags(c, 0, col);
-        c.sync();
     }
     const std::size_t ncs = z(c.nc);
     c.U.alloc(5 * ncs);
@@ -899,13 +1026,12 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
     c.U.zero(s);
     c.res.zero(s);
     c.lam.zero(s);
-    c.values.alloc(c.h_cols.size() * 25 * sizeof(double));
-    c.values.zero(s);
-    c.lu.alloc(ncs * 25 * sizeof(double));
-    c.piv.alloc(ncs * 5);
+    alloc_blocks(c, cfdg::kStoreF64);
+    alloc_lu(c, 0);
+    c.sell_piv.alloc(z(c.n_slices()) * cfdg::kSellRows);
     c.singular.alloc(1);
-    for (DBuf<double>* v : {&c.b, &c.x, &c.r, &c.r0, &c.p, &c.v, &c.s, &c.t, &c.ph, &c.sh}) {
-        v->alloc(5 * ncs);
+    for (DBuf<double>* v : {&c.r, &c.r0, &c.p, &c.v, &c.s, &c.t, &c.ph, &c.sh, &c.bs, &c.xs, &c.b, &c.x}) {
+        v->alloc(v == &c.b || v == &c.x ? 5 * ncs : c.vector_alloc());
         v->zero(s);
     }
     c.partial.alloc(static_cast<std::size_t>(cfdg::kReduceBlocks) * 5);
@@ -923,10 +1049,13 @@ void implicit_step(cfdg_ctx& c, const cfdg_linparams& lp, cfdg_step_result* out)
     cfdg::gnn_step_features(c);
     assemble_jacobian(c);
     cfdg_iter_result lr{};
-    linear_solve(c, lp, nullptr, nullptr, nullptr, &lr);
+    const bool sliced = linear_solve(c, lp, nullptr, nullptr, nullptr, &lr).sliced();
     double l2[5];
     residual_norms(c, l2);
-    cfdg::launch_state_update(c.nc, c.nc, c.x.get(), c.U.get(), c.stream);
+    if (sliced)
+        cfdg::launch_sell_state_update(c.sellargs(), c.nc, c.xs.get(), c.U.get(), c.x.get(), c.stream);
+    else
+        cfdg::launch_state_update(c.nc, c.nc, c.x.get(), c.U.get(), c.stream);
     // module block: copied (implicit_euler.hpp:64-72) or point-implicit, then clamped
     if (c.sa_on())
         cfdg::launch_sa_update(c.nc, c.turb.update == CFDG_TURB_POINT_IMPLICIT, c.alpha.get(), c.sargs(), c.stream);
@@ -939,52 +1068,27 @@ void implicit_step(cfdg_ctx& c, const cfdg_linparams& lp, cfdg_step_result* out)
     out->linear = lr;
 }
 
-std::size_t storage_bytes(int storage) {
-    return storage == cfdg::kStoreF64 ? sizeof(double) : (storage == cfdg::kStoreF32 ? sizeof(float) : sizeof(cfdg::bf16));
-}
-
-// Stored values per block (bfloat16 blocks are padded, see BlockLayout).
-std::size_t block_stride(int storage) { return storage == cfdg::kStoreBF16 ? cfdg::BlockLayout<cfdg::bf16>::block : 25; }
-
-// Device-order block values as double (25 per block), whatever the storage.
-std::vector<double> download_values(cfdg_ctx& c) {
-    const std::size_t n = c.blk_dev.size() * 25;
-    std::vector<double> out(n);
-    if (c.storage == cfdg::kStoreF64) {
-        c.d2h(out.data(), reinterpret_cast<const double*>(c.values.get()), n);
-        c.sync();
-    } else if (c.storage == cfdg::kStoreF32) {
-        std::vector<float> h(n);
-        c.d2h(h.data(), reinterpret_cast<const float*>(c.values.get()), n);
-        c.sync();
-        for (std::size_t i = 0; i < n; ++i) out[i] = cfdg::to_f64(h[i]);
-    } else {
-        constexpr int kB = cfdg::BlockLayout<cfdg::bf16>::block, kR = cfdg::BlockLayout<cfdg::bf16>::row;
-        std::vector<cfdg::bf16> h(c.blk_dev.size() * kB);
-        c.d2h(h.data(), reinterpret_cast<const cfdg::bf16*>(c.values.get()), h.size());
-        c.sync();
-        for (std::size_t k = 0; k < c.blk_dev.size(); ++k)
-            for (int i = 0; i < 25; ++i) out[k * 25 + z(i)] = cfdg::to_f64(h[k * kB + z((i / 5) * kR + i % 5)]);
-    }
-    return out;
-}
-
-void upload_values(cfdg_ctx& c, const std::vector<double>& h) {
-    const std::size_t n = h.size();
-    if (c.storage == cfdg::kStoreF64) {
-        c.h2d(reinterpret_cast<double*>(c.values.get()), h.data(), n);
-        c.sync();
-    } else if (c.storage == cfdg::kStoreF32) {
-        std::vector<float> t(n);
-        for (std::size_t i = 0; i < n; ++i) t[i] = cfdg::cvt<float>(h[i]);
-        c.h2d(reinterpret_cast<float*>(c.values.get()), t.data(), n);
-        c.sync();
-    } else {
-        constexpr int kB = cfdg::BlockLayout<cfdg::bf16>::block, kR = cfdg::BlockLayout<cfdg::bf16>::row;
-        std::vector<cfdg::bf16> t(n / 25 * kB, cfdg::bf16{0});
-        for (std::size_t k = 0; k < n / 25; ++k)
-            for (int i = 0; i < 25; ++i) t[k * kB + z((i / 5) * kR + i % 5)] = cfdg::cvt<cfdg::bf16>(h[k * 25 + z(i)]);
-        c.h2d(reinterpret_cast<cfdg::bf16*>(c.values.get()), t.data(), t.size());
+// Blocks of the ABI's pattern as FP64 rows, in pieces of at most 2^22 blocks
+// (0.8 GB of staging): out != null reads them, in != null sets them.
+void transfer_blocks(cfdg_ctx& c, double* out, const double* in) {
+    const std::size_t nnzb = c.h_cols.size();
+    if (c.block_code.size() != nnzb) c.block_code.upload(mesh_block_codes(c), c.stream);
+    c.sync();
+    const std::size_t piece = std::min<std::size_t>(nnzb, 1u << 22);
+    DBuf<double> stage;
+    stage.alloc(piece * 25);
+    for (std::size_t k0 = 0; k0 < nnzb; k0 += piece) {
+        const std::size_t n = std::min(piece, nnzb - k0);
+        const int* code = c.block_code.get() + k0;
+        if (out) {
+            cfdg::launch_sell_get_blocks(code, static_cast<long long>(n), c.sellmatrix(), stage.get(), c.stream);
+            c.d2h(out + k0 * 25, stage.get(), n * 25);
+        } else {
+            c.h2d(stage.get(), in + k0 * 25, n * 25);
+            cfdg::launch_sell_set_blocks(code, static_cast<long long>(n), stage.get(), c.sell_off.get(),
+                                         c.sell_diag.get(), c.storage, c.stream);
+        }
+        c.check_launch();
         c.sync();
     }
 }
@@ -999,21 +1103,16 @@ void set_precision(cfdg_ctx& c, const cfdg_precision& p) {
     if (p.krylov == CFDG_PREC_FP32 && (p.max_outer < 1 || !(p.inner_rel_tol > 0.0 && p.inner_rel_tol < 1.0)))
         throw CfdgError(CFDG_ERR_CONFIG, "FP32 Krylov needs max_outer >= 1 and 0 < inner_rel_tol < 1");
     const int storage = p.block_storage;  // CFDG_PREC_* == kStore*
-    const std::size_t nnzb = c.blk_dev.size();
-    const std::size_t ncs = z(c.nc);
-    if (storage != c.storage || c.values.size() != nnzb * block_stride(storage) * storage_bytes(storage)) {
-        c.values.alloc(0);
-        c.values.alloc(nnzb * block_stride(storage) * storage_bytes(storage));
-        c.values.zero(c.stream);
+    if (storage != c.storage || c.sell_off.size() != z(c.sell.n_slots) * cfdg::sell_slot_bytes(storage)) {
+        alloc_blocks(c, storage);
         c.have_jacobian = false;
     }
     const int lu_f32 = (p.krylov == CFDG_PREC_FP32) ? 1 : 0;
-    c.lu.alloc(0);
-    c.lu.alloc(ncs * 25 * (lu_f32 ? sizeof(float) : sizeof(double)));
+    alloc_lu(c, lu_f32);
     if (p.krylov == CFDG_PREC_FP32) {
         auto& f = c.f32;
         for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh}) {
-            if (v->size() != 5 * ncs) v->alloc(5 * ncs);
+            if (v->size() != c.vector_alloc()) v->alloc(c.vector_alloc());
             v->zero(c.stream);
         }
     } else {
@@ -1195,19 +1294,15 @@ int cfdg_get_bsr_pattern(cfdg_ctx* c, int32_t* row_ptr, int32_t* cols, int32_t* 
 int cfdg_get_bsr_values(cfdg_ctx* c, double* values) {
     return guarded(c, [&] {
         if (!values) throw CfdgError(CFDG_ERR_ARG, "null output");
-        const std::vector<double> h = download_values(*c);
-        for (std::size_t k = 0; k < c->blk_dev.size(); ++k)
-            std::memcpy(values + k * 25, h.data() + z(c->blk_dev[k]) * 25, 25 * sizeof(double));
+        transfer_blocks(*c, values, nullptr);
     });
 }
 
 int cfdg_set_bsr_values(cfdg_ctx* c, const double* values) {
     return guarded(c, [&] {
         if (!values) throw CfdgError(CFDG_ERR_ARG, "null input");
-        std::vector<double> h(c->blk_dev.size() * 25);
-        for (std::size_t k = 0; k < c->blk_dev.size(); ++k)
-            std::memcpy(h.data() + z(c->blk_dev[k]) * 25, values + k * 25, 25 * sizeof(double));
-        upload_values(*c, h);
+        transfer_blocks(*c, nullptr, values);
+        c->have_csr = false;
         c->have_jacobian = true;
     });
 }
@@ -1230,7 +1325,9 @@ int cfdg_linear_solve(cfdg_ctx* c, const cfdg_linparams* lp, const double* b, co
                       cfdg_iter_result* res) {
     return guarded(c, [&] {
         if (!lp) throw CfdgError(CFDG_ERR_ARG, "null linear parameters");
-        linear_solve(*c, *lp, b, x0, x, res);
+        if (linear_solve(*c, *lp, b, x0, x, res).sliced())
+            cfdg::launch_sell_scatter(c->sellargs(), nullptr, c->xs.get(), c->x.get(), c->stream);
+        c->sync();
         c->have_prev_du = false;
     });
 }
@@ -1246,21 +1343,31 @@ int cfdg_sgs_apply(cfdg_ctx* c, int32_t sgs_order, const double* r, double* zout
         P.kind = CFDG_PRECOND_SGS;
         P.order = sgs_order;
         precond_setup(*c, P);
-        const auto d = c->vec_to_device(r);
-        c->h2d(c->s.get(), d.data(), n5);
+        const long long n = vector_size(*c, P);
+        if (P.sliced()) {
+            upload_sliced(*c, r, c->s.get());
+        } else {
+            const auto d = c->vec_to_device(r);
+            c->h2d(c->s.get(), d.data(), n5);
+            c->sync();
+        }
         if (c->prec.krylov == CFDG_PREC_FP32) {
-            cfdg::launch_cast_f64_to_f32(static_cast<long long>(n5), c->s.get(), c->f32.s.get(), c->stream);
+            cfdg::launch_cast_f64_to_f32(n, c->s.get(), c->f32.s.get(), c->stream);
             precond_apply<float>(*c, P, c->f32.s.get(), c->f32.sh.get());
-            cfdg::launch_cast_f32_to_f64(static_cast<long long>(n5), c->f32.sh.get(), c->sh.get(), c->stream);
+            cfdg::launch_cast_f32_to_f64(n, c->f32.sh.get(), c->sh.get(), c->stream);
         } else {
             precond_apply<double>(*c, P, c->s.get(), c->sh.get());
         }
-        std::vector<double> h(n5);
-        c->d2h(h.data(), c->sh.get(), n5);
         c->check_launch();
-        c->sync();
         precond_check(*c, P);
-        c->vec_to_mesh(h, zout);
+        if (P.sliced()) {
+            download_sliced(*c, c->sh.get(), zout);
+        } else {
+            std::vector<double> h(n5);
+            c->d2h(h.data(), c->sh.get(), n5);
+            c->sync();
+            c->vec_to_mesh(h, zout);
+        }
     });
 }
 
@@ -1269,16 +1376,33 @@ int cfdg_sgs_row_groups(cfdg_ctx* c, int32_t sgs_order, int32_t* fwd_group, int3
     return guarded(c, [&] {
         if (sgs_order != CFDG_SGS_MULTICOLOUR && sgs_order != CFDG_SGS_SEQUENTIAL)
             throw CfdgError(CFDG_ERR_CONFIG, "unknown SGS order");
-        if (sgs_order == CFDG_SGS_SEQUENTIAL) build_seq_groups(*c);
-        const int gf = (sgs_order == CFDG_SGS_SEQUENTIAL) ? 2 : 0;
+        if (sgs_order == CFDG_SGS_MULTICOLOUR) {
+            // the rows the kernels are handed, read back from the device: colour
+            // g forward, the colours in reverse backward
+            const auto& off = c->sell.colour_slice;
+            const int ng = static_cast<int>(off.size()) - 1;
+            std::vector<i32> rows(c->sell_row.size());
+            c->d2h(rows.data(), c->sell_row.get(), rows.size());
+            c->sync();
+            for (int k = 0; n_groups && k < 2; ++k) n_groups[k] = ng;
+            for (int g = 0; g < ng; ++g)
+                for (i32 p = off[z(g)] * cfdg::kSellRows; p < off[z(g) + 1] * cfdg::kSellRows; ++p) {
+                    if (rows[z(p)] < 0) continue;
+                    const std::size_t o = z(c->new2old[z(rows[z(p)])]);
+                    if (fwd_group) fwd_group[o] = g;
+                    if (bwd_group) bwd_group[o] = ng - 1 - g;
+                }
+            return;
+        }
+        build_seq_groups(*c);
         for (int sweep = 0; sweep < 2; ++sweep) {
-            const auto& off = c->h_gofs[gf + sweep];
+            const auto& off = c->h_gofs[sweep];
             int32_t* out = sweep == 0 ? fwd_group : bwd_group;
             if (n_groups) n_groups[sweep] = static_cast<int32_t>(off.size()) - 1;
             if (!out) continue;
             // the rows the kernels are handed, read back from the device
-            std::vector<i32> rows(c->grows[gf + sweep].size());
-            c->d2h(rows.data(), c->grows[gf + sweep].get(), rows.size());
+            std::vector<i32> rows(c->grows[sweep].size());
+            c->d2h(rows.data(), c->grows[sweep].get(), rows.size());
             c->sync();
             std::fill(out, out + c->nc, -1);
             for (std::size_t g = 0; g + 1 < off.size(); ++g)
@@ -1291,15 +1415,11 @@ int cfdg_spmv(cfdg_ctx* c, const double* x, double* y) {
     return guarded(c, [&] {
         if (!x || !y) throw CfdgError(CFDG_ERR_ARG, "null vector");
         require_jacobian(*c);
-        const std::size_t n5 = 5ULL * z(c->nc);
-        const auto d = c->vec_to_device(x);
-        c->h2d(c->s.get(), d.data(), n5);
-        spmv_stored<double>(*c, c->s.get(), c->t.get());
-        std::vector<double> h(n5);
-        c->d2h(h.data(), c->t.get(), n5);
+        use_layout(*c, true);
+        upload_sliced(*c, x, c->s.get());
+        cfdg::launch_sell_spmv<double>(c->sellargs(), c->sellmatrix(), c->s.get(), c->t.get(), c->stream);
         c->check_launch();
-        c->sync();
-        c->vec_to_mesh(h, y);
+        download_sliced(*c, c->t.get(), y);
     });
 }
 

@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -12,6 +13,7 @@
 #include "capi_internal.hpp"
 #include "cfdg.h"
 #include "kernels.hpp"
+#include "kernels_sell.hpp"
 #include "setup.hpp"
 
 namespace cfdg {
@@ -104,32 +106,46 @@ struct cfdg_ctx {
     bool have_residual = false;
     bool have_dt = false;
     bool have_jacobian = false;  // block values set (assembled, or given) in the current storage
-    // BSR: mesh-order pattern for the ABI, device-order pattern for the kernels
+    // BSR: mesh-order pattern for the ABI
     std::vector<std::int32_t> h_row_ptr, h_cols, h_diag;
-    std::vector<long long> blk_dev;  // mesh block k -> device block
-    DBuf<int> row_ptr, cols, diag, cf_blk;
-    // per block: 1 when its column lies in an earlier group of the forward SGS
-    // sweep than its row ([0] multicolour groups, [1] dependency levels)
-    DBuf<std::uint8_t> blk_lower[2];
-    // per device row: 1 when it lies in the forward sweep's first group (same slots)
-    DBuf<std::uint8_t> row_first[2];
-    // block values and diagonal LU as raw bytes in the storage of the precision form
-    DBuf<std::uint8_t> values, lu;
+    // sliced block matrix (setup.hpp, SellPlan): the plan's device arrays, the
+    // blocks in the storage of the precision form as raw bytes, the diagonal LU
+    cfdg::SellPlan sell;  // host copy without the Jacobian's visits
+    DBuf<int4> sell_slice;
+    DBuf<int> sell_row, sell_pos, sell_cols, sell_tile_pos, sell_visit_base;
+    DBuf<std::uint32_t> sell_count, sell_visit;
+    DBuf<std::uint16_t> sell_piv;
+    DBuf<std::uint8_t> sell_off, sell_diag, lu;
+    DBuf<int> mesh_of_row;  // device row -> mesh cell
+    DBuf<int> block_code;   // where each block of the ABI's pattern is stored, made on first use
     int storage = cfdg::kStoreF64;
     int lu_f32 = 0;
     cfdg_precision prec{CFDG_PREC_FP64, CFDG_PREC_FP64, 8, 0, 0.1};
-    DBuf<std::uint8_t> piv;
     DBuf<int> singular;
-    // SGS row groups (device rows): 0 multicolour fwd, 1 multicolour bwd, 2 sequential fwd, 3 sequential bwd
-    std::vector<std::int32_t> h_gofs[4];
-    DBuf<int> grows[4];
+    // row-major copy of the matrix in device row order with its LU, for the
+    // sequential SGS order and the solve without preconditioner: made from the
+    // sliced blocks when such a solve needs it (have_csr: up to date)
+    DBuf<int> row_ptr, cols, diag, csr_code;
+    DBuf<std::uint8_t> values, lu_csr, piv;
+    bool have_csr = false;
+    // per block: 1 when its column lies in an earlier dependency level of the
+    // forward sweep than its row; per device row: 1 when in the first level
+    DBuf<std::uint8_t> blk_lower, row_first;
+    // dependency levels of the sequential SGS sweeps (device rows): 0 forward, 1 backward
+    std::vector<std::int32_t> h_gofs[2];
+    DBuf<int> grows[2];
     cfdg::Csr ccf_mesh;
     bool have_seq_groups = false;
-    // Krylov work vectors (AoS, 5 nc, device order); FP32 set for the FP32 form
-    DBuf<double> b, x, r, r0, p, v, s, t, ph, sh;
+    // Krylov work vectors; FP32 set for the FP32 form.  Layout of a solve: 5
+    // per row in device order, or sliced (then zero past a slice's rows).
+    bool vectors_sliced = true;
+    DBuf<double> r, r0, p, v, s, t, ph, sh;
     struct F32 {
         DBuf<float> b, x, r, r0, p, v, s, t, ph, sh;
     } f32;
+    DBuf<double> b, x;    // right-hand side and solution, 5 per cell in device order
+    DBuf<double> bs, xs;  // the same in the sliced layout
+    DBuf<double> stage;   // 5 per cell in mesh order: vectors crossing the ABI
     DBuf<double> partial, dots;
     double* h_dots = nullptr;  // pinned
     DBuf<double> ks;           // device-driven BiCGSTAB state block (kernels_linalg.hpp)
@@ -246,9 +262,29 @@ struct cfdg_ctx {
         a.row_ptr = row_ptr.get();
         a.cols = cols.get();
         a.diag = diag.get();
-        a.cf_blk = cf_blk.get();
         return a;
     }
+    cfdg::SellArgs sellargs() const {
+        cfdg::SellArgs a{};
+        a.n = nc;
+        a.nslices = static_cast<int>(sell.slices.size());
+        a.slice = sell_slice.get();
+        a.row = sell_row.get();
+        a.pos = sell_pos.get();
+        a.count = sell_count.get();
+        a.cols = sell_cols.get();
+        a.tile_pos = sell_tile_pos.get();
+        a.visit = sell_visit.get();
+        a.visit_base = sell_visit_base.get();
+        return a;
+    }
+    cfdg::SellMatrix sellmatrix() const {
+        return {sell_off.get(), sell_diag.get(), storage, lu.get(), sell_piv.get()};
+    }
+    int n_slices() const { return static_cast<int>(sell.slices.size()); }
+    // elements of a Krylov vector in the sliced layout
+    long long sliced_size() const { return cfdg::sell_vector_size(n_slices()); }
+    std::size_t vector_alloc() const { return z(std::max(sliced_size(), 5LL * nc)); }
     void sync() { hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize"); }
     void check_launch() { hip_check(hipGetLastError(), "kernel launch"); }
     template <typename T>

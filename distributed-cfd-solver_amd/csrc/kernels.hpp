@@ -182,15 +182,47 @@ struct BcTable {
     BcDev bc[kMaxPatches];
 };
 
+// Block matrix in row-major device-row order (CSR): the layout of the
+// sequential SGS order and of the solve without preconditioner.
 struct BsrArgs {
     int n;
     const int* row_ptr;
     const int* cols;
     const int* diag;
-    // per entry of the cell -> face lists (MeshArgs::cf_off order): the block
-    // (row = the cell, column = the face's other cell) of an interior face, -1
-    // at a boundary face
-    const int* cf_blk;
+};
+
+// Block matrix in sliced colour order (setup.hpp, SellPlan): the layout the
+// Jacobian writes and the multicolour sweeps read.  Entry e of the block in
+// (slot, lane) is element (slot * 25 + e) * 64 + lane (SellLayout), so the 64
+// lanes of a wave, each on a row of its own, read and write whole cache
+// lines.  Vectors of this layout hold component v of the row at (slice, lane)
+// at (slice * 5 + v) * 64 + lane, zero past a slice's rows.
+constexpr int kSellRows = 64;
+struct SellArgs {
+    int n;                    // rows
+    int nslices;
+    const int4* slice;        // first slot, lower slots, upper slots, rows
+    const int* row;           // position -> device row, -1 past a slice's rows
+    const int* pos;           // device row -> position
+    const std::uint32_t* count;  // per position: lower blocks | upper blocks << 16
+    const int* cols;          // per (slot, lane): position of the column
+    const int* tile_pos;      // the Jacobian's rows and visits (SellPlan)
+    const std::uint32_t* visit;
+    const int* visit_base;
+};
+constexpr unsigned kSellVisitNone = 0xffffffffu, kSellVisitNeighbour = 0x8000u;
+
+// Words per block of the sliced layout: one per entry, and for bfloat16 two
+// entries per 4-byte word (entry 2 q in the low half of word q).
+template <class TS>
+struct SellLayout {
+    typedef TS word;
+    static constexpr int words = 25;
+};
+template <>
+struct SellLayout<bf16> {
+    typedef std::uint32_t word;
+    static constexpr int words = 13;
 };
 
 // Bijective block -> work-item map that gives each XCD one contiguous range of
@@ -230,9 +262,10 @@ void launch_explicit_update(const MeshArgs& m, const FieldArgs& f, const double*
 // dual time stepping: R += V (c0 U + c1 U^n [+ c2 U^{n-1}]), bdf = 1 or 2
 void launch_unsteady_source(const MeshArgs& m, const FieldArgs& f, int bdf, double inv_dt, const double* Un,
                             const double* Unm1, hipStream_t s);
-// values: nnzb x 25 entries of the storage type (kStoreF64 / kStoreF32 / kStoreBF16)
-void launch_jacobian(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const BsrArgs& b,
-                     const double* alpha, void* values, int storage, hipStream_t s);
+// off / diag: the off-diagonal and the diagonal blocks of the sliced layout in
+// the storage type (kStoreF64 / kStoreF32 / kStoreBF16)
+void launch_jacobian(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const SellArgs& b,
+                     const double* alpha, void* off, void* diag, int storage, hipStream_t s);
 
 // --- Spalart-Allmaras module (kernels_sa.hip) --------------------------------
 void launch_sa_prepare(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const SaArgs& sa, hipStream_t s);

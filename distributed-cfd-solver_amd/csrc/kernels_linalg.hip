@@ -1,4 +1,7 @@
-// Block-sparse (5x5 BSR) linear-algebra kernels for the implicit step (gfx950).
+// Block-sparse (5x5 BSR) linear-algebra kernels for the implicit step (gfx950):
+// the vector operations and reductions of every solve, and the matrix kernels
+// on row-major blocks that the sequential SGS order and the solve without
+// preconditioner use (the multicolour order has its own, kernels_sell.hip).
 //
 //   k_lu_factor   diagonal-block LU with partial pivoting (bsr_helpers.hpp:278-321)
 //   k_spmv        y = A x, five lanes per block row (bsr_helpers.hpp:139-203)
@@ -23,6 +26,7 @@
 #include <stdexcept>
 
 #include "kernels.hpp"
+#include "kernels_krylov.hpp"
 #include "kernels_linalg.hpp"
 
 // Scratch of the allocation-free residual norms (residual_norms_noalloc):
@@ -287,28 +291,6 @@ __global__ void __launch_bounds__(kBlock) k_update_xr(long long n, double alpha,
 // iterations enqueued after convergence or breakdown change nothing and the
 // result is the one the per-iteration host loop of bicgstab.cpp:42-201 gives.
 
-// Start of an iteration (bicgstab.cpp:97-109): iteration limit, it += 1,
-// beta = (rho / rho_old)(alpha / omega) from the second iteration on.  Run
-// at the end of the step before it (the start of the solve, or the end of the
-// previous iteration), since nothing in between reads or writes the state.
-__device__ void bicg_begin(double* ks) {
-    if (ks[kKsIt] >= ks[kKsMaxIt]) {
-        ks[kKsStatus] = kKsMaxIter;
-        return;
-    }
-    ks[kKsIt] += 1.0;
-    ks[kKsFirst] = (ks[kKsIt] == 1.0) ? 1.0 : 0.0;
-    if (ks[kKsFirst] == 0.0) {
-        const double beta = (ks[kKsRho] / ks[kKsRhoOld]) * (ks[kKsAlpha] / ks[kKsOmega]);
-        if (!isfinite(beta)) {
-            ks[kKsStatus] = kKsDiverged;
-            return;
-        }
-        ks[kKsBeta] = beta;
-        ks[kKsNbo] = -beta * ks[kKsOmega];
-    }
-}
-
 // Start of a solve (bicgstab.cpp:56-92): norms, tolerance, initial status,
 // then the start of the first iteration.
 __global__ void k_bicg_init(double* ks, const double* dots, int x_zero, int fallback, double abs_tol,
@@ -375,73 +357,9 @@ __device__ void bicg_omega(double* ks, const double* dots) {
     ks[kKsRhoNew] = r0s - omega_new * r0t;
 }
 
-// After x and r are updated (bicgstab.cpp:160-195): breakdown checks, the
-// true residual norm when rr is given (every 32nd iteration), convergence;
-// then the start of the next iteration.
-__device__ void bicg_post(double* ks, const double* rr) {
-    double rnorm = ks[kKsRnNew];
-    const double omega_new = ks[kKsOmegaNew];
-    ks[kKsRnorm] = rnorm;
-    if (!isfinite(rnorm) || !isfinite(omega_new) || omega_new == 0.0) {
-        ks[kKsStatus] = kKsDiverged;
-        return;
-    }
-    if (rr) rnorm = sqrt(rr[0]);
-    ks[kKsRnorm] = rnorm;
-    if (rnorm <= ks[kKsTol]) {
-        ks[kKsStatus] = kKsConverged;
-        return;
-    }
-    const double rho_new = ks[kKsRhoNew];
-    if (!isfinite(rho_new) || rho_new == 0.0) {
-        ks[kKsStatus] = kKsDiverged;
-        return;
-    }
-    ks[kKsRhoOld] = ks[kKsRho];
-    ks[kKsRho] = rho_new;
-    ks[kKsOmega] = omega_new;
-    bicg_begin(ks);
-}
-
 __global__ void k_bicg_post(double* ks) {
     if (ks[kKsStatus] != 0.0) return;
     bicg_post(ks, nullptr);
-}
-
-// p = r on the first iteration, else p = ((p beta) + (-beta omega) v) + r
-template <class T>
-__device__ __forceinline__ T p_entry_of(double first, double beta, double nbo, T ri, const T* v, const T* p,
-                                        long long i) {
-    if (first != 0.0) return ri;
-    T t = p[i] * static_cast<T>(beta);
-    t += static_cast<T>(nbo) * v[i];
-    t += static_cast<T>(1.0) * ri;
-    return t;
-}
-template <class T>
-__device__ __forceinline__ T p_entry(const double* ks, const T* r, const T* v, const T* p, long long i) {
-    return p_entry_of(ks[kKsFirst], ks[kKsBeta], ks[kKsNbo], r[i], v, p, i);
-}
-
-// x = (x + alpha ph) + omega sh, written; returns r = s + (-omega) t
-// (bicgstab.cpp:145-149)
-template <class T>
-__device__ __forceinline__ T xr_entry(const double* ks, const T* ph, const T* sh, const T* sv, const T* t, T* x,
-                                      long long i) {
-    const double alpha = ks[kKsAlpha], omega = ks[kKsOmegaNew];
-    T xv = x[i];
-    xv += static_cast<T>(alpha) * ph[i];
-    xv += static_cast<T>(omega) * sh[i];
-    x[i] = xv;
-    T rv = sv[i];
-    rv += static_cast<T>(-omega) * t[i];
-    return rv;
-}
-
-// s = r + (-alpha) v
-template <class T>
-__device__ __forceinline__ T s_entry(const double* ks, const T* r, const T* v, long long i) {
-    return r[i] + static_cast<T>(-ks[kKsAlpha]) * v[i];
 }
 
 template <class T>
@@ -514,24 +432,7 @@ __global__ void __launch_bounds__(kBlock) k_xr_next(int nrows, const double* ks_
                                                     const TV* v, TV* p, const std::uint8_t* first, const TL* lu,
                                                     const std::uint8_t* piv) {
     __shared__ double next[4];  // status, first, beta, nbo of the next iteration
-    const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
-    if (ks_in[kKsStatus] != 0.0) {  // ended before: carry the state over
-        if (lead)
-            for (int k = 0; k < kKsCount; ++k) ks_out[k] = ks_in[k];
-        return;
-    }
-    if (threadIdx.x == 0) {
-        double st[kKsCount];
-        for (int k = 0; k < kKsCount; ++k) st[k] = ks_in[k];
-        bicg_post(st, nullptr);
-        next[0] = st[kKsStatus];
-        next[1] = st[kKsFirst];
-        next[2] = st[kKsBeta];
-        next[3] = st[kKsNbo];
-        if (lead)
-            for (int k = 0; k < kKsCount; ++k) ks_out[k] = st[k];
-    }
-    __syncthreads();
+    if (!next_iteration(ks_in, ks_out, next)) return;
     const int lane = static_cast<int>(threadIdx.x & 63);
     const int rw = lane / 5;
     const int ii = lane - rw * 5;

@@ -941,72 +941,23 @@ __global__ void __launch_bounds__(kBlock) k_unsteady_source(int nc, const double
     }
 }
 
-// Store one 5x5 block (values v, sign +1 or -1 applied as 0.0 + v / 0.0 - v,
-// or as is) in the storage layout; bfloat16 rows go out as three 4-byte words.
+// Stores one 5x5 block (values v, sign +1 or -1 applied as 0.0 + v / 0.0 - v,
+// or as is) in the sliced layout: its words at dst, dst + 64, ...; the lanes of a wave
+// write consecutive words.
 template <class TS>
-__device__ __forceinline__ void store_block(TS* dst, const double v[25], int sign) {
-    for (int i = 0; i < 25; ++i) {
-        const double x = sign > 0 ? 0.0 + v[i] : (sign < 0 ? 0.0 - v[i] : v[i]);
-        dst[(i / 5) * BlockLayout<TS>::row + i % 5] = cvt<TS>(x);
-    }
-}
-template <>
-__device__ __forceinline__ void store_block<bf16>(bf16* dst, const double v[25], int sign) {
-    std::uint32_t* w = reinterpret_cast<std::uint32_t*>(dst);
-    for (int a = 0; a < 5; ++a) {
-        std::uint32_t h[6];
-        for (int q = 0; q < 5; ++q) {
-            const double x = sign > 0 ? 0.0 + v[a * 5 + q] : (sign < 0 ? 0.0 - v[a * 5 + q] : v[a * 5 + q]);
-            h[q] = cvt<bf16>(x).u;
+__device__ __forceinline__ void store_sell_block(typename SellLayout<TS>::word* dst, const double v[25], int sign) {
+    const auto signed_value = [&](int k) { return sign > 0 ? 0.0 + v[k] : (sign < 0 ? 0.0 - v[k] : v[k]); };
+    if constexpr (sizeof(TS) == sizeof(bf16)) {
+#pragma unroll
+        for (int q = 0; q < SellLayout<TS>::words; ++q) {
+            const std::uint32_t lo = cvt<bf16>(signed_value(2 * q)).u;
+            const std::uint32_t hi = 2 * q + 1 < 25 ? cvt<bf16>(signed_value(2 * q + 1)).u : 0;
+            dst[q * kSellRows] = lo | (hi << 16);
         }
-        h[5] = 0;
-        for (int q = 0; q < 3; ++q) w[a * 3 + q] = h[2 * q] | (h[2 * q + 1] << 16);
+    } else {
+#pragma unroll
+        for (int k = 0; k < 25; ++k) dst[k * kSellRows] = cvt<TS>(signed_value(k));
     }
-}
-
-// Block of the storage type TS as storage words (8 bytes for FP64, 4 for FP32
-// and BF16), the unit of the Jacobian kernel's coalesced block stores.
-template <class TS>
-struct BlockWords {
-    typedef std::uint32_t word;
-    static constexpr int n = BlockLayout<TS>::block * static_cast<int>(sizeof(TS)) / 4;
-};
-template <>
-struct BlockWords<double> {
-    typedef unsigned long long word;
-    static constexpr int n = 25;
-};
-
-// The words of one block as store_block writes it (sign: +1 -> 0 + v,
-// -1 -> 0 - v, 0 -> v); a BF16 block's padding word is zero.
-template <class TS>
-__device__ __forceinline__ void block_words(const double v[25], int sign, typename BlockWords<TS>::word* w);
-template <>
-__device__ __forceinline__ void block_words<double>(const double v[25], int sign, unsigned long long* w) {
-    for (int k = 0; k < 25; ++k) {
-        const double x = sign > 0 ? 0.0 + v[k] : (sign < 0 ? 0.0 - v[k] : v[k]);
-        w[k] = static_cast<unsigned long long>(__double_as_longlong(x));
-    }
-}
-template <>
-__device__ __forceinline__ void block_words<float>(const double v[25], int sign, std::uint32_t* w) {
-    for (int k = 0; k < 25; ++k) {
-        const double x = sign > 0 ? 0.0 + v[k] : (sign < 0 ? 0.0 - v[k] : v[k]);
-        w[k] = f32_bits(cvt<float>(x));
-    }
-}
-template <>
-__device__ __forceinline__ void block_words<bf16>(const double v[25], int sign, std::uint32_t* w) {
-    for (int a = 0; a < 5; ++a) {
-        std::uint32_t h[6];
-        for (int q = 0; q < 5; ++q) {
-            const double x = sign > 0 ? 0.0 + v[a * 5 + q] : (sign < 0 ? 0.0 - v[a * 5 + q] : v[a * 5 + q]);
-            h[q] = cvt<bf16>(x).u;
-        }
-        h[5] = 0;
-        for (int q = 0; q < 3; ++q) w[a * 3 + q] = h[2 * q] | (h[2 * q + 1] << 16);
-    }
-    w[15] = 0;
 }
 
 // J += Jv (plus) or J -= Jv for the dense viscous block Jv of
@@ -1115,95 +1066,66 @@ __device__ __forceinline__ bool jacobian_face(const MeshArgs& m, const FieldArgs
 // loads; each of a row's faces is read from the tile face-list stream (normal,
 // area, centroid, packed cell ids: contiguous per tile), so only the halo or
 // ghost side of a face on the tile boundary is gathered from the cell planes.
-// Row c forms, per face in ascending face index, the face's dF of its own
-// side (added to the diagonal: + dFL as owner, - dFR as neighbour) and, at an
-// interior face, the other side's dF, the off-diagonal block at the position
-// precomputed at set-up (cf_blk): + dFR as owner, - dFL as neighbour.
-// The rows advance through their faces in lock step (round r = each row's
-// r-th face, then a last round for the diagonal blocks); each round's blocks
-// go through LDS, and each wave stores its 64 blocks word by word with
-// consecutive lanes on consecutive words, so a store instruction writes a few
-// contiguous runs instead of 64 scattered words.
-// The arithmetic and its order are those of the reference's face loop, so the
+// Row c forms, per face, the face's dF of its own side (added to the diagonal:
+// + dFL as owner, - dFR as neighbour) and, at an interior face, the other
+// side's dF, the off-diagonal block: + dFR as owner, - dFL as neighbour.
+// The threads take the tile's rows in the order of the sliced matrix layout,
+// so in a round (each row's r-th face in ascending face index) a wave's 64
+// blocks lie on consecutive lanes of a slot -- on a hexahedral mesh, where a
+// row's blocks keep the face order -- and every store instruction writes whole
+// cache lines.  (Row-major blocks staged through LDS and stored word by word
+// covered cache lines only partly at first touch and made the L2 fetch them:
+// 2.64 GB read for 0.9 GB of inputs, and the stage's 51 KB of LDS; on the
+// 2.1M-cell plate FP64 1,429 -> 985 us.)  Two waves per SIMD at 178 registers: a third
+// wave at 168 spills ten of them and gains nothing (262,144 cells FP64 138 / 147 us,
+// 524,288 cells 271 / 268, 663,552 tetrahedra with eddy viscosity 301 / 317).  The
+// arithmetic and its order are those of the reference's face loop, so the
 // blocks are the reference's bit for bit; each block has a single writer.
-// Waves per SIMD: three where the LDS leaves room for three workgroups per
-// CU (FP32 blocks without eddy viscosity, BF16 blocks: 52 KB and 45 KB), at
-// 168 registers; two otherwise (FP64 blocks: 78 KB; FP32 with eddy
-// viscosity: 54 KB), where a lower register cap would only add spills.
 template <class TS, bool kTurb>
 __global__ void __launch_bounds__(kTileCells)
-__attribute__((amdgpu_waves_per_eu((sizeof(TS) == 8 || (sizeof(TS) == 4 && kTurb)) ? 2 : 3)))
-k_jacobian(MeshArgs m, FieldArgs f, NumArgs nm, BsrArgs b,
-                                                         const double* alpha, TS* values) {
-    typedef typename BlockWords<TS>::word word;
-    constexpr int kW = BlockWords<TS>::n;
+__attribute__((amdgpu_waves_per_eu(2)))
+k_jacobian(MeshArgs m, FieldArgs f, NumArgs nm, SellArgs b, const double* alpha,
+           typename SellLayout<TS>::word* off, typename SellLayout<TS>::word* diag) {
+    constexpr long long kW = SellLayout<TS>::words;
     __shared__ double sq[8 * kTileCells];  // q (0-4) and centroid (5-7) of the tile's cells, one plane each
     __shared__ double smut[kTurb ? kTileCells : 1];
-    __shared__ int scf[kTileCells + 1 + 2 * kTileFaces];  // the tile's cf_off (rebased), then its cf_slot entries
-    __shared__ word sblk[kTileCells * kW];  // one block per row for the round's store
-    __shared__ int spos[kTileCells];        // its destination block, -1 for none
-    __shared__ int srounds;
     const int t = xcd_block(blockIdx.x, gridDim.x);
     const int c0 = m.tile_off[t], nt = m.tile_off[t + 1] - c0;
     const int fb = m.tile_face_off[t];
-    const int i = threadIdx.x;
-    const int e0 = m.cf_off[c0];
-    if (i == 0) srounds = 0;
-    if (i < nt) {
+    const int th = threadIdx.x;
+    if (th < nt) {
         typedef double pair_t __attribute__((ext_vector_type(2)));
         for (int p = 0; p < 4; ++p) {
-            const pair_t v = *reinterpret_cast<const pair_t*>(f.cs + plane_at(2 * p, f.ld, c0 + i));
-            sq[(2 * p) * kTileCells + i] = v.x;
-            sq[(2 * p + 1) * kTileCells + i] = v.y;
+            const pair_t v = *reinterpret_cast<const pair_t*>(f.cs + plane_at(2 * p, f.ld, c0 + th));
+            sq[(2 * p) * kTileCells + th] = v.x;
+            sq[(2 * p + 1) * kTileCells + th] = v.y;
         }
-        if (kTurb) smut[i] = f.mut[c0 + i];
-    }
-    {
-        // nt + 1 offsets (up to kTileCells + 1, one more than the threads)
-        const int ne = m.cf_off[c0 + nt] - e0;  // at most two entries per tile face
-        for (int k = i; k <= nt; k += kTileCells) scf[k] = m.cf_off[c0 + k] - e0;
-        for (int e = i; e < ne; e += kTileCells) scf[kTileCells + 1 + e] = m.cf_slot[e0 + e];
+        if (kTurb) smut[th] = f.mut[c0 + th];
     }
     __syncthreads();
-    const bool row = i < nt;
-    const int nfc = row ? scf[i + 1] - scf[i] : 0;
-    if (nfc > 0) atomicMax(&srounds, nfc);  // integer maximum: the tile's longest face list
-    const int c = c0 + (row ? i : 0);
+    if (th >= nt) return;
+    const int p = b.tile_pos[c0 + th];
+    const int c = b.row[p], i = c - c0;
+    const int4 sl = b.slice[p / kSellRows];
+    const int lane = p % kSellRows;
+    const int nl = static_cast<int>(b.count[p] & 0xffffu);
+    const int vb = b.visit_base[t], rounds = (b.visit_base[t + 1] - vb) / nt;
     double dg[25];
     for (int k = 0; k < 25; ++k) dg[k] = 0.0;
-    __syncthreads();
-    const int rounds = srounds;
-    const int lane = i & 63, wbase = i & ~63;
-    for (int rr = 0; rr <= rounds; ++rr) {
-        int pos = -1;
-        if (rr < nfc) {
-            const int e = scf[i] + rr;
-            const int sl = scf[kTileCells + 1 + e];
-            const bool own = sl >= 0;
-            double J[25];
-            if (jacobian_face<kTurb>(m, f, nm, sq, smut, i, c0, nt, fb + (own ? sl : -sl - 1), own, dg, J)) {
-                pos = b.cf_blk[e0 + e];
-                block_words<TS>(J, own ? 1 : -1, sblk + i * kW);
-            }
-        } else if (rr == rounds && row) {  // last round: the diagonal block
-            const double a = alpha[c];
-            for (int k = 0; k < 5; ++k) dg[k * 6] += a;
-            pos = b.diag[c];
-            block_words<TS>(dg, 0, sblk + i * kW);
+    for (int rr = 0; rr < rounds; ++rr) {
+        const unsigned v = b.visit[vb + rr * nt + th];
+        if (v == kSellVisitNone) break;  // no face follows
+        const bool own = (v & kSellVisitNeighbour) == 0;
+        double J[25];
+        if (jacobian_face<kTurb>(m, f, nm, sq, smut, i, c0, nt, fb + static_cast<int>(v & 0x7fffu), own, dg, J)) {
+            const int blk = static_cast<int>(v >> 16);
+            const long long slot = blk < nl ? sl.x + blk : sl.x + sl.y + (blk - nl);
+            store_sell_block<TS>(off + slot * kW * kSellRows + lane, J, own ? 1 : -1);
         }
-        spos[i] = pos;
-        __syncthreads();
-        // this wave's 64 blocks, word by word: consecutive lanes on consecutive words
-        word* out = reinterpret_cast<word*>(values);
-#pragma unroll 1
-        for (int q = 0; q < kW; ++q) {
-            const int w = q * 64 + lane;
-            const int blk = w / kW, o = w - blk * kW;
-            const int dst = spos[wbase + blk];
-            if (dst >= 0) out[static_cast<long long>(dst) * kW + o] = sblk[(wbase + blk) * kW + o];
-        }
-        __syncthreads();  // the next round reuses sblk / spos
     }
+    const double a = alpha[c];
+    for (int k = 0; k < 5; ++k) dg[k * 6] += a;
+    store_sell_block<TS>(diag + (p / kSellRows) * kW * kSellRows + lane, dg, 0);
 }
 
 // Per-patch boundary integrals (residual_kernel.hpp:96-169 forms F[0] and
@@ -1323,24 +1245,28 @@ void launch_unsteady_source(const MeshArgs& m, const FieldArgs& f, int bdf, doub
                            Un, Unm1, f.res);
 }
 
-void launch_jacobian(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const BsrArgs& b,
-                     const double* alpha, void* values, int storage, hipStream_t s) {
-    if (m.nc <= 0) return;
+template <class TS>
+static void launch_jacobian_as(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const SellArgs& b,
+                               const double* alpha, void* off, void* diag, hipStream_t s) {
+    typedef typename SellLayout<TS>::word word;
     const dim3 grid(static_cast<unsigned>(m.ntiles)), block(kTileCells);
-    const bool turb = f.mut != nullptr;
-    if (storage == kStoreF32) {
-        float* v = static_cast<float*>(values);
-        if (turb) hipLaunchKernelGGL((k_jacobian<float, true>), grid, block, 0, s, m, f, nm, b, alpha, v);
-        else hipLaunchKernelGGL((k_jacobian<float, false>), grid, block, 0, s, m, f, nm, b, alpha, v);
-    } else if (storage == kStoreBF16) {
-        bf16* v = static_cast<bf16*>(values);
-        if (turb) hipLaunchKernelGGL((k_jacobian<bf16, true>), grid, block, 0, s, m, f, nm, b, alpha, v);
-        else hipLaunchKernelGGL((k_jacobian<bf16, false>), grid, block, 0, s, m, f, nm, b, alpha, v);
-    } else {
-        double* v = static_cast<double*>(values);
-        if (turb) hipLaunchKernelGGL((k_jacobian<double, true>), grid, block, 0, s, m, f, nm, b, alpha, v);
-        else hipLaunchKernelGGL((k_jacobian<double, false>), grid, block, 0, s, m, f, nm, b, alpha, v);
-    }
+    if (f.mut)
+        hipLaunchKernelGGL((k_jacobian<TS, true>), grid, block, 0, s, m, f, nm, b, alpha, static_cast<word*>(off),
+                           static_cast<word*>(diag));
+    else
+        hipLaunchKernelGGL((k_jacobian<TS, false>), grid, block, 0, s, m, f, nm, b, alpha, static_cast<word*>(off),
+                           static_cast<word*>(diag));
+}
+
+void launch_jacobian(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const SellArgs& b,
+                     const double* alpha, void* off, void* diag, int storage, hipStream_t s) {
+    if (m.nc <= 0) return;
+    if (storage == kStoreF32)
+        launch_jacobian_as<float>(m, f, nm, b, alpha, off, diag, s);
+    else if (storage == kStoreBF16)
+        launch_jacobian_as<bf16>(m, f, nm, b, alpha, off, diag, s);
+    else
+        launch_jacobian_as<double>(m, f, nm, b, alpha, off, diag, s);
 }
 
 }  // namespace cfdg

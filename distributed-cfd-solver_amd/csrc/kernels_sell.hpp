@@ -1,0 +1,75 @@
+// Launch wrappers of the multicolour Krylov kernels on the sliced block layout
+// (kernels_sell.hip).  Blocks are passed untyped with their storage kind;
+// vectors (5 values per row at (slice * 5 + v) * 64 + lane, SellArgs) are typed
+// and fix the arithmetic type.
+#pragma once
+
+#include <hip/hip_runtime.h>
+
+#include <cstdint>
+
+#include "kernels.hpp"
+#include "kernels_linalg.hpp"
+
+namespace cfdg {
+
+// One matrix in the sliced layout: off-diagonal blocks, diagonal blocks, and
+// the diagonal LU factors (25 entries of the LU type per row) with their pivots
+// (five 3-bit row numbers per row).
+struct SellMatrix {
+    const void* off = nullptr;
+    const void* diag = nullptr;
+    int storage = kStoreF64;
+    const void* lu = nullptr;
+    const std::uint16_t* piv = nullptr;
+};
+
+// Elements of a vector of the layout.
+inline long long sell_vector_size(int nslices) { return 5LL * kSellRows * nslices; }
+// Bytes of one slot of blocks (64 blocks) in a storage type.
+inline std::size_t sell_slot_bytes(int storage) {
+    return storage == kStoreF64 ? 64 * 25 * 8 : (storage == kStoreF32 ? 64 * 25 * 4 : 64 * 13 * 4);
+}
+
+// LU factors with partial pivoting of the stored diagonal blocks, factorised in
+// FP64 and kept in FP64 (lu_f32 = 0, FP64 blocks only) or FP32; singular takes
+// the largest device row + 1 with a zero pivot.
+void launch_sell_lu(const SellArgs& b, const SellMatrix& m, void* lu, int lu_f32, std::uint16_t* piv, int* singular,
+                    hipStream_t s);
+// y = A x.  TV = float needs FP32 vectors, any storage; TV = double any storage.
+template <class TV>
+void launch_sell_spmv(const SellArgs& b, const SellMatrix& m, const TV* x, TV* y, hipStream_t s,
+                      const double* gate = nullptr);
+// One sweep step over the slices [first, first + count) of a colour:
+// z_i = D_i^-1 (r_i - sum A_ij z_j) over the row's lower blocks, or with all
+// set over all its off-diagonal blocks.
+template <class TV>
+void launch_sell_sweep(const SellArgs& b, const SellMatrix& m, int first, int count, bool all, const TV* r, TV* z,
+                       hipStream_t s, const double* gate = nullptr);
+// The Krylov vector updates of launch_vec_sgs_first / launch_xr_next
+// (kernels_linalg.hpp) with the rows of the first colour, slices [0, first),
+// solved in the same launch.
+template <class TV>
+void launch_sell_vec_first(int op, const SellArgs& b, const SellMatrix& m, int first, const double* ks, const TV* r,
+                           const TV* v, TV* y, TV* z, hipStream_t s);
+template <class TV>
+void launch_sell_xr_next(const SellArgs& b, const SellMatrix& m, int first, const double* ks_in, double* ks_out,
+                         TV* ph, const TV* sh, const TV* sv, const TV* t, TV* x, TV* r, const TV* v, TV* p,
+                         hipStream_t s);
+// dst (sliced) = src (5 values per cell, cell src_of[device row], or the device
+// row itself when src_of is null), and back.
+void launch_sell_gather(const SellArgs& b, const int* src_of, const double* src, double* dst, hipStream_t s);
+void launch_sell_scatter(const SellArgs& b, const int* dst_of, const double* src, double* dst, hipStream_t s);
+// b = -R in the sliced layout; U += du with du in the sliced layout, du also
+// written per cell (5 values, device order).
+void launch_sell_rhs(const SellArgs& b, int ld, const double* res, double* rhs, hipStream_t s);
+void launch_sell_state_update(const SellArgs& b, int ld, const double* du, double* U, double* du_cells, hipStream_t s);
+// Row-major 25-entry blocks k0 .. k0 + n of a list of block codes (setup.hpp,
+// sell_block_codes) from and to the sliced layout; to_csr keeps the storage
+// type (block layout of precision.hpp).
+void launch_sell_get_blocks(const int* code, long long n, const SellMatrix& m, double* out, hipStream_t s);
+void launch_sell_set_blocks(const int* code, long long n, const double* in, void* off, void* diag, int storage,
+                            hipStream_t s);
+void launch_sell_to_csr(const int* code, long long n, const SellMatrix& m, void* values, hipStream_t s);
+
+}  // namespace cfdg

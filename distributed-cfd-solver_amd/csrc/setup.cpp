@@ -570,6 +570,152 @@ std::vector<i32> split_tiles(const std::vector<i32>& tile_off, const Csr& dev_cc
     return out;
 }
 
+SellPlan sell_plan(const Tiling& t, const std::vector<i32>& colour_mesh, i32 n_colours, const Csr& dev_cf,
+                   const TileFaces& tf, const std::vector<i32>& face_owner_dev, const std::vector<i32>& face_other_dev,
+                   i32 n_inner_faces) {
+    SellPlan p;
+    const i32 n = static_cast<i32>(t.new2old.size());
+    const std::size_t ntiles = t.tile_off.size() - 1;
+    const std::size_t nc = z(n_colours);
+    std::vector<i32> colour(z(n)), lower(z(n)), blocks(z(n));
+    std::vector<std::uint32_t> mask(z(n));  // bit k: the row's k-th block in face order is lower (first 32)
+    const auto other = [&](i32 f, i32 r) { return face_owner_dev[z(f)] == r ? face_other_dev[z(f)] : face_owner_dev[z(f)]; };
+    parallel_for(z(n), [&](std::size_t r, int) { colour[r] = colour_mesh[z(t.new2old[r])]; }, 4096);
+    // rows of each (colour, tile), and the tile's rows sorted by (colour, lower, row)
+    std::vector<i32> first(nc * ntiles + 1, 0);
+    p.tile_pos.resize(z(n));
+    parallel_for(ntiles, [&](std::size_t k, int) {
+        for (i32 r = t.tile_off[k]; r < t.tile_off[k + 1]; ++r) {
+            i32 lo = 0, nb = 0;
+            std::uint32_t mk = 0;
+            for (i32 e = dev_cf.off[z(r)]; e < dev_cf.off[z(r) + 1]; ++e) {
+                const i32 f = dev_cf.idx[z(e)];
+                if (f >= n_inner_faces) continue;
+                const bool low = colour[z(other(f, r))] < colour[z(r)];
+                if (low && nb < 32) mk |= 1u << nb;
+                ++nb;
+                lo += low;
+            }
+            mask[z(r)] = mk;
+            lower[z(r)] = lo;
+            blocks[z(r)] = nb;
+            p.tile_pos[z(r)] = r;
+        }
+        std::sort(p.tile_pos.begin() + t.tile_off[k], p.tile_pos.begin() + t.tile_off[k + 1], [&](i32 a, i32 b) {
+            if (colour[z(a)] != colour[z(b)]) return colour[z(a)] < colour[z(b)];
+            if (lower[z(a)] != lower[z(b)]) return lower[z(a)] < lower[z(b)];
+            if (mask[z(a)] != mask[z(b)]) return mask[z(a)] < mask[z(b)];
+            return a < b;
+        });
+        for (i32 r = t.tile_off[k]; r < t.tile_off[k + 1]; ++r) ++first[z(colour[z(r)]) * ntiles + k];
+    }, 16);
+    // first position of each (colour, tile); a colour starts a new slice
+    p.colour_slice.assign(nc + 1, 0);
+    i32 at = 0;
+    for (std::size_t c = 0; c < nc; ++c) {
+        p.colour_slice[c] = at / kSliceRows;
+        for (std::size_t k = 0; k < ntiles; ++k) {
+            const i32 m = first[c * ntiles + k];
+            first[c * ntiles + k] = at;
+            at += m;
+        }
+        at = (at + kSliceRows - 1) / kSliceRows * kSliceRows;
+    }
+    const std::size_t ns = z(at / kSliceRows);
+    p.colour_slice[nc] = static_cast<i32>(ns);
+    p.row.assign(z(at), -1);
+    p.pos.resize(z(n));
+    p.count.assign(z(at), 0);
+    parallel_for(ntiles, [&](std::size_t k, int) {
+        i32 c = -1, q = 0;
+        for (i32 i = t.tile_off[k]; i < t.tile_off[k + 1]; ++i) {
+            const i32 r = p.tile_pos[z(i)];
+            if (colour[z(r)] != c) {
+                c = colour[z(r)];
+                q = first[z(c) * ntiles + k];
+            }
+            p.row[z(q)] = r;
+            p.pos[z(r)] = q;
+            p.count[z(q)] = static_cast<std::uint32_t>(lower[z(r)] | ((blocks[z(r)] - lower[z(r)]) << 16));
+            p.tile_pos[z(i)] = q++;
+        }
+    }, 16);
+    p.slices.resize(ns);
+    parallel_for(ns, [&](std::size_t s, int) {
+        Slice& sl = p.slices[s];
+        sl = Slice{0, 0, 0, 0};
+        for (std::size_t l = 0; l < static_cast<std::size_t>(kSliceRows); ++l) {
+            const std::size_t q = s * static_cast<std::size_t>(kSliceRows) + l;
+            if (p.row[q] < 0) break;
+            sl.lower = std::max(sl.lower, static_cast<i32>(p.count[q] & 0xffffu));
+            sl.upper = std::max(sl.upper, static_cast<i32>(p.count[q] >> 16));
+            ++sl.rows;
+        }
+    }, 256);
+    for (Slice& s : p.slices) {
+        if (p.n_slots > INT32_MAX / kSliceRows - 512) throw std::runtime_error("the block matrix is too large");
+        s.base = p.n_slots;
+        p.n_slots += s.lower + s.upper;
+    }
+    p.cols.assign(z(p.n_slots) * static_cast<std::size_t>(kSliceRows), 0);
+    // block columns and the Jacobian's visits
+    p.visit_base.assign(ntiles + 1, 0);
+    for (std::size_t k = 0; k < ntiles; ++k) {
+        i32 w = 0;
+        for (i32 r = t.tile_off[k]; r < t.tile_off[k + 1]; ++r) w = std::max(w, dev_cf.off[z(r) + 1] - dev_cf.off[z(r)]);
+        p.visit_base[k + 1] = p.visit_base[k] + w * (t.tile_off[k + 1] - t.tile_off[k]);
+    }
+    p.visit.assign(z(p.visit_base.back()), kVisitNone);
+    parallel_for(ntiles, [&](std::size_t k, int) {
+        const i32 c0 = t.tile_off[k], nt = t.tile_off[k + 1] - c0;
+        for (i32 i = 0; i < nt; ++i) {
+            const i32 q = p.tile_pos[z(c0 + i)], r = p.row[z(q)];
+            const Slice& sl = p.slices[z(q / kSliceRows)];
+            const i32 lane = q % kSliceRows, nl = lower[z(r)];
+            i32 kl = 0, ku = 0, j = 0;
+            for (i32 e = dev_cf.off[z(r)]; e < dev_cf.off[z(r) + 1]; ++e) {
+                const i32 f = dev_cf.idx[z(e)], s = tf.cell_slot[z(e)];
+                std::uint32_t v = static_cast<std::uint32_t>(s >= 0 ? s : -s - 1) | (s >= 0 ? 0 : kVisitNeighbour);
+                if (f < n_inner_faces) {
+                    const bool low = colour[z(other(f, r))] < colour[z(r)];
+                    const i32 blk = low ? kl++ : nl + ku++;
+                    const i32 slot = low ? sl.base + blk : sl.base + sl.lower + (blk - nl);
+                    v |= static_cast<std::uint32_t>(blk) << 16;
+                    p.cols[z(slot) * static_cast<std::size_t>(kSliceRows) + z(lane)] = p.pos[z(other(f, r))];
+                }
+                p.visit[z(p.visit_base[k] + j++ * nt + i)] = v;
+            }
+        }
+    }, 16);
+    return p;
+}
+
+std::vector<i32> sell_block_codes(const SellPlan& p, const std::vector<i32>& row_ptr, const std::vector<i32>& cols,
+                                  const std::vector<i32>& old2new) {
+    std::vector<i32> code(cols.size());
+    std::atomic<bool> missing{false};
+    parallel_for(old2new.size(), [&](std::size_t o, int) {
+        const i32 q = p.pos[z(old2new[o])];
+        const Slice& sl = p.slices[z(q / kSliceRows)];
+        const i32 lane = q % kSliceRows;
+        const i32 nl = static_cast<i32>(p.count[z(q)] & 0xffffu), nu = static_cast<i32>(p.count[z(q)] >> 16);
+        for (i32 k = row_ptr[o]; k < row_ptr[o + 1]; ++k) {
+            const i32 c = p.pos[z(old2new[z(cols[z(k)])])];
+            i32 found = -1 - q;
+            if (c != q) {
+                for (i32 b = 0; b < nl + nu; ++b) {
+                    const i32 slot = b < nl ? sl.base + b : sl.base + sl.lower + (b - nl);
+                    if (p.cols[z(slot) * static_cast<std::size_t>(kSliceRows) + z(lane)] == c) found = slot * kSliceRows + lane;
+                }
+                if (found < 0) missing = true;
+            }
+            code[z(k)] = found;
+        }
+    }, 1024);
+    if (missing) throw std::runtime_error("a block of the pattern is missing from the matrix");
+    return code;
+}
+
 std::vector<i32> backward_levels(const Csr& ccf, i32 n, i32& n_levels) {
     std::vector<i32> lev(z(n), 0);
     n_levels = (n > 0) ? 1 : 0;

@@ -143,6 +143,51 @@ TileStencil tile_stencil(const std::vector<std::int32_t>& tile_off, const Csr& d
 // The largest slot count (cells + stencil halo) of any tile, without the slot lists.
 std::int32_t tile_max_slots(const std::vector<std::int32_t>& tile_off, const Csr& dev_ccn, const Csr& dev_ccf);
 
+// Storage order of the block matrix for the multicolour sweeps.  Rows are
+// sorted by colour (each colour starting a new slice), inside a colour by tile
+// and then by the number of blocks whose column has an earlier colour
+// ("lower" blocks), and cut into slices of kSliceRows rows, one per lane of a
+// wave: position p = slice * kSliceRows + lane.  The off-diagonal blocks of a
+// slice are stored slot by slot, first its lower slots, then its upper ones;
+// a row's lower blocks fill the first lower slots in ascending face order, its
+// upper blocks the first upper slots.  The diagonal blocks are kept apart.
+constexpr int kSliceRows = 64;
+struct Slice {
+    std::int32_t base;   // first slot
+    std::int32_t lower;  // lower slots
+    std::int32_t upper;  // upper slots
+    std::int32_t rows;   // rows in the slice (the first lanes)
+};
+struct SellPlan {
+    std::vector<Slice> slices;
+    std::vector<std::int32_t> colour_slice;  // colours + 1: first slice of each colour
+    std::vector<std::int32_t> row;           // position -> device row, -1 past a slice's rows
+    std::vector<std::int32_t> pos;           // device row -> position
+    std::vector<std::uint32_t> count;        // per position: lower blocks | upper blocks << 16
+    std::vector<std::int32_t> cols;          // slot * kSliceRows + lane -> position of the block's column
+    std::int32_t n_slots = 0;
+    // the Jacobian's visits, per flux tile: the tile's i-th row in position
+    // order is tile_pos[tile_off[t] + i]; its j-th visited face is
+    // visit[visit_base[t] + j nt + i] (nt = rows of the tile), faces in
+    // ascending index: the face's index in the tile's face list (low 15 bits),
+    // kVisitNeighbour when the row is the face's neighbour, and in the high
+    // half, for an interior face, which of the row's blocks is its (lower
+    // blocks first); kVisitNone past the row's faces.
+    std::vector<std::int32_t> tile_pos;
+    std::vector<std::uint32_t> visit;
+    std::vector<std::int32_t> visit_base;  // tiles + 1
+};
+constexpr std::uint32_t kVisitNone = 0xffffffffu, kVisitNeighbour = 0x8000u;
+SellPlan sell_plan(const Tiling& t, const std::vector<std::int32_t>& colour_mesh, std::int32_t n_colours,
+                   const Csr& dev_cf, const TileFaces& tf, const std::vector<std::int32_t>& face_owner_dev,
+                   const std::vector<std::int32_t>& face_other_dev, std::int32_t n_inner_faces);
+// Where the block of every entry of a BSR pattern in mesh order is stored:
+// slot * kSliceRows + lane of an off-diagonal block, -1 - position of a
+// diagonal block.
+std::vector<std::int32_t> sell_block_codes(const SellPlan& p, const std::vector<std::int32_t>& row_ptr,
+                                           const std::vector<std::int32_t>& cols,
+                                           const std::vector<std::int32_t>& old2new);
+
 // Splits each tile (a range of device cells) into consecutive sub-ranges whose
 // cells plus stencil halo take at most max_slots LDS slots, for meshes whose
 // full tiles do not fit (tetrahedra: about 70 vertex neighbours per cell).
