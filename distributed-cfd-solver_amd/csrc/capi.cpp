@@ -3,7 +3,10 @@
 // stream.  Every entry point catches exceptions and returns a status code.
 //
 // Internally cells live in the device (tile) order of setup.hpp; every array
-// crossing the ABI is in mesh order and is permuted here, on the host.
+// crossing the ABI is in mesh order.  States, block values and the multicolour
+// solve's vectors are permuted on the device from and to a staging buffer (2.1M
+// cells: set_state and get_state 2.8 ms each, where a permutation on the host and
+// a pageable copy took about 40 ms each); the rest is permuted here, on the host.
 #include "cfdg.h"
 
 #include <hip/hip_runtime.h>
@@ -663,18 +666,27 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
 
 // Mesh-order vectors of the ABI (5 per cell) into the sliced layout and back.
 void upload_sliced(cfdg_ctx& c, const double* h, double* dst) {
-    const std::size_t n5 = 5ULL * z(c.nc);
-    if (c.stage.size() != n5) c.stage.alloc(n5);
-    c.h2d(c.stage.get(), h, n5);
+    c.pipe.to_device(c.stage.get(), h, c.stage.size() * sizeof(double), c.stream);
     cfdg::launch_sell_gather(c.sellargs(), c.mesh_of_row.get(), c.stage.get(), dst, c.stream);
     c.sync();
 }
 void download_sliced(cfdg_ctx& c, const double* src, double* h) {
-    const std::size_t n5 = 5ULL * z(c.nc);
-    if (c.stage.size() != n5) c.stage.alloc(n5);
     cfdg::launch_sell_scatter(c.sellargs(), c.mesh_of_row.get(), src, c.stage.get(), c.stream);
-    c.d2h(h, c.stage.get(), n5);
-    c.sync();
+    c.check_launch();
+    c.pipe.to_host(h, c.stage.get(), c.stage.size() * sizeof(double), c.stream);
+}
+
+// copy(plane of the staging buffer, offset of the caller's plane, bytes) over the
+// five planes of a caller's state with leading dimension ld: one copy where they
+// are contiguous.
+template <class F>
+void state_planes(cfdg_ctx& c, std::int64_t ld, F&& copy) {
+    const std::size_t n = z(c.nc);
+    if (ld == c.nc) {
+        copy(c.stage.get(), 0, 5 * n * sizeof(double));
+        return;
+    }
+    for (int v = 0; v < 5; ++v) copy(c.stage.get() + z(v) * n, v * ld, n * sizeof(double));
 }
 
 // The solution stays in c.xs (multicolour SGS) or c.x; returns which Krylov
@@ -1017,6 +1029,8 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
     }
     const std::size_t ncs = z(c.nc);
     c.U.alloc(5 * ncs);
+    c.stage.alloc(5 * ncs);
+    c.pipe.reserve(5 * ncs * sizeof(double));
     c.res.alloc(5 * ncs);
     c.lam.alloc(ncs);
     c.bflux.alloc(5 * static_cast<std::size_t>(std::max(c.nbf, 1)));
@@ -1163,10 +1177,11 @@ int cfdg_sizes(const cfdg_ctx* ctx, int32_t* n_cells, int32_t* n_total, int64_t*
 int cfdg_set_state(cfdg_ctx* c, const double* U, int64_t ld) {
     return guarded(c, [&] {
         if (!U || ld < c->nc) throw CfdgError(CFDG_ERR_ARG, "set_state: bad array");
-        std::vector<double> h(5 * z(c->nc));
-        for (int v = 0; v < 5; ++v)
-            for (int r = 0; r < c->nc; ++r) h[z(v) * z(c->nc) + z(r)] = U[v * ld + c->new2old[z(r)]];
-        c->h2d(c->U.get(), h.data(), h.size());
+        state_planes(*c, ld, [&](double* dev, std::ptrdiff_t at, std::size_t bytes) {
+            c->pipe.to_device(dev, U + at, bytes, c->stream);
+        });
+        cfdg::launch_planes_to_device(c->nc, c->mesh_of_row.get(), c->stage.get(), c->U.get(), c->stream);
+        c->check_launch();
         c->sync();
         c->have_residual = false;
         c->have_dt = false;
@@ -1177,11 +1192,11 @@ int cfdg_set_state(cfdg_ctx* c, const double* U, int64_t ld) {
 int cfdg_get_state(cfdg_ctx* c, double* U, int64_t ld) {
     return guarded(c, [&] {
         if (!U || ld < c->nc) throw CfdgError(CFDG_ERR_ARG, "get_state: bad array");
-        std::vector<double> h(5 * z(c->nc));
-        c->d2h(h.data(), c->U.get(), h.size());
-        c->sync();
-        for (int v = 0; v < 5; ++v)
-            for (int r = 0; r < c->nc; ++r) U[v * ld + c->new2old[z(r)]] = h[z(v) * z(c->nc) + z(r)];
+        cfdg::launch_planes_to_mesh(c->nc, c->mesh_of_row.get(), c->U.get(), c->stage.get(), c->stream);
+        c->check_launch();
+        state_planes(*c, ld, [&](double* dev, std::ptrdiff_t at, std::size_t bytes) {
+            c->pipe.to_host(U + at, dev, bytes, c->stream);
+        });
     });
 }
 

@@ -15,6 +15,7 @@
 #include "kernels.hpp"
 #include "kernels_sell.hpp"
 #include "setup.hpp"
+#include "transfer.hpp"
 
 namespace cfdg {
 
@@ -145,7 +146,8 @@ struct cfdg_ctx {
     } f32;
     DBuf<double> b, x;    // right-hand side and solution, 5 per cell in device order
     DBuf<double> bs, xs;  // the same in the sliced layout
-    DBuf<double> stage;   // 5 per cell in mesh order: vectors crossing the ABI
+    DBuf<double> stage;   // 5 per cell in mesh order: states and vectors crossing the ABI
+    cfdg::HostPipe pipe;  // their copies from and to the caller's arrays
     DBuf<double> partial, dots;
     double* h_dots = nullptr;  // pinned
     DBuf<double> ks;           // device-driven BiCGSTAB state block (kernels_linalg.hpp)

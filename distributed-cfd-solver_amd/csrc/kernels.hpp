@@ -255,6 +255,9 @@ void launch_dt(const MeshArgs& m, const FieldArgs& f, const double* lam, double 
 void launch_output_fields(int nc, const Gas& g, const double* U, double* out, hipStream_t s);
 // mdot[f] = mdot_tile[face_entry[f]] for every face (mesh order)
 void launch_gather_mdot(int nf, const int* face_entry, const double* mdot_tile, double* mdot, hipStream_t s);
+// five planes of nc from mesh order to device order and back
+void launch_planes_to_device(int nc, const int* mesh_of_row, const double* src, double* dst, hipStream_t s);
+void launch_planes_to_mesh(int nc, const int* mesh_of_row, const double* src, double* dst, hipStream_t s);
 // forward Euler: alpha = CFL / lambda, then U <- U - alpha R
 void launch_dt_explicit(const MeshArgs& m, const FieldArgs& f, const double* lam, double cfl, double* dt,
                         double* alpha, hipStream_t s);

@@ -910,6 +910,23 @@ __global__ void __launch_bounds__(kBlock) k_dt_explicit(int nc, const double* cs
     alpha[c] = cfl_over_l;
 }
 
+// Five planes of nc between mesh order and device order: dst[r] = src[map[r]]
+// (mesh cell of a device row), or back, dst[map[r]] = src[r].  A tile's rows are
+// runs of neighbouring mesh cells, so either side falls in few cache lines.
+template <bool kToDevice>
+__global__ void __launch_bounds__(kBlock) k_permute_planes(int nc, const int* map, const double* src, double* dst) {
+    const int r = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
+    if (r >= nc) return;
+    const int o = map[r];
+    for (int v = 0; v < 5; ++v) {
+        const long long p = static_cast<long long>(v) * nc;
+        if (kToDevice)
+            dst[p + r] = src[p + o];
+        else
+            dst[p + o] = src[p + r];
+    }
+}
+
 // Forward Euler update U <- U - alpha R (update_ops.hpp:28-44)
 __global__ void __launch_bounds__(kBlock) k_explicit_update(int nc, const double* alpha, const double* res, double* U) {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1232,6 +1249,14 @@ void launch_dt_explicit(const MeshArgs& m, const FieldArgs& f, const double* lam
                         double* alpha, hipStream_t s) {
     if (m.nc > 0)
         hipLaunchKernelGGL(k_dt_explicit, grid_for(m.nc), dim3(kBlock), 0, s, m.nc, f.cs, f.ld, lam, cfl, dt, alpha);
+}
+
+void launch_planes_to_device(int nc, const int* mesh_of_row, const double* src, double* dst, hipStream_t s) {
+    if (nc > 0) hipLaunchKernelGGL(k_permute_planes<true>, grid_for(nc), dim3(kBlock), 0, s, nc, mesh_of_row, src, dst);
+}
+
+void launch_planes_to_mesh(int nc, const int* mesh_of_row, const double* src, double* dst, hipStream_t s) {
+    if (nc > 0) hipLaunchKernelGGL(k_permute_planes<false>, grid_for(nc), dim3(kBlock), 0, s, nc, mesh_of_row, src, dst);
 }
 
 void launch_explicit_update(const MeshArgs& m, const FieldArgs& f, const double* alpha, double* U, hipStream_t s) {
