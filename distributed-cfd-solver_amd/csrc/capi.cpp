@@ -25,6 +25,7 @@
 #include "ctx.hpp"
 #include "kernels.hpp"
 #include "kernels_linalg.hpp"
+#include "kernels_reduced.hpp"
 #include "kernels_sell.hpp"
 #include "mesh.hpp"
 #include "setup.hpp"
@@ -335,16 +336,14 @@ struct Precond {
 long long vector_size(const cfdg_ctx& c, const Precond& P) { return P.sliced() ? c.sliced_size() : 5LL * c.nc; }
 
 // Work vectors of one Krylov precision.
-template <class T>
-struct KVecs {
-    T *r, *r0, *p, *v, *s, *t, *ph, *sh;
-};
-KVecs<double> kvecs64(cfdg_ctx& c) {
-    return {c.r.get(), c.r0.get(), c.p.get(), c.v.get(), c.s.get(), c.t.get(), c.ph.get(), c.sh.get()};
+cfdg::RedVecs<double> kvecs64(cfdg_ctx& c) {
+    return {c.r.get(), c.r0.get(), c.p.get(),  c.v.get(),  c.s.get(),
+            c.t.get(), c.ph.get(), c.sh.get(), c.rd.get(), c.rg.get()};
 }
-KVecs<float> kvecs32(cfdg_ctx& c) {
+cfdg::RedVecs<float> kvecs32(cfdg_ctx& c) {
     auto& f = c.f32;
-    return {f.r.get(), f.r0.get(), f.p.get(), f.v.get(), f.s.get(), f.t.get(), f.ph.get(), f.sh.get()};
+    return {f.r.get(), f.r0.get(), f.p.get(),  f.v.get(),  f.s.get(),
+            f.t.get(), f.ph.get(), f.sh.get(), f.rd.get(), f.rg.get()};
 }
 
 template <class T>
@@ -364,7 +363,7 @@ void spmv_stored(cfdg_ctx& c, const Precond& P, const T* x, T* y, const double* 
 // sweep ended with: those rows read only neighbours that the forward sweep
 // already left final, so their backward update equals their forward one bit
 // for bit and is skipped.  first_done: the forward sweep's first group was
-// already solved by the kernel that formed r (vec_sgs_first).
+// already solved by the kernel that formed r (launch_vec_sgs_first).
 template <class T>
 void precond_apply(cfdg_ctx& c, const Precond& P, const T* r, T* z, const double* gate = nullptr,
                    bool first_done = false) {
@@ -395,17 +394,6 @@ void precond_apply(cfdg_ctx& c, const Precond& P, const T* r, T* z, const double
             cfdg::launch_sgs_group<T>(c.grows[sweep].get() + off[k], off[k + 1] - off[k], b, c.values.get(), c.storage,
                                       c.lu_csr.get(), c.piv.get(), lower, r, z, c.stream, gate);
     }
-}
-
-// y = p (op 0) or s (op 1) and the first group's z = M^-1 y in one launch.
-template <class T>
-void vec_sgs_first(cfdg_ctx& c, const Precond& P, int op, const double* ks, const T* r, const T* v, T* y, T* z) {
-    if (P.sliced())
-        cfdg::launch_sell_vec_first<T>(op, c.sellargs(), c.sellmatrix(), c.sell.colour_slice[1], ks, r, v, y, z,
-                                       c.stream);
-    else
-        cfdg::launch_vec_sgs_first<T>(op, c.nc, ks, r, v, y, c.row_first.get(), c.storage, c.lu_csr.get(),
-                                      c.piv.get(), z, c.stream);
 }
 
 // Diagonal-block LU of the SGS preconditioner (preconditioners.cpp:62-93).
@@ -441,13 +429,24 @@ void precond_check(cfdg_ctx& c, const Precond& P) {
 // Right-preconditioned BiCGSTAB (bicgstab.cpp:42-201) on device vectors of
 // type T (FP64: the reference's arithmetic; FP32: the inner solve of the
 // defect correction).  x holds the initial guess on entry and the solution on
-// exit.  Scalars and dot products are FP64.
+// exit.  Scalars and dot products are FP64.  The multicolour order runs in the
+// reduced form (kernels_reduced.hip), with two exceptions: one colour only, and
+// reduce = false.  A solve whose s vanishes exactly is repeated so, because the
+// reference ends there as broken down unless the rounding of its product, which
+// the reduced form does not have, leaves a remainder to go on with.
 template <class T>
-cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& P, const KVecs<T>& w, T* x,
-                          const T* bvec, bool zero_fallback = false, bool x_zero = false) {
+cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& P, const cfdg::RedVecs<T>& w, T* x,
+                          const T* bvec, bool zero_fallback = false, bool x_zero = false, bool reduce = true) {
     const long long N = vector_size(c, P);
     const std::size_t bytes = static_cast<std::size_t>(N) * sizeof(T);
     cfdg_iter_result res{CFDG_MAX_ITERATIONS, 0, 0.0, 0.0};
+    const int* cs = c.sell.colour_slice.data();
+    const int colours = static_cast<int>(c.sell.colour_slice.size()) - 1;
+    const bool reduced = P.sliced() && reduce && colours > 1;
+    // entries of the first colour, which the reduced form leaves out of its vectors
+    const long long skip = reduced ? cfdg::sell_vector_size(cs[1]) : 0;
+    const auto b = c.sellargs();
+    const auto m = c.sellmatrix();
     // two state blocks: an iteration that ends in launch_xr_next reads one and
     // leaves the next iteration's state in the other
     double* const kb[2] = {c.ks.get(), c.ks.get() + cfdg::kKsCount};
@@ -458,121 +457,143 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
     // device: no host round trip before the first batch of iterations
     {
         cfdg::DotPairsT<T> pr{};
-        pr.a[0] = bvec;
-        pr.b[0] = bvec;
-        if (x_zero) {
-            hip_check(hipMemcpyAsync(w.r, bvec, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
-        } else {
+        int nd = 0;
+        const auto pair = [&](const T* a, long long n) {
+            pr.a[nd] = a;
+            pr.b[nd] = a;
+            pr.n[nd++] = n;
+        };
+        const T* r = bvec;
+        pair(bvec, N);
+        if (!x_zero) {
             spmv_stored<T>(c, P, x, w.v);
             cfdg::launch_axpy_copy<T>(N, bvec, -1.0, w.v, w.r, c.stream);
-            pr.a[1] = w.r;
-            pr.b[1] = w.r;
+            r = w.r;
+            pair(r, N);
         }
-        cfdg::launch_dots(N, x_zero ? 1 : 2, pr, c.partial.get(), c.dots.get(), c.stream);
-        cfdg::launch_bicg_init(ks, c.dots.get(), x_zero ? 1 : 0, zero_fallback ? 1 : 0, lp.abs_tol, lp.rel_tol,
-                               lp.max_iter, c.stream);
+        if (reduced) pair(r, skip);
+        if (reduced && !x_zero) pair(bvec, skip);
+        cfdg::launch_dots(N, nd, pr, c.partial.get(), c.dots.get(), c.stream);
+        cfdg::launch_bicg_init(ks, c.dots.get(), x_zero ? 1 : 0, zero_fallback ? 1 : 0, reduced ? 1 : 0, lp.abs_tol,
+                               lp.rel_tol, lp.max_iter, c.stream);
         if (zero_fallback) cfdg::launch_bicg_reject<T>(N, ks, bvec, x, w.r, c.stream);
+        if (reduced) {
+            cfdg::launch_red_start<T>(b, m, cs, r, w, ks, c.stream);
+        } else {
+            if (x_zero) hip_check(hipMemcpyAsync(w.r, bvec, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
+            hip_check(hipMemcpyAsync(w.r0, w.r, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
+            hip_check(hipMemsetAsync(w.v, 0, bytes, c.stream), "memset");
+        }
     }
-    int it = 0;
-    double rnorm = 0.0;
-    {
-        hip_check(hipMemcpyAsync(w.r0, w.r, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
-        hip_check(hipMemsetAsync(w.v, 0, bytes, c.stream), "memset");
-        // The recurrence runs on the device: scalars in the state block ks,
-        // iterations enqueued in batches and the state read back once per
-        // batch; iterations past convergence or breakdown are no-ops.
-        const int slot = (sizeof(T) == sizeof(double)) ? 0 : 1;
-        int batch = std::max(1, c.last_iters[slot] - 1);
-        const bool sgs = P.kind == CFDG_PRECOND_SGS;
-        long long enq = 0;
-        double* rr = c.dots.get() + 5;
-        // with SGS, every iteration but the last of a batch (and the ones with
-        // the true residual norm) ends with launch_xr_next, which also forms
-        // the next iteration's p and the first group of its M^-1 p
-        bool p_ready = false;
-        while (true) {
-            for (int b = 0; b < batch && enq <= lp.max_iter; ++b) {
-                ++enq;
-                ks = kb[cur];
-                // p, and with SGS the first forward group of p^ = M^-1 p, in one launch
-                if (p_ready) {
-                    // formed by the previous iteration's launch_xr_next
-                } else if (sgs) {
-                    vec_sgs_first<T>(c, P, 0, ks, w.r, w.v, w.p, w.ph);
-                } else {
-                    cfdg::launch_update_p_g<T>(N, ks, w.r, w.v, w.p, c.stream);
-                }
-                precond_apply<T>(c, P, w.p, w.ph, ks, sgs);
-                spmv_stored<T>(c, P, w.ph, w.v, ks);
-                {
-                    cfdg::DotPairsT<T> pr{};
-                    pr.a[0] = w.r0;
-                    pr.b[0] = w.v;
-                    cfdg::launch_dots_step(N, 1, pr, c.partial.get(), c.dots.get(), ks, cfdg::kStepAlpha, c.stream);
-                }
-                if (sgs) {
-                    vec_sgs_first<T>(c, P, 1, ks, w.r, w.v, w.s, w.sh);
-                } else {
-                    cfdg::launch_axpy_alpha_g<T>(N, ks, w.r, w.v, w.s, c.stream);
-                }
-                precond_apply<T>(c, P, w.s, w.sh, ks, sgs);
-                spmv_stored<T>(c, P, w.sh, w.t, ks);
-                {
-                    cfdg::DotPairsT<T> pr{};
-                    const T* A[5] = {w.t, w.t, w.r0, w.r0, w.s};
-                    const T* B[5] = {w.t, w.s, w.t, w.s, w.s};
-                    for (int j = 0; j < 5; ++j) {
-                        pr.a[j] = A[j];
-                        pr.b[j] = B[j];
-                    }
-                    cfdg::launch_dots_step(N, 5, pr, c.partial.get(), c.dots.get(), ks, cfdg::kStepOmega, c.stream);
-                }
-                const bool next_in_batch = b + 1 < batch && enq <= lp.max_iter;
-                if (sgs && next_in_batch && enq % 32 != 0) {
-                    if (P.sliced())
-                        cfdg::launch_sell_xr_next<T>(c.sellargs(), c.sellmatrix(), c.sell.colour_slice[1], ks,
-                                                     kb[1 - cur], w.ph, w.sh, w.s, w.t, x, w.r, w.v, w.p, c.stream);
-                    else
-                        cfdg::launch_xr_next<T>(c.nc, ks, kb[1 - cur], w.ph, w.sh, w.s, w.t, x, w.r, w.v, w.p,
-                                                c.row_first.get(), c.storage, c.lu_csr.get(), c.piv.get(), c.stream);
-                    cur = 1 - cur;
-                    p_ready = true;
-                    continue;
-                }
-                p_ready = false;
-                cfdg::launch_update_xr_g<T>(N, ks, w.ph, w.sh, w.s, w.t, x, w.r, c.stream);
-                if (enq % 32 == 0) {  // true residual norm every 32 iterations
-                    cfdg::DotPairsT<T> pr{};
-                    pr.a[0] = w.r;
-                    pr.b[0] = w.r;
-                    cfdg::launch_dots_step(N, 1, pr, c.partial.get(), rr, ks, cfdg::kStepPost, c.stream);
-                } else {
-                    cfdg::launch_bicg_post(ks, c.stream);
-                }
-            }
-            c.check_launch();
+    // The recurrence runs on the device: scalars in the state block ks,
+    // iterations enqueued in batches and the state read back once per
+    // batch; iterations past convergence or breakdown are no-ops.
+    const int slot = (sizeof(T) == sizeof(double)) ? 0 : 1;
+    int batch = std::max(1, c.last_iters[slot] - 1);
+    // the dependency levels' first group is solved by the vector kernels
+    const bool levels = P.kind == CFDG_PRECOND_SGS && !P.sliced();
+    long long enq = 0;
+    double* rr = c.dots.get() + 5;
+    // with the reduced form and the dependency levels, every iteration but the last
+    // of a batch (and the ones with the true residual norm) ends with launch_xr_next,
+    // which also forms the next iteration's p and the first solves of its M^-1 p
+    bool p_ready = false;
+    // y = p (op 0) or s (op 1), z = M^-1 y, A z, and the dot products of the step
+    const auto product = [&](int op) {
+        if (reduced) {
+            if (!(op == 0 && p_ready)) cfdg::launch_red_vec<T>(op, b, m, cs, w, ks, c.stream);
+            cfdg::launch_red_product<T>(op, b, m, cs, colours, w, c.partial.get(), c.dots.get(), ks, c.stream);
+            return;
+        }
+        T* const y = op == 0 ? w.p : w.s;
+        T* const zv = op == 0 ? w.ph : w.sh;
+        T* const av = op == 0 ? w.v : w.t;
+        if (op == 0 && p_ready) {
+            // formed by the previous iteration's launch_xr_next
+        } else if (levels) {
+            cfdg::launch_vec_sgs_first<T>(op, c.nc, ks, w.r, w.v, y, c.row_first.get(), c.storage, c.lu_csr.get(),
+                                          c.piv.get(), zv, c.stream);
+        } else if (op == 0) {
+            cfdg::launch_update_p_g<T>(N, ks, w.r, w.v, w.p, c.stream);
+        } else {
+            cfdg::launch_axpy_alpha_g<T>(N, ks, w.r, w.v, w.s, c.stream);
+        }
+        precond_apply<T>(c, P, y, zv, ks, levels);
+        spmv_stored<T>(c, P, zv, av, ks);
+        cfdg::DotPairsT<T> pr{};
+        const T* A[5] = {w.t, w.t, w.r0, w.r0, w.s};
+        const T* B[5] = {w.t, w.s, w.t, w.s, w.s};
+        for (int j = 0; j < 5; ++j) {
+            pr.a[j] = op == 0 ? w.r0 : A[j];
+            pr.b[j] = op == 0 ? w.v : B[j];
+        }
+        cfdg::launch_dots_step(N, op == 0 ? 1 : 5, pr, c.partial.get(), c.dots.get(), ks,
+                               op == 0 ? cfdg::kStepAlpha : cfdg::kStepOmega, c.stream);
+    };
+    while (true) {
+        for (int k = 0; k < batch && enq <= lp.max_iter; ++k) {
+            ++enq;
             ks = kb[cur];
-            c.d2h(h, ks, cfdg::kKsCount);
-            c.sync();
-            if (h[cfdg::kKsStatus] != 0.0 || enq > lp.max_iter) break;
-            batch = 2;
+            product(0);
+            product(1);
+            const bool next_in_batch = k + 1 < batch && enq <= lp.max_iter;
+            p_ready = (reduced || levels) && next_in_batch && enq % 32 != 0;
+            if (p_ready) {
+                if (reduced)
+                    cfdg::launch_red_xr_next<T>(b, m, cs, w, x, ks, kb[1 - cur], c.stream);
+                else
+                    cfdg::launch_xr_next<T>(c.nc, ks, kb[1 - cur], w.ph, w.sh, w.s, w.t, x, w.r, w.v, w.p,
+                                            c.row_first.get(), c.storage, c.lu_csr.get(), c.piv.get(), c.stream);
+                cur = 1 - cur;
+                continue;
+            }
+            cfdg::launch_update_xr_g<T>(N - skip, ks, w.ph + skip, w.sh + skip, w.s + skip, w.t + skip, x + skip,
+                                        w.r + skip, c.stream);
+            if (enq % 32 == 0) {  // true residual norm every 32 iterations
+                cfdg::DotPairsT<T> pr{};
+                pr.a[0] = w.r + skip;
+                pr.b[0] = w.r + skip;
+                cfdg::launch_dots_step(N - skip, 1, pr, c.partial.get(), rr, ks, cfdg::kStepPost, c.stream);
+            } else {
+                cfdg::launch_bicg_post(ks, c.stream);
+            }
         }
-        it = static_cast<int>(h[cfdg::kKsIt]);
-        rnorm = h[cfdg::kKsRnorm];
-        const double st = h[cfdg::kKsStatus];
-        res.status = (st == cfdg::kKsConverged) ? CFDG_CONVERGED
-                                                 : (st == cfdg::kKsDiverged ? CFDG_DIVERGED : CFDG_MAX_ITERATIONS);
-        res.initial_residual = h[cfdg::kKsRnorm0];
-        if (zero_fallback) {
-            if (h[cfdg::kKsReject] != 0.0)
-                ++c.warm_rejected;
-            else
-                ++c.warm_used;
-        }
-        if (it > 0) c.last_iters[slot] = it;
+        c.check_launch();
+        ks = kb[cur];
+        c.d2h(h, ks, cfdg::kKsCount);
+        c.sync();
+        if (h[cfdg::kKsStatus] != 0.0 || enq > lp.max_iter) break;
+        batch = 2;
     }
-    c.check_launch();
-    c.sync();
+    int it = static_cast<int>(h[cfdg::kKsIt]);
+    double rnorm = h[cfdg::kKsRnorm];
+    const double st = h[cfdg::kKsStatus];
+    const double updates = h[cfdg::kKsUpdates];
+    res.status = (st == cfdg::kKsConverged) ? CFDG_CONVERGED
+                                             : (st == cfdg::kKsDiverged ? CFDG_DIVERGED : CFDG_MAX_ITERATIONS);
+    res.initial_residual = h[cfdg::kKsRnorm0];
+    bool rejected = false;
+    if (zero_fallback) {
+        rejected = h[cfdg::kKsReject] != 0.0;
+        if (rejected)
+            ++c.warm_rejected;
+        else
+            ++c.warm_used;
+    }
+    if (reduced && updates > 0.0) {
+        cfdg::launch_red_finish<T>(b, m, cs, bvec, w, x, ks, c.stream);
+        c.check_launch();
+    }
+    if (st == cfdg::kKsExact) {
+        cfdg_linparams rest = lp;
+        rest.max_iter = lp.max_iter - (it - 1);
+        const cfdg_iter_result r2 =
+            bicgstab<T>(c, rest, P, w, x, bvec, false, updates == 0.0 && (x_zero || rejected), false);
+        res.status = r2.status;
+        rnorm = r2.final_residual;
+        it += r2.iterations - 1;
+    }
+    if (it > 0) c.last_iters[slot] = it;
     res.iterations = it;
     res.final_residual = rnorm;
     return res;
@@ -623,7 +644,7 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
     }
     const double tol = std::max(lp.abs_tol, lp.rel_tol * ((bnorm > 0.0) ? bnorm : 1.0));
     res.initial_residual = rnorm;
-    const KVecs<float> w = kvecs32(c);
+    const cfdg::RedVecs<float> w = kvecs32(c);
     int total = 0;
     for (int pass = 0;; ++pass) {
         if (!std::isfinite(rnorm)) {
@@ -923,6 +944,7 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
         c.sell_row.upload(c.sell.row, s);
         c.sell_pos.upload(c.sell.pos, s);
         c.sell_count.upload(c.sell.count, s);
+        c.sell_lower0.upload(c.sell.lower0, s);
         c.sell_cols.upload(c.sell.cols, s);
         c.sell_tile_pos.upload(c.sell.tile_pos, s);
         c.sell_visit.upload(c.sell.visit, s);
@@ -931,6 +953,7 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
         c.sync();
         for (auto* v : {&c.sell.row, &c.sell.tile_pos, &c.sell.visit_base}) std::vector<i32>().swap(*v);
         std::vector<std::uint32_t>().swap(c.sell.visit);
+        std::vector<std::uint16_t>().swap(c.sell.lower0);
         const cfdg::Csr ccf_dev = to_device_rows(c.ccf_mesh, c.new2old, &c.old2new);
         c.ccf_off.upload(ccf_dev.off, s);
         c.ccf.upload(ccf_dev.idx, s);
@@ -1044,11 +1067,11 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
     alloc_lu(c, 0);
     c.sell_piv.alloc(z(c.n_slices()) * cfdg::kSellRows);
     c.singular.alloc(1);
-    for (DBuf<double>* v : {&c.r, &c.r0, &c.p, &c.v, &c.s, &c.t, &c.ph, &c.sh, &c.bs, &c.xs, &c.b, &c.x}) {
+    for (DBuf<double>* v : {&c.r, &c.r0, &c.p, &c.v, &c.s, &c.t, &c.ph, &c.sh, &c.rd, &c.rg, &c.bs, &c.xs, &c.b, &c.x}) {
         v->alloc(v == &c.b || v == &c.x ? 5 * ncs : c.vector_alloc());
         v->zero(s);
     }
-    c.partial.alloc(static_cast<std::size_t>(cfdg::kReduceBlocks) * 5);
+    c.partial.alloc(static_cast<std::size_t>(cfdg::kMaxPartials) * 5);
     c.dots.alloc(8);
     c.ks.alloc(2 * cfdg::kKsCount);
     c.sync();
@@ -1125,13 +1148,13 @@ void set_precision(cfdg_ctx& c, const cfdg_precision& p) {
     alloc_lu(c, lu_f32);
     if (p.krylov == CFDG_PREC_FP32) {
         auto& f = c.f32;
-        for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh}) {
+        for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh, &f.rd, &f.rg}) {
             if (v->size() != c.vector_alloc()) v->alloc(c.vector_alloc());
             v->zero(c.stream);
         }
     } else {
         auto& f = c.f32;
-        for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh}) v->alloc(0);
+        for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh, &f.rd, &f.rg}) v->alloc(0);
     }
     c.sync();
     c.storage = storage;

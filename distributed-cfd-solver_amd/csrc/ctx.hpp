@@ -115,7 +115,7 @@ struct cfdg_ctx {
     DBuf<int4> sell_slice;
     DBuf<int> sell_row, sell_pos, sell_cols, sell_tile_pos, sell_visit_base;
     DBuf<std::uint32_t> sell_count, sell_visit;
-    DBuf<std::uint16_t> sell_piv;
+    DBuf<std::uint16_t> sell_piv, sell_lower0;
     DBuf<std::uint8_t> sell_off, sell_diag, lu;
     DBuf<int> mesh_of_row;  // device row -> mesh cell
     DBuf<int> block_code;   // where each block of the ABI's pattern is stored, made on first use
@@ -141,8 +141,9 @@ struct cfdg_ctx {
     // per row in device order, or sliced (then zero past a slice's rows).
     bool vectors_sliced = true;
     DBuf<double> r, r0, p, v, s, t, ph, sh;
+    DBuf<double> rd, rg;  // d and g of the reduced form (kernels_reduced.hpp)
     struct F32 {
-        DBuf<float> b, x, r, r0, p, v, s, t, ph, sh;
+        DBuf<float> b, x, r, r0, p, v, s, t, ph, sh, rd, rg;
     } f32;
     DBuf<double> b, x;    // right-hand side and solution, 5 per cell in device order
     DBuf<double> bs, xs;  // the same in the sliced layout
@@ -274,6 +275,7 @@ struct cfdg_ctx {
         a.row = sell_row.get();
         a.pos = sell_pos.get();
         a.count = sell_count.get();
+        a.lower0 = sell_lower0.get();
         a.cols = sell_cols.get();
         a.tile_pos = sell_tile_pos.get();
         a.visit = sell_visit.get();

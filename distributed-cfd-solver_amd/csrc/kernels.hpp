@@ -205,6 +205,7 @@ struct SellArgs {
     const int* row;           // position -> device row, -1 past a slice's rows
     const int* pos;           // device row -> position
     const std::uint32_t* count;  // per position: lower blocks | upper blocks << 16
+    const std::uint16_t* lower0;  // per position: lower blocks with a column of the first colour, before the others
     const int* cols;          // per (slot, lane): position of the column
     const int* tile_pos;      // the Jacobian's rows and visits (SellPlan)
     const std::uint32_t* visit;

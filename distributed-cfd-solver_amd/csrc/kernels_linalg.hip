@@ -293,7 +293,7 @@ __global__ void __launch_bounds__(kBlock) k_update_xr(long long n, double alpha,
 
 // Start of a solve (bicgstab.cpp:56-92): norms, tolerance, initial status,
 // then the start of the first iteration.
-__global__ void k_bicg_init(double* ks, const double* dots, int x_zero, int fallback, double abs_tol,
+__global__ void k_bicg_init(double* ks, const double* dots, int x_zero, int fallback, int reduced, double abs_tol,
                             double rel_tol, int max_iter) {
     const double bnorm = sqrt(dots[0]);
     double rnorm = x_zero ? bnorm : sqrt(dots[1]);
@@ -314,6 +314,14 @@ __global__ void k_bicg_init(double* ks, const double* dots, int x_zero, int fall
     ks[kKsRnorm] = rnorm;
     ks[kKsRnorm0] = rnorm;
     ks[kKsReject] = reject;
+    if (reduced) {
+        const double b0 = dots[x_zero ? 1 : (reject != 0.0 ? 3 : 2)];
+        ks[kKsReduced] = 1.0;
+        if (b0 > 0.0) {
+            ks[kKsB0] = b0;
+            ks[kKsAr] = 1.0;
+        }
+    }
     if (!isfinite(rnorm))
         ks[kKsStatus] = kKsDiverged;
     else if (rnorm <= tol)
@@ -334,27 +342,31 @@ __global__ void __launch_bounds__(kBlock) k_bicg_reject(long long n, const doubl
 
 // gamma = (r0, v); alpha = rho / gamma (bicgstab.cpp:113-120)
 __device__ void bicg_alpha(double* ks, const double* dots) {
-    const double gamma = dots[0];
+    const double gamma = dots[0] + ks[kKsAp] * ks[kKsB0];
     if (!isfinite(gamma) || gamma == 0.0) {
         ks[kKsStatus] = kKsDiverged;
         return;
     }
     ks[kKsAlpha] = ks[kKsRho] / gamma;
+    ks[kKsAs] = ks[kKsAr] - ks[kKsAlpha] * ks[kKsAp];  // s = r - alpha v with v = p
 }
 
 // omega = (t, s) / (t, t); the recurrence norm of the new r and rho_new
 // (bicgstab.cpp:126-160); dots = (t,t), (t,s), (r0,t), (r0,s), (s,s)
 __device__ void bicg_omega(double* ks, const double* dots) {
-    const double tt = dots[0], ts = dots[1], r0t = dots[2], r0s = dots[3], ss = dots[4];
+    // the first colour's t = s: (t,t) = (t,s) = (s,s) and (r0,t) = (r0,s)
+    const double first = ks[kKsAs] * ks[kKsAs] * ks[kKsB0];
+    const double tt = dots[0] + first, ts = dots[1] + first, r0t = dots[2], r0s = dots[3], ss = dots[4];
     if (!isfinite(ts) || !isfinite(tt) || tt == 0.0) {
-        ks[kKsStatus] = kKsDiverged;
+        ks[kKsStatus] = (ks[kKsReduced] != 0.0 && tt == 0.0 && ss == 0.0) ? kKsExact : kKsDiverged;
         return;
     }
     const double omega_new = ts / tt;
-    const double rn2 = ss - 2.0 * omega_new * ts + omega_new * omega_new * tt;
+    const double rest = 1.0 - omega_new;
+    const double rn2 = (ss - 2.0 * omega_new * dots[1] + omega_new * omega_new * dots[0]) + first * (rest * rest);
     ks[kKsOmegaNew] = omega_new;
     ks[kKsRnNew] = sqrt(rn2 > 0.0 ? rn2 : 0.0);
-    ks[kKsRhoNew] = r0s - omega_new * r0t;
+    ks[kKsRhoNew] = (r0s - omega_new * r0t) + ks[kKsAs] * rest * ks[kKsB0];
 }
 
 __global__ void k_bicg_post(double* ks) {
@@ -431,7 +443,7 @@ __global__ void __launch_bounds__(kBlock) k_xr_next(int nrows, const double* ks_
                                                     const TV* sh, const TV* sv, const TV* t, TV* x, TV* r,
                                                     const TV* v, TV* p, const std::uint8_t* first, const TL* lu,
                                                     const std::uint8_t* piv) {
-    __shared__ double next[4];  // status, first, beta, nbo of the next iteration
+    __shared__ double next[kNextCount];  // status, first, beta, nbo of the next iteration
     if (!next_iteration(ks_in, ks_out, next)) return;
     const int lane = static_cast<int>(threadIdx.x & 63);
     const int rw = lane / 5;
@@ -495,18 +507,20 @@ __device__ __forceinline__ double wave_sum(double v) {
     return v;
 }
 
-// Block-level sum in a fixed tree order; result valid in thread 0.
-__device__ __forceinline__ double block_sum(double v, double* lds) {
-    v = wave_sum(v);
-    const int lane = threadIdx.x & 63;
-    const int wid = threadIdx.x >> 6;
-    if (lane == 0) lds[wid] = v;
-    __syncthreads();
-    double s = 0.0;
-    if (threadIdx.x == 0) {
-        for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) s += lds[w];
+// Sums over the workgroup of the first ncomp components, each in a fixed tree
+// order (the waves' sums in wave order); sum j valid in thread j.  lds: 5 per wave.
+__device__ __forceinline__ double block_sums(const double v[5], int ncomp, double* lds) {
+    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+#pragma unroll
+    for (int j = 0; j < 5; ++j) {
+        if (j >= ncomp) break;
+        const double s = wave_sum(v[j]);
+        if (lane == 0) lds[wid * 5 + j] = s;
     }
     __syncthreads();
+    double s = 0.0;
+    if (static_cast<int>(threadIdx.x) < ncomp)
+        for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) s += lds[w * 5 + static_cast<int>(threadIdx.x)];
     return s;
 }
 
@@ -515,23 +529,20 @@ template <class T>
 __global__ void __launch_bounds__(kBlock) k_dots(long long n, int ndot, DotPairsT<T> pr, double* partial,
                                                  const double* gate) {
     if (gate && gate[kKsStatus] != 0.0) return;
-    __shared__ double lds[kBlock / 64];
+    __shared__ double lds[kBlock / 64 * 5];
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
     for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
         for (int j = 0; j < 5; ++j)
-            if (j < ndot) acc[j] += static_cast<double>(pr.a[j][i]) * static_cast<double>(pr.b[j][i]);
+            if (j < ndot && i < pr.n[j]) acc[j] += static_cast<double>(pr.a[j][i]) * static_cast<double>(pr.b[j][i]);
     }
-    for (int j = 0; j < 5; ++j) {
-        if (j >= ndot) break;
-        const double s = block_sum(acc[j], lds);
-        if (threadIdx.x == 0) partial[blockIdx.x * 5 + j] = s;
-    }
+    const double s = block_sums(acc, ndot, lds);
+    if (static_cast<int>(threadIdx.x) < ndot) partial[blockIdx.x * 5 + threadIdx.x] = s;
 }
 
 // Sum of squares of the five residual planes (solver.hpp:740-756)
 __global__ void __launch_bounds__(kBlock) k_res_sq(int nc, int ld, const double* res, double* partial) {
-    __shared__ double lds[kBlock / 64];
+    __shared__ double lds[kBlock / 64 * 5];
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     const int stride = gridDim.x * blockDim.x;
     for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < nc; i += stride) {
@@ -540,24 +551,30 @@ __global__ void __launch_bounds__(kBlock) k_res_sq(int nc, int ld, const double*
             acc[v] += r * r;
         }
     }
-    for (int v = 0; v < 5; ++v) {
-        const double s = block_sum(acc[v], lds);
-        if (threadIdx.x == 0) partial[blockIdx.x * 5 + v] = s;
-    }
+    const double s = block_sums(acc, 5, lds);
+    if (threadIdx.x < 5) partial[blockIdx.x * 5 + threadIdx.x] = s;
 }
 
 // Adds nblocks partial 5-vectors: thread t sums blocks t, t + 256, ... in
-// order, then the block tree adds the 256 thread sums in a fixed order.
+// order, then the block tree adds the 256 thread sums in a fixed order; sum j in
+// thread j.  Bound by latency: the components' loads are in flight together and
+// their trees share the barriers (one component after the other took 7 us for five
+// components of 1,024 partials).
+__device__ __forceinline__ double sum_partials(int nblocks, int ncomp, const double* partial, double* lds) {
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int b = threadIdx.x; b < nblocks; b += kBlock)
+#pragma unroll
+        for (int j = 0; j < 5; ++j)
+            if (j < ncomp) acc[j] += partial[b * 5 + j];
+    return block_sums(acc, ncomp, lds);
+}
+
 __global__ void __launch_bounds__(kBlock) k_reduce_partials(int nblocks, int ncomp, const double* partial,
                                                             double* out, const double* gate) {
     if (gate && gate[kKsStatus] != 0.0) return;
-    __shared__ double lds[kBlock / 64];
-    for (int j = 0; j < ncomp; ++j) {
-        double s = 0.0;
-        for (int b = threadIdx.x; b < nblocks; b += kBlock) s += partial[b * 5 + j];
-        s = block_sum(s, lds);
-        if (threadIdx.x == 0) out[j] = s;
-    }
+    __shared__ double lds[kBlock / 64 * 5];
+    const double s = sum_partials(nblocks, ncomp, partial, lds);
+    if (static_cast<int>(threadIdx.x) < ncomp) out[threadIdx.x] = s;
 }
 
 // k_reduce_partials followed, in thread 0, by the scalar step of the
@@ -568,30 +585,24 @@ template <int kStep>
 __global__ void __launch_bounds__(kBlock) k_reduce_step(int nblocks, int ncomp, const double* partial, double* out,
                                                         double* ks) {
     if (ks[kKsStatus] != 0.0) return;
-    __shared__ double lds[kBlock / 64];
-    for (int j = 0; j < ncomp; ++j) {
-        double s = 0.0;
-        for (int b = threadIdx.x; b < nblocks; b += kBlock) s += partial[b * 5 + j];
-        s = block_sum(s, lds);
-        if (threadIdx.x == 0) out[j] = s;
-    }
+    __shared__ double lds[kBlock / 64 * 5];
+    __shared__ double sums[5];
+    const double s = sum_partials(nblocks, ncomp, partial, lds);
+    if (static_cast<int>(threadIdx.x) < ncomp) out[threadIdx.x] = sums[threadIdx.x] = s;
+    __syncthreads();
     if (threadIdx.x != 0) return;
-    if constexpr (kStep == kStepAlpha) bicg_alpha(ks, out);
-    if constexpr (kStep == kStepOmega) bicg_omega(ks, out);
-    if constexpr (kStep == kStepPost) bicg_post(ks, out);
+    if constexpr (kStep == kStepAlpha) bicg_alpha(ks, sums);
+    if constexpr (kStep == kStepOmega) bicg_omega(ks, sums);
+    if constexpr (kStep == kStepPost) bicg_post(ks, sums);
 }
 
 // The partial sums of k_res_sq added in k_reduce_partials' order, then
 // l2[v] = sqrt(sum_v * scale) (solver.hpp:740-756) written to device memory.
 __global__ void __launch_bounds__(kBlock) k_norms_finish(int nblocks, const double* partial, double scale,
                                                          double* l2) {
-    __shared__ double lds[kBlock / 64];
-    for (int j = 0; j < 5; ++j) {
-        double s = 0.0;
-        for (int b = threadIdx.x; b < nblocks; b += kBlock) s += partial[b * 5 + j];
-        s = block_sum(s, lds);
-        if (threadIdx.x == 0) l2[j] = sqrt(s * scale);
-    }
+    __shared__ double lds[kBlock / 64 * 5];
+    const double s = sum_partials(nblocks, 5, partial, lds);
+    if (threadIdx.x < 5) l2[threadIdx.x] = sqrt(s * scale);
 }
 
 // b = -R (AoS), the implicit right-hand side (implicit_euler.hpp:81-92)
@@ -727,11 +738,19 @@ int reduction_blocks(long long n) {
     return static_cast<int>(b);
 }
 
+// a pair without a length of its own is as long as the vectors
+template <class T>
+static DotPairsT<T> whole(long long n, DotPairsT<T> pr) {
+    for (long long& k : pr.n)
+        if (k == 0) k = n;
+    return pr;
+}
+
 template <class T>
 void launch_dots(long long n, int ndot, const DotPairsT<T>& pr, double* partial, double* out, hipStream_t s,
                  const double* gate) {
     const int nb = reduction_blocks(n);
-    hipLaunchKernelGGL(k_dots<T>, dim3(nb), dim3(kBlock), 0, s, n, ndot, pr, partial, gate);
+    hipLaunchKernelGGL(k_dots<T>, dim3(nb), dim3(kBlock), 0, s, n, ndot, whole(n, pr), partial, gate);
     hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kBlock), 0, s, nb, ndot, partial, out, gate);
 }
 
@@ -744,7 +763,15 @@ template <class T>
 void launch_dots_step(long long n, int ndot, const DotPairsT<T>& pr, double* partial, double* out, double* ks,
                       int step, hipStream_t s) {
     const int nb = reduction_blocks(n);
-    hipLaunchKernelGGL(k_dots<T>, dim3(nb), dim3(kBlock), 0, s, n, ndot, pr, partial, ks);
+    hipLaunchKernelGGL(k_dots<T>, dim3(nb), dim3(kBlock), 0, s, n, ndot, whole(n, pr), partial, ks);
+    launch_reduce_step(nb, ndot, partial, out, ks, step, s);
+}
+template void launch_dots_step<double>(long long, int, const DotPairsT<double>&, double*, double*, double*, int,
+                                       hipStream_t);
+template void launch_dots_step<float>(long long, int, const DotPairsT<float>&, double*, double*, double*, int,
+                                      hipStream_t);
+
+void launch_reduce_step(int nb, int ndot, const double* partial, double* out, double* ks, int step, hipStream_t s) {
     if (step == kStepAlpha)
         hipLaunchKernelGGL(k_reduce_step<kStepAlpha>, dim3(1), dim3(kBlock), 0, s, nb, ndot, partial, out, ks);
     else if (step == kStepOmega)
@@ -752,14 +779,11 @@ void launch_dots_step(long long n, int ndot, const DotPairsT<T>& pr, double* par
     else
         hipLaunchKernelGGL(k_reduce_step<kStepPost>, dim3(1), dim3(kBlock), 0, s, nb, ndot, partial, out, ks);
 }
-template void launch_dots_step<double>(long long, int, const DotPairsT<double>&, double*, double*, double*, int,
-                                       hipStream_t);
-template void launch_dots_step<float>(long long, int, const DotPairsT<float>&, double*, double*, double*, int,
-                                      hipStream_t);
 
-void launch_bicg_init(double* ks, const double* dots, int x_zero, int fallback, double abs_tol, double rel_tol,
-                      int max_iter, hipStream_t s) {
-    hipLaunchKernelGGL(k_bicg_init, dim3(1), dim3(1), 0, s, ks, dots, x_zero, fallback, abs_tol, rel_tol, max_iter);
+void launch_bicg_init(double* ks, const double* dots, int x_zero, int fallback, int reduced, double abs_tol,
+                      double rel_tol, int max_iter, hipStream_t s) {
+    hipLaunchKernelGGL(k_bicg_init, dim3(1), dim3(1), 0, s, ks, dots, x_zero, fallback, reduced, abs_tol, rel_tol,
+                       max_iter);
 }
 
 template <class T>

@@ -14,20 +14,27 @@
 namespace cfdg {
 
 constexpr int kReduceBlocks = 1024;  // partial sums per reduction (fixed -> deterministic)
+constexpr int kMaxPartials = 1536;   // of the reductions fused into a product (one per slice, kernels_reduced.hip)
 
 // State block of the device-driven BiCGSTAB (doubles).  kKsStatus is 0 while
 // the solve runs, then one of the codes below; every gated kernel returns at
 // once when it is not 0.
 enum : int {
     kKsStatus = 0, kKsIt, kKsMaxIt, kKsTol, kKsRho, kKsRhoOld, kKsAlpha, kKsOmega, kKsBeta, kKsNbo, kKsFirst,
-    kKsOmegaNew, kKsRnNew, kKsRhoNew, kKsRnorm, kKsRnorm0, kKsReject, kKsCount = 24
+    kKsOmegaNew, kKsRnNew, kKsRhoNew, kKsRnorm, kKsRnorm0, kKsReject,
+    // the reduced form (kernels_reduced.hip; zero in the others): multiples of the
+    // first colour's initial residual in r, p and s, its squared norm, whether the
+    // form is in use; and the updates of x so far
+    kKsAr, kKsAp, kKsAs, kKsB0, kKsReduced, kKsUpdates, kKsCount = 24
 };
-constexpr double kKsConverged = 1.0, kKsDiverged = 2.0, kKsMaxIter = 3.0;
+// kKsExact: the reduced form met s = 0 exactly
+constexpr double kKsConverged = 1.0, kKsDiverged = 2.0, kKsMaxIter = 3.0, kKsExact = 4.0;
 
 template <class T>
 struct DotPairsT {
     const T* a[5];
     const T* b[5];
+    long long n[5];  // entries of the pair, 0 for all
 };
 using DotPairs = DotPairsT<double>;
 
@@ -57,7 +64,7 @@ void launch_cast_f64_to_f32(long long n, const double* src, float* dst, hipStrea
 void launch_cast_f32_to_f64(long long n, const float* src, double* dst, hipStream_t s);
 void launch_add_f32(long long n, const float* e, double* x, hipStream_t s);
 int reduction_blocks(long long n);
-// out[0..ndot) = dot products accumulated in FP64; partial needs kReduceBlocks * 5 doubles
+// out[0..ndot) = dot products accumulated in FP64; partial needs kMaxPartials * 5 doubles
 template <class T>
 void launch_dots(long long n, int ndot, const DotPairsT<T>& pr, double* partial, double* out, hipStream_t s,
                  const double* gate = nullptr);
@@ -67,9 +74,10 @@ void launch_dots(long long n, int ndot, const DotPairsT<T>& pr, double* partial,
 // Start of a solve from dots = (b, b) and, unless x_zero, (r, r) with r = b - A x:
 // tolerance max(abs_tol, rel_tol ||b||), status, rho; with fallback, a guess
 // whose residual exceeds ||b|| is marked rejected (launch_bicg_reject then
-// restarts from zero).
-void launch_bicg_init(double* ks, const double* dots, int x_zero, int fallback, double abs_tol, double rel_tol,
-                      int max_iter, hipStream_t s);
+// restarts from zero).  reduced: dots go on with (r, r) -- or x_zero, (b, b) --
+// of the first colour, and unless x_zero with its (b, b).
+void launch_bicg_init(double* ks, const double* dots, int x_zero, int fallback, int reduced, double abs_tol,
+                      double rel_tol, int max_iter, hipStream_t s);
 template <class T>
 void launch_bicg_reject(long long n, const double* ks, const T* b, T* x, T* r, hipStream_t s);
 // dot products as launch_dots, gated by ks, then the scalar step that uses them
@@ -80,6 +88,8 @@ enum { kStepAlpha = 1, kStepOmega = 2, kStepPost = 3 };
 template <class T>
 void launch_dots_step(long long n, int ndot, const DotPairsT<T>& pr, double* partial, double* out, double* ks,
                       int step, hipStream_t s);
+// the second half of it: nb partial sums of ndot products, then the scalar step
+void launch_reduce_step(int nb, int ndot, const double* partial, double* out, double* ks, int step, hipStream_t s);
 // the end of an iteration with the recurrence's residual norm
 void launch_bicg_post(double* ks, hipStream_t s);
 template <class T>

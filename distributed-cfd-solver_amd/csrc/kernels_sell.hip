@@ -9,7 +9,11 @@
 //   k_sell_lu      diagonal-block LU with partial pivoting (bsr_helpers.hpp:278-321)
 //   k_sell_spmv    y = A x
 //   k_sell_sweep   one Gauss-Seidel step of a colour (bsr_helpers.hpp:390-435)
-//   k_sell_vec_first, k_sell_xr_next   Krylov vector updates with the first colour's solves
+//
+// The iterations of the solve run on kernels_reduced.hip, which needs neither a
+// whole product nor a whole sweep; these serve the residuals of the defect
+// correction, the ABI's product and preconditioner calls, and the solves that the
+// reduced form leaves (bicgstab, capi.cpp).
 //
 // Arithmetic per row component: products summed over the block's columns, the
 // block sums added or subtracted in the order of the row's slots.
@@ -27,94 +31,18 @@
 #include <type_traits>
 
 #include "kernels.hpp"
-#include "kernels_krylov.hpp"
 #include "kernels_sell.hpp"
+#include "kernels_sell_device.hpp"
 
 namespace cfdg {
 
 namespace {
 
-constexpr int kBlock = 256;
-constexpr int kBlockSlices = kBlock / kSellRows;  // slices per workgroup, one per wave
+constexpr int kBlock = kSellBlock;
 
 inline dim3 grid_for(long long n) { return dim3(static_cast<unsigned>((n + kBlock - 1) / kBlock)); }
-inline dim3 grid_for_slices(int n) { return dim3(static_cast<unsigned>((n + kBlockSlices - 1) / kBlockSlices)); }
 
 [[noreturn]] void throw_bad_combination(const char* what) { throw std::invalid_argument(what); }
-
-template <class TS>
-using word_t = typename SellLayout<TS>::word;
-
-// The 25 entries of the block in (slot, lane) as storage words.
-template <class TS>
-__device__ __forceinline__ void load_words(const word_t<TS>* v, long long slot, int lane, word_t<TS> w[]) {
-    const word_t<TS>* p = v + slot * (SellLayout<TS>::words * kSellRows) + lane;
-#pragma unroll
-    for (int q = 0; q < SellLayout<TS>::words; ++q) w[q] = p[q * kSellRows];
-}
-// Entry e of a loaded block in the arithmetic type.
-template <class TS, class TV>
-__device__ __forceinline__ TV entry(const word_t<TS> w[], int e) {
-    if constexpr (sizeof(TS) == sizeof(bf16)) {
-        const std::uint32_t u = w[e >> 1];
-        return static_cast<TV>(f32_from_bits((e & 1) ? (u & 0xffff0000u) : (u << 16)));
-    } else {
-        return load_as<TV>(w[e]);
-    }
-}
-
-// Component 0 of the row at a position; component v follows at v * 64.
-__device__ __forceinline__ long long vec_at(int position) {
-    return static_cast<long long>(position >> 6) * (5 * kSellRows) + (position & (kSellRows - 1));
-}
-
-// t = A x of one block: t_a = a0 x0 + a1 x1 + ... in column order
-template <class TS, class TV>
-__device__ __forceinline__ void block_times(const word_t<TS> w[], const TV x[5], TV t[5]) {
-#pragma unroll
-    for (int a = 0; a < 5; ++a) {
-        TV s = entry<TS, TV>(w, a * 5) * x[0];
-#pragma unroll
-        for (int b = 1; b < 5; ++b) s += entry<TS, TV>(w, a * 5 + b) * x[b];
-        t[a] = s;
-    }
-}
-
-// Solution of (LU) x = s with partial pivoting (lu_solve_block<5>,
-// bsr_helpers.hpp:325-353); pivots as five 3-bit row numbers.
-template <class TV>
-__device__ __forceinline__ void lu_solve(TV s[5], const TV L[25], unsigned piv) {
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-        const int pk = static_cast<int>((piv >> (3 * k)) & 7u);
-        const TV sk = s[k];
-        TV sp = sk;
-#pragma unroll
-        for (int q = k + 1; q < 5; ++q) {
-            const bool sw = q == pk;
-            sp = sw ? s[q] : sp;
-            s[q] = sw ? sk : s[q];
-        }
-        s[k] = sp;
-    }
-#pragma unroll
-    for (int a = 1; a < 5; ++a)
-#pragma unroll
-        for (int b = 0; b < a; ++b) s[a] -= L[a * 5 + b] * s[b];
-#pragma unroll
-    for (int a = 4; a >= 0; --a) {
-#pragma unroll
-        for (int b = a + 1; b < 5; ++b) s[a] -= L[a * 5 + b] * s[b];
-        s[a] = s[a] / L[a * 5 + a];
-    }
-}
-
-template <class TL, class TV>
-__device__ __forceinline__ void load_lu(const TL* lu, int slice, int lane, TV L[25]) {
-    const TL* p = lu + static_cast<long long>(slice) * (25 * kSellRows) + lane;
-#pragma unroll
-    for (int k = 0; k < 25; ++k) L[k] = load_as<TV>(p[k * kSellRows]);
-}
 
 template <class TS, class TL>
 __global__ void __launch_bounds__(kBlock) k_sell_lu(SellArgs b, const word_t<TS>* diag, TL* lu, std::uint16_t* piv,
@@ -178,77 +106,6 @@ __global__ void __launch_bounds__(kBlock) k_sell_lu(SellArgs b, const word_t<TS>
     piv[p] = static_cast<std::uint16_t>(pv);
 }
 
-// t = A x for the row's block in a slot.
-template <class TS, class TV>
-__device__ __forceinline__ void slot_times(const word_t<TS>* off, const int* cols, long long slot, int lane,
-                                           const TV* x, TV t[5]) {
-    word_t<TS> w[SellLayout<TS>::words];
-    const TV* xb = x + vec_at(cols[slot * kSellRows + lane]);
-    load_words<TS>(off, slot, lane, w);
-    TV xv[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) xv[v] = xb[v * kSellRows];
-    block_times<TS, TV>(w, xv, t);
-}
-
-// Whether the row with block counts n (lower | upper << 16) has a block in the
-// j-th slot of its slice.
-__device__ __forceinline__ bool has_block(const int4& sl, unsigned n, int j) {
-    return j < sl.y ? j < static_cast<int>(n & 0xffffu) : j - sl.y < static_cast<int>(n >> 16);
-}
-
-// The products of slots [0, slots) of a slice with x, handed to add(t) in slot
-// order.  kSplit = 1: by the wave alone, one slot after the other.  kSplit > 1:
-// the kSplit waves of the workgroup, all on the same slice, form kSplit slots at a
-// time into LDS and the first wave adds them, in the same order.
-template <int kSplit, class TS, class TV, class F>
-__device__ __forceinline__ void for_slots(const word_t<TS>* off, const int* cols, const int4& sl, unsigned n, int slots,
-                                          int lane, const TV* x, TV* lds, F&& add) {
-    if constexpr (kSplit == 1) {
-        for (int j = 0; j < slots; ++j) {
-            if (!has_block(sl, n, j)) continue;
-            TV t[5];
-            slot_times<TS, TV>(off, cols, sl.x + j, lane, x, t);
-            add(t);
-        }
-    } else {
-        const int w = threadIdx.x >> 6;
-        for (int j0 = 0; j0 < slots; j0 += kSplit) {
-            const int j = j0 + w;
-            if (j < slots && has_block(sl, n, j)) {
-                TV t[5];
-                slot_times<TS, TV>(off, cols, sl.x + j, lane, x, t);
-#pragma unroll
-                for (int v = 0; v < 5; ++v) lds[(w * 5 + v) * kSellRows + lane] = t[v];
-            }
-            __syncthreads();
-            if (w == 0)
-                for (int k = 0; k < kSplit && j0 + k < slots; ++k) {
-                    if (!has_block(sl, n, j0 + k)) continue;
-                    TV t[5];
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) t[v] = lds[(k * 5 + v) * kSellRows + lane];
-                    add(t);
-                }
-            if (j0 + kSplit < slots) __syncthreads();
-        }
-    }
-}
-template <int kSplit>
-constexpr int slice_threads() {
-    return kSplit == 1 ? kBlock : kSplit * kSellRows;
-}
-template <int kSplit, class TV>
-constexpr int split_lds() {
-    return kSplit == 1 ? 1 : kSplit * 5 * kSellRows;
-}
-// The slice of this wave among count, or count and above for none.
-template <int kSplit>
-__device__ __forceinline__ int wave_slice() {
-    const int b = xcd_block(blockIdx.x, gridDim.x);
-    return kSplit == 1 ? b * kBlockSlices + static_cast<int>(threadIdx.x >> 6) : b;
-}
-
 template <class TS, class TV, int kSplit>
 __global__ void __launch_bounds__(slice_threads<kSplit>()) k_sell_spmv(SellArgs b, const word_t<TS>* off,
                                                                        const word_t<TS>* diag, const TV* x, TV* y,
@@ -272,7 +129,7 @@ __global__ void __launch_bounds__(slice_threads<kSplit>()) k_sell_spmv(SellArgs 
         for (int v = 0; v < 5; ++v) xv[v] = x[at + v * kSellRows];
         block_times<TS, TV>(w, xv, acc);
     }
-    for_slots<kSplit, TS, TV>(off, b.cols, sl, n, sl.y + sl.z, lane, x, lds, [&](const TV t[5]) {
+    for_slots<kSplit, TS, TV>(off, b.cols, sl, n, 0, sl.y + sl.z, 0, lane, x, lds, [&](const TV t[5]) {
 #pragma unroll
         for (int v = 0; v < 5; ++v) acc[v] += t[v];
     });
@@ -304,7 +161,7 @@ __global__ void __launch_bounds__(slice_threads<kSplit>()) k_sell_sweep(SellArgs
         for (int v = 0; v < 5; ++v) acc[v] = r[at + v * kSellRows];
         if (kSplit > 1) load_lu<TL, TV>(lu, slice, lane, L);  // in flight with the slots
     }
-    for_slots<kSplit, TS, TV>(off, b.cols, sl, n, all ? sl.y + sl.z : sl.y, lane, z, lds, [&](const TV t[5]) {
+    for_slots<kSplit, TS, TV>(off, b.cols, sl, n, 0, all ? sl.y + sl.z : sl.y, 0, lane, z, lds, [&](const TV t[5]) {
 #pragma unroll
         for (int v = 0; v < 5; ++v) acc[v] -= t[v];
     });
@@ -313,66 +170,6 @@ __global__ void __launch_bounds__(slice_threads<kSplit>()) k_sell_sweep(SellArgs
     lu_solve(acc, L, piv[slice * kSellRows + lane]);
 #pragma unroll
     for (int v = 0; v < 5; ++v) z[at + v * kSellRows] = acc[v];
-}
-
-// y = p (kOp 0) or s (kOp 1), and z_i = D_i^-1 y_i for the rows of the first
-// colour, whose forward sweep reads no off-diagonal block.
-template <int kOp, class TL, class TV>
-__global__ void __launch_bounds__(kBlock) k_sell_vec_first(SellArgs b, int first, const double* ks, const TV* r,
-                                                           const TV* v, TV* y, const TL* lu,
-                                                           const std::uint16_t* piv, TV* z) {
-    if (ks[kKsStatus] != 0.0) return;
-    const int slice = xcd_block(blockIdx.x, gridDim.x) * kBlockSlices + (threadIdx.x >> 6);
-    if (slice >= b.nslices) return;
-    const int lane = threadIdx.x & 63;
-    if (lane >= b.slice[slice].w) return;
-    const long long at = static_cast<long long>(slice) * (5 * kSellRows) + lane;
-    TV s[5];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-        const long long e = at + k * kSellRows;
-        s[k] = (kOp == 0) ? p_entry(ks, r, v, y, e) : s_entry(ks, r, v, e);
-        y[e] = s[k];
-    }
-    if (slice >= first) return;
-    TV L[25];
-    load_lu<TL, TV>(lu, slice, lane, L);
-    lu_solve(s, L, piv[slice * kSellRows + lane]);
-#pragma unroll
-    for (int k = 0; k < 5; ++k) z[at + k * kSellRows] = s[k];
-}
-
-// The end of one iteration and the start of the next (k_xr_next,
-// kernels_linalg.hip) on the sliced vectors.
-template <class TL, class TV>
-__global__ void __launch_bounds__(kBlock) k_sell_xr_next(SellArgs b, int first, const double* ks_in, double* ks_out,
-                                                         TV* ph, const TV* sh, const TV* sv, const TV* t, TV* x, TV* r,
-                                                         const TV* v, TV* p, const TL* lu, const std::uint16_t* piv) {
-    __shared__ double next[4];  // status, first, beta, nbo of the next iteration
-    if (!next_iteration(ks_in, ks_out, next)) return;
-    const int slice = xcd_block(blockIdx.x, gridDim.x) * kBlockSlices + (threadIdx.x >> 6);
-    if (slice >= b.nslices) return;
-    const int lane = threadIdx.x & 63;
-    if (lane >= b.slice[slice].w) return;
-    const long long at = static_cast<long long>(slice) * (5 * kSellRows) + lane;
-    const bool go = next[0] == 0.0;  // uniform over the grid
-    TV s[5];
-#pragma unroll
-    for (int k = 0; k < 5; ++k) {
-        const long long e = at + k * kSellRows;
-        const TV rv = xr_entry(ks_in, ph, sh, sv, t, x, e);
-        r[e] = rv;
-        if (go) {
-            s[k] = p_entry_of(next[1], next[2], next[3], rv, v, p, e);
-            p[e] = s[k];
-        }
-    }
-    if (!go || slice >= first) return;
-    TV L[25];
-    load_lu<TL, TV>(lu, slice, lane, L);
-    lu_solve(s, L, piv[slice * kSellRows + lane]);
-#pragma unroll
-    for (int k = 0; k < 5; ++k) ph[at + k * kSellRows] = s[k];
 }
 
 __global__ void __launch_bounds__(kBlock) k_sell_gather(SellArgs b, const int* src_of, const double* src, double* dst) {
@@ -474,39 +271,6 @@ __global__ void __launch_bounds__(kBlock) k_sell_to_csr(const int* code, long lo
         block_entry<TS>(block_words_of<TS>(code[k], off, diag), e);
 }
 
-// Waves per slice.  A launch over few slices is bound by the latency of a row's
-// chain of slots, so eight waves share a slice (a hexahedron's or tetrahedron's
-// slots all at once); over many slices one wave each fills the chip and the
-// split only adds barriers.  The line lies where the two cross (1,536 slices =
-// 1.5 waves per SIMD), per BiCGSTAB iteration with one wave / with eight: 24,576-cell
-// plate (192 slices per colour) FP64 108 / 77 us, BF16 80 / 61 us; 93,765 cells (735) 147 /
-// 151, 96 / 92; 156,849 cells (1,226) 250 / 231, 114 / 115; 262,144 cells (2,048) 370 /
-// 393, 144 / 156.
-constexpr int kSplitWaves = 8, kSplitSlices = 1536;
-template <int kSplit>
-dim3 slice_grid(int slices) {
-    return kSplit == 1 ? grid_for_slices(slices) : dim3(static_cast<unsigned>(slices));
-}
-// f(std::integral_constant<int, waves per slice>) for a launch over that many slices
-template <class F>
-void with_split(int slices, F&& f) {
-    if (slices <= kSplitSlices)
-        f(std::integral_constant<int, kSplitWaves>{});
-    else
-        f(std::integral_constant<int, 1>{});
-}
-
-// f(TS{}) for the storage kind
-template <class F>
-void with_storage(int storage, F&& f) {
-    if (storage == kStoreF32)
-        f(float{});
-    else if (storage == kStoreBF16)
-        f(bf16{});
-    else
-        f(double{});
-}
-
 }  // namespace
 
 void launch_sell_lu(const SellArgs& b, const SellMatrix& m, void* lu, int lu_f32, std::uint16_t* piv, int* singular,
@@ -569,39 +333,6 @@ template void launch_sell_sweep<double>(const SellArgs&, const SellMatrix&, int,
                                         hipStream_t, const double*);
 template void launch_sell_sweep<float>(const SellArgs&, const SellMatrix&, int, int, bool, const float*, float*,
                                        hipStream_t, const double*);
-
-// The LU type follows the vector type: FP64 factors with FP64 vectors, FP32
-// factors with FP32 vectors.
-template <class TV>
-void launch_sell_vec_first(int op, const SellArgs& b, const SellMatrix& m, int first, const double* ks, const TV* r,
-                           const TV* v, TV* y, TV* z, hipStream_t s) {
-    if (b.nslices <= 0) return;
-    const dim3 g = grid_for_slices(b.nslices), blk(kBlock);
-    const TV* L = static_cast<const TV*>(m.lu);
-    if (op == 0)
-        hipLaunchKernelGGL((k_sell_vec_first<0, TV, TV>), g, blk, 0, s, b, first, ks, r, v, y, L, m.piv, z);
-    else
-        hipLaunchKernelGGL((k_sell_vec_first<1, TV, TV>), g, blk, 0, s, b, first, ks, r, v, y, L, m.piv, z);
-}
-template void launch_sell_vec_first<double>(int, const SellArgs&, const SellMatrix&, int, const double*, const double*,
-                                            const double*, double*, double*, hipStream_t);
-template void launch_sell_vec_first<float>(int, const SellArgs&, const SellMatrix&, int, const double*, const float*,
-                                           const float*, float*, float*, hipStream_t);
-
-template <class TV>
-void launch_sell_xr_next(const SellArgs& b, const SellMatrix& m, int first, const double* ks_in, double* ks_out,
-                         TV* ph, const TV* sh, const TV* sv, const TV* t, TV* x, TV* r, const TV* v, TV* p,
-                         hipStream_t s) {
-    if (b.nslices <= 0) return;
-    hipLaunchKernelGGL((k_sell_xr_next<TV, TV>), grid_for_slices(b.nslices), dim3(kBlock), 0, s, b, first, ks_in,
-                       ks_out, ph, sh, sv, t, x, r, v, p, static_cast<const TV*>(m.lu), m.piv);
-}
-template void launch_sell_xr_next<double>(const SellArgs&, const SellMatrix&, int, const double*, double*, double*,
-                                          const double*, const double*, const double*, double*, double*,
-                                          const double*, double*, hipStream_t);
-template void launch_sell_xr_next<float>(const SellArgs&, const SellMatrix&, int, const double*, double*, float*,
-                                         const float*, const float*, const float*, float*, float*, const float*,
-                                         float*, hipStream_t);
 
 void launch_sell_gather(const SellArgs& b, const int* src_of, const double* src, double* dst, hipStream_t s) {
     if (b.nslices > 0)

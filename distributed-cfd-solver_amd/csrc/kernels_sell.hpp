@@ -46,16 +46,6 @@ void launch_sell_spmv(const SellArgs& b, const SellMatrix& m, const TV* x, TV* y
 template <class TV>
 void launch_sell_sweep(const SellArgs& b, const SellMatrix& m, int first, int count, bool all, const TV* r, TV* z,
                        hipStream_t s, const double* gate = nullptr);
-// The Krylov vector updates of launch_vec_sgs_first / launch_xr_next
-// (kernels_linalg.hpp) with the rows of the first colour, slices [0, first),
-// solved in the same launch.
-template <class TV>
-void launch_sell_vec_first(int op, const SellArgs& b, const SellMatrix& m, int first, const double* ks, const TV* r,
-                           const TV* v, TV* y, TV* z, hipStream_t s);
-template <class TV>
-void launch_sell_xr_next(const SellArgs& b, const SellMatrix& m, int first, const double* ks_in, double* ks_out,
-                         TV* ph, const TV* sh, const TV* sv, const TV* t, TV* x, TV* r, const TV* v, TV* p,
-                         hipStream_t s);
 // dst (sliced) = src (5 values per cell, cell src_of[device row], or the device
 // row itself when src_of is null), and back.
 void launch_sell_gather(const SellArgs& b, const int* src_of, const double* src, double* dst, hipStream_t s);
