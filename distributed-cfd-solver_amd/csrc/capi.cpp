@@ -162,6 +162,41 @@ void upload_groups(cfdg_ctx& c, int slot, const std::vector<i32>& label_mesh, i3
     c.sync();  // rows is released on return
 }
 
+// The chunks of SgsLevels: a row's blocks are stored in ascending mesh column
+// order (ensure_csr), the lower ones before the diagonal and the upper ones after.
+void build_level_chunks(cfdg_ctx& c) {
+    std::vector<i32> begin(z(c.nc) + 1, 0);
+    for (i32 r = 0; r < c.nc; ++r) {
+        const i32 o = c.new2old[z(r)];
+        begin[z(r) + 1] = begin[z(r)] + (c.h_row_ptr[z(o) + 1] - c.h_row_ptr[z(o)]);
+    }
+    constexpr i32 kRows = cfdg::kSgsRowsPerWave;
+    for (int sweep = 0; sweep < 2; ++sweep) {
+        const auto& off = c.h_gofs[sweep];
+        std::vector<i32> rows(c.grows[sweep].size());
+        c.d2h(rows.data(), c.grows[sweep].get(), rows.size());
+        c.sync();
+        std::vector<int4> desc;
+        i32 level = 0;
+        for (std::size_t g = sweep == 0 ? 0 : 1; g + 1 < off.size(); ++g, ++level)
+            for (i32 k = off[g]; k < off[g + 1]; k += kRows)
+                for (i32 q = k; q < k + kRows; ++q) {
+                    if (q >= off[g + 1]) {
+                        desc.push_back(int4{-1, 0, 0, level});
+                        continue;
+                    }
+                    const i32 r = rows[z(q)], o = c.new2old[z(r)];
+                    const i32 d = c.h_diag[z(o)] - c.h_row_ptr[z(o)], n = begin[z(r) + 1] - begin[z(r)];
+                    const i32 first = begin[z(r)] + (sweep == 0 ? 0 : d + 1), count = sweep == 0 ? d : n - d - 1;
+                    desc.push_back(int4{r, count > 0 ? first : 0, count, level});
+                }
+        c.level_count[sweep] = level;
+        c.level_chunks[sweep] = static_cast<int>(desc.size()) / kRows;
+        c.level_desc[sweep].upload(desc, c.stream);
+        c.sync();  // desc is released at the end of the pass
+    }
+}
+
 void build_seq_groups(cfdg_ctx& c) {
     if (c.have_seq_groups) return;
     i32 nfw = 0, nbw = 0;
@@ -169,6 +204,7 @@ void build_seq_groups(cfdg_ctx& c) {
     const auto lb = cfdg::backward_levels(c.ccf_mesh, c.nc, nbw);
     upload_groups(c, 0, lf, nfw, false);
     upload_groups(c, 1, lb, nbw, false);
+    if (c.nc <= cfdg::sgs_levels_capacity(1)) build_level_chunks(c);
     // forward-sweep flags of every block (device order): 1 when the column's
     // level precedes the row's; and of every device row: 1 in the first level
     std::vector<std::uint8_t> f(c.h_cols.size(), 0), first(z(c.nc), 0);
@@ -387,6 +423,14 @@ void precond_apply(cfdg_ctx& c, const Precond& P, const T* r, T* z, const double
         return;
     }
     const auto b = c.bargs();
+    // Small systems: both sweeps in one launch wherever z fits LDS.  That is also
+    // where it is faster: at the capacity (4,096 rows FP64) the widest levels hold a
+    // few hundred rows, which one workgroup still passes in less than a launch.
+    if (c.nc <= cfdg::sgs_levels_capacity(c.lu_f32)) {
+        cfdg::launch_sgs_levels<T>(c.nc, c.sgs_levels(), c.cols.get(), c.values.get(), c.storage, c.lu_csr.get(),
+                                   c.piv.get(), r, z, c.stream, gate);
+        return;
+    }
     for (int sweep = 0; sweep < 2; ++sweep) {
         const auto& off = c.h_gofs[sweep];
         const std::uint8_t* lower = sweep == 0 ? c.blk_lower.get() : nullptr;

@@ -13,6 +13,7 @@
 #include "capi_internal.hpp"
 #include "cfdg.h"
 #include "kernels.hpp"
+#include "kernels_linalg.hpp"
 #include "kernels_sell.hpp"
 #include "setup.hpp"
 #include "transfer.hpp"
@@ -135,6 +136,17 @@ struct cfdg_ctx {
     // dependency levels of the sequential SGS sweeps (device rows): 0 forward, 1 backward
     std::vector<std::int32_t> h_gofs[2];
     DBuf<int> grows[2];
+    DBuf<int4> level_desc[2];  // the levels' chunks where both sweeps run in one launch (SgsLevels)
+    int level_chunks[2] = {0, 0}, level_count[2] = {0, 0};
+    cfdg::SgsLevels sgs_levels() const {
+        cfdg::SgsLevels l{};
+        for (int k = 0; k < 2; ++k) {
+            l.desc[k] = level_desc[k].get();
+            l.chunks[k] = level_chunks[k];
+            l.levels[k] = level_count[k];
+        }
+        return l;
+    }
     cfdg::Csr ccf_mesh;
     bool have_seq_groups = false;
     // Krylov work vectors; FP32 set for the FP32 form.  Layout of a solve: 5

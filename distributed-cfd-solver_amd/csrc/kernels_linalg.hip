@@ -24,6 +24,7 @@
 #include <cstdint>
 #include <mutex>
 #include <stdexcept>
+#include <string>
 
 #include "kernels.hpp"
 #include "kernels_krylov.hpp"
@@ -158,8 +159,6 @@ __global__ void __launch_bounds__(kBlock) k_spmv(int n, const int* row_ptr, cons
 // five lanes and every lane performs the same 5x5 LU solve
 // (lu_solve_block<5>, bsr_helpers.hpp:325-353) and keeps its component.  The
 // arithmetic and its order per component are those of one thread per row.
-constexpr int kSgsRowsPerWave = 12;
-
 // Component ii of the solution of (LU) x = s with partial pivoting
 // (lu_solve_block<5>, bsr_helpers.hpp:325-353): row swaps, forward then
 // backward substitution over the five values every lane of a row holds.
@@ -246,6 +245,130 @@ __global__ void __launch_bounds__(kBlock) k_sgs_group(const int* rows, int count
         for (int q = 0; q < 5; ++q) pv[q] = p[q];
     }
     z[static_cast<long long>(i) * 5 + ii] = lu_solve_component(s, Lr, pv, ii);
+}
+
+// Both sweeps of z = M^-1 r over the dependency levels in one launch of one
+// workgroup, z in LDS, for systems that fit it.  A level of a small system holds a
+// few dozen rows, so a launch per level (k_sgs_group) is all latency: 5 to 7 us for
+// each of the 2 x 66 levels of a 48 x 16 x 4 mesh, 950 us for M^-1 r.  Here a level
+// costs a barrier, the products of LDS reads and a 5x5 solve; everything that does
+// not depend on z -- blocks, factors, right-hand side -- is in flight before its
+// level begins: the waves take the chunks of twelve rows (kSgsRowsPerWave) in turn,
+// and a wave requests its next chunk when it has finished one.  The barriers wait for
+// LDS alone, so these loads pass them.
+//
+// Arithmetic and order per row are those of k_sgs_group.  The columns of a row
+// ascend in mesh numbering, so its lower blocks come first, and the backward sweep
+// meets them with the forward values: their sum is the forward sweep's, kept in z's
+// device array until the end.
+constexpr int kLevelThreads = 768, kLevelWaves = kLevelThreads / 64;
+constexpr int kLevelBlocks = 3;  // blocks per row requested ahead (a hexahedron's lower or upper ones)
+
+__device__ __forceinline__ void lds_barrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+template <class TS, class TL, class TV>
+struct LevelRow {
+    TV acc, a[kLevelBlocks][5], L[25];
+    int col[kLevelBlocks];
+    std::uint32_t piv;  // as loaded: four of the five
+    std::uint8_t piv4;
+};
+
+template <class TS, class TL, class TV>
+__device__ __forceinline__ void level_fetch(const int4& d, int ii, const int* cols, const TS* values, const TL* lu,
+                                            const std::uint8_t* piv, const TV* rhs, LevelRow<TS, TL, TV>& w) {
+    // without branches, so that the waits behind it can count the loads: what a row
+    // does not have is read from its first block, or from the first row
+#pragma unroll
+    for (int q = 0; q < kLevelBlocks; ++q) {
+        const int k = d.y + (q < d.z ? q : 0);
+        w.col[q] = cols[k];
+        block_row(values, k, ii, w.a[q]);
+    }
+    const int row = d.x < 0 ? 0 : d.x;
+    w.acc = rhs[static_cast<long long>(row) * 5 + ii];
+    const TL* L = lu + static_cast<long long>(row) * 25;
+    const std::uint8_t* p = piv + static_cast<long long>(row) * 5;
+#pragma unroll
+    for (int q = 0; q < 25; ++q) w.L[q] = load_as<TV>(L[q]);
+    __builtin_memcpy(&w.piv, p, 4);
+    w.piv4 = p[4];
+}
+
+template <class TV>
+__device__ __forceinline__ TV level_product(const TV a[5], const TV* zb) {
+    TV tt = 0;
+    tt += a[0] * zb[0];
+    tt += a[1] * zb[1];
+    tt += a[2] * zb[2];
+    tt += a[3] * zb[3];
+    tt += a[4] * zb[4];
+    return tt;
+}
+
+template <class TS, class TL, class TV>
+__global__ void __launch_bounds__(kLevelThreads) k_sgs_levels(int n, SgsLevels lv, const int* cols, const TS* values,
+                                                              const TL* lu, const std::uint8_t* piv, const TV* r,
+                                                              TV* z, const double* gate) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char level_lds[];
+    TV* zl = reinterpret_cast<TV*>(level_lds);
+    if (gate && gate[kKsStatus] != 0.0) return;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int lane = static_cast<int>(threadIdx.x & 63);
+    const int rw = lane / 5, ii = lane - rw * 5;  // lanes 60-63: a thirteenth row, idle
+    const bool on = rw < kSgsRowsPerWave;
+    const int base = rw * 5;
+    for (int sweep = 0; sweep < 2; ++sweep) {
+        const int4* desc = lv.desc[sweep];
+        const int chunks = lv.chunks[sweep], levels = lv.levels[sweep];
+        const TV* rhs = sweep == 0 ? r : z;
+        const auto row_of = [&](int c) {
+            const int last = chunks - 1;
+            return desc[(c < last ? c : last) * kSgsRowsPerWave + (on ? rw : 0)];
+        };
+        int level = 0;
+        if (wave < chunks) {
+            int4 d = row_of(wave), dn = row_of(wave + kLevelWaves);
+            LevelRow<TS, TL, TV> w;
+            level_fetch<TS, TL, TV>(d, ii, cols, values, lu, piv, rhs, w);
+            int at = __builtin_amdgcn_readfirstlane(d.w);
+            for (int c = wave; c < chunks; c += kLevelWaves) {
+                for (; level < at; ++level) lds_barrier();
+                const bool has = on && d.x >= 0;
+                TV acc = 0;
+                if (has) {
+                    acc = w.acc;
+#pragma unroll
+                    for (int q = 0; q < kLevelBlocks; ++q)
+                        if (q < d.z) acc -= level_product(w.a[q], zl + w.col[q] * 5);
+                    for (int q = kLevelBlocks; q < d.z; ++q) {
+                        TV a[5];
+                        block_row(values, d.y + q, ii, a);
+                        acc -= level_product(a, zl + cols[d.y + q] * 5);
+                    }
+                    if (sweep == 0) z[static_cast<long long>(d.x) * 5 + ii] = acc;
+                }
+                TV s[5];
+                for (int q = 0; q < 5; ++q) s[q] = __shfl(acc, (base + q) & 63, 64);
+                int pv[5];
+#pragma unroll
+                for (int q = 0; q < 4; ++q) pv[q] = static_cast<int>((w.piv >> (8 * q)) & 0xffu);
+                pv[4] = w.piv4;
+                if (has) zl[d.x * 5 + ii] = lu_solve_component(s, w.L, pv, ii);
+                d = dn;
+                at = __builtin_amdgcn_readfirstlane(d.w);
+                dn = row_of(c + 2 * kLevelWaves);
+                level_fetch<TS, TL, TV>(d, ii, cols, values, lu, piv, rhs, w);
+            }
+        }
+        for (; level < levels; ++level) lds_barrier();
+        __syncthreads();  // the sums kept in z
+    }
+    for (int e = static_cast<int>(threadIdx.x); e < 5 * n; e += kLevelThreads) z[e] = zl[e];
 }
 
 // p = ((p * beta) + (-beta * omega) v) + r           (bicgstab.cpp:104-109)
@@ -693,6 +816,44 @@ template void launch_sgs_group<double>(const int*, int, const BsrArgs&, const vo
 template void launch_sgs_group<float>(const int*, int, const BsrArgs&, const void*, int, const void*,
                                       const std::uint8_t*, const std::uint8_t*, const float*, float*, hipStream_t,
                                       const double*);
+
+int sgs_levels_capacity(int lu_f32) { return (160 * 1024) / (5 * static_cast<int>(lu_f32 ? sizeof(float) : sizeof(double))); }
+
+template <class TS, class TL, class TV>
+static void launch_sgs_levels_as(int n, const SgsLevels& lv, const int* cols, const void* values, const void* lu,
+                                 const std::uint8_t* piv, const TV* r, TV* z, hipStream_t s, const double* gate) {
+    const std::size_t lds = static_cast<std::size_t>(n) * 5 * sizeof(TV);
+    const auto kernel = k_sgs_levels<TS, TL, TV>;
+    if (lds > 64 * 1024) {
+        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
+        if (e != hipSuccess) throw std::runtime_error(std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
+    }
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kLevelThreads), lds, s, n, lv, cols, static_cast<const TS*>(values),
+                       static_cast<const TL*>(lu), piv, r, z, gate);
+}
+
+template <class TV>
+void launch_sgs_levels(int n, const SgsLevels& lv, const int* cols, const void* values, int storage, const void* lu,
+                       const std::uint8_t* piv, const TV* r, TV* z, hipStream_t s, const double* gate) {
+    if (n <= 0) return;
+    if (n > sgs_levels_capacity(sizeof(TV) == sizeof(float) ? 1 : 0)) throw_bad_combination("SGS levels: too many rows");
+    if constexpr (sizeof(TV) == sizeof(double)) {
+        if (storage != kStoreF64) throw_bad_combination("FP64 SGS needs FP64 blocks");
+        launch_sgs_levels_as<double, double, double>(n, lv, cols, values, lu, piv, r, z, s, gate);
+    } else {
+        if (storage == kStoreF32)
+            launch_sgs_levels_as<float, float, float>(n, lv, cols, values, lu, piv, r, z, s, gate);
+        else if (storage == kStoreBF16)
+            launch_sgs_levels_as<bf16, float, float>(n, lv, cols, values, lu, piv, r, z, s, gate);
+        else
+            launch_sgs_levels_as<double, float, float>(n, lv, cols, values, lu, piv, r, z, s, gate);
+    }
+}
+template void launch_sgs_levels<double>(int, const SgsLevels&, const int*, const void*, int, const void*,
+                                        const std::uint8_t*, const double*, double*, hipStream_t, const double*);
+template void launch_sgs_levels<float>(int, const SgsLevels&, const int*, const void*, int, const void*,
+                                       const std::uint8_t*, const float*, float*, hipStream_t, const double*);
 
 template <class T>
 void launch_update_p(long long n, double beta, double nbo, const T* r, const T* v, T* p, hipStream_t s) {

@@ -53,6 +53,20 @@ template <class TV>
 void launch_sgs_group(const int* rows, int count, const BsrArgs& b, const void* values, int storage, const void* lu,
                       const std::uint8_t* piv, const std::uint8_t* lower, const TV* r, TV* z, hipStream_t s,
                       const double* gate = nullptr);
+// The sweeps' rows over the dependency levels, forward (0) and backward (1, its
+// first level left out), in chunks of twelve rows of one level: device row (-1 past
+// a level's rows), first (0 if none) and number of the blocks the sweep reads, level.
+struct SgsLevels {
+    const int4* desc[2];
+    int chunks[2], levels[2];
+};
+// Rows up to which both sweeps run in one launch (z in the 160 KB of LDS).
+int sgs_levels_capacity(int lu_f32);
+// z = M^-1 r over the dependency levels for such a system, first level included
+template <class TV>
+void launch_sgs_levels(int n, const SgsLevels& lv, const int* cols, const void* values, int storage, const void* lu,
+                       const std::uint8_t* piv, const TV* r, TV* z, hipStream_t s, const double* gate = nullptr);
+constexpr int kSgsRowsPerWave = 12;  // five lanes a row
 template <class T>
 void launch_update_p(long long n, double beta, double nbo, const T* r, const T* v, T* p, hipStream_t s);
 template <class T>
