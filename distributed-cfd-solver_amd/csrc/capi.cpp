@@ -274,69 +274,62 @@ void use_layout(cfdg_ctx& c, bool sliced) {
     c.vectors_sliced = sliced;
 }
 
-void eval_residual(cfdg_ctx& c) {
+// in_step: the caller's next launch stamps the end of the stage, and waits later.
+void eval_residual(cfdg_ctx& c, bool in_step) {
     c.have_features = false;
     const auto m = c.margs();
     const auto f = c.fargs();
-    hip_check(hipEventRecord(c.ev[0], c.stream), "event");
-    cfdg::launch_primitives(m, f, c.nargs, c.stream);
-    cfdg::launch_ghosts(m, f, c.nargs, c.bcs, c.stream);
+    cfdg::launch_primitives(m, f, c.nargs, c.bcs, c.stream);
     // module ghosts, then density / nu_tilde / eddy viscosity (solver.hpp:195-204)
     if (c.sa_on()) {
         cfdg::launch_sa_prepare(m, f, c.nargs, c.sargs(), c.stream);
         c.sa_evaluated = true;
     }
-    hip_check(hipEventRecord(c.ev[1], c.stream), "event");
     const bool need_grad = c.nargs.muscl || c.nargs.viscous;
     if (need_grad) {
         const cfdg::SaArgs sa = c.sargs();
         const bool sa_done = cfdg::launch_gradient_limiter(m, f, c.nargs, c.stream, c.sa_on() ? &sa : nullptr);
-        hip_check(hipEventRecord(c.ev[2], c.stream), "event");
         cfdg::launch_ghost_gradients(m, f, c.nargs, c.bcs, c.stream);
         if (c.sa_on() && !sa_done) cfdg::launch_sa_gradient(m, f, c.nargs, sa, c.stream);
-    } else {
-        hip_check(hipEventRecord(c.ev[2], c.stream), "event");
     }
-    hip_check(hipEventRecord(c.ev[3], c.stream), "event");
     cfdg::launch_flux(m, f, c.nargs, c.stream);
     // module face sweep on the recorded mass flux, then its sources (solver.hpp:233-241)
     if (c.sa_on()) cfdg::launch_sa_residual(m, f, c.nargs, c.sargs(), c.stream);
     // BDF pseudo-source of dual time stepping (solver.hpp:243-246)
     if (c.bdf_order > 0)
         cfdg::launch_unsteady_source(m, f, c.bdf_cur, 1.0 / c.phys_dt, c.Un.get(), c.Unm1.get(), c.stream);
-    hip_check(hipEventRecord(c.ev[4], c.stream), "event");
-    c.check_launch();
-    c.sync();
-    float ms = 0.f;
-    for (int k = 0; k < 4; ++k) {
-        hip_check(hipEventElapsedTime(&ms, c.ev[k], c.ev[k + 1]), "elapsed");
-        c.stage_ms[k] = ms;
+    if (!in_step) {
+        cfdg::launch_stamp(c.stamp.get(), cfdg::kStampFluxEnd, -1, c.stream);
+        c.finish();
     }
+    c.check_launch();
+    c.timed_residual = true;
+    c.timed_gradients = need_grad;
     c.have_residual = true;
 }
 
-void compute_dt(cfdg_ctx& c) {
+void compute_dt(cfdg_ctx& c, bool in_step) {
     if (!c.have_residual) throw CfdgError(CFDG_ERR_STATE, "compute_dt before eval_residual");
     const double unsteady = (c.bdf_order > 0) ? ((c.bdf_cur == 2) ? 1.5 : 1.0) / c.phys_dt : 0.0;
-    cfdg::launch_dt(c.margs(), c.fargs(), c.lam.get(), c.num.cfl, unsteady, c.dt.get(), c.alpha.get(), c.stream);
+    cfdg::launch_dt(c.margs(), c.fargs(), c.lam.get(), c.num.cfl, unsteady, c.dt.get(), c.alpha.get(), in_step,
+                    c.stream);
+    if (!in_step) c.finish();
     c.check_launch();
-    c.sync();
     c.have_dt = true;
 }
 
-void assemble_jacobian(cfdg_ctx& c) {
+void assemble_jacobian(cfdg_ctx& c, bool in_step) {
     if (!c.have_dt) throw CfdgError(CFDG_ERR_STATE, "assemble_jacobian before compute_dt");
-    hip_check(hipEventRecord(c.ev[5], c.stream), "event");
     cfdg::launch_jacobian(c.margs(), c.fargs(), c.nargs, c.sellargs(), c.alpha.get(), c.sell_off.get(),
                           c.sell_diag.get(), c.storage, c.stream);
     c.have_csr = false;
-    hip_check(hipEventRecord(c.ev[6], c.stream), "event");
+    if (!in_step) {
+        cfdg::launch_stamp(c.stamp.get(), cfdg::kStampJacobianEnd, -1, c.stream);
+        c.finish();
+    }
     c.check_launch();
-    c.sync();
     c.have_jacobian = true;
-    float ms = 0.f;
-    hip_check(hipEventElapsedTime(&ms, c.ev[5], c.ev[6]), "elapsed");
-    c.stage_ms[4] = ms;
+    c.timed_jacobian = true;
 }
 
 void require_jacobian(const cfdg_ctx& c) {
@@ -345,19 +338,15 @@ void require_jacobian(const cfdg_ctx& c) {
                         "no block values in the current storage: cfdg_assemble_jacobian or cfdg_set_bsr_values first");
 }
 
-void fetch_dots(cfdg_ctx& c, int n) {
-    c.d2h(c.h_dots, c.dots.get(), static_cast<std::size_t>(n));
-    c.sync();
-}
-
 template <class T>
 double dot_device(cfdg_ctx& c, long long n, const T* a, const T* b) {
     cfdg::DotPairsT<T> pr{};
     pr.a[0] = a;
     pr.b[0] = b;
-    cfdg::launch_dots(n, 1, pr, c.partial.get(), c.dots.get(), c.stream);
-    fetch_dots(c, 1);
-    return c.h_dots[0];
+    cfdg::launch_dots(n, 1, pr, c.partial.get(), c.dots.get(), c.stream, c.publish());
+    c.check_launch();
+    c.wait();
+    return c.blk->v[0];
 }
 
 struct Precond {
@@ -444,11 +433,13 @@ void precond_apply(cfdg_ctx& c, const Precond& P, const T* r, T* z, const double
 // The singular-pivot flag is read with the solve's result (precond_check):
 // a zero pivot makes the solve produce non-finite values, and the error names
 // the row either way.
-void precond_setup(cfdg_ctx& c, const Precond& P) {
+// singular_clear: the flag is zero already.
+void precond_setup(cfdg_ctx& c, const Precond& P, bool singular_clear = false) {
     use_layout(c, P.sliced());
     if (!P.sliced()) ensure_csr(c);
+    c.singular_known = false;
     if (P.kind != CFDG_PRECOND_SGS) return;
-    c.singular.zero(c.stream);
+    if (!singular_clear) c.singular.zero(c.stream);
     if (P.sliced()) {
         cfdg::launch_sell_lu(c.sellargs(), c.sellmatrix(), c.lu.get(), c.lu_f32, c.sell_piv.get(), c.singular.get(),
                              c.stream);
@@ -463,8 +454,12 @@ void precond_setup(cfdg_ctx& c, const Precond& P) {
 void precond_check(cfdg_ctx& c, const Precond& P) {
     if (P.kind != CFDG_PRECOND_SGS) return;
     int sing = 0;
-    c.d2h(&sing, c.singular.get(), 1);
-    c.sync();
+    if (c.singular_known) {
+        sing = static_cast<int>(c.blk->v[cfdg::kKsCount + 5]);
+    } else {
+        c.d2h(&sing, c.singular.get(), 1);
+        c.sync();
+    }
     if (sing != 0)
         throw CfdgError(CFDG_ERR_SINGULAR,
                         "SGS: singular diagonal block at row " + std::to_string(c.new2old[z(sing - 1)]));
@@ -475,12 +470,14 @@ void precond_check(cfdg_ctx& c, const Precond& P) {
 // defect correction).  x holds the initial guess on entry and the solution on
 // exit.  Scalars and dot products are FP64.  The multicolour order runs in the
 // reduced form (kernels_reduced.hip), with two exceptions: one colour only, and
-// reduce = false.  A solve whose s vanishes exactly is repeated so, because the
+// reduce = false.  parts: the number of partial sums that the kernel which formed bvec
+// left for launch_bicg_start, 0 for none.  A solve whose s vanishes exactly is repeated so, because the
 // reference ends there as broken down unless the rounding of its product, which
 // the reduced form does not have, leaves a remainder to go on with.
 template <class T>
 cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& P, const cfdg::RedVecs<T>& w, T* x,
-                          const T* bvec, bool zero_fallback = false, bool x_zero = false, bool reduce = true) {
+                          const T* bvec, bool zero_fallback = false, bool x_zero = false, int parts = 0,
+                          bool reduce = true) {
     const long long N = vector_size(c, P);
     const std::size_t bytes = static_cast<std::size_t>(N) * sizeof(T);
     cfdg_iter_result res{CFDG_MAX_ITERATIONS, 0, 0.0, 0.0};
@@ -496,38 +493,37 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
     double* const kb[2] = {c.ks.get(), c.ks.get() + cfdg::kKsCount};
     int cur = 0;
     double* ks = kb[0];
-    double* h = c.h_ks;
+    double h[cfdg::kKsCount];
     // r = b - A x (r = b for a zero guess), norms, tolerance and status on the
     // device: no host round trip before the first batch of iterations
-    {
+    const T* r = bvec;
+    if (!x_zero) {
+        spmv_stored<T>(c, P, x, w.v);
+        cfdg::launch_axpy_copy<T>(N, bvec, -1.0, w.v, w.r, c.stream);
+        r = w.r;
+    }
+    if (reduced) {
+        double* const part = c.partial.get();
+        if (parts == 0) parts = cfdg::launch_sell_squares<T>(b, bvec, cs[1], part, c.stream);
+        if (!x_zero) cfdg::launch_sell_squares<T>(b, r, cs[1], part + cfdg::kSquares, c.stream);
+        // FP32: the norms are the outer right-hand side's, not this one's
+        cfdg::launch_bicg_start(parts, part, !x_zero, sizeof(T) == sizeof(double) ? c.norms.get() : nullptr, ks,
+                                zero_fallback, lp.abs_tol, lp.rel_tol, lp.max_iter, cfdg::Publish{}, c.stream);
+    } else {
         cfdg::DotPairsT<T> pr{};
-        int nd = 0;
-        const auto pair = [&](const T* a, long long n) {
-            pr.a[nd] = a;
-            pr.b[nd] = a;
-            pr.n[nd++] = n;
-        };
-        const T* r = bvec;
-        pair(bvec, N);
-        if (!x_zero) {
-            spmv_stored<T>(c, P, x, w.v);
-            cfdg::launch_axpy_copy<T>(N, bvec, -1.0, w.v, w.r, c.stream);
-            r = w.r;
-            pair(r, N);
-        }
-        if (reduced) pair(r, skip);
-        if (reduced && !x_zero) pair(bvec, skip);
-        cfdg::launch_dots(N, nd, pr, c.partial.get(), c.dots.get(), c.stream);
-        cfdg::launch_bicg_init(ks, c.dots.get(), x_zero ? 1 : 0, zero_fallback ? 1 : 0, reduced ? 1 : 0, lp.abs_tol,
-                               lp.rel_tol, lp.max_iter, c.stream);
-        if (zero_fallback) cfdg::launch_bicg_reject<T>(N, ks, bvec, x, w.r, c.stream);
-        if (reduced) {
-            cfdg::launch_red_start<T>(b, m, cs, r, w, ks, c.stream);
-        } else {
-            if (x_zero) hip_check(hipMemcpyAsync(w.r, bvec, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
-            hip_check(hipMemcpyAsync(w.r0, w.r, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
-            hip_check(hipMemsetAsync(w.v, 0, bytes, c.stream), "memset");
-        }
+        pr.a[0] = pr.b[0] = bvec;
+        pr.a[1] = pr.b[1] = r;
+        cfdg::launch_dots(N, x_zero ? 1 : 2, pr, c.partial.get(), c.dots.get(), c.stream);
+        cfdg::launch_bicg_init(ks, c.dots.get(), x_zero ? 1 : 0, zero_fallback ? 1 : 0, lp.abs_tol, lp.rel_tol,
+                               lp.max_iter, c.stream);
+    }
+    if (zero_fallback) cfdg::launch_bicg_reject<T>(N, ks, bvec, x, w.r, c.stream);
+    if (reduced) {
+        cfdg::launch_red_start<T>(b, m, cs, r, w, ks, c.stream);
+    } else {
+        if (x_zero) hip_check(hipMemcpyAsync(w.r, bvec, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
+        hip_check(hipMemcpyAsync(w.r0, w.r, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
+        hip_check(hipMemsetAsync(w.v, 0, bytes, c.stream), "memset");
     }
     // The recurrence runs on the device: scalars in the state block ks,
     // iterations enqueued in batches and the state read back once per
@@ -593,19 +589,22 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
             }
             cfdg::launch_update_xr_g<T>(N - skip, ks, w.ph + skip, w.sh + skip, w.s + skip, w.t + skip, x + skip,
                                         w.r + skip, c.stream);
-            if (enq % 32 == 0) {  // true residual norm every 32 iterations
+            const bool true_norm = enq % 32 == 0;  // of the residual, every 32 iterations
+            if (true_norm) {
                 cfdg::DotPairsT<T> pr{};
                 pr.a[0] = w.r + skip;
                 pr.b[0] = w.r + skip;
                 cfdg::launch_dots_step(N - skip, 1, pr, c.partial.get(), rr, ks, cfdg::kStepPost, c.stream);
-            } else {
-                cfdg::launch_bicg_post(ks, c.stream);
             }
+            if (!true_norm || !next_in_batch)
+                cfdg::launch_bicg_post(ks, !true_norm, c.norms.get(), c.singular.get(),
+                                       next_in_batch ? cfdg::Publish{} : c.publish(), c.stream);
         }
         c.check_launch();
+        c.wait();
         ks = kb[cur];
-        c.d2h(h, ks, cfdg::kKsCount);
-        c.sync();
+        std::copy(c.blk->v, c.blk->v + cfdg::kKsCount, h);
+        c.norms_known = c.singular_known = true;
         if (h[cfdg::kKsStatus] != 0.0 || enq > lp.max_iter) break;
         batch = 2;
     }
@@ -632,7 +631,7 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
         cfdg_linparams rest = lp;
         rest.max_iter = lp.max_iter - (it - 1);
         const cfdg_iter_result r2 =
-            bicgstab<T>(c, rest, P, w, x, bvec, false, updates == 0.0 && (x_zero || rejected), false);
+            bicgstab<T>(c, rest, P, w, x, bvec, false, updates == 0.0 && (x_zero || rejected), 0, false);
         res.status = r2.status;
         rnorm = r2.final_residual;
         it += r2.iterations - 1;
@@ -647,33 +646,45 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
 // x (FP64, initial guess on entry), b (FP64).  Every pass forms r = b - A x in
 // FP64 arithmetic over the stored blocks and solves A e = r in FP32 from e = 0.
 cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& P, double* x,
-                                   const double* bvec, bool zero_fallback = false, bool x_zero = false) {
+                                   const double* bvec, bool zero_fallback = false, bool x_zero = false,
+                                   int parts = 0) {
     const long long N = vector_size(c, P);
     cfdg_iter_result res{CFDG_MAX_ITERATIONS, 0, 0.0, 0.0};
+    const double* r = c.r.get();  // the outer residual
     const auto outer_residual = [&]() {
         spmv_stored<double>(c, P, x, c.v.get());
         cfdg::launch_axpy_copy<double>(N, bvec, -1.0, c.v.get(), c.r.get(), c.stream);
         return std::sqrt(dot_device<double>(c, N, c.r.get(), c.r.get()));
     };
-    // ||b|| and the first outer residual in one reduction (r = b for a zero guess)
+    // ||b|| and the first outer residual's norm (r = b for a zero guess)
     double bnorm = 0.0, rnorm = 0.0;
     {
-        cfdg::DotPairsT<double> pr{};
-        pr.a[0] = bvec;
-        pr.b[0] = bvec;
         if (x_zero) {
-            hip_check(hipMemcpyAsync(c.r.get(), bvec, static_cast<std::size_t>(N) * sizeof(double),
-                                     hipMemcpyDeviceToDevice, c.stream), "copy");
+            r = bvec;
         } else {
             spmv_stored<double>(c, P, x, c.v.get());
             cfdg::launch_axpy_copy<double>(N, bvec, -1.0, c.v.get(), c.r.get(), c.stream);
-            pr.a[1] = c.r.get();
-            pr.b[1] = c.r.get();
         }
-        cfdg::launch_dots(N, x_zero ? 1 : 2, pr, c.partial.get(), c.dots.get(), c.stream);
-        fetch_dots(c, x_zero ? 1 : 2);
-        bnorm = std::sqrt(c.h_dots[0]);
-        rnorm = x_zero ? bnorm : std::sqrt(c.h_dots[1]);
+        const cfdg::Publish pub = c.publish();
+        if (P.sliced()) {
+            const auto b = c.sellargs();
+            double* const part = c.partial.get();
+            const bool rhs = parts > 0;  // an implicit step's: its norms
+            if (!rhs) parts = cfdg::launch_sell_squares<double>(b, bvec, 0, part, c.stream);
+            if (!x_zero) cfdg::launch_sell_squares<double>(b, r, 0, part + cfdg::kSquares, c.stream);
+            cfdg::launch_bicg_start(parts, part, !x_zero, rhs ? c.norms.get() : nullptr, nullptr, false, 0.0, 0.0, 0,
+                                    pub, c.stream);
+            c.norms_known = rhs;
+        } else {
+            cfdg::DotPairsT<double> pr{};
+            pr.a[0] = pr.b[0] = bvec;
+            pr.a[1] = pr.b[1] = r;
+            cfdg::launch_dots(N, 2, pr, c.partial.get(), c.dots.get(), c.stream, pub);
+        }
+        c.check_launch();
+        c.wait();
+        bnorm = std::sqrt(c.blk->v[0]);
+        rnorm = std::sqrt(c.blk->v[1]);
     }
     if (zero_fallback) {
         if (!(rnorm <= bnorm)) {
@@ -703,8 +714,14 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
             res.status = CFDG_MAX_ITERATIONS;
             break;
         }
-        cfdg::launch_cast_f64_to_f32(N, c.r.get(), c.f32.b.get(), c.stream);
-        c.f32.x.zero(c.stream);
+        int inner_parts = 0;
+        if (P.sliced()) {
+            inner_parts = cfdg::launch_sell_inner_rhs(c.sellargs(), r, c.f32.b.get(), c.f32.x.get(),
+                                                      c.sell.colour_slice[1], c.partial.get(), c.stream);
+        } else {
+            cfdg::launch_cast_f64_to_f32(N, r, c.f32.b.get(), c.stream);
+            c.f32.x.zero(c.stream);
+        }
         cfdg_linparams in = lp;
         // stop the inner solve at max(inner_rel_tol ||r||, 0.9 tol): no further
         // than the caller's tolerance needs (the FP64 outer residual of the
@@ -713,17 +730,17 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
         in.rel_tol = c.prec.inner_rel_tol;
         in.abs_tol = 0.9 * tol;
         in.max_iter = lp.max_iter - total;
-        const cfdg_iter_result ir = bicgstab<float>(c, in, P, w, c.f32.x.get(), c.f32.b.get(), false, true);
+        const cfdg_iter_result ir = bicgstab<float>(c, in, P, w, c.f32.x.get(), c.f32.b.get(), false, true, inner_parts);
         total += ir.iterations;
         if (ir.iterations == 0 && ir.status != CFDG_CONVERGED) {
             res.status = CFDG_DIVERGED;
             break;
         }
         cfdg::launch_add_f32(N, c.f32.x.get(), x, c.stream);
+        r = c.r.get();
         rnorm = outer_residual();
     }
     c.check_launch();
-    c.sync();
     res.iterations = total;
     res.final_residual = rnorm;
     return res;
@@ -755,9 +772,10 @@ void state_planes(cfdg_ctx& c, std::int64_t ld, F&& copy) {
 }
 
 // The solution stays in c.xs (multicolour SGS) or c.x; returns which Krylov
-// layout the solve used.
+// layout the solve used.  in_step: directly after the Jacobian; the caller's next
+// launch stamps the end, and waits later.
 Precond linear_solve(cfdg_ctx& c, const cfdg_linparams& lp, const double* hb, const double* hx0, double* hx,
-                     cfdg_iter_result* out) {
+                     cfdg_iter_result* out, bool in_step) {
     if (lp.preconditioner != CFDG_PRECOND_NONE && lp.preconditioner != CFDG_PRECOND_SGS)
         throw CfdgError(CFDG_ERR_CONFIG, "unknown preconditioner");
     if (lp.sgs_order != CFDG_SGS_MULTICOLOUR && lp.sgs_order != CFDG_SGS_SEQUENTIAL)
@@ -780,14 +798,21 @@ Precond linear_solve(cfdg_ctx& c, const cfdg_linparams& lp, const double* hb, co
         c.h2d(dst, d.data(), n5);
         c.sync();
     };
+    const int first = c.sell.colour_slice.size() > 2 ? c.sell.colour_slice[1] : 0;
+    int parts = 0;
+    c.norms_known = false;
     if (hb) {
         upload(hb, b);
+        cfdg::launch_stamp(c.stamp.get(), cfdg::kStampLinear, -1, c.stream);
     } else {
         if (!c.have_residual) throw CfdgError(CFDG_ERR_STATE, "implicit right-hand side needs a residual");
-        if (sliced)
-            cfdg::launch_sell_rhs(c.sellargs(), c.nc, c.res.get(), b, c.stream);
-        else
-            cfdg::launch_rhs(c.nc, c.nc, c.res.get(), b, c.stream);
+        if (sliced) {
+            parts = cfdg::launch_sell_rhs(c.sellargs(), c.nc, c.res.get(), b, x, first, c.partial.get(),
+                                          c.singular.get(), c.stamp.get(), in_step, c.stream);
+        } else {
+            cfdg::launch_stamp(c.stamp.get(), cfdg::kStampLinear, in_step ? cfdg::kStampJacobianEnd : -1, c.stream);
+            cfdg::launch_rhs(c.nc, c.nc, c.res.get(), b, c.partial.get(), c.norms.get(), c.stream);
+        }
     }
     bool learned = false, x_zero = false;
     if (hx0) {
@@ -796,18 +821,23 @@ Precond linear_solve(cfdg_ctx& c, const cfdg_linparams& lp, const double* hb, co
         learned = cfdg::gnn_warm_guess(c, c.x.get());
         if (sliced) cfdg::launch_sell_gather(c.sellargs(), nullptr, c.x.get(), x, c.stream);
     } else {
-        hip_check(hipMemsetAsync(x, 0, static_cast<std::size_t>(vector_size(c, P)) * sizeof(double), c.stream),
-                  "memset");
+        // the sliced right-hand side cleared x as well
+        if (hb || !sliced)
+            hip_check(hipMemsetAsync(x, 0, static_cast<std::size_t>(vector_size(c, P)) * sizeof(double), c.stream),
+                      "memset");
         x_zero = true;
     }
-    hip_check(hipEventRecord(c.ev[5], c.stream), "event");
-    precond_setup(c, P);
+    if (parts > 0 && first == 0 && c.prec.krylov != CFDG_PREC_FP32) {  // one colour: no launch_bicg_start to add them
+        cfdg::launch_reduce_partials(parts, 5, c.partial.get(), c.norms.get(), cfdg::Publish{}, c.stream);
+        parts = 0;
+    }
+    precond_setup(c, P, !hb && sliced);
     const cfdg_iter_result r = (c.prec.krylov == CFDG_PREC_FP32)
-                                   ? defect_correction(c, lp, P, x, b, learned, x_zero)
-                                   : bicgstab<double>(c, lp, P, kvecs64(c), x, b, learned, x_zero);
-    hip_check(hipEventRecord(c.ev[6], c.stream), "event");
-    c.sync();
+                                   ? defect_correction(c, lp, P, x, b, learned, x_zero, parts)
+                                   : bicgstab<double>(c, lp, P, kvecs64(c), x, b, learned, x_zero, parts);
     precond_check(c, P);
+    c.timed_linear = true;
+    if (!in_step) cfdg::launch_stamp(c.stamp.get(), cfdg::kStampLinearEnd, -1, c.stream);
     if (hx && sliced) {
         download_sliced(c, x, hx);
     } else if (hx) {
@@ -816,19 +846,22 @@ Precond linear_solve(cfdg_ctx& c, const cfdg_linparams& lp, const double* hb, co
         c.sync();
         c.vec_to_mesh(d, hx);
     }
-    float ms = 0.f;
-    hip_check(hipEventElapsedTime(&ms, c.ev[5], c.ev[6]), "elapsed");
-    c.stage_ms[5] = ms;
     if (out) *out = r;
     return P;
 }
 
+// l2 from the sums of the squared residuals (solver.hpp:740-756)
+void norms_of(const cfdg_ctx& c, const double* sums, double l2[5]) {
+    const double scale = 1.0 / static_cast<double>(std::max(c.nc, 1));
+    for (int v = 0; v < 5; ++v) l2[v] = std::sqrt(sums[v] * scale);
+}
+
 void residual_norms(cfdg_ctx& c, double l2[5]) {
     if (!c.have_residual) throw CfdgError(CFDG_ERR_STATE, "residual norms before eval_residual");
-    cfdg::launch_res_sq(c.nc, c.nc, c.res.get(), c.partial.get(), c.dots.get(), c.stream);
-    fetch_dots(c, 5);
-    const double scale = 1.0 / static_cast<double>(std::max(c.nc, 1));
-    for (int v = 0; v < 5; ++v) l2[v] = std::sqrt(c.h_dots[v] * scale);
+    cfdg::launch_res_sq(c.nc, c.nc, c.res.get(), c.partial.get(), c.dots.get(), c.publish(), c.stream);
+    c.check_launch();
+    c.wait();
+    norms_of(c, c.blk->v, l2);
 }
 
 void check_numerics(const cfdg_numerics* num) {
@@ -876,8 +909,9 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
     if (ndev < 1) throw CfdgError(CFDG_ERR_HIP, "no HIP device");
     hip_check(hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking), "hipStreamCreate");
     for (auto& e : c.ev) hip_check(hipEventCreate(&e), "hipEventCreate");
-    hip_check(hipHostMalloc(reinterpret_cast<void**>(&c.h_dots), 8 * sizeof(double)), "hipHostMalloc");
-    hip_check(hipHostMalloc(reinterpret_cast<void**>(&c.h_ks), cfdg::kKsCount * sizeof(double)), "hipHostMalloc");
+    hip_check(hipHostMalloc(reinterpret_cast<void**>(&c.blk), sizeof(cfdg::HostBlock)), "hipHostMalloc");
+    *c.blk = cfdg::HostBlock{};
+    hip_check(hipHostGetDevicePointer(reinterpret_cast<void**>(&c.blk_dev), c.blk, 0), "hipHostGetDevicePointer");
 
     c.num = *num;
     c.nc = m.n_cells;
@@ -1115,8 +1149,13 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
         v->alloc(v == &c.b || v == &c.x ? 5 * ncs : c.vector_alloc());
         v->zero(s);
     }
-    c.partial.alloc(static_cast<std::size_t>(cfdg::kMaxPartials) * 5);
+    c.partial.alloc(2 * static_cast<std::size_t>(cfdg::kSquares));
     c.dots.alloc(8);
+    c.norms.alloc(5);
+    c.norms.zero(s);
+    c.stamp.alloc(cfdg::kStampCount);
+    c.stamp.zero(s);
+    c.singular.zero(s);
     c.ks.alloc(2 * cfdg::kKsCount);
     c.sync();
 }
@@ -1124,28 +1163,35 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
 // BackwardEuler::advance (implicit_euler.hpp:34-76): residual, dt, Jacobian,
 // (alpha I + J) du = -R, U <- U + du; the step proceeds whatever the linear
 // solver's status (implicit_euler.hpp:45-47).  out->l2 = norms of R(U^n).
+// The host waits for the linear solve only; the rest is enqueued (the caller waits).
 void implicit_step(cfdg_ctx& c, const cfdg_linparams& lp, cfdg_step_result* out) {
-    eval_residual(c);
-    compute_dt(c);
+    eval_residual(c, true);
+    compute_dt(c, true);
     cfdg::gnn_step_features(c);
-    assemble_jacobian(c);
+    assemble_jacobian(c, true);
     cfdg_iter_result lr{};
-    const bool sliced = linear_solve(c, lp, nullptr, nullptr, nullptr, &lr).sliced();
-    double l2[5];
-    residual_norms(c, l2);
-    if (sliced)
-        cfdg::launch_sell_state_update(c.sellargs(), c.nc, c.xs.get(), c.U.get(), c.x.get(), c.stream);
-    else
+    const bool sliced = linear_solve(c, lp, nullptr, nullptr, nullptr, &lr, true).sliced();
+    double sums[5];
+    if (c.norms_known) {
+        std::copy(c.blk->v + cfdg::kKsCount, c.blk->v + cfdg::kKsCount + 5, sums);
+    } else {
+        c.d2h(sums, c.norms.get(), 5);
+        c.sync();
+    }
+    if (sliced) {
+        cfdg::launch_sell_state_update(c.sellargs(), c.nc, c.xs.get(), c.U.get(), c.x.get(), c.stamp.get(), c.stream);
+    } else {
+        cfdg::launch_stamp(c.stamp.get(), cfdg::kStampLinearEnd, -1, c.stream);
         cfdg::launch_state_update(c.nc, c.nc, c.x.get(), c.U.get(), c.stream);
+    }
     // module block: copied (implicit_euler.hpp:64-72) or point-implicit, then clamped
     if (c.sa_on())
         cfdg::launch_sa_update(c.nc, c.turb.update == CFDG_TURB_POINT_IMPLICIT, c.alpha.get(), c.sargs(), c.stream);
     c.check_launch();
-    c.sync();
     c.have_residual = false;
     c.have_dt = false;
     c.have_prev_du = true;
-    for (int v = 0; v < 5; ++v) out->l2[v] = l2[v];
+    norms_of(c, sums, out->l2);
     out->linear = lr;
 }
 
@@ -1293,7 +1339,7 @@ int cfdg_init_uniform(cfdg_ctx* c, double rho, const double vel[3], double p) {
 
 int cfdg_eval_residual(cfdg_ctx* c) {
     return guarded(c, [&] {
-        eval_residual(*c);
+        eval_residual(*c, false);
         c->have_dt = false;
     });
 }
@@ -1348,7 +1394,7 @@ int cfdg_residual_norms(cfdg_ctx* c, double l2[5]) {
     });
 }
 
-int cfdg_compute_dt(cfdg_ctx* c) { return guarded(c, [&] { compute_dt(*c); }); }
+int cfdg_compute_dt(cfdg_ctx* c) { return guarded(c, [&] { compute_dt(*c, false); }); }
 
 int cfdg_get_dt(cfdg_ctx* c, double* dt, double* alpha) {
     return guarded(c, [&] {
@@ -1363,7 +1409,7 @@ int cfdg_get_dt(cfdg_ctx* c, double* dt, double* alpha) {
     });
 }
 
-int cfdg_assemble_jacobian(cfdg_ctx* c) { return guarded(c, [&] { assemble_jacobian(*c); }); }
+int cfdg_assemble_jacobian(cfdg_ctx* c) { return guarded(c, [&] { assemble_jacobian(*c, false); }); }
 
 int cfdg_get_bsr_pattern(cfdg_ctx* c, int32_t* row_ptr, int32_t* cols, int32_t* diag_idx) {
     return guarded(c, [&] {
@@ -1407,7 +1453,7 @@ int cfdg_linear_solve(cfdg_ctx* c, const cfdg_linparams* lp, const double* b, co
                       cfdg_iter_result* res) {
     return guarded(c, [&] {
         if (!lp) throw CfdgError(CFDG_ERR_ARG, "null linear parameters");
-        if (linear_solve(*c, *lp, b, x0, x, res).sliced())
+        if (linear_solve(*c, *lp, b, x0, x, res, false).sliced())
             cfdg::launch_sell_scatter(c->sellargs(), nullptr, c->xs.get(), c->x.get(), c->stream);
         c->sync();
         c->have_prev_du = false;
@@ -1510,6 +1556,7 @@ int cfdg_implicit_step(cfdg_ctx* c, const cfdg_linparams* lp, cfdg_step_result* 
         if (!lp) throw CfdgError(CFDG_ERR_ARG, "null linear parameters");
         cfdg_step_result st{};
         implicit_step(*c, *lp, &st);
+        c->finish();
         if (out) *out = st;
     });
 }
@@ -1518,15 +1565,15 @@ int cfdg_explicit_step(cfdg_ctx* c, cfdg_step_result* out) {
     return guarded(c, [&] {
         if (c->sa_on()) throw CfdgError(CFDG_ERR_CONFIG, "explicit stepping with the turbulence module is not supported");
         if (c->bdf_order > 0) throw CfdgError(CFDG_ERR_STATE, "explicit stepping in dual time is not supported");
-        eval_residual(*c);
-        cfdg::launch_dt_explicit(c->margs(), c->fargs(), c->lam.get(), c->num.cfl, c->dt.get(), c->alpha.get(),
-                                 c->stream);
+        eval_residual(*c, true);
+        const int nb = cfdg::launch_explicit_step(c->margs(), c->fargs(), c->lam.get(), c->num.cfl, c->dt.get(),
+                                                  c->alpha.get(), c->U.get(), c->partial.get(), c->stream);
         c->have_dt = false;  // alpha holds the explicit dt / V, not the implicit diagonal shift
-        double l2[5];
-        residual_norms(*c, l2);
-        cfdg::launch_explicit_update(c->margs(), c->fargs(), c->alpha.get(), c->U.get(), c->stream);
+        cfdg::launch_reduce_partials(nb, 5, c->partial.get(), c->dots.get(), c->publish(), c->stream);
         c->check_launch();
-        c->sync();
+        c->wait();
+        double l2[5];
+        norms_of(*c, c->blk->v, l2);
         c->have_residual = false;
         if (out) {
             *out = cfdg_step_result{};
@@ -1596,8 +1643,8 @@ int cfdg_run_unsteady(cfdg_ctx* c, const cfdg_linparams* lp, int64_t steps, int6
             if (c->bdf_order == 2) c->Unm1.swap(c->Un);
             hip_check(hipMemcpyAsync(c->Un.get(), c->U.get(), n * sizeof(double), hipMemcpyDeviceToDevice, c->stream),
                       "copy");
-            c->sync();
         }
+        c->finish();
     });
 }
 
@@ -1797,6 +1844,7 @@ int cfdg_run_steady(cfdg_ctx* c, const cfdg_linparams* lp, const cfdg_steady_par
                 break;
             }
         }
+        c->finish();
         out->seconds = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();
     });
 }
@@ -1804,7 +1852,22 @@ int cfdg_run_steady(cfdg_ctx* c, const cfdg_linparams* lp, const cfdg_steady_par
 int cfdg_stage_times(cfdg_ctx* c, double ms[6]) {
     return guarded(c, [&] {
         if (!ms) throw CfdgError(CFDG_ERR_ARG, "null output");
-        for (int i = 0; i < 6; ++i) ms[i] = c->stage_ms[i];
+        int device = 0, khz = 0;
+        hip_check(hipGetDevice(&device), "hipGetDevice");
+        hip_check(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device), "hipDeviceGetAttribute");
+        unsigned long long t[cfdg::kStampCount];
+        c->d2h(t, c->stamp.get(), cfdg::kStampCount);
+        c->sync();
+        const auto span = [&](bool timed, int a, int b) {
+            return timed && t[b] > t[a] ? static_cast<double>(t[b] - t[a]) / khz : 0.0;
+        };
+        const bool r = c->timed_residual, g = r && c->timed_gradients;
+        ms[0] = span(r, cfdg::kStampPrimitives, g ? cfdg::kStampGradients : cfdg::kStampFlux);
+        ms[1] = span(g, cfdg::kStampGradients, cfdg::kStampGhostGradients);
+        ms[2] = span(g, cfdg::kStampGhostGradients, cfdg::kStampFlux);
+        ms[3] = span(r, cfdg::kStampFlux, cfdg::kStampFluxEnd);
+        ms[4] = span(c->timed_jacobian, cfdg::kStampJacobian, cfdg::kStampJacobianEnd);
+        ms[5] = span(c->timed_linear, cfdg::kStampLinear, cfdg::kStampLinearEnd);
     });
 }
 
@@ -1814,13 +1877,13 @@ int cfdg_time_flux_kernel(cfdg_ctx* c, int32_t reps, double* ms_per_launch) {
         if (!c->have_residual) throw CfdgError(CFDG_ERR_STATE, "time_flux_kernel needs an evaluated residual");
         const auto m = c->margs();
         const auto f = c->fargs();
-        hip_check(hipEventRecord(c->ev[6], c->stream), "event");
+        hip_check(hipEventRecord(c->ev[0], c->stream), "event");
         for (int i = 0; i < reps; ++i) cfdg::launch_flux(m, f, c->nargs, c->stream);
-        hip_check(hipEventRecord(c->ev[7], c->stream), "event");
+        hip_check(hipEventRecord(c->ev[1], c->stream), "event");
         c->check_launch();
         c->sync();
         float ms = 0.f;
-        hip_check(hipEventElapsedTime(&ms, c->ev[6], c->ev[7]), "elapsed");
+        hip_check(hipEventElapsedTime(&ms, c->ev[0], c->ev[1]), "elapsed");
         *ms_per_launch = static_cast<double>(ms) / reps;
     });
 }

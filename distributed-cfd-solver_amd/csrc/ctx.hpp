@@ -6,6 +6,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <chrono>
 #include <cstdint>
 #include <string>
 #include <vector>
@@ -161,10 +162,13 @@ struct cfdg_ctx {
     DBuf<double> bs, xs;  // the same in the sliced layout
     DBuf<double> stage;   // 5 per cell in mesh order: states and vectors crossing the ABI
     cfdg::HostPipe pipe;  // their copies from and to the caller's arrays
-    DBuf<double> partial, dots;
-    double* h_dots = nullptr;  // pinned
+    DBuf<double> partial, dots, norms;  // norms: sums of the squared residuals of an implicit step
+    // results handed over by the kernels (Publish), pinned; the number of the last hand-over
+    cfdg::HostBlock* blk = nullptr;
+    cfdg::HostBlock* blk_dev = nullptr;
+    unsigned long long seq = 0;
+    bool norms_known = false, singular_known = false;  // blk holds this solve's
     DBuf<double> ks;           // device-driven BiCGSTAB state block (kernels_linalg.hpp)
-    double* h_ks = nullptr;    // pinned copy
     int last_iters[2] = {4, 4};  // iterations of the last FP64 / FP32 solve: the first batch size
     // learned warm start (gnn.hpp)
     std::uint64_t uid = 0;              // identity of this context's graph in recorded samples
@@ -220,8 +224,9 @@ struct cfdg_ctx {
         return a;
     }
     // timing
-    hipEvent_t ev[8] = {};
-    double stage_ms[6] = {0, 0, 0, 0, 0, 0};
+    hipEvent_t ev[2] = {};
+    DBuf<unsigned long long> stamp;  // kStamp...
+    bool timed_residual = false, timed_gradients = false, timed_jacobian = false, timed_linear = false;
 
     cfdg::MeshArgs margs() const {
         cfdg::MeshArgs a{};
@@ -269,6 +274,7 @@ struct cfdg_ctx {
         f.mut = has_mut() ? sa_mut.get() : nullptr;
         f.mdot = sa_on() ? sa_mdot.get() : nullptr;
         f.mdot_tile = has_mut() ? sa_mdot_tile.get() : nullptr;
+        f.stamp = stamp.get();
         return f;
     }
     cfdg::BsrArgs bargs() const {
@@ -302,6 +308,27 @@ struct cfdg_ctx {
     long long sliced_size() const { return cfdg::sell_vector_size(n_slices()); }
     std::size_t vector_alloc() const { return z(std::max(sliced_size(), 5LL * nc)); }
     void sync() { hip_check(hipStreamSynchronize(stream), "hipStreamSynchronize"); }
+    cfdg::Publish publish() { return {blk_dev, ++seq}; }
+    // Until the last hand-over is there.  Spins for 2 ms, about the longest stretch that
+    // a runtime wait's 10 to 20 us are noticed in, then waits in the runtime, which also
+    // reports a failed kernel.
+    void wait() {
+        const auto here = [&] { return __atomic_load_n(&blk->seq, __ATOMIC_ACQUIRE) == seq; };
+        const auto t0 = std::chrono::steady_clock::now();
+        while (!here()) {
+            for (int k = 0; k < 64 && !here(); ++k) __builtin_ia32_pause();
+            if (std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) break;
+        }
+        if (here()) return;
+        sync();
+        if (!here()) throw cfdg::CfdgError(CFDG_ERR_HIP, "the device work ended without its results");
+    }
+    // Waits for all work enqueued so far.
+    void finish() {
+        cfdg::launch_publish(publish(), stream);
+        check_launch();
+        wait();
+    }
     void check_launch() { hip_check(hipGetLastError(), "kernel launch"); }
     template <typename T>
     void d2h(T* dst, const T* src, std::size_t n) {
@@ -333,8 +360,7 @@ struct cfdg_ctx {
     ~cfdg_ctx() {
         for (auto& e : ev)
             if (e) (void)hipEventDestroy(e);
-        if (h_dots) (void)hipHostFree(h_dots);
-        if (h_ks) (void)hipHostFree(h_ks);
+        if (blk) (void)hipHostFree(blk);
         if (stream) (void)hipStreamDestroy(stream);
     }
 };

@@ -147,7 +147,21 @@ struct FieldArgs {
     const double* mut;  // eddy viscosity (cells + ghosts, ghosts zero), null without turbulence
     double* mdot;       // mass flux F[0] of every face (mesh order), gathered from mdot_tile on request
     double* mdot_tile;  // mass flux per tile face-list entry (tile stream order), written when mut is set
+    unsigned long long* stamp;  // device clock at the stage boundaries (kStamp...)
 };
+
+// Stage times without events (an event between two kernels costs the stream 4 us,
+// as much as a small kernel): the first workgroup of the kernel that starts a stage
+// writes the device clock.
+enum : int {
+    kStampPrimitives = 0, kStampGradients, kStampGhostGradients, kStampFlux, kStampFluxEnd, kStampJacobian,
+    kStampJacobianEnd, kStampLinear, kStampLinearEnd, kStampCount
+};
+__device__ __forceinline__ void stamp_stage(unsigned long long* stamp, int k) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) stamp[k] = wall_clock64();
+}
+// stamp[k] (and stamp[k2] unless negative) by a launch of its own
+void launch_stamp(unsigned long long* stamp, int k, int k2, hipStream_t s);
 
 // Zone treatment of nu_tilde at a boundary face (spalart_allmaras.hpp:54-59)
 constexpr int kZoneWall = 0, kZoneSymmetry = 1, kZoneInflow = 2, kZoneOutflow = 3;
@@ -236,8 +250,8 @@ __host__ __device__ __forceinline__ int xcd_block(int b, int nb) {
 }
 
 // --- residual stages (kernels_residual.hip) ---------------------------------
-void launch_primitives(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, hipStream_t s);
-void launch_ghosts(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const BcTable& bcs, hipStream_t s);
+// primitives of the cells and of the boundary ghosts
+void launch_primitives(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const BcTable& bcs, hipStream_t s);
 // With sa given and the LDS-staged kernel in use, the module's nu_tilde gradient
 // is formed in the same pass; returns whether it was.
 bool launch_gradient_limiter(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, hipStream_t s,
@@ -249,9 +263,10 @@ void launch_ghost_gradients(const MeshArgs& m, const FieldArgs& f, const NumArgs
 void launch_flux(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, hipStream_t s);
 // out[5 p + v] = sum of F[v] over the boundary faces of patch p, p < n_patches
 void launch_boundary_integrals(const MeshArgs& m, const FieldArgs& f, int n_patches, double* out, hipStream_t s);
-// unsteady = c0 / dt of dual time stepping (0 in steady mode)
+// unsteady = c0 / dt of dual time stepping (0 in steady mode); flux_end: the launch
+// directly after the flux stage, whose end it stamps
 void launch_dt(const MeshArgs& m, const FieldArgs& f, const double* lam, double cfl, double unsteady, double* dt,
-               double* alpha, hipStream_t s);
+               double* alpha, bool flux_end, hipStream_t s);
 // rho, u, v, w, p, Mach of every cell (6 planes of nc, device order) for the solution files
 void launch_output_fields(int nc, const Gas& g, const double* U, double* out, hipStream_t s);
 // mdot[f] = mdot_tile[face_entry[f]] for every face (mesh order)
@@ -259,10 +274,10 @@ void launch_gather_mdot(int nf, const int* face_entry, const double* mdot_tile, 
 // five planes of nc from mesh order to device order and back
 void launch_planes_to_device(int nc, const int* mesh_of_row, const double* src, double* dst, hipStream_t s);
 void launch_planes_to_mesh(int nc, const int* mesh_of_row, const double* src, double* dst, hipStream_t s);
-// forward Euler: alpha = CFL / lambda, then U <- U - alpha R
-void launch_dt_explicit(const MeshArgs& m, const FieldArgs& f, const double* lam, double cfl, double* dt,
-                        double* alpha, hipStream_t s);
-void launch_explicit_update(const MeshArgs& m, const FieldArgs& f, const double* alpha, double* U, hipStream_t s);
+// forward Euler step: alpha = CFL / lambda, U <- U - alpha R, and the partial sums
+// (5 per workgroup, returned count, at most kReduceBlocks) of the squared residuals
+int launch_explicit_step(const MeshArgs& m, const FieldArgs& f, const double* lam, double cfl, double* dt,
+                         double* alpha, double* U, double* partial, hipStream_t s);
 // dual time stepping: R += V (c0 U + c1 U^n [+ c2 U^{n-1}]), bdf = 1 or 2
 void launch_unsteady_source(const MeshArgs& m, const FieldArgs& f, int bdf, double inv_dt, const double* Un,
                             const double* Unm1, hipStream_t s);

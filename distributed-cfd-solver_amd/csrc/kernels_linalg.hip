@@ -29,6 +29,7 @@
 #include "kernels.hpp"
 #include "kernels_krylov.hpp"
 #include "kernels_linalg.hpp"
+#include "reduce_device.hpp"
 
 // Scratch of the allocation-free residual norms (residual_norms_noalloc):
 // kReduceBlocks partial 5-vectors, 40 KiB per GPU, held until the process
@@ -416,8 +417,8 @@ __global__ void __launch_bounds__(kBlock) k_update_xr(long long n, double alpha,
 
 // Start of a solve (bicgstab.cpp:56-92): norms, tolerance, initial status,
 // then the start of the first iteration.
-__global__ void k_bicg_init(double* ks, const double* dots, int x_zero, int fallback, int reduced, double abs_tol,
-                            double rel_tol, int max_iter) {
+__device__ void bicg_init(double* ks, const double* dots, int x_zero, int fallback, int reduced, double abs_tol,
+                          double rel_tol, int max_iter) {
     const double bnorm = sqrt(dots[0]);
     double rnorm = x_zero ? bnorm : sqrt(dots[1]);
     double reject = 0.0;
@@ -451,6 +452,11 @@ __global__ void k_bicg_init(double* ks, const double* dots, int x_zero, int fall
         ks[kKsStatus] = kKsConverged;
     else
         bicg_begin(ks);
+}
+
+__global__ void k_bicg_init(double* ks, const double* dots, int x_zero, int fallback, double abs_tol, double rel_tol,
+                            int max_iter) {
+    bicg_init(ks, dots, x_zero, fallback, 0, abs_tol, rel_tol, max_iter);
 }
 
 // A rejected guess restarts from zero: x = 0, r = b.
@@ -492,10 +498,21 @@ __device__ void bicg_omega(double* ks, const double* dots) {
     ks[kKsRhoNew] = (r0s - omega_new * r0t) + ks[kKsAs] * rest * ks[kKsB0];
 }
 
-__global__ void k_bicg_post(double* ks) {
-    if (ks[kKsStatus] != 0.0) return;
-    bicg_post(ks, nullptr);
+// The end of the iteration, unless the step that formed the true residual norm took
+// it (post = 0), and the hand-over of a batch: the state, then the residual norms'
+// sums and the singular row that the solve was started with.
+__global__ void __launch_bounds__(64) k_bicg_post(double* ks, int post, const double* norms, const int* singular,
+                                                  Publish pub) {
+    if (threadIdx.x == 0 && post && ks[kKsStatus] == 0.0) bicg_post(ks, nullptr);
+    if (!pub.host) return;
+    __syncthreads();
+    if (threadIdx.x < kKsCount) pub.host->v[threadIdx.x] = ks[threadIdx.x];
+    if (threadIdx.x < 5) pub.host->v[kKsCount + threadIdx.x] = norms[threadIdx.x];
+    if (threadIdx.x == 5) pub.host->v[kKsCount + 5] = static_cast<double>(*singular);
+    publish_seq(pub);
 }
+
+__global__ void __launch_bounds__(64) k_publish(Publish pub) { publish_seq(pub); }
 
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_update_p_g(long long n, const double* ks, const T* r, const T* v, T* p) {
@@ -625,28 +642,6 @@ __global__ void __launch_bounds__(kBlock) k_add_f32(long long n, const float* e,
     x[i] = x[i] + static_cast<double>(e[i]);
 }
 
-__device__ __forceinline__ double wave_sum(double v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    return v;
-}
-
-// Sums over the workgroup of the first ncomp components, each in a fixed tree
-// order (the waves' sums in wave order); sum j valid in thread j.  lds: 5 per wave.
-__device__ __forceinline__ double block_sums(const double v[5], int ncomp, double* lds) {
-    const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-#pragma unroll
-    for (int j = 0; j < 5; ++j) {
-        if (j >= ncomp) break;
-        const double s = wave_sum(v[j]);
-        if (lane == 0) lds[wid * 5 + j] = s;
-    }
-    __syncthreads();
-    double s = 0.0;
-    if (static_cast<int>(threadIdx.x) < ncomp)
-        for (int w = 0; w < static_cast<int>(blockDim.x >> 6); ++w) s += lds[w * 5 + static_cast<int>(threadIdx.x)];
-    return s;
-}
-
 // Up to five dot products of flat vectors in one pass; partial[b * 5 + j].
 template <class T>
 __global__ void __launch_bounds__(kBlock) k_dots(long long n, int ndot, DotPairsT<T> pr, double* partial,
@@ -657,7 +652,7 @@ __global__ void __launch_bounds__(kBlock) k_dots(long long n, int ndot, DotPairs
     const long long stride = static_cast<long long>(gridDim.x) * blockDim.x;
     for (long long i = static_cast<long long>(blockIdx.x) * blockDim.x + threadIdx.x; i < n; i += stride) {
         for (int j = 0; j < 5; ++j)
-            if (j < ndot && i < pr.n[j]) acc[j] += static_cast<double>(pr.a[j][i]) * static_cast<double>(pr.b[j][i]);
+            if (j < ndot) acc[j] += static_cast<double>(pr.a[j][i]) * static_cast<double>(pr.b[j][i]);
     }
     const double s = block_sums(acc, ndot, lds);
     if (static_cast<int>(threadIdx.x) < ndot) partial[blockIdx.x * 5 + threadIdx.x] = s;
@@ -678,26 +673,15 @@ __global__ void __launch_bounds__(kBlock) k_res_sq(int nc, int ld, const double*
     if (threadIdx.x < 5) partial[blockIdx.x * 5 + threadIdx.x] = s;
 }
 
-// Adds nblocks partial 5-vectors: thread t sums blocks t, t + 256, ... in
-// order, then the block tree adds the 256 thread sums in a fixed order; sum j in
-// thread j.  Bound by latency: the components' loads are in flight together and
-// their trees share the barriers (one component after the other took 7 us for five
-// components of 1,024 partials).
-__device__ __forceinline__ double sum_partials(int nblocks, int ncomp, const double* partial, double* lds) {
-    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int b = threadIdx.x; b < nblocks; b += kBlock)
-#pragma unroll
-        for (int j = 0; j < 5; ++j)
-            if (j < ncomp) acc[j] += partial[b * 5 + j];
-    return block_sums(acc, ncomp, lds);
-}
-
 __global__ void __launch_bounds__(kBlock) k_reduce_partials(int nblocks, int ncomp, const double* partial,
-                                                            double* out, const double* gate) {
-    if (gate && gate[kKsStatus] != 0.0) return;
+                                                            double* out, Publish pub) {
     __shared__ double lds[kBlock / 64 * 5];
     const double s = sum_partials(nblocks, ncomp, partial, lds);
-    if (static_cast<int>(threadIdx.x) < ncomp) out[threadIdx.x] = s;
+    const bool mine = static_cast<int>(threadIdx.x) < ncomp;
+    if (mine) out[threadIdx.x] = s;
+    if (!pub.host) return;
+    if (mine) pub.host->v[threadIdx.x] = s;
+    publish_seq(pub);
 }
 
 // k_reduce_partials followed, in thread 0, by the scalar step of the
@@ -719,6 +703,52 @@ __global__ void __launch_bounds__(kBlock) k_reduce_step(int nblocks, int ncomp, 
     if constexpr (kStep == kStepPost) bicg_post(ks, sums);
 }
 
+// The start of a reduced solve from the squares of its right-hand side and, for a
+// guess, of its residual: partial sums per component (norms takes the right-hand
+// side's) and behind them the first colour's.
+__device__ __forceinline__ void sum_squares(int nblocks, const double* partial, double* lds, double sums[6]) {
+    const double s = sum_partials(nblocks, 5, partial, lds);
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int b = threadIdx.x; b < nblocks; b += kBlock) acc[0] += partial[5 * kMaxPartials + b];
+    __syncthreads();  // lds
+    const double s0 = block_sums(acc, 1, lds);
+    if (threadIdx.x < 5) sums[threadIdx.x] = s;
+    if (threadIdx.x == 0) sums[5] = s0;
+    __syncthreads();
+}
+__device__ __forceinline__ double total_square(const double sums[6]) {
+    return (((sums[0] + sums[1]) + sums[2]) + sums[3]) + sums[4];
+}
+__global__ void __launch_bounds__(kBlock) k_bicg_start(int nblocks, const double* partial, int guess, double* norms,
+                                                       double* ks, int fallback, double abs_tol, double rel_tol,
+                                                       int max_iter, Publish pub) {
+    __shared__ double lds[kBlock / 64 * 5];
+    __shared__ double sb[6], sr[6];
+    sum_squares(nblocks, partial, lds, sb);
+    if (guess) sum_squares(nblocks, partial + kSquares, lds, sr);
+    if (threadIdx.x == 0) {
+        const double bb = total_square(sb), rr = guess ? total_square(sr) : bb;
+        if (ks) {
+            if (guess) {
+                const double dots[4] = {bb, rr, sr[5], sb[5]};
+                bicg_init(ks, dots, 0, fallback, 1, abs_tol, rel_tol, max_iter);
+            } else {
+                const double dots[2] = {bb, sb[5]};
+                bicg_init(ks, dots, 1, fallback, 1, abs_tol, rel_tol, max_iter);
+            }
+        }
+        if (pub.host) {
+            pub.host->v[0] = bb;
+            pub.host->v[1] = rr;
+        }
+    }
+    if (threadIdx.x < 5) {
+        if (norms) norms[threadIdx.x] = sb[threadIdx.x];
+        if (pub.host) pub.host->v[kKsCount + threadIdx.x] = sb[threadIdx.x];
+    }
+    if (pub.host) publish_seq(pub);
+}
+
 // The partial sums of k_res_sq added in k_reduce_partials' order, then
 // l2[v] = sqrt(sum_v * scale) (solver.hpp:740-756) written to device memory.
 __global__ void __launch_bounds__(kBlock) k_norms_finish(int nblocks, const double* partial, double scale,
@@ -728,11 +758,20 @@ __global__ void __launch_bounds__(kBlock) k_norms_finish(int nblocks, const doub
     if (threadIdx.x < 5) l2[threadIdx.x] = sqrt(s * scale);
 }
 
-// b = -R (AoS), the implicit right-hand side (implicit_euler.hpp:81-92)
-__global__ void __launch_bounds__(kBlock) k_rhs(int nc, int ld, const double* res, double* b) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nc) return;
-    for (int v = 0; v < 5; ++v) b[static_cast<long long>(c) * 5 + v] = -res[static_cast<long long>(v) * ld + c];
+// b = -R (AoS), the implicit right-hand side (implicit_euler.hpp:81-92), with the
+// partial sums of k_res_sq
+__global__ void __launch_bounds__(kBlock) k_rhs(int nc, int ld, const double* res, double* b, double* partial) {
+    __shared__ double lds[kBlock / 64 * 5];
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    const int stride = static_cast<int>(gridDim.x * blockDim.x);
+    for (int c = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); c < nc; c += stride)
+        for (int v = 0; v < 5; ++v) {
+            const double r = res[static_cast<long long>(v) * ld + c];
+            acc[v] += r * r;
+            b[static_cast<long long>(c) * 5 + v] = -r;
+        }
+    const double s = block_sums(acc, 5, lds);
+    if (threadIdx.x < 5) partial[blockIdx.x * 5 + threadIdx.x] = s;
 }
 
 // U = U + du (implicit_euler.hpp:53-61)
@@ -899,32 +938,36 @@ int reduction_blocks(long long n) {
     return static_cast<int>(b);
 }
 
-// a pair without a length of its own is as long as the vectors
-template <class T>
-static DotPairsT<T> whole(long long n, DotPairsT<T> pr) {
-    for (long long& k : pr.n)
-        if (k == 0) k = n;
-    return pr;
-}
-
 template <class T>
 void launch_dots(long long n, int ndot, const DotPairsT<T>& pr, double* partial, double* out, hipStream_t s,
-                 const double* gate) {
+                 const Publish& pub) {
     const int nb = reduction_blocks(n);
-    hipLaunchKernelGGL(k_dots<T>, dim3(nb), dim3(kBlock), 0, s, n, ndot, whole(n, pr), partial, gate);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kBlock), 0, s, nb, ndot, partial, out, gate);
+    hipLaunchKernelGGL(k_dots<T>, dim3(nb), dim3(kBlock), 0, s, n, ndot, pr, partial, nullptr);
+    launch_reduce_partials(nb, ndot, partial, out, pub, s);
 }
 
 template void launch_dots<double>(long long, int, const DotPairsT<double>&, double*, double*, hipStream_t,
-                                  const double*);
+                                  const Publish&);
 template void launch_dots<float>(long long, int, const DotPairsT<float>&, double*, double*, hipStream_t,
-                                 const double*);
+                                 const Publish&);
+
+void launch_reduce_partials(int nb, int ncomp, const double* partial, double* out, const Publish& pub, hipStream_t s) {
+    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kBlock), 0, s, nb, ncomp, partial, out, pub);
+}
+
+void launch_bicg_start(int nb, const double* partial, bool guess, double* norms, double* ks, bool fallback,
+                       double abs_tol, double rel_tol, int max_iter, const Publish& pub, hipStream_t s) {
+    hipLaunchKernelGGL(k_bicg_start, dim3(1), dim3(kBlock), 0, s, nb, partial, guess ? 1 : 0, norms, ks,
+                       fallback ? 1 : 0, abs_tol, rel_tol, max_iter, pub);
+}
+
+void launch_publish(const Publish& pub, hipStream_t s) { hipLaunchKernelGGL(k_publish, dim3(1), dim3(64), 0, s, pub); }
 
 template <class T>
 void launch_dots_step(long long n, int ndot, const DotPairsT<T>& pr, double* partial, double* out, double* ks,
                       int step, hipStream_t s) {
     const int nb = reduction_blocks(n);
-    hipLaunchKernelGGL(k_dots<T>, dim3(nb), dim3(kBlock), 0, s, n, ndot, whole(n, pr), partial, ks);
+    hipLaunchKernelGGL(k_dots<T>, dim3(nb), dim3(kBlock), 0, s, n, ndot, pr, partial, ks);
     launch_reduce_step(nb, ndot, partial, out, ks, step, s);
 }
 template void launch_dots_step<double>(long long, int, const DotPairsT<double>&, double*, double*, double*, int,
@@ -941,10 +984,9 @@ void launch_reduce_step(int nb, int ndot, const double* partial, double* out, do
         hipLaunchKernelGGL(k_reduce_step<kStepPost>, dim3(1), dim3(kBlock), 0, s, nb, ndot, partial, out, ks);
 }
 
-void launch_bicg_init(double* ks, const double* dots, int x_zero, int fallback, int reduced, double abs_tol,
-                      double rel_tol, int max_iter, hipStream_t s) {
-    hipLaunchKernelGGL(k_bicg_init, dim3(1), dim3(1), 0, s, ks, dots, x_zero, fallback, reduced, abs_tol, rel_tol,
-                       max_iter);
+void launch_bicg_init(double* ks, const double* dots, int x_zero, int fallback, double abs_tol, double rel_tol,
+                      int max_iter, hipStream_t s) {
+    hipLaunchKernelGGL(k_bicg_init, dim3(1), dim3(1), 0, s, ks, dots, x_zero, fallback, abs_tol, rel_tol, max_iter);
 }
 
 template <class T>
@@ -954,7 +996,10 @@ void launch_bicg_reject(long long n, const double* ks, const T* b, T* x, T* r, h
 template void launch_bicg_reject<double>(long long, const double*, const double*, double*, double*, hipStream_t);
 template void launch_bicg_reject<float>(long long, const double*, const float*, float*, float*, hipStream_t);
 
-void launch_bicg_post(double* ks, hipStream_t s) { hipLaunchKernelGGL(k_bicg_post, dim3(1), dim3(1), 0, s, ks); }
+void launch_bicg_post(double* ks, bool post, const double* norms, const int* singular, const Publish& pub,
+                      hipStream_t s) {
+    hipLaunchKernelGGL(k_bicg_post, dim3(1), dim3(64), 0, s, ks, post ? 1 : 0, norms, singular, pub);
+}
 
 template <class T>
 void launch_update_p_g(long long n, const double* ks, const T* r, const T* v, T* p, hipStream_t s) {
@@ -1030,10 +1075,11 @@ template void launch_update_xr_g<double>(long long, const double*, const double*
 template void launch_update_xr_g<float>(long long, const double*, const float*, const float*, const float*,
                                         const float*, float*, float*, hipStream_t);
 
-void launch_res_sq(int nc, int ld, const double* res, double* partial, double* out, hipStream_t s) {
+void launch_res_sq(int nc, int ld, const double* res, double* partial, double* out, const Publish& pub,
+                   hipStream_t s) {
     const int nb = reduction_blocks(nc);
     hipLaunchKernelGGL(k_res_sq, dim3(nb), dim3(kBlock), 0, s, nc, ld, res, partial);
-    hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kBlock), 0, s, nb, 5, partial, out, nullptr);
+    launch_reduce_partials(nb, 5, partial, out, pub, s);
 }
 
 namespace {
@@ -1076,8 +1122,10 @@ hipError_t residual_norms_noalloc(int nc, int ld, const double* res, double* l2,
     return hipGetLastError();
 }
 
-void launch_rhs(int nc, int ld, const double* res, double* b, hipStream_t s) {
-    if (nc > 0) hipLaunchKernelGGL(k_rhs, grid_for(nc), dim3(kBlock), 0, s, nc, ld, res, b);
+void launch_rhs(int nc, int ld, const double* res, double* b, double* partial, double* norms, hipStream_t s) {
+    const int nb = reduction_blocks(nc);
+    hipLaunchKernelGGL(k_rhs, dim3(nb), dim3(kBlock), 0, s, nc, ld, res, b, partial);
+    launch_reduce_partials(nb, 5, partial, norms, Publish{}, s);
 }
 
 void launch_state_update(int nc, int ld, const double* du, double* U, hipStream_t s) {

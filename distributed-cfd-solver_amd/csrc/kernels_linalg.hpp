@@ -30,11 +30,23 @@ enum : int {
 // kKsExact: the reduced form met s = 0 exactly
 constexpr double kKsConverged = 1.0, kKsDiverged = 2.0, kKsMaxIter = 3.0, kKsExact = 4.0;
 
+// Results for the host without a copy and a stream synchronisation, which cost 13 to
+// 20 us after a short kernel: the kernel that ends a stretch of work writes them to
+// pinned host memory, then seq, which the host polls (cfdg_ctx::wait).
+struct HostBlock {
+    double v[kKsCount + 8];
+    unsigned long long seq;
+};
+struct Publish {
+    HostBlock* host = nullptr;  // null: nothing is handed over
+    unsigned long long seq = 0;
+};
+void launch_publish(const Publish& pub, hipStream_t s);
+
 template <class T>
 struct DotPairsT {
     const T* a[5];
     const T* b[5];
-    long long n[5];  // entries of the pair, 0 for all
 };
 using DotPairs = DotPairsT<double>;
 
@@ -78,20 +90,30 @@ void launch_cast_f64_to_f32(long long n, const double* src, float* dst, hipStrea
 void launch_cast_f32_to_f64(long long n, const float* src, double* dst, hipStream_t s);
 void launch_add_f32(long long n, const float* e, double* x, hipStream_t s);
 int reduction_blocks(long long n);
-// out[0..ndot) = dot products accumulated in FP64; partial needs kMaxPartials * 5 doubles
+// out[0..ndot) = dot products accumulated in FP64, handed over in v[0..ndot); partial
+// needs kMaxPartials * 5 doubles
 template <class T>
 void launch_dots(long long n, int ndot, const DotPairsT<T>& pr, double* partial, double* out, hipStream_t s,
-                 const double* gate = nullptr);
+                 const Publish& pub = {});
+// the second half of it
+void launch_reduce_partials(int nb, int ncomp, const double* partial, double* out, const Publish& pub, hipStream_t s);
 // device-driven BiCGSTAB: scalar steps on the state block ks and gated vector
 // updates.  The start of each iteration (iteration limit, beta) is taken at
 // the end of the step before it, so an iteration begins with its p update.
 // Start of a solve from dots = (b, b) and, unless x_zero, (r, r) with r = b - A x:
 // tolerance max(abs_tol, rel_tol ||b||), status, rho; with fallback, a guess
 // whose residual exceeds ||b|| is marked rejected (launch_bicg_reject then
-// restarts from zero).  reduced: dots go on with (r, r) -- or x_zero, (b, b) --
-// of the first colour, and unless x_zero with its (b, b).
-void launch_bicg_init(double* ks, const double* dots, int x_zero, int fallback, int reduced, double abs_tol,
-                      double rel_tol, int max_iter, hipStream_t s);
+// restarts from zero).
+void launch_bicg_init(double* ks, const double* dots, int x_zero, int fallback, double abs_tol, double rel_tol,
+                      int max_iter, hipStream_t s);
+// launch_bicg_init of a reduced solve from the nb partial sums of the right-hand side's
+// squares and, with a guess, kSquares further those of b - A x: 5 per workgroup by
+// component (the right-hand side's sums also go to norms, unless null), and from 5
+// kMaxPartials on one per workgroup for the first colour.  Hand-over: v[0] = (b, b),
+// v[1] = (r, r), norms from v[kKsCount].  ks null: the sums only.
+constexpr int kSquares = 6 * kMaxPartials;
+void launch_bicg_start(int nb, const double* partial, bool guess, double* norms, double* ks, bool fallback,
+                       double abs_tol, double rel_tol, int max_iter, const Publish& pub, hipStream_t s);
 template <class T>
 void launch_bicg_reject(long long n, const double* ks, const T* b, T* x, T* r, hipStream_t s);
 // dot products as launch_dots, gated by ks, then the scalar step that uses them
@@ -104,8 +126,10 @@ void launch_dots_step(long long n, int ndot, const DotPairsT<T>& pr, double* par
                       int step, hipStream_t s);
 // the second half of it: nb partial sums of ndot products, then the scalar step
 void launch_reduce_step(int nb, int ndot, const double* partial, double* out, double* ks, int step, hipStream_t s);
-// the end of an iteration with the recurrence's residual norm
-void launch_bicg_post(double* ks, hipStream_t s);
+// the end of an iteration with the recurrence's residual norm (post), and of a batch:
+// v = the state block, norms (5), *singular
+void launch_bicg_post(double* ks, bool post, const double* norms, const int* singular, const Publish& pub,
+                      hipStream_t s);
 template <class T>
 void launch_update_p_g(long long n, const double* ks, const T* r, const T* v, T* p, hipStream_t s);
 template <class T>
@@ -128,12 +152,15 @@ void launch_vec_sgs_first(int op, int nrows, const double* ks, const TV* r, cons
 template <class T>
 void launch_update_xr_g(long long n, const double* ks, const T* ph, const T* sh, const T* sv, const T* t, T* x, T* r,
                         hipStream_t s);
-void launch_res_sq(int nc, int ld, const double* res, double* partial, double* out, hipStream_t s);
+// out = v[0..5) = the sums of the squared residuals
+void launch_res_sq(int nc, int ld, const double* res, double* partial, double* out, const Publish& pub,
+                   hipStream_t s);
 // l2 (5 doubles, device) = residual norms of res (5 planes of ld, nc cells,
 // device), with the partial sums in the library's static scratch array: no
 // device allocation, no host synchronisation; stream-ordered on s.
 hipError_t residual_norms_noalloc(int nc, int ld, const double* res, double* l2, hipStream_t s);
-void launch_rhs(int nc, int ld, const double* res, double* b, hipStream_t s);
+// b = -R and norms = the sums of the squared residuals
+void launch_rhs(int nc, int ld, const double* res, double* b, double* partial, double* norms, hipStream_t s);
 void launch_state_update(int nc, int ld, const double* du, double* U, hipStream_t s);
 
 }  // namespace cfdg

@@ -43,6 +43,7 @@
 #include "kernels_krylov.hpp"
 #include "kernels_reduced.hpp"
 #include "kernels_sell_device.hpp"
+#include "reduce_device.hpp"
 
 namespace cfdg {
 
@@ -249,11 +250,6 @@ __global__ void __launch_bounds__(slice_threads<kSplit>()) k_red_backward(SellAr
         d[e] = acc[k];
         if (update) z[e] += acc[k];
     }
-}
-
-__device__ __forceinline__ double wave_sum(double v) {
-    for (int off = 32; off > 0; off >>= 1) v += __shfl_down(v, off, 64);
-    return v;
 }
 
 // The product, (2), with the dot products of its step: v and (r0, v) (kOp 0), or

@@ -3,8 +3,8 @@
 // Data: cell and face planes (structure of arrays, kernels.hpp).  Cells are
 // in the device (tile) order; faces keep their mesh index.
 //
-//   k_primitives        U -> (p,u,v,w,T) into the cell records
-//   k_ghosts            boundary ghost states, one thread per boundary face
+//   k_primitives        U -> (p,u,v,w,T) into the cell records; boundary ghost
+//                       states, one thread per boundary face
 //   k_gradient_limiter  cell gradient (node-stencil least squares with the
 //                       3x3 normal equations rebuilt per cell from neighbour
 //                       centroids, or Green-Gauss) + MUSCL limiter, one thread
@@ -22,6 +22,8 @@
 #include <hip/hip_runtime.h>
 
 #include "kernels.hpp"
+#include "kernels_linalg.hpp"
+#include "reduce_device.hpp"
 
 namespace cfdg {
 
@@ -36,17 +38,6 @@ __device__ __forceinline__ FaceRef frec(const MeshArgs& m, int f) { return FaceR
 __device__ __forceinline__ CellRef crec(const FieldArgs& f, int c) { return CellRef{f.cs, f.ld, c}; }
 __device__ __forceinline__ CellRefW crecw(const FieldArgs& f, int c) { return CellRefW{f.cs, f.ld, c}; }
 
-// U -> q for the cells (solver.hpp:185-188)
-__global__ void __launch_bounds__(kBlock) k_primitives(MeshArgs m, FieldArgs f, NumArgs nm) {
-    const int c = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
-    if (c >= m.nc) return;
-    double U[5], q[5];
-    for (int v = 0; v < 5; ++v) U[v] = f.U[static_cast<long long>(v) * m.nc + c];
-    cons_to_prim(nm.gas, U, q);
-    const CellRefW r = crecw(f, c);
-    for (int v = 0; v < 5; ++v) r[kRQ + v] = q[v];
-}
-
 // 1 / max((x_f - x_c) . n, 1e-14)   (boundary_traversal.hpp:98-108)
 template <class FR, class CR>
 __device__ __forceinline__ double rcfn_inverse(const FR& fr, const CR& cr) {
@@ -55,18 +46,24 @@ __device__ __forceinline__ double rcfn_inverse(const FR& fr, const CR& cr) {
     return 1.0 / dmax(r, 1.0e-14);
 }
 
+__device__ __forceinline__ void cell_primitives(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, int c,
+                                                double q[5]) {
+    double U[5];
+    for (int v = 0; v < 5; ++v) U[v] = f.U[static_cast<long long>(v) * m.nc + c];
+    cons_to_prim(nm.gas, U, q);
+}
+
 // Ghost primitive states (bc/physical/*.hpp value kernels)
-__global__ void __launch_bounds__(kBlock) k_ghosts(MeshArgs m, FieldArgs f, NumArgs nm, BcTable bt) {
-    const int bf = blockIdx.x * blockDim.x + threadIdx.x;
-    const int nbf = m.nf - m.ninner;
-    if (bf >= nbf) return;
+__device__ __forceinline__ void ghost_primitives(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm,
+                                                 const BcTable& bt, int bf) {
     const int fc = m.ninner + bf;
     const FaceRef fr = frec(m, fc);
-    const CellRef ri = crec(f, face_owner(m, fc));
+    const int owner = face_owner(m, fc);
+    const CellRef ri = crec(f, owner);
     const CellRefW rg = crecw(f, m.nc + bf);
     const BcDev bp = bt.bc[m.bface_bc[bf]];
     double qi[5], qg[5];
-    for (int v = 0; v < 5; ++v) qi[v] = ri[kRQ + v];
+    cell_primitives(m, f, nm, owner, qi);
     const double nx = fr[kFN], ny = fr[kFN + 1], nz = fr[kFN + 2];
     switch (bp.type) {
         case kSupIn: {
@@ -129,6 +126,26 @@ __global__ void __launch_bounds__(kBlock) k_ghosts(MeshArgs m, FieldArgs f, NumA
             break;
     }
     for (int v = 0; v < 5; ++v) rg[kRQ + v] = qg[v];
+}
+
+// U -> q for the cells (solver.hpp:185-188), the first cell_blocks workgroups, and
+// the ghosts, the others: a ghost forms its owner's primitives itself, so the two
+// need no order and one launch does both.
+__global__ void __launch_bounds__(kBlock) k_primitives(MeshArgs m, FieldArgs f, NumArgs nm, BcTable bt,
+                                                       int cell_blocks) {
+    stamp_stage(f.stamp, kStampPrimitives);
+    const int blk = static_cast<int>(blockIdx.x);
+    if (blk >= cell_blocks) {
+        const int bf = (blk - cell_blocks) * kBlock + static_cast<int>(threadIdx.x);
+        if (bf < m.nf - m.ninner) ghost_primitives(m, f, nm, bt, bf);
+        return;
+    }
+    const int c = xcd_block(blk, cell_blocks) * kBlock + static_cast<int>(threadIdx.x);
+    if (c >= m.nc) return;
+    double q[5];
+    cell_primitives(m, f, nm, c, q);
+    const CellRefW r = crecw(f, c);
+    for (int v = 0; v < 5; ++v) r[kRQ + v] = q[v];
 }
 
 // Inverse of the weighted least-squares normal matrix of cell c over its
@@ -339,6 +356,7 @@ __device__ __forceinline__ void store_and_limit(const MeshArgs& m, const FieldAr
 
 // One thread per cell, neighbours gathered from the records in HBM.
 __global__ void __launch_bounds__(kBlock) k_gradient_limiter(MeshArgs m, FieldArgs f, NumArgs nm) {
+    stamp_stage(f.stamp, kStampGradients);
     const int c = xcd_block(blockIdx.x, gridDim.x) * kBlock + threadIdx.x;
     if (c >= m.nc) return;
     gradient_limiter_cell(
@@ -381,6 +399,7 @@ struct LdsSlot {
 // and face neighbours from there.
 template <bool kSA, int kSlots>
 __global__ void __launch_bounds__(kTileCells) k_gradient_limiter_lds(MeshArgs m, FieldArgs f, NumArgs nm, SaArgs sa) {
+    stamp_stage(f.stamp, kStampGradients);
     __shared__ __attribute__((aligned(16))) double sq[(kSA ? 9 : 8) * kSlots];  // 4 plane pairs (+ nu_tilde)
     const int t = xcd_block(blockIdx.x, gridDim.x);
     const int c0 = m.gtile_off[t], nt = m.gtile_off[t + 1] - c0;
@@ -454,6 +473,7 @@ __global__ void __launch_bounds__(kTileCells) k_gradient_limiter_lds(MeshArgs m,
 template <bool kSA>
 __global__ void __launch_bounds__(2 * kTileCells) k_gradient_limiter_pair(MeshArgs m, FieldArgs f, NumArgs nm,
                                                                           SaArgs sa) {
+    stamp_stage(f.stamp, kStampGradients);
     constexpr int kSlots = kGradSlotsBig;
     __shared__ __attribute__((aligned(16))) double sq[(kSA ? 9 : 8) * kSlots];
     const int t = xcd_block(blockIdx.x, gridDim.x);
@@ -587,6 +607,7 @@ __device__ __forceinline__ void grad_slip(double* g, const double* gi, double qi
 
 // Ghost gradients (bc/physical/*.hpp gradient kernels, boundary_gradients.hpp)
 __global__ void __launch_bounds__(kBlock) k_ghost_gradients(MeshArgs m, FieldArgs f, NumArgs nm, BcTable bt) {
+    stamp_stage(f.stamp, kStampGhostGradients);
     const int bf = blockIdx.x * blockDim.x + threadIdx.x;
     const int nbf = m.nf - m.ninner;
     if (bf >= nbf) return;
@@ -750,6 +771,7 @@ struct TileFaceRef {
 // cells (residual_kernel.hpp:229-230, 282-283).
 template <bool kTurb>
 __global__ void __launch_bounds__(kFluxThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) k_flux(MeshArgs m, FieldArgs f, NumArgs nm) {
+    stamp_stage(f.stamp, kStampFlux);
     __shared__ double sc[kFluxPlanes * kTileCells];  // staged planes, then the fluxes sF[6][kTileFaces]
     __shared__ double smut[kTurb ? kTileCells : 1];
     __shared__ int scf[kTileCells + 1 + 2 * kTileFaces];  // the tile's cf_off (rebased), then its cf_slot entries
@@ -857,7 +879,9 @@ __global__ void __launch_bounds__(kFluxThreads) __attribute__((amdgpu_waves_per_
 // Implicit local time step and diagonal shift (solver.hpp:256-287); unsteady
 // = c0 / dt of dual time stepping (0 in steady mode)
 __global__ void __launch_bounds__(kBlock) k_dt(int nc, const double* cs, long long ld, const double* lam, double cfl,
-                                               double unsteady, double* dt, double* alpha) {
+                                               double unsteady, double* dt, double* alpha,
+                                               unsigned long long* flux_end) {
+    if (flux_end) stamp_stage(flux_end, kStampFluxEnd);
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
     if (c >= nc) return;
     const double vol = cs[plane_at(kRVol, ld, c)];
@@ -899,17 +923,6 @@ __global__ void __launch_bounds__(kBlock) k_output_fields(int nc, Gas g, const d
     o[5LL * nc] = sqrt(u[1] * u[1] + u[2] * u[2] + u[3] * u[3]) / (r * a);
 }
 
-// Explicit local time step: alpha = dt / V = CFL / lambda (solver.hpp:278-285)
-__global__ void __launch_bounds__(kBlock) k_dt_explicit(int nc, const double* cs, long long ld, const double* lam,
-                                                        double cfl, double* dt, double* alpha) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nc) return;
-    const double l = dmax(lam[c], 1.0e-14);
-    const double cfl_over_l = cfl / l;
-    dt[c] = cfl_over_l * cs[plane_at(kRVol, ld, c)];
-    alpha[c] = cfl_over_l;
-}
-
 // Five planes of nc between mesh order and device order: dst[r] = src[map[r]]
 // (mesh cell of a device row), or back, dst[map[r]] = src[r].  A tile's rows are
 // runs of neighbouring mesh cells, so either side falls in few cache lines.
@@ -927,15 +940,36 @@ __global__ void __launch_bounds__(kBlock) k_permute_planes(int nc, const int* ma
     }
 }
 
-// Forward Euler update U <- U - alpha R (update_ops.hpp:28-44)
-__global__ void __launch_bounds__(kBlock) k_explicit_update(int nc, const double* alpha, const double* res, double* U) {
-    const int c = blockIdx.x * blockDim.x + threadIdx.x;
-    if (c >= nc) return;
-    const double a = alpha[c];
-    for (int v = 0; v < 5; ++v) {
-        const long long k = static_cast<long long>(v) * nc + c;
-        U[k] = U[k] - a * res[k];
+// Forward Euler step in one pass over the residual: local time step alpha = dt / V
+// = CFL / lambda (solver.hpp:278-285), U <- U - alpha R (update_ops.hpp:28-44) and
+// the residual's squares (solver.hpp:740-756), summed as k_res_sq does.  Bound: HBM
+// (three kernels read the residual twice and alpha back: 80 us at 2.1M cells).
+__global__ void __launch_bounds__(kBlock) k_explicit_step(int nc, const double* cs, long long ld, const double* lam,
+                                                          double cfl, const double* res, double* dt, double* alpha,
+                                                          double* U, double* partial, unsigned long long* stamp) {
+    __shared__ double lds[kBlock / 64 * 5];
+    stamp_stage(stamp, kStampFluxEnd);
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    const int stride = static_cast<int>(gridDim.x * blockDim.x);
+    for (int c = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); c < nc; c += stride) {
+        const double l = dmax(lam[c], 1.0e-14);
+        const double a = cfl / l;
+        dt[c] = a * cs[plane_at(kRVol, ld, c)];
+        alpha[c] = a;
+        for (int v = 0; v < 5; ++v) {
+            const long long k = static_cast<long long>(v) * nc + c;
+            const double r = res[k];
+            acc[v] += r * r;
+            U[k] = U[k] - a * r;
+        }
     }
+    const double s = block_sums(acc, 5, lds);
+    if (threadIdx.x < 5) partial[blockIdx.x * 5 + threadIdx.x] = s;
+}
+
+__global__ void k_stamp(unsigned long long* stamp, int k, int k2) {
+    stamp_stage(stamp, k);
+    if (k2 >= 0) stamp_stage(stamp, k2);
 }
 
 // BDF pseudo-source of dual time stepping, R += V (c0 U + c1 U^n [+ c2 U^{n-1}])
@@ -1103,6 +1137,7 @@ __global__ void __launch_bounds__(kTileCells)
 __attribute__((amdgpu_waves_per_eu(2)))
 k_jacobian(MeshArgs m, FieldArgs f, NumArgs nm, SellArgs b, const double* alpha,
            typename SellLayout<TS>::word* off, typename SellLayout<TS>::word* diag) {
+    stamp_stage(f.stamp, kStampJacobian);
     constexpr long long kW = SellLayout<TS>::words;
     __shared__ double sq[8 * kTileCells];  // q (0-4) and centroid (5-7) of the tile's cells, one plane each
     __shared__ double smut[kTurb ? kTileCells : 1];
@@ -1174,13 +1209,11 @@ inline dim3 grid_for(long long n) { return dim3(static_cast<unsigned>((n + kBloc
 
 }  // namespace
 
-void launch_primitives(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, hipStream_t s) {
-    if (m.nc > 0) hipLaunchKernelGGL(k_primitives, grid_for(m.nc), dim3(kBlock), 0, s, m, f, nm);
-}
-
-void launch_ghosts(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const BcTable& bcs, hipStream_t s) {
-    const int nbf = m.nf - m.ninner;
-    if (nbf > 0) hipLaunchKernelGGL(k_ghosts, grid_for(nbf), dim3(kBlock), 0, s, m, f, nm, bcs);
+void launch_primitives(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const BcTable& bcs, hipStream_t s) {
+    const int cells = (m.nc + kBlock - 1) / kBlock, ghosts = (m.nf - m.ninner + kBlock - 1) / kBlock;
+    if (cells + ghosts > 0)
+        hipLaunchKernelGGL(k_primitives, dim3(static_cast<unsigned>(cells + ghosts)), dim3(kBlock), 0, s, m, f, nm, bcs,
+                           cells);
 }
 
 bool launch_gradient_limiter(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, hipStream_t s,
@@ -1240,15 +1273,10 @@ void launch_gather_mdot(int nf, const int* face_entry, const double* mdot_tile, 
 }
 
 void launch_dt(const MeshArgs& m, const FieldArgs& f, const double* lam, double cfl, double unsteady, double* dt,
-               double* alpha, hipStream_t s) {
+               double* alpha, bool flux_end, hipStream_t s) {
     if (m.nc > 0)
-        hipLaunchKernelGGL(k_dt, grid_for(m.nc), dim3(kBlock), 0, s, m.nc, f.cs, f.ld, lam, cfl, unsteady, dt, alpha);
-}
-
-void launch_dt_explicit(const MeshArgs& m, const FieldArgs& f, const double* lam, double cfl, double* dt,
-                        double* alpha, hipStream_t s) {
-    if (m.nc > 0)
-        hipLaunchKernelGGL(k_dt_explicit, grid_for(m.nc), dim3(kBlock), 0, s, m.nc, f.cs, f.ld, lam, cfl, dt, alpha);
+        hipLaunchKernelGGL(k_dt, grid_for(m.nc), dim3(kBlock), 0, s, m.nc, f.cs, f.ld, lam, cfl, unsteady, dt, alpha,
+                           flux_end ? f.stamp : nullptr);
 }
 
 void launch_planes_to_device(int nc, const int* mesh_of_row, const double* src, double* dst, hipStream_t s) {
@@ -1259,8 +1287,16 @@ void launch_planes_to_mesh(int nc, const int* mesh_of_row, const double* src, do
     if (nc > 0) hipLaunchKernelGGL(k_permute_planes<false>, grid_for(nc), dim3(kBlock), 0, s, nc, mesh_of_row, src, dst);
 }
 
-void launch_explicit_update(const MeshArgs& m, const FieldArgs& f, const double* alpha, double* U, hipStream_t s) {
-    if (m.nc > 0) hipLaunchKernelGGL(k_explicit_update, grid_for(m.nc), dim3(kBlock), 0, s, m.nc, alpha, f.res, U);
+int launch_explicit_step(const MeshArgs& m, const FieldArgs& f, const double* lam, double cfl, double* dt,
+                         double* alpha, double* U, double* partial, hipStream_t s) {
+    const int nb = reduction_blocks(m.nc);
+    hipLaunchKernelGGL(k_explicit_step, dim3(nb), dim3(kBlock), 0, s, m.nc, f.cs, f.ld, lam, cfl, f.res, dt, alpha, U,
+                       partial, f.stamp);
+    return nb;
+}
+
+void launch_stamp(unsigned long long* stamp, int k, int k2, hipStream_t s) {
+    hipLaunchKernelGGL(k_stamp, dim3(1), dim3(1), 0, s, stamp, k, k2);
 }
 
 void launch_unsteady_source(const MeshArgs& m, const FieldArgs& f, int bdf, double inv_dt, const double* Un,

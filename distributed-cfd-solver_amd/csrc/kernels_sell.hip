@@ -33,6 +33,7 @@
 #include "kernels.hpp"
 #include "kernels_sell.hpp"
 #include "kernels_sell_device.hpp"
+#include "reduce_device.hpp"
 
 namespace cfdg {
 
@@ -190,19 +191,91 @@ __global__ void __launch_bounds__(kBlock) k_sell_scatter(SellArgs b, const int* 
     for (int v = 0; v < 5; ++v) d[v] = u[v * kSellRows];
 }
 
-// b = -R, the implicit right-hand side (implicit_euler.hpp:81-92)
-__global__ void __launch_bounds__(kBlock) k_sell_rhs(SellArgs b, int ld, const double* res, double* rhs) {
-    const int p = blockIdx.x * kBlock + threadIdx.x;
-    if (p >= b.nslices * kSellRows) return;
-    const int row = b.row[p];
-    if (row < 0) return;
-    double* d = rhs + vec_at(p);
-    for (int v = 0; v < 5; ++v) d[v * kSellRows] = -res[static_cast<long long>(v) * ld + row];
+// The positions of the sliced layout in grid-stride order, f(position, device row)
+// for those that hold a row and as many workgroups as a reduction has partial sums.
+template <class F>
+__device__ __forceinline__ void for_rows(const SellArgs& b, F&& f) {
+    const int end = b.nslices * kSellRows, stride = static_cast<int>(gridDim.x * blockDim.x);
+    for (int p = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); p < end; p += stride) {
+        const int row = b.row[p];
+        if (row >= 0) f(p, row);
+    }
+}
+
+// Partial sums of squares for launch_bicg_start: by component, and the total of the
+// positions before first_end.
+struct Squares {
+    double all[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, first = 0.0;
+    __device__ __forceinline__ void store(double* partial) const {
+        __shared__ double lds[2][kBlock / 64 * 5];
+        const double f[5] = {first, 0.0, 0.0, 0.0, 0.0};
+        const double s = block_sums(all, 5, lds[0]);
+        const double s0 = block_sums(f, 1, lds[1]);
+        if (threadIdx.x < 5) partial[blockIdx.x * 5 + threadIdx.x] = s;
+        if (threadIdx.x == 0) partial[5 * kMaxPartials + blockIdx.x] = s0;
+    }
+};
+
+// b = -R, the implicit right-hand side (implicit_euler.hpp:81-92), x = 0, and the
+// squares of R: one pass where the norms and (b, b) took one each and x a fill.
+__global__ void __launch_bounds__(kBlock) k_sell_rhs(SellArgs b, int ld, const double* res, double* rhs, double* x,
+                                                     int first_end, double* partial, int* singular,
+                                                     unsigned long long* stamp, int jacobian_end) {
+    stamp_stage(stamp, kStampLinear);
+    if (jacobian_end) stamp_stage(stamp, kStampJacobianEnd);
+    if (blockIdx.x == 0 && threadIdx.x == 0) *singular = 0;
+    Squares q;
+    for_rows(b, [&](int p, int row) {
+        const long long at = vec_at(p);
+        for (int v = 0; v < 5; ++v) {
+            const double r = res[static_cast<long long>(v) * ld + row];
+            rhs[at + v * kSellRows] = -r;
+            x[at + v * kSellRows] = 0.0;
+            q.all[v] += r * r;
+            if (p < first_end) q.first += r * r;
+        }
+    });
+    q.store(partial);
+}
+
+// The squares of a vector, added as the kernels above and below add theirs.
+template <class TV>
+__global__ void __launch_bounds__(kBlock) k_sell_squares(SellArgs b, const TV* u, int first_end, double* partial) {
+    Squares q;
+    for_rows(b, [&](int p, int) {
+        const long long at = vec_at(p);
+        for (int v = 0; v < 5; ++v) {
+            const double d = static_cast<double>(u[at + v * kSellRows]);
+            q.all[v] += d * d;
+            if (p < first_end) q.first += d * d;
+        }
+    });
+    q.store(partial);
+}
+
+// The right-hand side of a defect correction's inner solve, b = r in FP32, x = 0, and
+// the squares of b.
+__global__ void __launch_bounds__(kBlock) k_sell_inner_rhs(SellArgs b, const double* r, float* rhs, float* x,
+                                                           int first_end, double* partial) {
+    Squares q;
+    for_rows(b, [&](int p, int) {
+        const long long at = vec_at(p);
+        for (int v = 0; v < 5; ++v) {
+            const float f = static_cast<float>(r[at + v * kSellRows]);
+            rhs[at + v * kSellRows] = f;
+            x[at + v * kSellRows] = 0.0f;
+            const double d = static_cast<double>(f);
+            q.all[v] += d * d;
+            if (p < first_end) q.first += d * d;
+        }
+    });
+    q.store(partial);
 }
 
 // U = U + du (implicit_euler.hpp:53-61)
 __global__ void __launch_bounds__(kBlock) k_sell_state_update(SellArgs b, int ld, const double* du, double* U,
-                                                              double* du_cells) {
+                                                              double* du_cells, unsigned long long* stamp) {
+    stamp_stage(stamp, kStampLinearEnd);
     const int row = blockIdx.x * kBlock + threadIdx.x;
     if (row >= b.n) return;
     const double* d = du + vec_at(b.pos[row]);
@@ -343,14 +416,34 @@ void launch_sell_scatter(const SellArgs& b, const int* dst_of, const double* src
     if (b.n > 0) hipLaunchKernelGGL(k_sell_scatter, grid_for(b.n), dim3(kBlock), 0, s, b, dst_of, src, dst);
 }
 
-void launch_sell_rhs(const SellArgs& b, int ld, const double* res, double* rhs, hipStream_t s) {
-    if (b.nslices > 0)
-        hipLaunchKernelGGL(k_sell_rhs, grid_for_slices(b.nslices), dim3(kBlock), 0, s, b, ld, res, rhs);
+int launch_sell_rhs(const SellArgs& b, int ld, const double* res, double* rhs, double* x, int first_slices,
+                    double* partial, int* singular, unsigned long long* stamp, bool jacobian_end, hipStream_t s) {
+    const int nb = reduction_blocks(static_cast<long long>(b.nslices) * kSellRows);
+    hipLaunchKernelGGL(k_sell_rhs, dim3(nb), dim3(kBlock), 0, s, b, ld, res, rhs, x, first_slices * kSellRows, partial,
+                       singular, stamp, jacobian_end ? 1 : 0);
+    return nb;
+}
+
+template <class TV>
+int launch_sell_squares(const SellArgs& b, const TV* u, int first_slices, double* partial, hipStream_t s) {
+    const int nb = reduction_blocks(static_cast<long long>(b.nslices) * kSellRows);
+    hipLaunchKernelGGL(k_sell_squares<TV>, dim3(nb), dim3(kBlock), 0, s, b, u, first_slices * kSellRows, partial);
+    return nb;
+}
+template int launch_sell_squares<double>(const SellArgs&, const double*, int, double*, hipStream_t);
+template int launch_sell_squares<float>(const SellArgs&, const float*, int, double*, hipStream_t);
+
+int launch_sell_inner_rhs(const SellArgs& b, const double* r, float* rhs, float* x, int first_slices, double* partial,
+                          hipStream_t s) {
+    const int nb = reduction_blocks(static_cast<long long>(b.nslices) * kSellRows);
+    hipLaunchKernelGGL(k_sell_inner_rhs, dim3(nb), dim3(kBlock), 0, s, b, r, rhs, x, first_slices * kSellRows, partial);
+    return nb;
 }
 
 void launch_sell_state_update(const SellArgs& b, int ld, const double* du, double* U, double* du_cells,
-                              hipStream_t s) {
-    if (b.n > 0) hipLaunchKernelGGL(k_sell_state_update, grid_for(b.n), dim3(kBlock), 0, s, b, ld, du, U, du_cells);
+                              unsigned long long* stamp, hipStream_t s) {
+    if (b.n > 0)
+        hipLaunchKernelGGL(k_sell_state_update, grid_for(b.n), dim3(kBlock), 0, s, b, ld, du, U, du_cells, stamp);
 }
 
 void launch_sell_get_blocks(const int* code, long long n, const SellMatrix& m, double* out, hipStream_t s) {

@@ -50,10 +50,21 @@ void launch_sell_sweep(const SellArgs& b, const SellMatrix& m, int first, int co
 // row itself when src_of is null), and back.
 void launch_sell_gather(const SellArgs& b, const int* src_of, const double* src, double* dst, hipStream_t s);
 void launch_sell_scatter(const SellArgs& b, const int* dst_of, const double* src, double* dst, hipStream_t s);
-// b = -R in the sliced layout; U += du with du in the sliced layout, du also
-// written per cell (5 values, device order).
-void launch_sell_rhs(const SellArgs& b, int ld, const double* res, double* rhs, hipStream_t s);
-void launch_sell_state_update(const SellArgs& b, int ld, const double* du, double* U, double* du_cells, hipStream_t s);
+// b = -R and x = 0 in the sliced layout, *singular = 0, with the partial sums for
+// launch_bicg_start (their number is returned); jacobian_end: the launch directly
+// after the Jacobian's.
+int launch_sell_rhs(const SellArgs& b, int ld, const double* res, double* rhs, double* x, int first_slices,
+                    double* partial, int* singular, unsigned long long* stamp, bool jacobian_end, hipStream_t s);
+// the partial sums alone, of any vector of the layout
+template <class TV>
+int launch_sell_squares(const SellArgs& b, const TV* u, int first_slices, double* partial, hipStream_t s);
+// b = r in FP32 and x = 0, likewise
+int launch_sell_inner_rhs(const SellArgs& b, const double* r, float* rhs, float* x, int first_slices, double* partial,
+                          hipStream_t s);
+// U += du with du in the sliced layout, du also written per cell (5 values, device
+// order); stamps the solve's end.
+void launch_sell_state_update(const SellArgs& b, int ld, const double* du, double* U, double* du_cells,
+                              unsigned long long* stamp, hipStream_t s);
 // Row-major 25-entry blocks k0 .. k0 + n of a list of block codes (setup.hpp,
 // sell_block_codes) from and to the sliced layout; to_csr keeps the storage
 // type (block layout of precision.hpp).
