@@ -529,7 +529,12 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
     // iterations enqueued in batches and the state read back once per
     // batch; iterations past convergence or breakdown are no-ops.
     const int slot = (sizeof(T) == sizeof(double)) ? 0 : 1;
-    int batch = std::max(1, c.last_iters[slot] - 1);
+    // An iteration too many costs 8 empty launches, 20 us, one too few a wait and a batch
+    // more.  Solves of up to three iterations mostly take as many as the last one (3k-cell
+    // ramp 12.3 -> 10.5 ms for 60 steps); longer ones vary, and one less with two to
+    // follow is the better guess (dual time at 94k cells 15.3 against 15.8 ms).
+    const int last = c.last_iters[slot];
+    int batch = std::max(1, last <= 3 ? last : last - 1);
     // the dependency levels' first group is solved by the vector kernels
     const bool levels = P.kind == CFDG_PRECOND_SGS && !P.sliced();
     long long enq = 0;
@@ -1294,8 +1299,7 @@ int cfdg_set_state(cfdg_ctx* c, const double* U, int64_t ld) {
             c->pipe.to_device(dev, U + at, bytes, c->stream);
         });
         cfdg::launch_planes_to_device(c->nc, c->mesh_of_row.get(), c->stage.get(), c->U.get(), c->stream);
-        c->check_launch();
-        c->sync();
+        c->finish();
         c->have_residual = false;
         c->have_dt = false;
         c->have_prev_du = false;

@@ -460,34 +460,84 @@ __global__ void __launch_bounds__(kTileCells) k_gradient_limiter_lds(MeshArgs m,
     }
 }
 
-// The wide staged form with two lanes per cell (workgroups of up to 512
-// lanes): its 1,088 LDS slots allow two workgroups per CU, so one lane per
-// cell would leave two waves per SIMD to hide the stencil loop's latencies.
-// The two lanes of a cell (adjacent lanes) split the cell's vertex stencil by
-// chunks of four entries (lane h takes chunks h, h + 2, ...), each adding
-// its entries in stencil order with the arithmetic of gradient_limiter_cell;
-// the second lane's sums are then added to the first lane's, which stores the
-// gradients and forms the limiter.  The sums are therefore those of the
-// one-lane form up to the order of that one addition.  Node LSQ only (the
+// The second half of gradient_limiter_cell by kLanes lanes of one cell, lane h taking
+// the variables h, h + kLanes, ...: the same operations per variable.
+template <int kLanes, class Self, class NbF, class FVec>
+__device__ __forceinline__ void store_and_limit_split(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, int c,
+                                                      int h, const Self& self, const double (&g)[5][3], NbF nbf,
+                                                      FVec fvec) {
+    constexpr int kRounds = (5 + kLanes - 1) / kLanes;
+    const CellRefW rc = crecw(f, c);
+    int var[kRounds];
+    bool on[kRounds];
+    double gv[kRounds][3], qc[kRounds], qmax[kRounds], qmin[kRounds], ph[kRounds];
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int v = h + r * kLanes;
+        on[r] = v < 5;
+        var[r] = on[r] ? v : 4;
+        for (int d = 0; d < 3; ++d) {
+            gv[r][d] = g[0][d];
+            for (int w = 1; w < 5; ++w) gv[r][d] = (var[r] == w) ? g[w][d] : gv[r][d];
+            if (on[r]) rc[kRG + 3 * var[r] + d] = gv[r][d];
+        }
+        qc[r] = self[kRQ + var[r]];
+        qmax[r] = qmin[r] = qc[r];
+        ph[r] = 1.0;
+    }
+    if (!nm.muscl) return;
+    for (int j = m.ccf_off[c], k = 0; j < m.ccf_off[c + 1]; ++j, ++k) {
+        const auto rn = nbf(j, k);
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
+            const double qn = rn[kRQ + var[r]];
+            qmax[r] = dmax(qmax[r], qn);
+            qmin[r] = dmin(qmin[r], qn);
+        }
+    }
+    const double x0 = self[kRC], y0 = self[kRC + 1], z0 = self[kRC + 2];
+    const double eps2 = nm.k3 * rc[kRVol];
+    for (int e = m.cf_off[c], k = 0; e < m.cf_off[c + 1]; ++e, ++k) {
+        double ex, ey, ez;
+        fvec(e, k, x0, y0, z0, ex, ey, ez);
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
+            const double df = gv[r][0] * ex + gv[r][1] * ey + gv[r][2] * ez;
+            const double dnb = (df > 0.0) ? (qmax[r] - qc[r]) : (qmin[r] - qc[r]);
+            ph[r] = dmin(ph[r], limiter_phi(nm.limiter, dnb, df, eps2));
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r)
+        if (on[r]) rc[kRPhi + var[r]] = ph[r];
+}
+
+// The staged forms with two lanes per cell (workgroups of up to 512 lanes), where one lane per cell leaves too few waves to hide the
+// stencil loop's latencies (launch_gradient_limiter).  The lanes of a cell (adjacent
+// lanes) split the cell's vertex stencil by chunks of four entries (lane h takes
+// chunks h, h + kLanes, ...), each adding its entries in stencil order with the
+// arithmetic of gradient_limiter_cell; the two lanes' sums are then added.  The sums
+// are therefore those of the one-lane form up to the order of that one addition.  The
+// limiter's variables are split over the lanes.  Node LSQ only (the
 // only gradient the staged forms serve).
-template <bool kSA>
-__global__ void __launch_bounds__(2 * kTileCells) k_gradient_limiter_pair(MeshArgs m, FieldArgs f, NumArgs nm,
-                                                                          SaArgs sa) {
+template <bool kSA, int kSlots>
+__global__ void __launch_bounds__(2 * kTileCells) k_gradient_limiter_lanes(MeshArgs m, FieldArgs f, NumArgs nm,
+                                                                           SaArgs sa) {
+    constexpr int kLanes = 2;
     stamp_stage(f.stamp, kStampGradients);
-    constexpr int kSlots = kGradSlotsBig;
     __shared__ __attribute__((aligned(16))) double sq[(kSA ? 9 : 8) * kSlots];
     const int t = xcd_block(blockIdx.x, gridDim.x);
     const int c0 = m.gtile_off[t], nt = m.gtile_off[t + 1] - c0;
     const int hb = m.tile_halo_off[t], ns = nt + (m.tile_halo_off[t + 1] - hb);
-    const int cell = static_cast<int>(threadIdx.x >> 1), half = static_cast<int>(threadIdx.x & 1);
+    const int cell = static_cast<int>(threadIdx.x) / kLanes, h = static_cast<int>(threadIdx.x) % kLanes;
     const bool live = cell < nt;
     const int nchn = (m.ccn_base[t + 1] - m.ccn_base[t]) / (4 * nt);
     const SlotChunk* chn = reinterpret_cast<const SlotChunk*>(m.ccn_slot + m.ccn_base[t]) + cell;
     // this lane's first two vertex-slot chunks, requested before the staging
     SlotChunk cur = 0, nxt = 0;
     if (live) {
-        if (half < nchn) cur = chn[half * nt];
-        if (half + 2 < nchn) nxt = chn[(half + 2) * nt];
+        if (h < nchn) cur = chn[h * nt];
+        if (h + kLanes < nchn) nxt = chn[(h + kLanes) * nt];
     }
     for (int sl = threadIdx.x; sl < ns; sl += blockDim.x) {
         const int src = (sl < nt) ? c0 + sl : m.tile_halo[hb + sl - nt];
@@ -511,10 +561,10 @@ __global__ void __launch_bounds__(2 * kTileCells) k_gradient_limiter_pair(MeshAr
         const CellRef ri{f.cs, f.ld, c};
         const double i0 = ri[kRInv], i1 = ri[kRInv + 1], i2 = ri[kRInv + 2], i4 = ri[kRInv + 3], i5 = ri[kRInv + 4],
                      i8 = ri[kRInv + 5];
-        for (int q = half; 4 * q < cnt; q += 2) {
+        for (int q = h; 4 * q < cnt; q += kLanes) {
             const SlotChunk ch = cur;
             cur = nxt;
-            if (q + 4 < nchn) nxt = chn[(q + 4) * nt];
+            if (q + 2 * kLanes < nchn) nxt = chn[(q + 2 * kLanes) * nt];
             for (int e = 0; e < 4 && 4 * q + e < cnt; ++e) {
                 const int slot = chunk_slot(ch, e);
                 const LdsSlot<kSlots> rn{sq, slot};
@@ -540,17 +590,22 @@ __global__ void __launch_bounds__(2 * kTileCells) k_gradient_limiter_pair(MeshAr
             }
         }
     }
-    // the second lane's sums added to the first lane's (every lane takes part)
-    for (int v = 0; v < 5; ++v)
-        for (int d = 0; d < 3; ++d) g[v][d] += __shfl_xor(g[v][d], 1, 64);
-    if constexpr (kSA)
-        for (int d = 0; d < 3; ++d) gs[d] += __shfl_xor(gs[d], 1, 64);
-    if (!live || half != 0) return;
+    // the lanes' sums added (every lane takes part)
+#pragma unroll
+    for (int x = 1; x < kLanes; x <<= 1) {
+        for (int v = 0; v < 5; ++v)
+            for (int d = 0; d < 3; ++d) g[v][d] += __shfl_xor(g[v][d], x, 64);
+        if constexpr (kSA)
+            for (int d = 0; d < 3; ++d) gs[d] += __shfl_xor(gs[d], x, 64);
+    }
+    if (!live) return;
     if constexpr (kSA) {
         const long long nc = m.nc;
-        sa.g[c] = gs[0];
-        sa.g[nc + c] = gs[1];
-        sa.g[2 * nc + c] = gs[2];
+        if (h == 0) {
+            sa.g[c] = gs[0];
+            sa.g[nc + c] = gs[1];
+            sa.g[2 * nc + c] = gs[2];
+        }
     }
     // the limiter's face neighbours and face vectors, in order, as the one-lane form reads them
     const int nchf = (m.ccf_base[t + 1] - m.ccf_base[t]) / (4 * nt);
@@ -573,7 +628,7 @@ __global__ void __launch_bounds__(2 * kTileCells) k_gradient_limiter_pair(MeshAr
         ey = fvp[(vw + k) * nt];
         ez = fvp[(2 * vw + k) * nt];
     };
-    store_and_limit(m, f, nm, c, self, g, nbf, fvec);
+    store_and_limit_split<kLanes>(m, f, nm, c, h, self, g, nbf, fvec);
 }
 
 __device__ __forceinline__ void grad_dirichlet(double* g, const double* gi, double qin, double qfix, double nx,
@@ -769,14 +824,14 @@ struct TileFaceRef {
 // With turbulence the kernel also records each face's mass flux F[0] (from
 // the tile that owns the face's owner cell); eddy viscosity follows the
 // cells (residual_kernel.hpp:229-230, 282-283).
-template <bool kTurb>
-__global__ void __launch_bounds__(kFluxThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) k_flux(MeshArgs m, FieldArgs f, NumArgs nm) {
+template <bool kTurb, int kThreads>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4, 4))) k_flux(MeshArgs m, FieldArgs f, NumArgs nm) {
     stamp_stage(f.stamp, kStampFlux);
     __shared__ double sc[kFluxPlanes * kTileCells];  // staged planes, then the fluxes sF[6][kTileFaces]
     __shared__ double smut[kTurb ? kTileCells : 1];
     __shared__ int scf[kTileCells + 1 + 2 * kTileFaces];  // the tile's cf_off (rebased), then its cf_slot entries
     static_assert(6 * kTileFaces <= kFluxPlanes * kTileCells, "flux area must fit the staging area");
-    constexpr int kPerLane = kTileFaces / kFluxThreads;  // faces per lane
+    constexpr int kPerLane = kTileFaces / kThreads;  // faces per lane
     const int t = xcd_block(blockIdx.x, gridDim.x);
     const int c0 = m.tile_off[t], nt = m.tile_off[t + 1] - c0;
     const int fb = m.tile_face_off[t], nfl = m.tile_face_off[t + 1] - fb;
@@ -785,7 +840,7 @@ __global__ void __launch_bounds__(kFluxThreads) __attribute__((amdgpu_waves_per_
     double fz[kPerLane];
 #pragma unroll
     for (int r = 0; r < kPerLane; ++r) {  // this lane's faces: cells (and index), issued before the staging loads
-        const int j = i + r * kFluxThreads;
+        const int j = i + r * kThreads;
         cx[r] = cy[r] = 0;
         fz[r] = 0.0;
         if (j < nfl) {
@@ -802,7 +857,7 @@ __global__ void __launch_bounds__(kFluxThreads) __attribute__((amdgpu_waves_per_
     // and limiter (2-6) for MUSCL, gradients (7-14) for MUSCL or viscous terms
     {
         const int sl = i % kTileCells, g = i / kTileCells;
-        constexpr int kGroups = kFluxThreads / kTileCells, kPairs = kFluxPlanes / 2;
+        constexpr int kGroups = kThreads / kTileCells, kPairs = kFluxPlanes / 2;
         const int p_hi = (nm.muscl || nm.viscous) ? kPairs : 3;
         if (sl < nt) {
             for (int p = g; p < p_hi; p += kGroups) {
@@ -816,13 +871,13 @@ __global__ void __launch_bounds__(kFluxThreads) __attribute__((amdgpu_waves_per_
         // (at most two entries per tile face); ne > 2 kTileFaces cannot occur
         const int e0 = m.cf_off[c0], ne = m.cf_off[c0 + nt] - e0;
         if (i <= nt) scf[i] = m.cf_off[c0 + i] - e0;
-        for (int e = i; e < ne; e += kFluxThreads) scf[kTileCells + 1 + e] = m.cf_slot[e0 + e];
+        for (int e = i; e < ne; e += kThreads) scf[kTileCells + 1 + e] = m.cf_slot[e0 + e];
     }
     __syncthreads();
     double F[kPerLane][6];
 #pragma unroll
     for (int r = 0; r < kPerLane; ++r) {
-        const int j = i + r * kFluxThreads;
+        const int j = i + r * kThreads;
         for (int v = 0; v < 6; ++v) F[r][v] = 0.0;
         if (j >= nfl) break;  // later faces of the lane are out of range too
         const TileFaceRef fr{m.tf, m.tld, fb + j, fz[r]};
@@ -852,7 +907,7 @@ __global__ void __launch_bounds__(kFluxThreads) __attribute__((amdgpu_waves_per_
     double* sF = sc;
 #pragma unroll
     for (int r = 0; r < kPerLane; ++r) {
-        const int j = i + r * kFluxThreads;
+        const int j = i + r * kThreads;
         if (j < nfl)
             for (int v = 0; v < 6; ++v) sF[v * kTileFaces + j] = F[r][v];
     }
@@ -1216,25 +1271,36 @@ void launch_primitives(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm,
                            cells);
 }
 
+// Tiles up to which each has a CU of its own.
+constexpr int kFewTiles = 256;
+
+template <bool kSA>
+static void launch_staged_gradient(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const SaArgs& sa,
+                                   hipStream_t s) {
+    const unsigned cells = static_cast<unsigned>(m.gblock);
+    const dim3 g(static_cast<unsigned>(m.ngtiles));
+    // Two lanes per cell in the wide form, whose LDS leaves room for two workgroups per
+    // CU, and where there is no second workgroup for a CU anyway.  The narrow form with
+    // one / two lanes: 12 tiles 17.2 / 14.5 us, 106 tiles 21.8 / 18.7, 384 tiles 27.8 /
+    // 28.2, 1,024 tiles 44.8 / 52.4, 8,192 tiles 330 / 432 (four lanes are slower from
+    // the start: 17.6, 21.1, 41).
+    if (m.gslots > kGradSlots)
+        hipLaunchKernelGGL((k_gradient_limiter_lanes<kSA, kGradSlotsBig>), g, dim3(2 * cells), 0, s, m, f, nm, sa);
+    else if (m.ngtiles <= kFewTiles)
+        hipLaunchKernelGGL((k_gradient_limiter_lanes<kSA, kGradSlots>), g, dim3(2 * cells), 0, s, m, f, nm, sa);
+    else
+        hipLaunchKernelGGL((k_gradient_limiter_lds<kSA, kGradSlots>), g, dim3(cells), 0, s, m, f, nm, sa);
+}
+
 bool launch_gradient_limiter(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, hipStream_t s,
                              const SaArgs* sa) {
     if (m.nc <= 0) return false;
     if (m.tile_halo_off != nullptr) {
-        const dim3 g(static_cast<unsigned>(m.ngtiles)), b(static_cast<unsigned>(m.gblock));
-        const bool big = m.gslots > kGradSlots;
-        const dim3 b2(2u * static_cast<unsigned>(m.gblock));  // the wide form: two lanes per cell
-        if (sa) {
-            if (big)
-                hipLaunchKernelGGL((k_gradient_limiter_pair<true>), g, b2, 0, s, m, f, nm, *sa);
-            else
-                hipLaunchKernelGGL((k_gradient_limiter_lds<true, kGradSlots>), g, b, 0, s, m, f, nm, *sa);
-            return true;
-        }
-        if (big)
-            hipLaunchKernelGGL((k_gradient_limiter_pair<false>), g, b2, 0, s, m, f, nm, SaArgs{});
+        if (sa)
+            launch_staged_gradient<true>(m, f, nm, *sa, s);
         else
-            hipLaunchKernelGGL((k_gradient_limiter_lds<false, kGradSlots>), g, b, 0, s, m, f, nm, SaArgs{});
-        return false;
+            launch_staged_gradient<false>(m, f, nm, SaArgs{}, s);
+        return sa != nullptr;
     }
     hipLaunchKernelGGL(k_gradient_limiter, grid_for(m.nc), dim3(kBlock), 0, s, m, f, nm);
     return false;
@@ -1250,12 +1316,25 @@ void launch_ghost_gradients(const MeshArgs& m, const FieldArgs& f, const NumArgs
     if (nbf > 0) hipLaunchKernelGGL(k_ghost_gradients, grid_for(nbf), dim3(kBlock), 0, s, m, f, nm, bcs);
 }
 
+template <int kThreads>
+static void launch_flux_as(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, hipStream_t s) {
+    const dim3 g(static_cast<unsigned>(m.ntiles)), b(kThreads);
+    if (f.mut)
+        hipLaunchKernelGGL((k_flux<true, kThreads>), g, b, 0, s, m, f, nm);
+    else
+        hipLaunchKernelGGL((k_flux<false, kThreads>), g, b, 0, s, m, f, nm);
+}
+
 void launch_flux(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, hipStream_t s) {
     if (m.ntiles <= 0) return;
-    if (f.mut)
-        hipLaunchKernelGGL(k_flux<true>, dim3(static_cast<unsigned>(m.ntiles)), dim3(kFluxThreads), 0, s, m, f, nm);
+    // One face per lane where every tile has a CU of its own, else two, so that two
+    // tiles share a CU.  Two / one per lane: 12 tiles 16.2 / 14.9 us, 106 tiles 19.1 / 17.1,
+    // 188 tiles of tetrahedra with eddy viscosity 35 / 29, 384 tiles 26.6 / 30.7, 1,024
+    // tiles 54 / 63.
+    if (m.ntiles <= kFewTiles)
+        launch_flux_as<2 * kFluxThreads>(m, f, nm, s);
     else
-        hipLaunchKernelGGL(k_flux<false>, dim3(static_cast<unsigned>(m.ntiles)), dim3(kFluxThreads), 0, s, m, f, nm);
+        launch_flux_as<kFluxThreads>(m, f, nm, s);
 }
 
 void launch_boundary_integrals(const MeshArgs& m, const FieldArgs& f, int n_patches, double* out, hipStream_t s) {
