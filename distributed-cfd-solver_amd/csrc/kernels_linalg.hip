@@ -6,9 +6,9 @@
 //   k_lu_factor   diagonal-block LU with partial pivoting (bsr_helpers.hpp:278-321)
 //   k_spmv        y = A x, five lanes per block row (bsr_helpers.hpp:139-203)
 //   k_sgs_group   one Gauss-Seidel row update for every row of one row group
-//                 (bsr_helpers.hpp:390-435 for a single row), eight lanes per
-//                 row; a sweep launches the groups in order (colours, or
-//                 dependency levels)
+//                 (bsr_helpers.hpp:390-435 for a single row), five lanes per
+//                 row; a sweep launches the groups (dependency levels) in order
+//   k_sgs_levels  both sweeps of a small system in one launch
 //   vector ops    the BiCGSTAB updates of bicgstab.cpp:97-177, fused
 //   reductions    dot products: per-block partial sums in a fixed order, then
 //                 one block adds the partials in a fixed order -> the result
@@ -252,7 +252,8 @@ __global__ void __launch_bounds__(kBlock) k_sgs_group(const int* rows, int count
 // workgroup, z in LDS, for systems that fit it.  A level of a small system holds a
 // few dozen rows, so a launch per level (k_sgs_group) is all latency: 5 to 7 us for
 // each of the 2 x 66 levels of a 48 x 16 x 4 mesh, 950 us for M^-1 r.  Here a level
-// costs a barrier, the products of LDS reads and a 5x5 solve; everything that does
+// costs a barrier, the products of LDS reads and a 5x5 solve (1 us for a row, 2 us for
+// 64 rows, whose six waves share the SIMDs: 265 us for M^-1 r); everything that does
 // not depend on z -- blocks, factors, right-hand side -- is in flight before its
 // level begins: the waves take the chunks of twelve rows (kSgsRowsPerWave) in turn,
 // and a wave requests its next chunk when it has finished one.  The barriers wait for

@@ -1,6 +1,6 @@
 // Device functions and launch rules of the kernels on the sliced block layout
 // (kernels_sell.hip, kernels_reduced.hip): block and factor loads, the 5x5
-// solve, and the walk over a slice's slots by one wave or by eight.
+// solve, and the walk over a slice's slots by one wave, four or eight.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -165,14 +165,14 @@ __device__ __forceinline__ int wave_slice() {
 }
 
 // Waves per slice.  A launch over few slices is bound by the latency of a row's
-// chain of slots, so eight waves share a slice (a hexahedron's or tetrahedron's
-// slots all at once); over many slices one wave each fills the chip and the
-// split only adds barriers.  The line lies where the two cross (1,536 slices =
-// 1.5 waves per SIMD), per BiCGSTAB iteration with one wave / with eight: 24,576-cell
-// plate (192 slices per colour) FP64 108 / 77 us, BF16 80 / 61 us; 93,765 cells (735) 147 /
-// 151, 96 / 92; 156,849 cells (1,226) 250 / 231, 114 / 115; 262,144 cells (2,048) 370 /
-// 393, 144 / 156.
-constexpr int kSplitWaves = 8, kSplitSlices = 1536;
+// chain of slots, so eight or four waves share a slice (a hexahedron's or tetrahedron's
+// slots all at once, or in two goes); over many slices one wave each fills the chip and
+// the split only adds barriers.  Per BiCGSTAB iteration with one / four / eight waves
+// (slices of a colour): 24,576-cell plate (192) FP64 70 / 47 / 45 us, BF16 41 / 33 / 31;
+// 93,765 cells (735) 80 / 77 / 81, 53 / 51 / 49; 156,849 cells (1,226) 132 / 116 / 116,
+// 62 / 62 / 64; 196,608 cells (1,536) 157 / 153 / 160, 65 / 68 / 71; 162,000 tetrahedra
+// (four colours) 157 / 151 / 166, 102 / 100 / 102; 262,144 cells (2,048) 193 / - / -, 73.
+constexpr int kEightSlices = 384, kSplitSlices = 1536;
 static_assert(kSplitSlices <= kMaxPartials, "a product over that many slices leaves one partial sum each");
 template <int kSplit>
 dim3 slice_grid(int slices) {
@@ -181,8 +181,10 @@ dim3 slice_grid(int slices) {
 // f(std::integral_constant<int, waves per slice>) for a launch over that many slices
 template <class F>
 void with_split(int slices, F&& f) {
-    if (slices <= kSplitSlices)
-        f(std::integral_constant<int, kSplitWaves>{});
+    if (slices <= kEightSlices)
+        f(std::integral_constant<int, 8>{});
+    else if (slices <= kSplitSlices)
+        f(std::integral_constant<int, 4>{});
     else
         f(std::integral_constant<int, 1>{});
 }

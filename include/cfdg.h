@@ -540,8 +540,8 @@ int cfdg_set_warm_start(cfdg_ctx* ctx, cfdg_gnn* gnn);
 /* Solves since cfdg_set_warm_start that kept / rejected the prediction. */
 int cfdg_warm_start_stats(cfdg_ctx* ctx, int64_t* used, int64_t* rejected);
 
-/* Device time (milliseconds, HIP events on the context stream) of the last
-   call of each stage: 0 primitives+ghosts, 1 gradients, 2 limiter,
+/* Device time (milliseconds, device clock at the stage boundaries) of the last
+   call of each stage, 0 before the first: 0 primitives+ghosts, 1 gradients, 2 limiter,
    3 flux residual, 4 Jacobian assembly, 5 linear solve. */
 int cfdg_stage_times(cfdg_ctx* ctx, double ms[6]);
 /* Launches the flux-residual kernel reps times back to back on the context

@@ -47,7 +47,7 @@ def _bicgstab(A, M, b, x, iterations):
 
 @pytest.mark.parametrize("guess", [False, True])
 @pytest.mark.parametrize("kind, size", [("hex", (3, 2, 1)), ("hex", (13, 11, 3)), ("tet", (2, 1, 3)), ("tet", (7, 6, 5)),
-                                        ("tet", (11, 13, 9)), ("hex", (64, 64, 49))])
+                                        ("tet", (11, 13, 9)), ("hex", (41, 40, 31)), ("hex", (64, 64, 49))])
 def test_iterates_match_numpy(kind, size, guess):
     mesh, s, rp, cols, dg, v = _solver(kind, size, "fp64")
     colour = s.sgs_row_groups(cfdg.SGS_MULTICOLOUR)[0]
@@ -66,7 +66,7 @@ def test_iterates_match_numpy(kind, size, guess):
 
 
 @pytest.mark.parametrize("form", sorted(FORMS))
-@pytest.mark.parametrize("kind, size", [("hex", (13, 11, 3)), ("tet", (7, 6, 5)), ("tet", (41, 23, 19)),
+@pytest.mark.parametrize("kind, size", [("hex", (13, 11, 3)), ("tet", (7, 6, 5)), ("tet", (41, 23, 19)), ("hex", (41, 40, 31)),
                                         ("hex", (64, 64, 49))])
 def test_forms_reach_the_tolerance(kind, size, form):
     """More iterations than a batch, past the 32nd (true residual norm); the
