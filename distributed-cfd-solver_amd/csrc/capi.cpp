@@ -647,6 +647,26 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
     return res;
 }
 
+// An inner solve that broke off with a grown residual (BiCGSTAB at its iteration limit;
+// seen with residuals up to 300 times the right-hand side on the plate at CFL 1000, where
+// the step then left the range of the state) has been added to x: keeps the multiple of
+// the correction e with the smallest residual, theta = (r_old, A e) / (A e, A e), instead.
+// On entry c.r is the residual with the whole of e; returns the norm of the new one.
+double shorten_correction(cfdg_ctx& c, const Precond& P, long long N, double* x) {
+    double* const e = c.s.get();
+    double* const ae = c.t.get();
+    double* const r = c.r.get();
+    cfdg::launch_cast_f32_to_f64(N, c.f32.x.get(), e, c.stream);
+    spmv_stored<double>(c, P, e, ae);
+    const double ee = dot_device<double>(c, N, ae, ae);
+    const double back = ee > 0.0 ? -dot_device<double>(c, N, r, ae) / ee : 0.0;  // 1 - theta
+    if (std::isfinite(back)) {
+        cfdg::launch_axpy_copy<double>(N, x, -back, e, x, c.stream);
+        cfdg::launch_axpy_copy<double>(N, r, back, ae, r, c.stream);
+    }
+    return std::sqrt(dot_device<double>(c, N, r, r));
+}
+
 // FP64 defect correction around FP32 BiCGSTAB + SGS (the FP32 precision form):
 // x (FP64, initial guess on entry), b (FP64).  Every pass forms r = b - A x in
 // FP64 arithmetic over the stored blocks and solves A e = r in FP32 from e = 0.
@@ -743,7 +763,9 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
         }
         cfdg::launch_add_f32(N, c.f32.x.get(), x, c.stream);
         r = c.r.get();
+        const double before = rnorm;
         rnorm = outer_residual();
+        if (std::isfinite(rnorm) && rnorm > before) rnorm = shorten_correction(c, P, N, x);
     }
     c.check_launch();
     res.iterations = total;
