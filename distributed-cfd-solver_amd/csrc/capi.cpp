@@ -25,7 +25,7 @@
 #include "ctx.hpp"
 #include "kernels.hpp"
 #include "kernels_linalg.hpp"
-#include "kernels_reduced.hpp"
+#include "kernels_multicolour.hpp"
 #include "kernels_sell.hpp"
 #include "mesh.hpp"
 #include "setup.hpp"
@@ -263,17 +263,6 @@ void ensure_csr(cfdg_ctx& c) {
     c.have_csr = true;
 }
 
-// The work vectors in the layout of the next solve; the sliced kernels and
-// reductions rely on zeros past a slice's rows.
-void use_layout(cfdg_ctx& c, bool sliced) {
-    if (sliced && !c.vectors_sliced) {
-        for (DBuf<double>* v : {&c.r, &c.r0, &c.p, &c.v, &c.s, &c.t, &c.ph, &c.sh}) v->zero(c.stream);
-        auto& f = c.f32;
-        for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh}) v->zero(c.stream);
-    }
-    c.vectors_sliced = sliced;
-}
-
 // in_step: the caller's next launch stamps the end of the stage, and waits later.
 void eval_residual(cfdg_ctx& c, bool in_step) {
     c.have_features = false;
@@ -338,17 +327,6 @@ void require_jacobian(const cfdg_ctx& c) {
                         "no block values in the current storage: cfdg_assemble_jacobian or cfdg_set_bsr_values first");
 }
 
-template <class T>
-double dot_device(cfdg_ctx& c, long long n, const T* a, const T* b) {
-    cfdg::DotPairsT<T> pr{};
-    pr.a[0] = a;
-    pr.b[0] = b;
-    cfdg::launch_dots(n, 1, pr, c.partial.get(), c.dots.get(), c.stream, c.publish());
-    c.check_launch();
-    c.wait();
-    return c.blk->v[0];
-}
-
 struct Precond {
     int kind = CFDG_PRECOND_NONE;
     int order = CFDG_SGS_MULTICOLOUR;
@@ -361,22 +339,36 @@ struct Precond {
 long long vector_size(const cfdg_ctx& c, const Precond& P) { return P.sliced() ? c.sliced_size() : 5LL * c.nc; }
 
 // Work vectors of one Krylov precision.
-cfdg::RedVecs<double> kvecs64(cfdg_ctx& c) {
-    return {c.r.get(), c.r0.get(), c.p.get(),  c.v.get(),  c.s.get(),
-            c.t.get(), c.ph.get(), c.sh.get(), c.rd.get(), c.rg.get()};
+cfdg::KrylovVecs<double> kvecs64(cfdg_ctx& c) {
+    return {c.r.get(), c.r0.get(), c.p.get(), c.v.get(), c.s.get(), c.t.get(), c.ph.get(), c.sh.get()};
 }
-cfdg::RedVecs<float> kvecs32(cfdg_ctx& c) {
+cfdg::KrylovVecs<float> kvecs32(cfdg_ctx& c) {
     auto& f = c.f32;
-    return {f.r.get(), f.r0.get(), f.p.get(),  f.v.get(),  f.s.get(),
-            f.t.get(), f.ph.get(), f.sh.get(), f.rd.get(), f.rg.get()};
+    return {f.r.get(), f.r0.get(), f.p.get(), f.v.get(), f.s.get(), f.t.get(), f.ph.get(), f.sh.get()};
 }
 
 template <class T>
 void spmv_stored(cfdg_ctx& c, const Precond& P, const T* x, T* y, const double* gate = nullptr) {
     if (P.sliced())
-        cfdg::launch_sell_spmv<T>(c.sellargs(), c.sellmatrix(), x, y, c.stream, gate);
+        cfdg::launch_sell_spmv<T>(c.sellargs(), c.sellmatrix(), 0, c.n_slices(), x, y, c.stream, gate);
     else
         cfdg::launch_spmv<T>(c.bargs(), c.values.get(), c.storage, x, y, c.stream, gate);
+}
+
+// (a, b) in the order of the device rows, handed over to the host.
+double dot_device(cfdg_ctx& c, const Precond& P, const double* a, const double* b) {
+    if (P.sliced()) {
+        const int nb = cfdg::launch_sell_dots<double>(c.sellargs(), 1, a, b, b, c.partial.get(), c.stream);
+        cfdg::launch_reduce_partials(nb, 1, c.partial.get(), c.dots.get(), c.publish(), c.stream);
+    } else {
+        cfdg::DotPairsT<double> pr{};
+        pr.a[0] = a;
+        pr.b[0] = b;
+        cfdg::launch_dots(5LL * c.nc, 1, pr, c.partial.get(), c.dots.get(), c.stream, c.publish());
+    }
+    c.check_launch();
+    c.wait();
+    return c.blk->v[0];
 }
 
 // z = M^-1 r: z = 0, forward groups, backward groups (preconditioners.cpp:171-194).
@@ -435,7 +427,6 @@ void precond_apply(cfdg_ctx& c, const Precond& P, const T* r, T* z, const double
 // the row either way.
 // singular_clear: the flag is zero already.
 void precond_setup(cfdg_ctx& c, const Precond& P, bool singular_clear = false) {
-    use_layout(c, P.sliced());
     if (!P.sliced()) ensure_csr(c);
     c.singular_known = false;
     if (P.kind != CFDG_PRECOND_SGS) return;
@@ -468,24 +459,17 @@ void precond_check(cfdg_ctx& c, const Precond& P) {
 // Right-preconditioned BiCGSTAB (bicgstab.cpp:42-201) on device vectors of
 // type T (FP64: the reference's arithmetic; FP32: the inner solve of the
 // defect correction).  x holds the initial guess on entry and the solution on
-// exit.  Scalars and dot products are FP64.  The multicolour order runs in the
-// reduced form (kernels_reduced.hip), with two exceptions: one colour only, and
-// reduce = false.  parts: the number of partial sums that the kernel which formed bvec
-// left for launch_bicg_start, 0 for none.  A solve whose s vanishes exactly is repeated so, because the
-// reference ends there as broken down unless the rounding of its product, which
-// the reduced form does not have, leaves a remainder to go on with.
+// exit.  Scalars and dot products are FP64.  parts: the partial sums that the kernel
+// which formed bvec left for launch_bicg_start (multicolour order, dots 0 for none).
 template <class T>
-cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& P, const cfdg::RedVecs<T>& w, T* x,
-                          const T* bvec, bool zero_fallback = false, bool x_zero = false, int parts = 0,
-                          bool reduce = true) {
+cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& P, const cfdg::KrylovVecs<T>& w, T* x,
+                          const T* bvec, bool zero_fallback = false, bool x_zero = false, cfdg::SellSums parts = {}) {
     const long long N = vector_size(c, P);
     const std::size_t bytes = static_cast<std::size_t>(N) * sizeof(T);
     cfdg_iter_result res{CFDG_MAX_ITERATIONS, 0, 0.0, 0.0};
+    const bool sliced = P.sliced();
     const int* cs = c.sell.colour_slice.data();
     const int colours = static_cast<int>(c.sell.colour_slice.size()) - 1;
-    const bool reduced = P.sliced() && reduce && colours > 1;
-    // entries of the first colour, which the reduced form leaves out of its vectors
-    const long long skip = reduced ? cfdg::sell_vector_size(cs[1]) : 0;
     const auto b = c.sellargs();
     const auto m = c.sellmatrix();
     // two state blocks: an iteration that ends in launch_xr_next reads one and
@@ -502,13 +486,11 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
         cfdg::launch_axpy_copy<T>(N, bvec, -1.0, w.v, w.r, c.stream);
         r = w.r;
     }
-    if (reduced) {
-        double* const part = c.partial.get();
-        if (parts == 0) parts = cfdg::launch_sell_squares<T>(b, bvec, cs[1], part, c.stream);
-        if (!x_zero) cfdg::launch_sell_squares<T>(b, r, cs[1], part + cfdg::kSquares, c.stream);
+    if (sliced) {
+        if (parts.dots == 0) parts.dots = cfdg::launch_sell_dots<T>(b, x_zero ? 1 : 2, bvec, r, r, c.partial.get(), c.stream);
         // FP32: the norms are the outer right-hand side's, not this one's
-        cfdg::launch_bicg_start(parts, part, !x_zero, sizeof(T) == sizeof(double) ? c.norms.get() : nullptr, ks,
-                                zero_fallback, lp.abs_tol, lp.rel_tol, lp.max_iter, cfdg::Publish{}, c.stream);
+        cfdg::launch_bicg_start(parts.dots, parts.norms, c.partial.get(), !x_zero, c.norms.get(), ks, zero_fallback,
+                                lp.abs_tol, lp.rel_tol, lp.max_iter, cfdg::Publish{}, c.stream);
     } else {
         cfdg::DotPairsT<T> pr{};
         pr.a[0] = pr.b[0] = bvec;
@@ -518,9 +500,7 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
                                lp.max_iter, c.stream);
     }
     if (zero_fallback) cfdg::launch_bicg_reject<T>(N, ks, bvec, x, w.r, c.stream);
-    if (reduced) {
-        cfdg::launch_red_start<T>(b, m, cs, r, w, ks, c.stream);
-    } else {
+    if (!sliced) {
         if (x_zero) hip_check(hipMemcpyAsync(w.r, bvec, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
         hip_check(hipMemcpyAsync(w.r0, w.r, bytes, hipMemcpyDeviceToDevice, c.stream), "copy");
         hip_check(hipMemsetAsync(w.v, 0, bytes, c.stream), "memset");
@@ -536,18 +516,20 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
     const int last = c.last_iters[slot];
     int batch = std::max(1, last <= 3 ? last : last - 1);
     // the dependency levels' first group is solved by the vector kernels
-    const bool levels = P.kind == CFDG_PRECOND_SGS && !P.sliced();
+    const bool levels = P.kind == CFDG_PRECOND_SGS && !sliced;
     long long enq = 0;
     double* rr = c.dots.get() + 5;
-    // with the reduced form and the dependency levels, every iteration but the last
-    // of a batch (and the ones with the true residual norm) ends with launch_xr_next,
-    // which also forms the next iteration's p and the first solves of its M^-1 p
-    bool p_ready = false;
+    // with SGS, every iteration but the last of a batch (and the ones with the true
+    // residual norm) ends with launch_xr_next, which also forms the next iteration's p
+    // and the first group of its M^-1 p; the multicolour order's start forms the first
+    bool p_ready = sliced;
+    if (sliced) cfdg::launch_mc_start<T>(b, m, cs, r, w, ks, c.stream);
     // y = p (op 0) or s (op 1), z = M^-1 y, A z, and the dot products of the step
     const auto product = [&](int op) {
-        if (reduced) {
-            if (!(op == 0 && p_ready)) cfdg::launch_red_vec<T>(op, b, m, cs, w, ks, c.stream);
-            cfdg::launch_red_product<T>(op, b, m, cs, colours, w, c.partial.get(), c.dots.get(), ks, c.stream);
+        if (sliced) {
+            if (!(op == 0 && p_ready)) cfdg::launch_mc_vec<T>(op, b, m, cs, w, ks, c.stream);
+            cfdg::launch_mc_product<T>(op, b, m, cs, colours, c.sell.first_slots, w, c.partial.get(), c.dots.get(), ks,
+                                       c.stream);
             return;
         }
         T* const y = op == 0 ? w.p : w.s;
@@ -582,24 +564,26 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
             product(0);
             product(1);
             const bool next_in_batch = k + 1 < batch && enq <= lp.max_iter;
-            p_ready = (reduced || levels) && next_in_batch && enq % 32 != 0;
+            p_ready = (sliced || levels) && next_in_batch && enq % 32 != 0;
             if (p_ready) {
-                if (reduced)
-                    cfdg::launch_red_xr_next<T>(b, m, cs, w, x, ks, kb[1 - cur], c.stream);
+                if (sliced)
+                    cfdg::launch_mc_xr_next<T>(b, m, cs, w, x, ks, kb[1 - cur], c.stream);
                 else
                     cfdg::launch_xr_next<T>(c.nc, ks, kb[1 - cur], w.ph, w.sh, w.s, w.t, x, w.r, w.v, w.p,
                                             c.row_first.get(), c.storage, c.lu_csr.get(), c.piv.get(), c.stream);
                 cur = 1 - cur;
                 continue;
             }
-            cfdg::launch_update_xr_g<T>(N - skip, ks, w.ph + skip, w.sh + skip, w.s + skip, w.t + skip, x + skip,
-                                        w.r + skip, c.stream);
+            cfdg::launch_update_xr_g<T>(N, ks, w.ph, w.sh, w.s, w.t, x, w.r, c.stream);
             const bool true_norm = enq % 32 == 0;  // of the residual, every 32 iterations
-            if (true_norm) {
+            if (true_norm && sliced) {
+                const int nb = cfdg::launch_sell_dots<T>(b, 1, w.r, w.r, w.r, c.partial.get(), c.stream, ks);
+                cfdg::launch_reduce_step(nb, 1, c.partial.get(), rr, ks, cfdg::kStepPost, c.stream);
+            } else if (true_norm) {
                 cfdg::DotPairsT<T> pr{};
-                pr.a[0] = w.r + skip;
-                pr.b[0] = w.r + skip;
-                cfdg::launch_dots_step(N - skip, 1, pr, c.partial.get(), rr, ks, cfdg::kStepPost, c.stream);
+                pr.a[0] = w.r;
+                pr.b[0] = w.r;
+                cfdg::launch_dots_step(N, 1, pr, c.partial.get(), rr, ks, cfdg::kStepPost, c.stream);
             }
             if (!true_norm || !next_in_batch)
                 cfdg::launch_bicg_post(ks, !true_norm, c.norms.get(), c.singular.get(),
@@ -613,37 +597,20 @@ cfdg_iter_result bicgstab(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& 
         if (h[cfdg::kKsStatus] != 0.0 || enq > lp.max_iter) break;
         batch = 2;
     }
-    int it = static_cast<int>(h[cfdg::kKsIt]);
-    double rnorm = h[cfdg::kKsRnorm];
+    const int it = static_cast<int>(h[cfdg::kKsIt]);
     const double st = h[cfdg::kKsStatus];
-    const double updates = h[cfdg::kKsUpdates];
     res.status = (st == cfdg::kKsConverged) ? CFDG_CONVERGED
                                              : (st == cfdg::kKsDiverged ? CFDG_DIVERGED : CFDG_MAX_ITERATIONS);
     res.initial_residual = h[cfdg::kKsRnorm0];
-    bool rejected = false;
     if (zero_fallback) {
-        rejected = h[cfdg::kKsReject] != 0.0;
-        if (rejected)
+        if (h[cfdg::kKsReject] != 0.0)
             ++c.warm_rejected;
         else
             ++c.warm_used;
     }
-    if (reduced && updates > 0.0) {
-        cfdg::launch_red_finish<T>(b, m, cs, bvec, w, x, ks, c.stream);
-        c.check_launch();
-    }
-    if (st == cfdg::kKsExact) {
-        cfdg_linparams rest = lp;
-        rest.max_iter = lp.max_iter - (it - 1);
-        const cfdg_iter_result r2 =
-            bicgstab<T>(c, rest, P, w, x, bvec, false, updates == 0.0 && (x_zero || rejected), 0, false);
-        res.status = r2.status;
-        rnorm = r2.final_residual;
-        it += r2.iterations - 1;
-    }
     if (it > 0) c.last_iters[slot] = it;
     res.iterations = it;
-    res.final_residual = rnorm;
+    res.final_residual = h[cfdg::kKsRnorm];
     return res;
 }
 
@@ -658,13 +625,13 @@ double shorten_correction(cfdg_ctx& c, const Precond& P, long long N, double* x)
     double* const r = c.r.get();
     cfdg::launch_cast_f32_to_f64(N, c.f32.x.get(), e, c.stream);
     spmv_stored<double>(c, P, e, ae);
-    const double ee = dot_device<double>(c, N, ae, ae);
-    const double back = ee > 0.0 ? -dot_device<double>(c, N, r, ae) / ee : 0.0;  // 1 - theta
+    const double ee = dot_device(c, P, ae, ae);
+    const double back = ee > 0.0 ? -dot_device(c, P, r, ae) / ee : 0.0;  // 1 - theta
     if (std::isfinite(back)) {
         cfdg::launch_axpy_copy<double>(N, x, -back, e, x, c.stream);
         cfdg::launch_axpy_copy<double>(N, r, back, ae, r, c.stream);
     }
-    return std::sqrt(dot_device<double>(c, N, r, r));
+    return std::sqrt(dot_device(c, P, r, r));
 }
 
 // FP64 defect correction around FP32 BiCGSTAB + SGS (the FP32 precision form):
@@ -672,14 +639,14 @@ double shorten_correction(cfdg_ctx& c, const Precond& P, long long N, double* x)
 // FP64 arithmetic over the stored blocks and solves A e = r in FP32 from e = 0.
 cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const Precond& P, double* x,
                                    const double* bvec, bool zero_fallback = false, bool x_zero = false,
-                                   int parts = 0) {
+                                   cfdg::SellSums parts = {}) {
     const long long N = vector_size(c, P);
     cfdg_iter_result res{CFDG_MAX_ITERATIONS, 0, 0.0, 0.0};
     const double* r = c.r.get();  // the outer residual
     const auto outer_residual = [&]() {
         spmv_stored<double>(c, P, x, c.v.get());
         cfdg::launch_axpy_copy<double>(N, bvec, -1.0, c.v.get(), c.r.get(), c.stream);
-        return std::sqrt(dot_device<double>(c, N, c.r.get(), c.r.get()));
+        return std::sqrt(dot_device(c, P, c.r.get(), c.r.get()));
     };
     // ||b|| and the first outer residual's norm (r = b for a zero guess)
     double bnorm = 0.0, rnorm = 0.0;
@@ -692,14 +659,12 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
         }
         const cfdg::Publish pub = c.publish();
         if (P.sliced()) {
-            const auto b = c.sellargs();
-            double* const part = c.partial.get();
-            const bool rhs = parts > 0;  // an implicit step's: its norms
-            if (!rhs) parts = cfdg::launch_sell_squares<double>(b, bvec, 0, part, c.stream);
-            if (!x_zero) cfdg::launch_sell_squares<double>(b, r, 0, part + cfdg::kSquares, c.stream);
-            cfdg::launch_bicg_start(parts, part, !x_zero, rhs ? c.norms.get() : nullptr, nullptr, false, 0.0, 0.0, 0,
-                                    pub, c.stream);
-            c.norms_known = rhs;
+            if (parts.dots == 0)
+                parts.dots = cfdg::launch_sell_dots<double>(c.sellargs(), x_zero ? 1 : 2, bvec, r, r, c.partial.get(),
+                                                            c.stream);
+            cfdg::launch_bicg_start(parts.dots, parts.norms, c.partial.get(), !x_zero, c.norms.get(), nullptr, false,
+                                    0.0, 0.0, 0, pub, c.stream);
+            c.norms_known = parts.norms > 0;  // an implicit step's
         } else {
             cfdg::DotPairsT<double> pr{};
             pr.a[0] = pr.b[0] = bvec;
@@ -724,7 +689,7 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
     }
     const double tol = std::max(lp.abs_tol, lp.rel_tol * ((bnorm > 0.0) ? bnorm : 1.0));
     res.initial_residual = rnorm;
-    const cfdg::RedVecs<float> w = kvecs32(c);
+    const cfdg::KrylovVecs<float> w = kvecs32(c);
     int total = 0;
     for (int pass = 0;; ++pass) {
         if (!std::isfinite(rnorm)) {
@@ -739,10 +704,10 @@ cfdg_iter_result defect_correction(cfdg_ctx& c, const cfdg_linparams& lp, const 
             res.status = CFDG_MAX_ITERATIONS;
             break;
         }
-        int inner_parts = 0;
+        cfdg::SellSums inner_parts{};
         if (P.sliced()) {
-            inner_parts = cfdg::launch_sell_inner_rhs(c.sellargs(), r, c.f32.b.get(), c.f32.x.get(),
-                                                      c.sell.colour_slice[1], c.partial.get(), c.stream);
+            inner_parts = cfdg::launch_sell_inner_rhs(c.sellargs(), r, c.f32.b.get(), c.f32.x.get(), c.partial.get(),
+                                                      c.stream);
         } else {
             cfdg::launch_cast_f64_to_f32(N, r, c.f32.b.get(), c.stream);
             c.f32.x.zero(c.stream);
@@ -825,8 +790,7 @@ Precond linear_solve(cfdg_ctx& c, const cfdg_linparams& lp, const double* hb, co
         c.h2d(dst, d.data(), n5);
         c.sync();
     };
-    const int first = c.sell.colour_slice.size() > 2 ? c.sell.colour_slice[1] : 0;
-    int parts = 0;
+    cfdg::SellSums parts{};
     c.norms_known = false;
     if (hb) {
         upload(hb, b);
@@ -834,7 +798,8 @@ Precond linear_solve(cfdg_ctx& c, const cfdg_linparams& lp, const double* hb, co
     } else {
         if (!c.have_residual) throw CfdgError(CFDG_ERR_STATE, "implicit right-hand side needs a residual");
         if (sliced) {
-            parts = cfdg::launch_sell_rhs(c.sellargs(), c.nc, c.res.get(), b, x, first, c.partial.get(),
+            // without a guess its (b, b) starts the solve
+            parts = cfdg::launch_sell_rhs(c.sellargs(), c.nc, c.res.get(), b, x, !hx0 && !c.warm, c.partial.get(),
                                           c.singular.get(), c.stamp.get(), in_step, c.stream);
         } else {
             cfdg::launch_stamp(c.stamp.get(), cfdg::kStampLinear, in_step ? cfdg::kStampJacobianEnd : -1, c.stream);
@@ -853,10 +818,6 @@ Precond linear_solve(cfdg_ctx& c, const cfdg_linparams& lp, const double* hb, co
             hip_check(hipMemsetAsync(x, 0, static_cast<std::size_t>(vector_size(c, P)) * sizeof(double), c.stream),
                       "memset");
         x_zero = true;
-    }
-    if (parts > 0 && first == 0 && c.prec.krylov != CFDG_PREC_FP32) {  // one colour: no launch_bicg_start to add them
-        cfdg::launch_reduce_partials(parts, 5, c.partial.get(), c.norms.get(), cfdg::Publish{}, c.stream);
-        parts = 0;
     }
     precond_setup(c, P, !hb && sliced);
     const cfdg_iter_result r = (c.prec.krylov == CFDG_PREC_FP32)
@@ -1049,7 +1010,8 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
         c.sell_row.upload(c.sell.row, s);
         c.sell_pos.upload(c.sell.pos, s);
         c.sell_count.upload(c.sell.count, s);
-        c.sell_lower0.upload(c.sell.lower0, s);
+        c.sell_before.upload(c.sell.before, s);
+        c.sell_order.upload(c.sell.order, s);
         c.sell_cols.upload(c.sell.cols, s);
         c.sell_tile_pos.upload(c.sell.tile_pos, s);
         c.sell_visit.upload(c.sell.visit, s);
@@ -1058,7 +1020,7 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
         c.sync();
         for (auto* v : {&c.sell.row, &c.sell.tile_pos, &c.sell.visit_base}) std::vector<i32>().swap(*v);
         std::vector<std::uint32_t>().swap(c.sell.visit);
-        std::vector<std::uint16_t>().swap(c.sell.lower0);
+        for (auto* v : {&c.sell.before, &c.sell.order}) std::vector<std::uint16_t>().swap(*v);
         const cfdg::Csr ccf_dev = to_device_rows(c.ccf_mesh, c.new2old, &c.old2new);
         c.ccf_off.upload(ccf_dev.off, s);
         c.ccf.upload(ccf_dev.idx, s);
@@ -1172,11 +1134,11 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
     alloc_lu(c, 0);
     c.sell_piv.alloc(z(c.n_slices()) * cfdg::kSellRows);
     c.singular.alloc(1);
-    for (DBuf<double>* v : {&c.r, &c.r0, &c.p, &c.v, &c.s, &c.t, &c.ph, &c.sh, &c.rd, &c.rg, &c.bs, &c.xs, &c.b, &c.x}) {
+    for (DBuf<double>* v : {&c.r, &c.r0, &c.p, &c.v, &c.s, &c.t, &c.ph, &c.sh, &c.bs, &c.xs, &c.b, &c.x}) {
         v->alloc(v == &c.b || v == &c.x ? 5 * ncs : c.vector_alloc());
         v->zero(s);
     }
-    c.partial.alloc(2 * static_cast<std::size_t>(cfdg::kSquares));
+    c.partial.alloc(cfdg::kNormPartials + 5 * static_cast<std::size_t>(cfdg::kReduceBlocks));
     c.dots.alloc(8);
     c.norms.alloc(5);
     c.norms.zero(s);
@@ -1265,13 +1227,13 @@ void set_precision(cfdg_ctx& c, const cfdg_precision& p) {
     alloc_lu(c, lu_f32);
     if (p.krylov == CFDG_PREC_FP32) {
         auto& f = c.f32;
-        for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh, &f.rd, &f.rg}) {
+        for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh}) {
             if (v->size() != c.vector_alloc()) v->alloc(c.vector_alloc());
             v->zero(c.stream);
         }
     } else {
         auto& f = c.f32;
-        for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh, &f.rd, &f.rg}) v->alloc(0);
+        for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh}) v->alloc(0);
     }
     c.sync();
     c.storage = storage;
@@ -1569,9 +1531,8 @@ int cfdg_spmv(cfdg_ctx* c, const double* x, double* y) {
     return guarded(c, [&] {
         if (!x || !y) throw CfdgError(CFDG_ERR_ARG, "null vector");
         require_jacobian(*c);
-        use_layout(*c, true);
         upload_sliced(*c, x, c->s.get());
-        cfdg::launch_sell_spmv<double>(c->sellargs(), c->sellmatrix(), c->s.get(), c->t.get(), c->stream);
+        cfdg::launch_sell_spmv<double>(c->sellargs(), c->sellmatrix(), 0, c->n_slices(), c->s.get(), c->t.get(), c->stream);
         c->check_launch();
         download_sliced(*c, c->t.get(), y);
     });

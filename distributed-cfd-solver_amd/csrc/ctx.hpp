@@ -117,7 +117,7 @@ struct cfdg_ctx {
     DBuf<int4> sell_slice;
     DBuf<int> sell_row, sell_pos, sell_cols, sell_tile_pos, sell_visit_base;
     DBuf<std::uint32_t> sell_count, sell_visit;
-    DBuf<std::uint16_t> sell_piv, sell_lower0;
+    DBuf<std::uint16_t> sell_piv, sell_before, sell_order;
     DBuf<std::uint8_t> sell_off, sell_diag, lu;
     DBuf<int> mesh_of_row;  // device row -> mesh cell
     DBuf<int> block_code;   // where each block of the ABI's pattern is stored, made on first use
@@ -151,12 +151,10 @@ struct cfdg_ctx {
     cfdg::Csr ccf_mesh;
     bool have_seq_groups = false;
     // Krylov work vectors; FP32 set for the FP32 form.  Layout of a solve: 5
-    // per row in device order, or sliced (then zero past a slice's rows).
-    bool vectors_sliced = true;
+    // per row in device order, or sliced.
     DBuf<double> r, r0, p, v, s, t, ph, sh;
-    DBuf<double> rd, rg;  // d and g of the reduced form (kernels_reduced.hpp)
     struct F32 {
-        DBuf<float> b, x, r, r0, p, v, s, t, ph, sh, rd, rg;
+        DBuf<float> b, x, r, r0, p, v, s, t, ph, sh;
     } f32;
     DBuf<double> b, x;    // right-hand side and solution, 5 per cell in device order
     DBuf<double> bs, xs;  // the same in the sliced layout
@@ -293,8 +291,9 @@ struct cfdg_ctx {
         a.row = sell_row.get();
         a.pos = sell_pos.get();
         a.count = sell_count.get();
-        a.lower0 = sell_lower0.get();
+        a.before = sell_before.get();
         a.cols = sell_cols.get();
+        a.order = sell_order.get();
         a.tile_pos = sell_tile_pos.get();
         a.visit = sell_visit.get();
         a.visit_base = sell_visit_base.get();

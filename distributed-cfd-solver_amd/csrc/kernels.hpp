@@ -210,7 +210,7 @@ struct BsrArgs {
 // (slot, lane) is element (slot * 25 + e) * 64 + lane (SellLayout), so the 64
 // lanes of a wave, each on a row of its own, read and write whole cache
 // lines.  Vectors of this layout hold component v of the row at (slice, lane)
-// at (slice * 5 + v) * 64 + lane, zero past a slice's rows.
+// at (slice * 5 + v) * 64 + lane; the elements past a slice's rows are never read.
 constexpr int kSellRows = 64;
 struct SellArgs {
     int n;                    // rows
@@ -219,8 +219,9 @@ struct SellArgs {
     const int* row;           // position -> device row, -1 past a slice's rows
     const int* pos;           // device row -> position
     const std::uint32_t* count;  // per position: lower blocks | upper blocks << 16
-    const std::uint16_t* lower0;  // per position: lower blocks with a column of the first colour, before the others
+    const std::uint16_t* before;  // per position: off-diagonal blocks whose mesh column precedes the row's
     const int* cols;          // per (slot, lane): position of the column
+    const std::uint16_t* order;  // slices with lower and upper slots: the slot of the row's k-th block in column order
     const int* tile_pos;      // the Jacobian's rows and visits (SellPlan)
     const std::uint32_t* visit;
     const int* visit_base;

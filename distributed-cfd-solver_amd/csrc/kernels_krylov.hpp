@@ -1,5 +1,5 @@
 // Device functions of the BiCGSTAB recurrence shared by the Krylov kernels
-// (kernels_linalg.hip, kernels_reduced.hip): the scalar steps on the state block and
+// (kernels_linalg.hip, kernels_multicolour.hip): the scalar steps on the state block and
 // the entry-wise vector updates.
 #pragma once
 
@@ -20,9 +20,7 @@ __device__ inline void bicg_begin(double* ks) {
     }
     ks[kKsIt] += 1.0;
     ks[kKsFirst] = (ks[kKsIt] == 1.0) ? 1.0 : 0.0;
-    if (ks[kKsFirst] != 0.0) {
-        ks[kKsAp] = ks[kKsAr];
-    } else {
+    if (ks[kKsFirst] == 0.0) {
         const double beta = (ks[kKsRho] / ks[kKsRhoOld]) * (ks[kKsAlpha] / ks[kKsOmega]);
         if (!isfinite(beta)) {
             ks[kKsStatus] = kKsDiverged;
@@ -30,8 +28,6 @@ __device__ inline void bicg_begin(double* ks) {
         }
         ks[kKsBeta] = beta;
         ks[kKsNbo] = -beta * ks[kKsOmega];
-        // p = r + beta (p - omega v) with v = p in the first colour
-        ks[kKsAp] = ks[kKsAr] + beta * (ks[kKsAp] * (1.0 - ks[kKsOmega]));
     }
 }
 
@@ -42,13 +38,11 @@ __device__ inline void bicg_post(double* ks, const double* rr) {
     double rnorm = ks[kKsRnNew];
     const double omega_new = ks[kKsOmegaNew];
     ks[kKsRnorm] = rnorm;
-    ks[kKsUpdates] += 1.0;
-    ks[kKsAr] = ks[kKsAs] * (1.0 - omega_new);  // r = s - omega t with t = s
     if (!isfinite(rnorm) || !isfinite(omega_new) || omega_new == 0.0) {
         ks[kKsStatus] = kKsDiverged;
         return;
     }
-    if (rr) rnorm = sqrt(rr[0] + ks[kKsAr] * ks[kKsAr] * ks[kKsB0]);
+    if (rr) rnorm = sqrt(rr[0]);
     ks[kKsRnorm] = rnorm;
     if (rnorm <= ks[kKsTol]) {
         ks[kKsStatus] = kKsConverged;
@@ -68,9 +62,9 @@ __device__ inline void bicg_post(double* ks, const double* rr) {
 // The end-of-iteration checks and the start of the next iteration inside a
 // vector kernel: formed by thread 0 of every workgroup from the state ks_in
 // alone, so every workgroup takes the same decision, workgroup 0 writing the
-// result to ks_out; next (LDS) = status, first, beta, nbo and the first colour's
-// multiple in p of the next iteration.  False when the solve had ended before.
-constexpr int kNextCount = 5;
+// result to ks_out; next (LDS) = status, first, beta, nbo of the next
+// iteration.  False when the solve had ended before.
+constexpr int kNextCount = 4;
 __device__ __forceinline__ bool next_iteration(const double* ks_in, double* ks_out, double next[kNextCount]) {
     const bool lead = blockIdx.x == 0 && threadIdx.x == 0;
     if (ks_in[kKsStatus] != 0.0) {  // ended before: carry the state over
@@ -86,7 +80,6 @@ __device__ __forceinline__ bool next_iteration(const double* ks_in, double* ks_o
         next[1] = st[kKsFirst];
         next[2] = st[kKsBeta];
         next[3] = st[kKsNbo];
-        next[4] = st[kKsAp];
         if (lead)
             for (int k = 0; k < kKsCount; ++k) ks_out[k] = st[k];
     }

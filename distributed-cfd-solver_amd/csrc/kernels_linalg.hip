@@ -418,8 +418,8 @@ __global__ void __launch_bounds__(kBlock) k_update_xr(long long n, double alpha,
 
 // Start of a solve (bicgstab.cpp:56-92): norms, tolerance, initial status,
 // then the start of the first iteration.
-__device__ void bicg_init(double* ks, const double* dots, int x_zero, int fallback, int reduced, double abs_tol,
-                          double rel_tol, int max_iter) {
+__device__ void bicg_init(double* ks, const double* dots, int x_zero, int fallback, double abs_tol, double rel_tol,
+                          int max_iter) {
     const double bnorm = sqrt(dots[0]);
     double rnorm = x_zero ? bnorm : sqrt(dots[1]);
     double reject = 0.0;
@@ -439,14 +439,6 @@ __device__ void bicg_init(double* ks, const double* dots, int x_zero, int fallba
     ks[kKsRnorm] = rnorm;
     ks[kKsRnorm0] = rnorm;
     ks[kKsReject] = reject;
-    if (reduced) {
-        const double b0 = dots[x_zero ? 1 : (reject != 0.0 ? 3 : 2)];
-        ks[kKsReduced] = 1.0;
-        if (b0 > 0.0) {
-            ks[kKsB0] = b0;
-            ks[kKsAr] = 1.0;
-        }
-    }
     if (!isfinite(rnorm))
         ks[kKsStatus] = kKsDiverged;
     else if (rnorm <= tol)
@@ -457,7 +449,7 @@ __device__ void bicg_init(double* ks, const double* dots, int x_zero, int fallba
 
 __global__ void k_bicg_init(double* ks, const double* dots, int x_zero, int fallback, double abs_tol, double rel_tol,
                             int max_iter) {
-    bicg_init(ks, dots, x_zero, fallback, 0, abs_tol, rel_tol, max_iter);
+    bicg_init(ks, dots, x_zero, fallback, abs_tol, rel_tol, max_iter);
 }
 
 // A rejected guess restarts from zero: x = 0, r = b.
@@ -472,31 +464,27 @@ __global__ void __launch_bounds__(kBlock) k_bicg_reject(long long n, const doubl
 
 // gamma = (r0, v); alpha = rho / gamma (bicgstab.cpp:113-120)
 __device__ void bicg_alpha(double* ks, const double* dots) {
-    const double gamma = dots[0] + ks[kKsAp] * ks[kKsB0];
+    const double gamma = dots[0];
     if (!isfinite(gamma) || gamma == 0.0) {
         ks[kKsStatus] = kKsDiverged;
         return;
     }
     ks[kKsAlpha] = ks[kKsRho] / gamma;
-    ks[kKsAs] = ks[kKsAr] - ks[kKsAlpha] * ks[kKsAp];  // s = r - alpha v with v = p
 }
 
 // omega = (t, s) / (t, t); the recurrence norm of the new r and rho_new
 // (bicgstab.cpp:126-160); dots = (t,t), (t,s), (r0,t), (r0,s), (s,s)
 __device__ void bicg_omega(double* ks, const double* dots) {
-    // the first colour's t = s: (t,t) = (t,s) = (s,s) and (r0,t) = (r0,s)
-    const double first = ks[kKsAs] * ks[kKsAs] * ks[kKsB0];
-    const double tt = dots[0] + first, ts = dots[1] + first, r0t = dots[2], r0s = dots[3], ss = dots[4];
+    const double tt = dots[0], ts = dots[1], r0t = dots[2], r0s = dots[3], ss = dots[4];
     if (!isfinite(ts) || !isfinite(tt) || tt == 0.0) {
-        ks[kKsStatus] = (ks[kKsReduced] != 0.0 && tt == 0.0 && ss == 0.0) ? kKsExact : kKsDiverged;
+        ks[kKsStatus] = kKsDiverged;
         return;
     }
     const double omega_new = ts / tt;
-    const double rest = 1.0 - omega_new;
-    const double rn2 = (ss - 2.0 * omega_new * dots[1] + omega_new * omega_new * dots[0]) + first * (rest * rest);
+    const double rn2 = ss - 2.0 * omega_new * ts + omega_new * omega_new * tt;
     ks[kKsOmegaNew] = omega_new;
     ks[kKsRnNew] = sqrt(rn2 > 0.0 ? rn2 : 0.0);
-    ks[kKsRhoNew] = (r0s - omega_new * r0t) + ks[kKsAs] * rest * ks[kKsB0];
+    ks[kKsRhoNew] = r0s - omega_new * r0t;
 }
 
 // The end of the iteration, unless the step that formed the true residual norm took
@@ -704,48 +692,27 @@ __global__ void __launch_bounds__(kBlock) k_reduce_step(int nblocks, int ncomp, 
     if constexpr (kStep == kStepPost) bicg_post(ks, sums);
 }
 
-// The start of a reduced solve from the squares of its right-hand side and, for a
-// guess, of its residual: partial sums per component (norms takes the right-hand
-// side's) and behind them the first colour's.
-__device__ __forceinline__ void sum_squares(int nblocks, const double* partial, double* lds, double sums[6]) {
-    const double s = sum_partials(nblocks, 5, partial, lds);
-    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    for (int b = threadIdx.x; b < nblocks; b += kBlock) acc[0] += partial[5 * kMaxPartials + b];
-    __syncthreads();  // lds
-    const double s0 = block_sums(acc, 1, lds);
-    if (threadIdx.x < 5) sums[threadIdx.x] = s;
-    if (threadIdx.x == 0) sums[5] = s0;
-    __syncthreads();
-}
-__device__ __forceinline__ double total_square(const double sums[6]) {
-    return (((sums[0] + sums[1]) + sums[2]) + sums[3]) + sums[4];
-}
-__global__ void __launch_bounds__(kBlock) k_bicg_start(int nblocks, const double* partial, int guess, double* norms,
-                                                       double* ks, int fallback, double abs_tol, double rel_tol,
-                                                       int max_iter, Publish pub) {
-    __shared__ double lds[kBlock / 64 * 5];
-    __shared__ double sb[6], sr[6];
-    sum_squares(nblocks, partial, lds, sb);
-    if (guess) sum_squares(nblocks, partial + kSquares, lds, sr);
-    if (threadIdx.x == 0) {
-        const double bb = total_square(sb), rr = guess ? total_square(sr) : bb;
-        if (ks) {
-            if (guess) {
-                const double dots[4] = {bb, rr, sr[5], sb[5]};
-                bicg_init(ks, dots, 0, fallback, 1, abs_tol, rel_tol, max_iter);
-            } else {
-                const double dots[2] = {bb, sb[5]};
-                bicg_init(ks, dots, 1, fallback, 1, abs_tol, rel_tol, max_iter);
-            }
-        }
-        if (pub.host) {
-            pub.host->v[0] = bb;
-            pub.host->v[1] = rr;
-        }
+// The start of a solve on the sliced layout from the partial sums of its kernels: the
+// dot products and, of an implicit step, the squared residuals.
+__global__ void __launch_bounds__(kBlock) k_bicg_start(int nb, int nnorms, const double* partial, int guess,
+                                                       double* norms, double* ks, int fallback, double abs_tol,
+                                                       double rel_tol, int max_iter, Publish pub) {
+    __shared__ double lds[2][kBlock / 64 * 5];
+    __shared__ double dots[5];
+    const double d = sum_partials(nb, guess ? 2 : 1, partial, lds[0]);
+    if (threadIdx.x < 2) dots[threadIdx.x] = d;
+    const double q = nnorms > 0 ? sum_partials(nnorms, 5, partial + kNormPartials, lds[1]) : 0.0;
+    if (threadIdx.x < 5 && nnorms > 0) {
+        norms[threadIdx.x] = q;
+        if (pub.host) pub.host->v[kKsCount + threadIdx.x] = q;
     }
-    if (threadIdx.x < 5) {
-        if (norms) norms[threadIdx.x] = sb[threadIdx.x];
-        if (pub.host) pub.host->v[kKsCount + threadIdx.x] = sb[threadIdx.x];
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (ks) bicg_init(ks, dots, guess ? 0 : 1, fallback, abs_tol, rel_tol, max_iter);
+        if (pub.host) {
+            pub.host->v[0] = dots[0];
+            pub.host->v[1] = guess ? dots[1] : dots[0];
+        }
     }
     if (pub.host) publish_seq(pub);
 }
@@ -956,9 +923,9 @@ void launch_reduce_partials(int nb, int ncomp, const double* partial, double* ou
     hipLaunchKernelGGL(k_reduce_partials, dim3(1), dim3(kBlock), 0, s, nb, ncomp, partial, out, pub);
 }
 
-void launch_bicg_start(int nb, const double* partial, bool guess, double* norms, double* ks, bool fallback,
+void launch_bicg_start(int nb, int nnorms, const double* partial, bool guess, double* norms, double* ks, bool fallback,
                        double abs_tol, double rel_tol, int max_iter, const Publish& pub, hipStream_t s) {
-    hipLaunchKernelGGL(k_bicg_start, dim3(1), dim3(kBlock), 0, s, nb, partial, guess ? 1 : 0, norms, ks,
+    hipLaunchKernelGGL(k_bicg_start, dim3(1), dim3(kBlock), 0, s, nb, nnorms, partial, guess ? 1 : 0, norms, ks,
                        fallback ? 1 : 0, abs_tol, rel_tol, max_iter, pub);
 }
 

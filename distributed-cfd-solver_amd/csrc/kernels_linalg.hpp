@@ -14,21 +14,15 @@
 namespace cfdg {
 
 constexpr int kReduceBlocks = 1024;  // partial sums per reduction (fixed -> deterministic)
-constexpr int kMaxPartials = 1536;   // of the reductions fused into a product (one per slice, kernels_reduced.hip)
 
 // State block of the device-driven BiCGSTAB (doubles).  kKsStatus is 0 while
 // the solve runs, then one of the codes below; every gated kernel returns at
 // once when it is not 0.
 enum : int {
     kKsStatus = 0, kKsIt, kKsMaxIt, kKsTol, kKsRho, kKsRhoOld, kKsAlpha, kKsOmega, kKsBeta, kKsNbo, kKsFirst,
-    kKsOmegaNew, kKsRnNew, kKsRhoNew, kKsRnorm, kKsRnorm0, kKsReject,
-    // the reduced form (kernels_reduced.hip; zero in the others): multiples of the
-    // first colour's initial residual in r, p and s, its squared norm, whether the
-    // form is in use; and the updates of x so far
-    kKsAr, kKsAp, kKsAs, kKsB0, kKsReduced, kKsUpdates, kKsCount = 24
+    kKsOmegaNew, kKsRnNew, kKsRhoNew, kKsRnorm, kKsRnorm0, kKsReject, kKsCount = 24
 };
-// kKsExact: the reduced form met s = 0 exactly
-constexpr double kKsConverged = 1.0, kKsDiverged = 2.0, kKsMaxIter = 3.0, kKsExact = 4.0;
+constexpr double kKsConverged = 1.0, kKsDiverged = 2.0, kKsMaxIter = 3.0;
 
 // Results for the host without a copy and a stream synchronisation, which cost 13 to
 // 20 us after a short kernel: the kernel that ends a stretch of work writes them to
@@ -91,7 +85,7 @@ void launch_cast_f32_to_f64(long long n, const float* src, double* dst, hipStrea
 void launch_add_f32(long long n, const float* e, double* x, hipStream_t s);
 int reduction_blocks(long long n);
 // out[0..ndot) = dot products accumulated in FP64, handed over in v[0..ndot); partial
-// needs kMaxPartials * 5 doubles
+// needs kReduceBlocks * 5 doubles
 template <class T>
 void launch_dots(long long n, int ndot, const DotPairsT<T>& pr, double* partial, double* out, hipStream_t s,
                  const Publish& pub = {});
@@ -106,13 +100,12 @@ void launch_reduce_partials(int nb, int ncomp, const double* partial, double* ou
 // restarts from zero).
 void launch_bicg_init(double* ks, const double* dots, int x_zero, int fallback, double abs_tol, double rel_tol,
                       int max_iter, hipStream_t s);
-// launch_bicg_init of a reduced solve from the nb partial sums of the right-hand side's
-// squares and, with a guess, kSquares further those of b - A x: 5 per workgroup by
-// component (the right-hand side's sums also go to norms, unless null), and from 5
-// kMaxPartials on one per workgroup for the first colour.  Hand-over: v[0] = (b, b),
-// v[1] = (r, r), norms from v[kKsCount].  ks null: the sums only.
-constexpr int kSquares = 6 * kMaxPartials;
-void launch_bicg_start(int nb, const double* partial, bool guess, double* norms, double* ks, bool fallback,
+// launch_bicg_init from the nb partial 5-vectors of the dot products (kernels_multicolour.hpp)
+// (b, b) and, with a guess, (r, r); and from nnorms > 0 more at kNormPartials the sums
+// of the squared residuals (to norms).  Hand-over: v[0] = (b, b), v[1] = (r, r), norms
+// from v[kKsCount].  ks null: the sums only.
+constexpr int kNormPartials = 5 * kReduceBlocks;
+void launch_bicg_start(int nb, int nnorms, const double* partial, bool guess, double* norms, double* ks, bool fallback,
                        double abs_tol, double rel_tol, int max_iter, const Publish& pub, hipStream_t s);
 template <class T>
 void launch_bicg_reject(long long n, const double* ks, const T* b, T* x, T* r, hipStream_t s);

@@ -10,20 +10,21 @@
 //   k_sell_spmv    y = A x
 //   k_sell_sweep   one Gauss-Seidel step of a colour (bsr_helpers.hpp:390-435)
 //
-// The iterations of the solve run on kernels_reduced.hip, which needs neither a
-// whole product nor a whole sweep; these serve the residuals of the defect
-// correction, the ABI's product and preconditioner calls, and the solves that the
-// reduced form leaves (bicgstab, capi.cpp).
+// with the vector kernels and sums of a solve's start and end.  The iterations of the
+// solve have some more (kernels_multicolour.hip).
 //
 // Arithmetic per row component: products summed over the block's columns, the
-// block sums added or subtracted in the order of the row's slots.
+// block sums added or subtracted in ascending mesh column, as on a row-major matrix;
+// sums over the vectors in the order of the device rows, 5 values each
+// (flat_dots).  Both are those of kernels_linalg.hip, so a solve's result does not
+// depend on the layout: a loosely converged solve magnifies rounding, and in a
+// sequence of time steps a different order of the sums shows within a few steps.
 //
 // Bound: HBM.  On the 2.1M-cell plate in FP64 (256 x 64 x 128) a sweep step moves
-// its 1.6 GB in 273 us and the product its 2.96 GB of blocks in 525 us (5.6-5.8
-// TB/s, against 6.0 TB/s of a reduction that only reads); five lanes per row on
-// row-major blocks in cell order took 384 and 612 us, because a colour's rows
-// alternated with the other colours' and with the diagonal blocks a sweep does not
-// read, at 200-byte blocks that start and end inside cache lines.
+// its 1.6 GB in 320 us (5.0 TB/s, against 6.0 TB/s of a reduction that only reads);
+// five lanes per row on row-major blocks in cell order took 1.4 times as long, because
+// a colour's rows alternated with the other colours' and with the diagonal blocks a
+// sweep does not read, at 200-byte blocks that start and end inside cache lines.
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
@@ -107,41 +108,36 @@ __global__ void __launch_bounds__(kBlock) k_sell_lu(SellArgs b, const word_t<TS>
     piv[p] = static_cast<std::uint16_t>(pv);
 }
 
+// y = A x in the rows of slices [first, first + count).
 template <class TS, class TV, int kSplit>
-__global__ void __launch_bounds__(slice_threads<kSplit>()) k_sell_spmv(SellArgs b, const word_t<TS>* off,
-                                                                       const word_t<TS>* diag, const TV* x, TV* y,
-                                                                       const double* gate) {
+__global__ void __launch_bounds__(slice_threads<kSplit>()) k_sell_spmv(SellArgs b, int first, int count,
+                                                                       const word_t<TS>* off, const word_t<TS>* diag,
+                                                                       const TV* x, TV* y, const double* gate) {
     __shared__ TV lds[split_lds<kSplit, TV>()];
     if (gate && gate[kKsStatus] != 0.0) return;
-    const int slice = wave_slice<kSplit>();
-    if (slice >= b.nslices) return;
-    const int lane = threadIdx.x & 63;
-    const int4 sl = b.slice[slice];
-    const bool lead = kSplit == 1 || threadIdx.x < kSellRows;
-    const bool on = lane < sl.w;
-    const unsigned n = on ? b.count[slice * kSellRows + lane] : 0;
-    const long long at = static_cast<long long>(slice) * (5 * kSellRows) + lane;
-    TV acc[5];
-    if (lead && on) {
-        word_t<TS> w[SellLayout<TS>::words];
-        load_words<TS>(diag, slice, lane, w);
+    const int ls = wave_slice<kSplit>();
+    if (ls >= count) return;
+    const Rows q = rows_of(b, first + ls);
+    const bool lead = lead_wave<kSplit>() && q.on;
+    const int before = lead ? b.before[q.slice * kSellRows + q.lane] : 0;
+    TV d[5];
+    RowSum<TV> sum;
+    if (lead) {
         TV xv[5];
 #pragma unroll
-        for (int v = 0; v < 5; ++v) xv[v] = x[at + v * kSellRows];
-        block_times<TS, TV>(w, xv, acc);
+        for (int v = 0; v < 5; ++v) xv[v] = x[q.at + v * kSellRows];
+        diagonal_times<TS, TV>(diag, q, xv, d);
     }
-    for_slots<kSplit, TS, TV>(off, b.cols, sl, n, 0, sl.y + sl.z, 0, lane, x, lds, [&](const TV t[5]) {
+    for_blocks<kSplit, true, TS, TV>(b, off, q, x, lds, [&](int k, const TV t[5]) { sum.add(k, t, before, d); });
+    if (!lead) return;
+    sum.finish(q.blocks(), before, d);
 #pragma unroll
-        for (int v = 0; v < 5; ++v) acc[v] += t[v];
-    });
-    if (!lead || !on) return;
-#pragma unroll
-    for (int v = 0; v < 5; ++v) y[at + v * kSellRows] = acc[v];
+    for (int v = 0; v < 5; ++v) y[q.at + v * kSellRows] = sum.s[v];
 }
 
 // z_i = D_i^-1 (r_i - sum A_ij z_j) for the rows of one colour.
-template <class TS, class TL, class TV, int kSplit>
-__global__ void __launch_bounds__(slice_threads<kSplit>()) k_sell_sweep(SellArgs b, int first, int count, int all,
+template <class TS, class TL, class TV, int kSplit, bool kAll>
+__global__ void __launch_bounds__(slice_threads<kSplit>()) k_sell_sweep(SellArgs b, int first, int count,
                                                                         const word_t<TS>* off, const TL* lu,
                                                                         const std::uint16_t* piv, const TV* r, TV* z,
                                                                         const double* gate) {
@@ -149,28 +145,23 @@ __global__ void __launch_bounds__(slice_threads<kSplit>()) k_sell_sweep(SellArgs
     if (gate && gate[kKsStatus] != 0.0) return;
     const int ls = wave_slice<kSplit>();
     if (ls >= count) return;
-    const int slice = first + ls;
-    const int lane = threadIdx.x & 63;
-    const int4 sl = b.slice[slice];
-    const bool lead = kSplit == 1 || threadIdx.x < kSellRows;
-    const bool on = lane < sl.w;
-    const unsigned n = on ? b.count[slice * kSellRows + lane] : 0;
-    const long long at = static_cast<long long>(slice) * (5 * kSellRows) + lane;
+    const Rows q = rows_of(b, first + ls);
+    const bool lead = lead_wave<kSplit>() && q.on;
     TV acc[5], L[25];
-    if (lead && on) {
+    if (lead) {
 #pragma unroll
-        for (int v = 0; v < 5; ++v) acc[v] = r[at + v * kSellRows];
-        if (kSplit > 1) load_lu<TL, TV>(lu, slice, lane, L);  // in flight with the slots
+        for (int v = 0; v < 5; ++v) acc[v] = r[q.at + v * kSellRows];
+        if (kSplit > 1) load_lu<TL, TV>(lu, q.slice, q.lane, L);  // in flight with the slots
     }
-    for_slots<kSplit, TS, TV>(off, b.cols, sl, n, 0, all ? sl.y + sl.z : sl.y, 0, lane, z, lds, [&](const TV t[5]) {
+    for_blocks<kSplit, kAll, TS, TV>(b, off, q, z, lds, [&](int, const TV t[5]) {
 #pragma unroll
         for (int v = 0; v < 5; ++v) acc[v] -= t[v];
     });
-    if (!lead || !on) return;
-    if (kSplit == 1) load_lu<TL, TV>(lu, slice, lane, L);
-    lu_solve(acc, L, piv[slice * kSellRows + lane]);
+    if (!lead) return;
+    if (kSplit == 1) load_lu<TL, TV>(lu, q.slice, q.lane, L);
+    lu_solve(acc, L, piv[q.slice * kSellRows + q.lane]);
 #pragma unroll
-    for (int v = 0; v < 5; ++v) z[at + v * kSellRows] = acc[v];
+    for (int v = 0; v < 5; ++v) z[q.at + v * kSellRows] = acc[v];
 }
 
 __global__ void __launch_bounds__(kBlock) k_sell_gather(SellArgs b, const int* src_of, const double* src, double* dst) {
@@ -191,85 +182,120 @@ __global__ void __launch_bounds__(kBlock) k_sell_scatter(SellArgs b, const int* 
     for (int v = 0; v < 5; ++v) d[v] = u[v * kSellRows];
 }
 
-// The positions of the sliced layout in grid-stride order, f(position, device row)
-// for those that hold a row and as many workgroups as a reduction has partial sums.
-template <class F>
-__device__ __forceinline__ void for_rows(const SellArgs& b, F&& f) {
-    const int end = b.nslices * kSellRows, stride = static_cast<int>(gridDim.x * blockDim.x);
-    for (int p = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x); p < end; p += stride) {
-        const int row = b.row[p];
-        if (row >= 0) f(p, row);
+// Partial dot products of vectors of the layout, in the order of k_dots
+// (kernels_linalg.hip) on flat vectors: element i is component i % 5 of device row
+// i / 5, thread t of workgroup blk takes i = blk 256 + t and every nb 256th from there.
+// load(row, component, v) gives an element's kVals factors; the products are v0 v0
+// (one factor), v0 v1, or (kDots 2) v0 v0 and v1 v1, or (kDots 5) v0 v0, v0 v1, v2 v0,
+// v2 v1, v1 v1.  Four elements are in flight at a time (eight are no faster).  5 rows < 2^32 in
+// 288 GB.
+template <int kDots, int kVals, class Load>
+__device__ __forceinline__ void flat_dots(int blk, int nb, int rows, double* partial, Load&& load) {
+    constexpr int kAhead = 4;
+    __shared__ double lds[kBlock / 64 * 5];
+    const unsigned n = 5u * static_cast<unsigned>(rows), stride = static_cast<unsigned>(nb) * kBlock;
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (unsigned long long i0 = static_cast<unsigned>(blk) * kBlock + threadIdx.x; i0 < n; i0 += kAhead * stride) {
+        double v[kAhead][kVals];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const unsigned long long i = i0 + static_cast<unsigned>(u) * static_cast<unsigned long long>(stride);
+            if (i < n) {
+                const unsigned row = static_cast<unsigned>(i) / 5u;
+                load(static_cast<int>(row), static_cast<int>(static_cast<unsigned>(i) - 5u * row), v[u]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if (i0 + static_cast<unsigned>(u) * static_cast<unsigned long long>(stride) >= n) break;
+            const double* e = v[u];
+            if constexpr (kDots == 1) {
+                acc[0] += e[0] * e[kVals - 1];
+            } else if constexpr (kDots == 2) {
+                acc[0] += e[0] * e[0];
+                acc[1] += e[1] * e[1];
+            } else {
+                acc[0] += e[0] * e[0];
+                acc[1] += e[0] * e[1];
+                acc[2] += e[2] * e[0];
+                acc[3] += e[2] * e[1];
+                acc[4] += e[1] * e[1];
+            }
+        }
     }
+    const double s = block_sums(acc, kDots, lds);
+    if (threadIdx.x < kDots) partial[blk * 5 + static_cast<int>(threadIdx.x)] = s;
 }
 
-// Partial sums of squares for launch_bicg_start: by component, and the total of the
-// positions before first_end.
-struct Squares {
-    double all[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, first = 0.0;
-    __device__ __forceinline__ void store(double* partial) const {
-        __shared__ double lds[2][kBlock / 64 * 5];
-        const double f[5] = {first, 0.0, 0.0, 0.0, 0.0};
-        const double s = block_sums(all, 5, lds[0]);
-        const double s0 = block_sums(f, 1, lds[1]);
-        if (threadIdx.x < 5) partial[blockIdx.x * 5 + threadIdx.x] = s;
-        if (threadIdx.x == 0) partial[5 * kMaxPartials + blockIdx.x] = s0;
-    }
-};
+// The dot products of a step or of a start: kDots 1 (v0, v1), 2 (v0, v0) and (v1, v1),
+// 5 with v0 = t, v1 = s, v2 = r0.  Bound: HBM at 2.1M cells (two vectors 43 us, three
+// 65 us, 3.9 TB/s: the rows' components are read in device order from colour order, in
+// runs of about 13 rows), latency below a million.  Workgroups in XCD order: neighbours
+// share lines.
+template <int kDots, class TV>
+__global__ void __launch_bounds__(kBlock) k_sell_dots(SellArgs b, const TV* v0, const TV* v1, const TV* v2,
+                                                      double* partial, const double* gate) {
+    if (gate && gate[kKsStatus] != 0.0) return;
+    constexpr int kVals = kDots == 5 ? 3 : 2;
+    const int nb = static_cast<int>(gridDim.x);
+    flat_dots<kDots, kVals>(xcd_block(blockIdx.x, nb), nb, b.n, partial, [&](int row, int k, double v[kVals]) {
+        const long long at = vec_at(b.pos[row]) + k * kSellRows;
+        v[0] = static_cast<double>(v0[at]);
+        v[1] = static_cast<double>(v1[at]);
+        if constexpr (kVals == 3) v[2] = static_cast<double>(v2[at]);
+    });
+}
 
-// b = -R, the implicit right-hand side (implicit_euler.hpp:81-92), x = 0, and the
-// squares of R: one pass where the norms and (b, b) took one each and x a fill.
+// b = -R, the implicit right-hand side (implicit_euler.hpp:81-92), x = 0 and the
+// squares of R by component (as k_res_sq adds them) in the first nb_norms workgroups,
+// (b, b) in the others: one launch where the norms, (b, b) and the fill took one each.
 __global__ void __launch_bounds__(kBlock) k_sell_rhs(SellArgs b, int ld, const double* res, double* rhs, double* x,
-                                                     int first_end, double* partial, int* singular,
+                                                     double* partial, int nb_norms, int* singular,
                                                      unsigned long long* stamp, int jacobian_end) {
     stamp_stage(stamp, kStampLinear);
     if (jacobian_end) stamp_stage(stamp, kStampJacobianEnd);
-    if (blockIdx.x == 0 && threadIdx.x == 0) *singular = 0;
-    Squares q;
-    for_rows(b, [&](int p, int row) {
-        const long long at = vec_at(p);
+    const int blk = static_cast<int>(blockIdx.x);
+    if (blk >= nb_norms) {
+        const int nb = static_cast<int>(gridDim.x) - nb_norms;
+        flat_dots<1, 1>(xcd_block(blk - nb_norms, nb), nb, b.n, partial, [&](int row, int k, double v[1]) {
+            v[0] = -res[static_cast<long long>(k) * ld + row];
+        });
+        return;
+    }
+    if (blk == 0 && threadIdx.x == 0) *singular = 0;
+    __shared__ double lds[kBlock / 64 * 5];
+    double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    for (int c = blk * kBlock + static_cast<int>(threadIdx.x); c < b.n; c += nb_norms * kBlock) {
+        const long long at = vec_at(b.pos[c]);
         for (int v = 0; v < 5; ++v) {
-            const double r = res[static_cast<long long>(v) * ld + row];
+            const double r = res[static_cast<long long>(v) * ld + c];
+            acc[v] += r * r;
             rhs[at + v * kSellRows] = -r;
             x[at + v * kSellRows] = 0.0;
-            q.all[v] += r * r;
-            if (p < first_end) q.first += r * r;
         }
-    });
-    q.store(partial);
+    }
+    const double s = block_sums(acc, 5, lds);
+    if (threadIdx.x < 5) partial[kNormPartials + blk * 5 + static_cast<int>(threadIdx.x)] = s;
 }
 
-// The squares of a vector, added as the kernels above and below add theirs.
-template <class TV>
-__global__ void __launch_bounds__(kBlock) k_sell_squares(SellArgs b, const TV* u, int first_end, double* partial) {
-    Squares q;
-    for_rows(b, [&](int p, int) {
-        const long long at = vec_at(p);
-        for (int v = 0; v < 5; ++v) {
-            const double d = static_cast<double>(u[at + v * kSellRows]);
-            q.all[v] += d * d;
-            if (p < first_end) q.first += d * d;
-        }
-    });
-    q.store(partial);
-}
-
-// The right-hand side of a defect correction's inner solve, b = r in FP32, x = 0, and
-// the squares of b.
+// The right-hand side of a defect correction's inner solve, b = r in FP32 and x = 0,
+// and (b, b), likewise.
 __global__ void __launch_bounds__(kBlock) k_sell_inner_rhs(SellArgs b, const double* r, float* rhs, float* x,
-                                                           int first_end, double* partial) {
-    Squares q;
-    for_rows(b, [&](int p, int) {
-        const long long at = vec_at(p);
-        for (int v = 0; v < 5; ++v) {
-            const float f = static_cast<float>(r[at + v * kSellRows]);
-            rhs[at + v * kSellRows] = f;
-            x[at + v * kSellRows] = 0.0f;
-            const double d = static_cast<double>(f);
-            q.all[v] += d * d;
-            if (p < first_end) q.first += d * d;
-        }
-    });
-    q.store(partial);
+                                                           double* partial, int nb_copy) {
+    const int blk = static_cast<int>(blockIdx.x);
+    if (blk >= nb_copy) {
+        const int nb = static_cast<int>(gridDim.x) - nb_copy;
+        flat_dots<1, 1>(xcd_block(blk - nb_copy, nb), nb, b.n, partial, [&](int row, int k, double v[1]) {
+            v[0] = static_cast<double>(static_cast<float>(r[vec_at(b.pos[row]) + k * kSellRows]));
+        });
+        return;
+    }
+    const long long end = 5LL * kSellRows * b.nslices;
+    for (long long e = static_cast<long long>(blk) * kBlock + threadIdx.x; e < end;
+         e += static_cast<long long>(nb_copy) * kBlock) {
+        rhs[e] = static_cast<float>(r[e]);
+        x[e] = 0.0f;
+    }
 }
 
 // U = U + du (implicit_euler.hpp:53-61)
@@ -364,42 +390,43 @@ void launch_sell_lu(const SellArgs& b, const SellMatrix& m, void* lu, int lu_f32
 }
 
 template <class TV>
-void launch_sell_spmv(const SellArgs& b, const SellMatrix& m, const TV* x, TV* y, hipStream_t s, const double* gate) {
-    if (b.nslices <= 0) return;
-    with_split(b.nslices, [&](auto split) {
+void launch_sell_spmv(const SellArgs& b, const SellMatrix& m, int first, int count, const TV* x, TV* y, hipStream_t s,
+                      const double* gate) {
+    if (count <= 0) return;
+    with_split(count, [&](auto split) {
         with_storage(m.storage, [&](auto ts) {
             typedef decltype(ts) TS;
             constexpr int kS = decltype(split)::value;
-            hipLaunchKernelGGL((k_sell_spmv<TS, TV, kS>), slice_grid<kS>(b.nslices), dim3(slice_threads<kS>()), 0, s,
-                               b, static_cast<const word_t<TS>*>(m.off), static_cast<const word_t<TS>*>(m.diag), x, y,
-                               gate);
+            hipLaunchKernelGGL((k_sell_spmv<TS, TV, kS>), slice_grid<kS>(count), dim3(slice_threads<kS>()), 0, s, b,
+                               first, count, static_cast<const word_t<TS>*>(m.off),
+                               static_cast<const word_t<TS>*>(m.diag), x, y, gate);
         });
     });
 }
-template void launch_sell_spmv<double>(const SellArgs&, const SellMatrix&, const double*, double*, hipStream_t,
-                                       const double*);
-template void launch_sell_spmv<float>(const SellArgs&, const SellMatrix&, const float*, float*, hipStream_t,
+template void launch_sell_spmv<double>(const SellArgs&, const SellMatrix&, int, int, const double*, double*,
+                                       hipStream_t, const double*);
+template void launch_sell_spmv<float>(const SellArgs&, const SellMatrix&, int, int, const float*, float*, hipStream_t,
                                       const double*);
 
 template <class TV>
 void launch_sell_sweep(const SellArgs& b, const SellMatrix& m, int first, int count, bool all, const TV* r, TV* z,
                        hipStream_t s, const double* gate) {
     if (count <= 0) return;
-    with_split(count, [&](auto split) {
+    const auto launch = [&](auto split, auto ts, auto whole) {
+        typedef decltype(ts) TS;
+        typedef std::conditional_t<sizeof(TV) == sizeof(double), double, float> TL;
         constexpr int kS = decltype(split)::value;
-        const dim3 g = slice_grid<kS>(count), blk(slice_threads<kS>());
-        if constexpr (sizeof(TV) == sizeof(double)) {
-            if (m.storage != kStoreF64) throw_bad_combination("FP64 SGS needs FP64 blocks");
-            hipLaunchKernelGGL((k_sell_sweep<double, double, double, kS>), g, blk, 0, s, b, first, count, all ? 1 : 0,
-                               static_cast<const double*>(m.off), static_cast<const double*>(m.lu), m.piv, r, z, gate);
-        } else {
-            with_storage(m.storage, [&](auto ts) {
-                typedef decltype(ts) TS;
-                hipLaunchKernelGGL((k_sell_sweep<TS, float, float, kS>), g, blk, 0, s, b, first, count, all ? 1 : 0,
-                                   static_cast<const word_t<TS>*>(m.off), static_cast<const float*>(m.lu), m.piv, r, z,
-                                   gate);
-            });
-        }
+        hipLaunchKernelGGL((k_sell_sweep<TS, TL, TV, kS, decltype(whole)::value>), slice_grid<kS>(count),
+                           dim3(slice_threads<kS>()), 0, s, b, first, count, static_cast<const word_t<TS>*>(m.off),
+                           static_cast<const TL*>(m.lu), m.piv, r, z, gate);
+    };
+    with_split(count, [&](auto split) {
+        with_form<TV>(m, [&](auto ts) {
+            if (all)
+                launch(split, ts, std::true_type{});
+            else
+                launch(split, ts, std::false_type{});
+        });
     });
 }
 template void launch_sell_sweep<double>(const SellArgs&, const SellMatrix&, int, int, bool, const double*, double*,
@@ -416,28 +443,39 @@ void launch_sell_scatter(const SellArgs& b, const int* dst_of, const double* src
     if (b.n > 0) hipLaunchKernelGGL(k_sell_scatter, grid_for(b.n), dim3(kBlock), 0, s, b, dst_of, src, dst);
 }
 
-int launch_sell_rhs(const SellArgs& b, int ld, const double* res, double* rhs, double* x, int first_slices,
-                    double* partial, int* singular, unsigned long long* stamp, bool jacobian_end, hipStream_t s) {
-    const int nb = reduction_blocks(static_cast<long long>(b.nslices) * kSellRows);
-    hipLaunchKernelGGL(k_sell_rhs, dim3(nb), dim3(kBlock), 0, s, b, ld, res, rhs, x, first_slices * kSellRows, partial,
-                       singular, stamp, jacobian_end ? 1 : 0);
-    return nb;
-}
-
 template <class TV>
-int launch_sell_squares(const SellArgs& b, const TV* u, int first_slices, double* partial, hipStream_t s) {
-    const int nb = reduction_blocks(static_cast<long long>(b.nslices) * kSellRows);
-    hipLaunchKernelGGL(k_sell_squares<TV>, dim3(nb), dim3(kBlock), 0, s, b, u, first_slices * kSellRows, partial);
+int launch_sell_dots(const SellArgs& b, int ndot, const TV* v0, const TV* v1, const TV* v2, double* partial,
+                     hipStream_t s, const double* gate) {
+    const int nb = reduction_blocks(5LL * b.n);
+    const dim3 g(static_cast<unsigned>(nb)), blk(kBlock);
+    if (ndot == 1)
+        hipLaunchKernelGGL((k_sell_dots<1, TV>), g, blk, 0, s, b, v0, v1, v2, partial, gate);
+    else if (ndot == 2)
+        hipLaunchKernelGGL((k_sell_dots<2, TV>), g, blk, 0, s, b, v0, v1, v2, partial, gate);
+    else
+        hipLaunchKernelGGL((k_sell_dots<5, TV>), g, blk, 0, s, b, v0, v1, v2, partial, gate);
     return nb;
 }
-template int launch_sell_squares<double>(const SellArgs&, const double*, int, double*, hipStream_t);
-template int launch_sell_squares<float>(const SellArgs&, const float*, int, double*, hipStream_t);
+template int launch_sell_dots<double>(const SellArgs&, int, const double*, const double*, const double*, double*,
+                                      hipStream_t, const double*);
+template int launch_sell_dots<float>(const SellArgs&, int, const float*, const float*, const float*, double*,
+                                     hipStream_t, const double*);
 
-int launch_sell_inner_rhs(const SellArgs& b, const double* r, float* rhs, float* x, int first_slices, double* partial,
-                          hipStream_t s) {
-    const int nb = reduction_blocks(static_cast<long long>(b.nslices) * kSellRows);
-    hipLaunchKernelGGL(k_sell_inner_rhs, dim3(nb), dim3(kBlock), 0, s, b, r, rhs, x, first_slices * kSellRows, partial);
-    return nb;
+SellSums launch_sell_rhs(const SellArgs& b, int ld, const double* res, double* rhs, double* x, bool square,
+                         double* partial, int* singular, unsigned long long* stamp, bool jacobian_end, hipStream_t s) {
+    const SellSums n{square ? reduction_blocks(5LL * b.n) : 0, reduction_blocks(b.n)};
+    hipLaunchKernelGGL(k_sell_rhs, dim3(static_cast<unsigned>(n.dots + n.norms)), dim3(kBlock), 0, s, b, ld, res, rhs, x,
+                       partial, n.norms, singular, stamp, jacobian_end ? 1 : 0);
+    return n;
+}
+
+SellSums launch_sell_inner_rhs(const SellArgs& b, const double* r, float* rhs, float* x, double* partial,
+                               hipStream_t s) {
+    const SellSums n{reduction_blocks(5LL * b.n), 0};
+    const int copy = reduction_blocks(5LL * kSellRows * b.nslices);
+    hipLaunchKernelGGL(k_sell_inner_rhs, dim3(static_cast<unsigned>(copy + n.dots)), dim3(kBlock), 0, s, b, r, rhs, x,
+                       partial, copy);
+    return n;
 }
 
 void launch_sell_state_update(const SellArgs& b, int ld, const double* du, double* U, double* du_cells,

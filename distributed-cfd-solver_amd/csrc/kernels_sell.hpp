@@ -36,9 +36,10 @@ inline std::size_t sell_slot_bytes(int storage) {
 // the largest device row + 1 with a zero pivot.
 void launch_sell_lu(const SellArgs& b, const SellMatrix& m, void* lu, int lu_f32, std::uint16_t* piv, int* singular,
                     hipStream_t s);
-// y = A x.  TV = float needs FP32 vectors, any storage; TV = double any storage.
+// y = A x in the rows of slices [first, first + count).  TV = float needs FP32
+// vectors, any storage; TV = double any storage.
 template <class TV>
-void launch_sell_spmv(const SellArgs& b, const SellMatrix& m, const TV* x, TV* y, hipStream_t s,
+void launch_sell_spmv(const SellArgs& b, const SellMatrix& m, int first, int count, const TV* x, TV* y, hipStream_t s,
                       const double* gate = nullptr);
 // One sweep step over the slices [first, first + count) of a colour:
 // z_i = D_i^-1 (r_i - sum A_ij z_j) over the row's lower blocks, or with all
@@ -50,17 +51,24 @@ void launch_sell_sweep(const SellArgs& b, const SellMatrix& m, int first, int co
 // row itself when src_of is null), and back.
 void launch_sell_gather(const SellArgs& b, const int* src_of, const double* src, double* dst, hipStream_t s);
 void launch_sell_scatter(const SellArgs& b, const int* dst_of, const double* src, double* dst, hipStream_t s);
-// b = -R and x = 0 in the sliced layout, *singular = 0, with the partial sums for
-// launch_bicg_start (their number is returned); jacobian_end: the launch directly
-// after the Jacobian's.
-int launch_sell_rhs(const SellArgs& b, int ld, const double* res, double* rhs, double* x, int first_slices,
-                    double* partial, int* singular, unsigned long long* stamp, bool jacobian_end, hipStream_t s);
-// the partial sums alone, of any vector of the layout
+// Partial sums left for launch_bicg_start: 5-vectors of dot products, and of squared
+// residuals.
+struct SellSums {
+    int dots = 0, norms = 0;
+};
+// Partial dot products (5 per workgroup, their number is returned): ndot 1 (v0, v1), 2
+// (v0, v0) and (v1, v1), 5 (v0, v0), (v0, v1), (v2, v0), (v2, v1), (v1, v1); vectors
+// that are not used repeat another.
 template <class TV>
-int launch_sell_squares(const SellArgs& b, const TV* u, int first_slices, double* partial, hipStream_t s);
-// b = r in FP32 and x = 0, likewise
-int launch_sell_inner_rhs(const SellArgs& b, const double* r, float* rhs, float* x, int first_slices, double* partial,
-                          hipStream_t s);
+int launch_sell_dots(const SellArgs& b, int ndot, const TV* v0, const TV* v1, const TV* v2, double* partial,
+                     hipStream_t s, const double* gate = nullptr);
+// b = -R and x = 0 in the sliced layout, *singular = 0, with the partial sums of the
+// norms and (square) of (b, b); jacobian_end: the launch directly after the Jacobian's.
+SellSums launch_sell_rhs(const SellArgs& b, int ld, const double* res, double* rhs, double* x, bool square,
+                         double* partial, int* singular, unsigned long long* stamp, bool jacobian_end, hipStream_t s);
+// b = r in FP32, x = 0 and the partial sums of (b, b)
+SellSums launch_sell_inner_rhs(const SellArgs& b, const double* r, float* rhs, float* x, double* partial,
+                               hipStream_t s);
 // U += du with du in the sliced layout, du also written per cell (5 values, device
 // order); stamps the solve's end.
 void launch_sell_state_update(const SellArgs& b, int ld, const double* du, double* U, double* du_cells,

@@ -1,11 +1,12 @@
 // Device functions and launch rules of the kernels on the sliced block layout
-// (kernels_sell.hip, kernels_reduced.hip): block and factor loads, the 5x5
+// (kernels_sell.hip, kernels_multicolour.hip): block and factor loads, the 5x5
 // solve, and the walk over a slice's slots by one wave, four or eight.
 #pragma once
 
 #include <hip/hip_runtime.h>
 
 #include <cstdint>
+#include <stdexcept>
 #include <type_traits>
 
 #include "kernels.hpp"
@@ -105,49 +106,103 @@ __device__ __forceinline__ void slot_times(const word_t<TS>* off, const int* col
     block_times<TS, TV>(w, xv, t);
 }
 
-// Whether the row with block counts n (lower | upper << 16) has a block in the
-// j-th slot of its slice.
-__device__ __forceinline__ bool has_block(const int4& sl, unsigned n, int j) {
-    return j < sl.y ? j < static_cast<int>(n & 0xffffu) : j - sl.y < static_cast<int>(n >> 16);
+// A wave's slice: its slots and rows, whether the lane holds a row, the row's blocks
+// (lower | upper << 16) and where component 0 of its vector entries is.
+struct Rows {
+    int slice, lane;
+    int4 sl;
+    bool on;
+    unsigned n;
+    long long at;
+    __device__ __forceinline__ int lower() const { return static_cast<int>(n & 0xffffu); }
+    __device__ __forceinline__ int blocks() const { return lower() + static_cast<int>(n >> 16); }
+};
+__device__ __forceinline__ Rows rows_of(const SellArgs& b, int slice) {
+    Rows q;
+    q.slice = slice;
+    q.lane = threadIdx.x & (kSellRows - 1);
+    q.sl = b.slice[slice];
+    q.on = q.lane < q.sl.w;
+    q.n = q.on ? b.count[slice * kSellRows + q.lane] : 0;
+    q.at = static_cast<long long>(slice) * (5 * kSellRows) + q.lane;
+    return q;
+}
+// The products with x of a row's lower blocks, or with kAll of all its off-diagonal
+// blocks, handed to add(k, t) in ascending mesh column (k counts them): the order of a
+// row-major matrix, so that a row's sums do not depend on the colours or on the layout.
+// In a slice with lower and upper slots that order is read from b.order; elsewhere the
+// slots are in it.  kSplit = 1: by the wave alone, one after the other.  kSplit > 1: the kSplit
+// waves of the workgroup, all on the same slice, form kSplit products at a time into LDS
+// and the first wave adds them.
+template <int kSplit, bool kAll, class TS, class TV, class F>
+__device__ __forceinline__ void for_blocks(const SellArgs& b, const word_t<TS>* off, const Rows& q, const TV* x,
+                                           TV* lds, F&& add) {
+    const int most = kAll ? q.sl.y + q.sl.z : q.sl.y, mine = kAll ? q.blocks() : q.lower();
+    const auto walk = [&](auto&& slot) {
+        if constexpr (kSplit == 1) {
+            for (int k = 0; k < most; ++k) {
+                if (k >= mine) continue;
+                TV t[5];
+                slot_times<TS, TV>(off, b.cols, slot(k), q.lane, x, t);
+                add(k, t);
+            }
+        } else {
+            const int w = threadIdx.x >> 6;
+            for (int k0 = 0; k0 < most; k0 += kSplit) {
+                if (k0 + w < mine) {
+                    TV t[5];
+                    slot_times<TS, TV>(off, b.cols, slot(k0 + w), q.lane, x, t);
+#pragma unroll
+                    for (int v = 0; v < 5; ++v) lds[(w * 5 + v) * kSellRows + q.lane] = t[v];
+                }
+                __syncthreads();
+                if (w == 0)
+                    for (int k = 0; k < kSplit && k0 + k < mine; ++k) {
+                        TV t[5];
+#pragma unroll
+                        for (int v = 0; v < 5; ++v) t[v] = lds[(k * 5 + v) * kSellRows + q.lane];
+                        add(k0 + k, t);
+                    }
+                if (k0 + kSplit < most) __syncthreads();
+            }
+        }
+    };
+    const long long base = q.sl.x;
+    if (kAll && q.sl.y > 0 && q.sl.z > 0)
+        walk([&](int k) { return base + b.order[(base + k) * kSellRows + q.lane]; });
+    else
+        walk([&](int k) { return base + k; });
 }
 
-// The products of slots [from, to) of a slice with x, of the row's blocks only
-// (has_block), handed to add(t) in slot order.  skip: the row's first lower blocks
-// that are left out.  kSplit = 1: by the wave alone, one slot after the other.  kSplit > 1:
-// the kSplit waves of the workgroup, all on the same slice, form kSplit slots at a
-// time into LDS and the first wave adds them, in the same order.
-template <int kSplit, class TS, class TV, class F>
-__device__ __forceinline__ void for_slots(const word_t<TS>* off, const int* cols, const int4& sl, unsigned n, int from,
-                                          int to, int skip, int lane, const TV* x, TV* lds, F&& add) {
-    if constexpr (kSplit == 1) {
-        for (int j = from; j < to; ++j) {
-            if (j < skip || !has_block(sl, n, j)) continue;
-            TV t[5];
-            slot_times<TS, TV>(off, cols, sl.x + j, lane, x, t);
-            add(t);
-        }
-    } else {
-        const int w = threadIdx.x >> 6;
-        for (int j0 = from; j0 < to; j0 += kSplit) {
-            const int j = j0 + w;
-            if (j < to && j >= skip && has_block(sl, n, j)) {
-                TV t[5];
-                slot_times<TS, TV>(off, cols, sl.x + j, lane, x, t);
+// The sum of a row's product y = A x: the off-diagonal products as for_blocks hands
+// them over, and the diagonal one, d, in its place among them (before: the number of
+// off-diagonal blocks that precede it).
+template <class TV>
+struct RowSum {
+    TV s[5] = {0, 0, 0, 0, 0};
+    __device__ __forceinline__ void add(const TV t[5]) {
 #pragma unroll
-                for (int v = 0; v < 5; ++v) lds[(w * 5 + v) * kSellRows + lane] = t[v];
-            }
-            __syncthreads();
-            if (w == 0)
-                for (int k = 0; k < kSplit && j0 + k < to; ++k) {
-                    if (j0 + k < skip || !has_block(sl, n, j0 + k)) continue;
-                    TV t[5];
-#pragma unroll
-                    for (int v = 0; v < 5; ++v) t[v] = lds[(k * 5 + v) * kSellRows + lane];
-                    add(t);
-                }
-            if (j0 + kSplit < to) __syncthreads();
-        }
+        for (int v = 0; v < 5; ++v) s[v] += t[v];
     }
+    __device__ __forceinline__ void add(int k, const TV t[5], int before, const TV d[5]) {
+        if (k == before) add(d);
+        add(t);
+    }
+    __device__ __forceinline__ void finish(int blocks, int before, const TV d[5]) {
+        if (blocks == before) add(d);
+    }
+};
+// d = D x for the row's diagonal block
+template <class TS, class TV>
+__device__ __forceinline__ void diagonal_times(const word_t<TS>* diag, const Rows& q, const TV x[5], TV d[5]) {
+    word_t<TS> w[SellLayout<TS>::words];
+    load_words<TS>(diag, q.slice, q.lane, w);
+    block_times<TS, TV>(w, x, d);
+}
+
+template <int kSplit>
+__device__ __forceinline__ bool lead_wave() {
+    return kSplit == 1 || threadIdx.x < kSellRows;
 }
 template <int kSplit>
 constexpr int slice_threads() {
@@ -168,12 +223,12 @@ __device__ __forceinline__ int wave_slice() {
 // chain of slots, so eight or four waves share a slice (a hexahedron's or tetrahedron's
 // slots all at once, or in two goes); over many slices one wave each fills the chip and
 // the split only adds barriers.  Per BiCGSTAB iteration with one / four / eight waves
-// (slices of a colour): 24,576-cell plate (192) FP64 70 / 47 / 45 us, BF16 41 / 33 / 31;
-// 93,765 cells (735) 80 / 77 / 81, 53 / 51 / 49; 156,849 cells (1,226) 132 / 116 / 116,
-// 62 / 62 / 64; 196,608 cells (1,536) 157 / 153 / 160, 65 / 68 / 71; 162,000 tetrahedra
-// (four colours) 157 / 151 / 166, 102 / 100 / 102; 262,144 cells (2,048) 193 / - / -, 73.
+// (slices of a colour): 24,576-cell plate (192) FP64 92 / 73 / 70 us, BF16 67 / 58 / 56;
+// 93,765 cells (735) 122 / 123 / 132, 87 / 80 / 79; 156,849 cells (1,226) 217 / 189 / 201,
+// 100 / 98 / 100; 196,608 cells (1,536) 241 / 230 / 244, 106 / 105 / 111; 162,000 tetrahedra
+// (four colours) 239 / 231 / 254, 153 / 131 / 137; 262,144 cells (2,048) 302 / 318 / 336,
+// 119 / 126 / 130.
 constexpr int kEightSlices = 384, kSplitSlices = 1536;
-static_assert(kSplitSlices <= kMaxPartials, "a product over that many slices leaves one partial sum each");
 template <int kSplit>
 dim3 slice_grid(int slices) {
     return kSplit == 1 ? grid_for_slices(slices) : dim3(static_cast<unsigned>(slices));
@@ -198,6 +253,18 @@ void with_storage(int storage, F&& f) {
         f(bf16{});
     else
         f(double{});
+}
+
+// f(storage type) with the LU type that follows the vector type, FP64 vectors only
+// with FP64 blocks.
+template <class TV, class F>
+void with_form(const SellMatrix& m, F&& f) {
+    if constexpr (sizeof(TV) == sizeof(double)) {
+        if (m.storage != kStoreF64) throw std::invalid_argument("FP64 SGS needs FP64 blocks");
+        f(double{});
+    } else {
+        with_storage(m.storage, f);
+    }
 }
 
 }  // namespace cfdg

@@ -577,36 +577,52 @@ SellPlan sell_plan(const Tiling& t, const std::vector<i32>& colour_mesh, i32 n_c
     const i32 n = static_cast<i32>(t.new2old.size());
     const std::size_t ntiles = t.tile_off.size() - 1;
     const std::size_t nc = z(n_colours);
-    std::vector<i32> colour(z(n)), lower(z(n)), lower0(z(n)), blocks(z(n));
-    std::vector<std::uint32_t> mask(z(n));  // bit k: the row's k-th block in face order is lower (first 32)
+    std::vector<i32> colour(z(n)), lower(z(n)), blocks(z(n));
+    std::vector<std::uint16_t> before(z(n));
+    std::vector<std::uint32_t> mask(z(n));  // bit k: the row's k-th block in column order is lower (first 32)
+    // per entry of the cell -> face lists, at an interior face: the rank of its block in
+    // the row's column order, and which of the row's blocks it is (lower ones first)
+    std::vector<std::uint16_t> rank(dev_cf.idx.size(), 0), block(dev_cf.idx.size(), 0);
     const auto other = [&](i32 f, i32 r) { return face_owner_dev[z(f)] == r ? face_other_dev[z(f)] : face_owner_dev[z(f)]; };
     parallel_for(z(n), [&](std::size_t r, int) { colour[r] = colour_mesh[z(t.new2old[r])]; }, 4096);
-    // rows of each (colour, tile), and the tile's rows sorted by (colour, lower, lower of colour 0, row)
+    // rows of each (colour, tile), and the tile's rows sorted by (colour, lower, mask, row)
     std::vector<i32> first(nc * ntiles + 1, 0);
     p.tile_pos.resize(z(n));
     parallel_for(ntiles, [&](std::size_t k, int) {
         for (i32 r = t.tile_off[k]; r < t.tile_off[k + 1]; ++r) {
-            i32 lo = 0, lo0 = 0, nb = 0;
+            const i32 e0 = dev_cf.off[z(r)], e1 = dev_cf.off[z(r) + 1], own = t.new2old[z(r)];
+            const auto inner = [&](i32 e) { return dev_cf.idx[z(e)] < n_inner_faces; };
+            const auto column = [&](i32 e) { return t.new2old[z(other(dev_cf.idx[z(e)], r))]; };
+            const auto is_lower = [&](i32 e) { return colour[z(other(dev_cf.idx[z(e)], r))] < colour[z(r)]; };
+            i32 lo = 0, nb = 0, bf = 0;
             std::uint32_t mk = 0;
-            for (i32 e = dev_cf.off[z(r)]; e < dev_cf.off[z(r) + 1]; ++e) {
-                const i32 f = dev_cf.idx[z(e)];
-                if (f >= n_inner_faces) continue;
-                const bool low = colour[z(other(f, r))] < colour[z(r)];
-                if (low && nb < 32) mk |= 1u << nb;
+            for (i32 e = e0; e < e1; ++e) {
+                if (!inner(e)) continue;
                 ++nb;
-                lo += low;
-                lo0 += low && colour[z(other(f, r))] == 0;
+                lo += is_lower(e);
+                bf += column(e) < own;
+            }
+            for (i32 e = e0; e < e1; ++e) {
+                if (!inner(e)) continue;
+                i32 q = 0, same = 0;  // blocks before this one, and those on its side of the diagonal
+                for (i32 g = e0; g < e1; ++g)
+                    if (inner(g) && column(g) < column(e)) {
+                        ++q;
+                        same += is_lower(g) == is_lower(e);
+                    }
+                rank[z(e)] = static_cast<std::uint16_t>(q);
+                block[z(e)] = static_cast<std::uint16_t>(is_lower(e) ? same : lo + same);
+                if (is_lower(e) && q < 32) mk |= 1u << q;
             }
             mask[z(r)] = mk;
             lower[z(r)] = lo;
-            lower0[z(r)] = lo0;
+            before[z(r)] = static_cast<std::uint16_t>(bf);
             blocks[z(r)] = nb;
             p.tile_pos[z(r)] = r;
         }
         std::sort(p.tile_pos.begin() + t.tile_off[k], p.tile_pos.begin() + t.tile_off[k + 1], [&](i32 a, i32 b) {
             if (colour[z(a)] != colour[z(b)]) return colour[z(a)] < colour[z(b)];
             if (lower[z(a)] != lower[z(b)]) return lower[z(a)] < lower[z(b)];
-            if (lower0[z(a)] != lower0[z(b)]) return lower0[z(a)] < lower0[z(b)];
             if (mask[z(a)] != mask[z(b)]) return mask[z(a)] < mask[z(b)];
             return a < b;
         });
@@ -629,7 +645,7 @@ SellPlan sell_plan(const Tiling& t, const std::vector<i32>& colour_mesh, i32 n_c
     p.row.assign(z(at), -1);
     p.pos.resize(z(n));
     p.count.assign(z(at), 0);
-    p.lower0.assign(z(at), 0);
+    p.before.assign(z(at), 0);
     parallel_for(ntiles, [&](std::size_t k, int) {
         i32 c = -1, q = 0;
         for (i32 i = t.tile_off[k]; i < t.tile_off[k + 1]; ++i) {
@@ -640,7 +656,7 @@ SellPlan sell_plan(const Tiling& t, const std::vector<i32>& colour_mesh, i32 n_c
             }
             p.row[z(q)] = r;
             p.pos[z(r)] = q;
-            p.lower0[z(q)] = static_cast<std::uint16_t>(lower0[z(r)]);
+            p.before[z(q)] = before[z(r)];
             p.count[z(q)] = static_cast<std::uint32_t>(lower[z(r)] | ((blocks[z(r)] - lower[z(r)]) << 16));
             p.tile_pos[z(i)] = q++;
         }
@@ -662,7 +678,10 @@ SellPlan sell_plan(const Tiling& t, const std::vector<i32>& colour_mesh, i32 n_c
         s.base = p.n_slots;
         p.n_slots += s.lower + s.upper;
     }
+    for (i32 k = 0; nc > 0 && k < p.colour_slice[1]; ++k) p.first_slots = std::max(p.first_slots, p.slices[z(k)].upper);
     p.cols.assign(z(p.n_slots) * static_cast<std::size_t>(kSliceRows), 0);
+    if (std::any_of(p.slices.begin(), p.slices.end(), [](const Slice& sl) { return sl.lower > 0 && sl.upper > 0; }))
+        p.order.assign(p.cols.size(), 0);
     // block columns and the Jacobian's visits
     p.visit_base.assign(ntiles + 1, 0);
     for (std::size_t k = 0; k < ntiles; ++k) {
@@ -677,16 +696,17 @@ SellPlan sell_plan(const Tiling& t, const std::vector<i32>& colour_mesh, i32 n_c
             const i32 q = p.tile_pos[z(c0 + i)], r = p.row[z(q)];
             const Slice& sl = p.slices[z(q / kSliceRows)];
             const i32 lane = q % kSliceRows, nl = lower[z(r)];
-            i32 k0 = 0, kl = lower0[z(r)], ku = 0, j = 0;
+            i32 j = 0;
             for (i32 e = dev_cf.off[z(r)]; e < dev_cf.off[z(r) + 1]; ++e) {
                 const i32 f = dev_cf.idx[z(e)], s = tf.cell_slot[z(e)];
                 std::uint32_t v = static_cast<std::uint32_t>(s >= 0 ? s : -s - 1) | (s >= 0 ? 0 : kVisitNeighbour);
                 if (f < n_inner_faces) {
-                    const bool low = colour[z(other(f, r))] < colour[z(r)];
-                    const i32 blk = !low ? nl + ku++ : (colour[z(other(f, r))] == 0 ? k0++ : kl++);
-                    const i32 slot = low ? sl.base + blk : sl.base + sl.lower + (blk - nl);
+                    const i32 blk = block[z(e)];
+                    const i32 slot = blk < nl ? blk : sl.lower + (blk - nl);
                     v |= static_cast<std::uint32_t>(blk) << 16;
-                    p.cols[z(slot) * static_cast<std::size_t>(kSliceRows) + z(lane)] = p.pos[z(other(f, r))];
+                    const auto at = [&](i32 q) { return z(sl.base + q) * static_cast<std::size_t>(kSliceRows) + z(lane); };
+                    p.cols[at(slot)] = p.pos[z(other(f, r))];
+                    if (!p.order.empty()) p.order[at(rank[z(e)])] = static_cast<std::uint16_t>(slot);
                 }
                 p.visit[z(p.visit_base[k] + j++ * nt + i)] = v;
             }

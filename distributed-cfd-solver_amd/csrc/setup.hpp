@@ -146,12 +146,14 @@ std::int32_t tile_max_slots(const std::vector<std::int32_t>& tile_off, const Csr
 // Storage order of the block matrix for the multicolour sweeps.  Rows are
 // sorted by colour (each colour starting a new slice), inside a colour by tile
 // and then by the number of blocks whose column has an earlier colour
-// ("lower" blocks) and of those with a column of the first colour, and cut into slices of kSliceRows rows, one per lane of a
-// wave: position p = slice * kSliceRows + lane.  The off-diagonal blocks of a
-// slice are stored slot by slot, first its lower slots, then its upper ones;
-// a row's lower blocks fill the first lower slots, those of the first colour
-// before the others and each in ascending face order, its upper blocks the first
-// upper slots.  The diagonal blocks are kept apart.
+// ("lower" blocks) and by which of the row's blocks these are, and cut into
+// slices of kSliceRows rows, one per lane of a wave: position p = slice *
+// kSliceRows + lane (sliced ELLPACK, the slices sorted for the sweeps).  The
+// off-diagonal blocks of a slice are stored slot by slot, first its lower
+// slots, then its upper ones; a row's lower blocks fill the first lower slots
+// and its upper blocks the first upper slots, each in ascending mesh column,
+// the order in which every product and sweep adds them.  The diagonal blocks
+// are kept apart.
 constexpr int kSliceRows = 64;
 struct Slice {
     std::int32_t base;   // first slot
@@ -165,9 +167,14 @@ struct SellPlan {
     std::vector<std::int32_t> row;           // position -> device row, -1 past a slice's rows
     std::vector<std::int32_t> pos;           // device row -> position
     std::vector<std::uint32_t> count;        // per position: lower blocks | upper blocks << 16
-    std::vector<std::uint16_t> lower0;       // per position: lower blocks whose column has the first colour
+    std::vector<std::uint16_t> before;       // per position: off-diagonal blocks whose mesh column precedes the row's
+    // slot * kSliceRows + lane, k-th slot of a slice that has lower and upper slots: the
+    // slot, counted from the slice's first, of the row's k-th off-diagonal block in
+    // ascending mesh column; empty when no slice has both
+    std::vector<std::uint16_t> order;
     std::vector<std::int32_t> cols;          // slot * kSliceRows + lane -> position of the block's column
     std::int32_t n_slots = 0;
+    std::int32_t first_slots = 0;  // the most slots of a slice of the first colour
     // the Jacobian's visits, per flux tile: the tile's i-th row in position
     // order is tile_pos[tile_off[t] + i]; its j-th visited face is
     // visit[visit_base[t] + j nt + i] (nt = rows of the tile), faces in

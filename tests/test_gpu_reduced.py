@@ -1,10 +1,8 @@
-"""BiCGSTAB with the multicolour sweeps in its reduced form (the first colour kept
-as scalars, products of the corrections only) against a plain float64 numpy
-BiCGSTAB with the full sweeps and products, iterate by iterate: from a zero and
-from a given guess, with two colours (hexahedra) and more (tetrahedra), ragged
-slices, and on either side of the slice count at which a launch changes its form.
-Where the reduced form does not apply -- one cell, and a system whose s vanishes
-exactly -- the solve falls back and must still end at the solution.
+"""BiCGSTAB with the multicolour sweeps against a plain float64 numpy BiCGSTAB with
+the full sweeps and products, iterate by iterate: from a zero and from a given guess,
+with two colours (hexahedra) and more (tetrahedra), ragged slices, and on either side
+of the slice count at which a launch changes its form.  One cell, and a system whose
+s vanishes when alpha rounds to 1, must end at the solution.
 
 Tolerance: the iterates of the dominant matrix (condition number below 10) differ
 by the rounding of a few hundred operations per row and iteration, and the
