@@ -460,27 +460,20 @@ __global__ void __launch_bounds__(kTileCells) k_gradient_limiter_lds(MeshArgs m,
     }
 }
 
-// The second half of gradient_limiter_cell by kLanes lanes of one cell, lane h taking
-// the variables h, h + kLanes, ...: the same operations per variable.
-template <int kLanes, class Self, class NbF, class FVec>
+// The second half of gradient_limiter_cell for the variables var (those with on set) and
+// their gradients gv of one of the two lanes of a cell: the same operations per variable.
+constexpr int kRounds = 3;  // of five variables, per lane
+template <class Self, class NbF, class FVec>
 __device__ __forceinline__ void store_and_limit_split(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, int c,
-                                                      int h, const Self& self, const double (&g)[5][3], NbF nbf,
-                                                      FVec fvec) {
-    constexpr int kRounds = (5 + kLanes - 1) / kLanes;
+                                                      const Self& self, const int (&var)[kRounds],
+                                                      const bool (&on)[kRounds], const double (&gv)[kRounds][3],
+                                                      NbF nbf, FVec fvec) {
     const CellRefW rc = crecw(f, c);
-    int var[kRounds];
-    bool on[kRounds];
-    double gv[kRounds][3], qc[kRounds], qmax[kRounds], qmin[kRounds], ph[kRounds];
+    double qc[kRounds], qmax[kRounds], qmin[kRounds], ph[kRounds];
 #pragma unroll
     for (int r = 0; r < kRounds; ++r) {
-        const int v = h + r * kLanes;
-        on[r] = v < 5;
-        var[r] = on[r] ? v : 4;
-        for (int d = 0; d < 3; ++d) {
-            gv[r][d] = g[0][d];
-            for (int w = 1; w < 5; ++w) gv[r][d] = (var[r] == w) ? g[w][d] : gv[r][d];
+        for (int d = 0; d < 3; ++d)
             if (on[r]) rc[kRG + 3 * var[r] + d] = gv[r][d];
-        }
         qc[r] = self[kRQ + var[r]];
         qmax[r] = qmin[r] = qc[r];
         ph[r] = 1.0;
@@ -512,32 +505,49 @@ __device__ __forceinline__ void store_and_limit_split(const MeshArgs& m, const F
         if (on[r]) rc[kRPhi + var[r]] = ph[r];
 }
 
-// The staged forms with two lanes per cell (workgroups of up to 512 lanes), where one lane per cell leaves too few waves to hide the
-// stencil loop's latencies (launch_gradient_limiter).  The lanes of a cell (adjacent
-// lanes) split the cell's vertex stencil by chunks of four entries (lane h takes
-// chunks h, h + kLanes, ...), each adding its entries in stencil order with the
-// arithmetic of gradient_limiter_cell; the two lanes' sums are then added.  The sums
-// are therefore those of the one-lane form up to the order of that one addition.  The
-// limiter's variables are split over the lanes.  Node LSQ only (the
-// only gradient the staged forms serve).
+// The neighbouring lane's value (lanes 2 k and 2 k + 1 exchange).
+__device__ __forceinline__ double other_lane(double v) {
+    constexpr int kSwapPairs = 0xb1;  // quad permutation 1, 0, 3, 2
+    const long long b = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, static_cast<int>(b), kSwapPairs, 0xf, 0xf, false);
+    const int hi = __builtin_amdgcn_update_dpp(0, static_cast<int>(b >> 32), kSwapPairs, 0xf, 0xf, false);
+    return __longlong_as_double((static_cast<long long>(hi) << 32) | static_cast<unsigned>(lo));
+}
+
+// The staged forms with two lanes per cell (adjacent lanes, workgroups of up to 512), where
+// one lane per cell leaves too few waves to hide the stencil loop's latencies
+// (launch_gradient_limiter).  Node LSQ only (the only gradient the staged forms serve).
+//
+// Wide: the lanes split the cell's vertex stencil by chunks of four entries (lane h takes
+// chunks h, h + 2, ...), each adding its entries in stencil order with the arithmetic of
+// gradient_limiter_cell; the two lanes' sums are then added.  The limiter's variables
+// are split over the lanes.
+//
+// Narrow: the lanes split the variables, lane 0 the first three, lane 1 the others (and
+// nu_tilde), and each adds every entry in stencil order; the entries' coefficients, with
+// the division the larger part of the work, are formed by the lanes in turn and
+// exchanged.  The sums are those of the one-lane form that takes over beyond few tiles, so
+// a cell's gradient does not depend on how many tiles the mesh has.
 template <bool kSA, int kSlots>
 __global__ void __launch_bounds__(2 * kTileCells) k_gradient_limiter_lanes(MeshArgs m, FieldArgs f, NumArgs nm,
                                                                            SaArgs sa) {
-    constexpr int kLanes = 2;
+    constexpr bool kByVariable = kSlots == kGradSlots;
+    constexpr int kStep = kByVariable ? 1 : 2;  // chunks of the stencil from one of a lane's to the next
     stamp_stage(f.stamp, kStampGradients);
     __shared__ __attribute__((aligned(16))) double sq[(kSA ? 9 : 8) * kSlots];
     const int t = xcd_block(blockIdx.x, gridDim.x);
     const int c0 = m.gtile_off[t], nt = m.gtile_off[t + 1] - c0;
     const int hb = m.tile_halo_off[t], ns = nt + (m.tile_halo_off[t + 1] - hb);
-    const int cell = static_cast<int>(threadIdx.x) / kLanes, h = static_cast<int>(threadIdx.x) % kLanes;
+    const int cell = static_cast<int>(threadIdx.x) / 2, h = static_cast<int>(threadIdx.x) % 2;
     const bool live = cell < nt;
     const int nchn = (m.ccn_base[t + 1] - m.ccn_base[t]) / (4 * nt);
     const SlotChunk* chn = reinterpret_cast<const SlotChunk*>(m.ccn_slot + m.ccn_base[t]) + cell;
     // this lane's first two vertex-slot chunks, requested before the staging
+    const int first = kByVariable ? 0 : h;
     SlotChunk cur = 0, nxt = 0;
     if (live) {
-        if (h < nchn) cur = chn[h * nt];
-        if (h + kLanes < nchn) nxt = chn[(h + kLanes) * nt];
+        if (first < nchn) cur = chn[first * nt];
+        if (first + kStep < nchn) nxt = chn[(first + kStep) * nt];
     }
     for (int sl = threadIdx.x; sl < ns; sl += blockDim.x) {
         const int src = (sl < nt) ? c0 + sl : m.tile_halo[hb + sl - nt];
@@ -550,58 +560,110 @@ __global__ void __launch_bounds__(2 * kTileCells) k_gradient_limiter_lanes(MeshA
     __syncthreads();
     const int c = c0 + cell;
     const LdsSlot<kSlots> self{sq, cell};
-    double g[5][3], gs[3] = {0.0, 0.0, 0.0};
-    for (int v = 0; v < 5; ++v) g[v][0] = g[v][1] = g[v][2] = 0.0;
-    if (live) {
-        double qc[5];
-        for (int v = 0; v < 5; ++v) qc[v] = self[kRQ + v];
-        const double x0 = self[kRC], y0 = self[kRC + 1], z0 = self[kRC + 2];
-        const double sc0 = kSA ? sq[8 * kSlots + cell] : 0.0;
-        const int cnt = m.ccn_off[c + 1] - m.ccn_off[c];
-        const CellRef ri{f.cs, f.ld, c};
-        const double i0 = ri[kRInv], i1 = ri[kRInv + 1], i2 = ri[kRInv + 2], i4 = ri[kRInv + 3], i5 = ri[kRInv + 4],
-                     i8 = ri[kRInv + 5];
-        for (int q = h; 4 * q < cnt; q += kLanes) {
+    int var[kRounds];
+    bool on[kRounds];
+    double gv[kRounds][3], gs[3] = {0.0, 0.0, 0.0};
+#pragma unroll
+    for (int r = 0; r < kRounds; ++r) {
+        const int v = kByVariable ? 3 * h + r : h + 2 * r;
+        on[r] = v < 5;
+        var[r] = on[r] ? v : 4;
+        gv[r][0] = gv[r][1] = gv[r][2] = 0.0;
+    }
+    const double x0 = self[kRC], y0 = self[kRC + 1], z0 = self[kRC + 2];
+    const double sc0 = kSA ? sq[8 * kSlots + cell] : 0.0;
+    const CellRef ri{f.cs, f.ld, c};
+    const int cnt = live ? m.ccn_off[c + 1] - m.ccn_off[c] : 0;
+    double inv[6] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
+    if (live)
+        for (int k = 0; k < 6; ++k) inv[k] = ri[kRInv + k];
+    // the coefficients of the stencil entry in a slot
+    const auto coefficients = [&](int slot, double k[3]) {
+        const LdsSlot<kSlots> rn{sq, slot};
+        const double dx = rn[kRC] - x0, dy = rn[kRC + 1] - y0, dz = rn[kRC + 2] - z0;
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        const double wgt = 1.0 / dmax(r2, 1.0e-30);
+        const double rx = wgt * dx, ry = wgt * dy, rz = wgt * dz;
+        k[0] = inv[0] * rx + inv[1] * ry + inv[2] * rz;
+        k[1] = inv[1] * rx + inv[3] * ry + inv[4] * rz;
+        k[2] = inv[2] * rx + inv[4] * ry + inv[5] * rz;
+    };
+    if constexpr (kByVariable) {
+        // where the lane's values lie in a slot; lane 1's third is nu_tilde, in a plane of its own
+        int at[kRounds], stride[kRounds];
+        double q0[kRounds];
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
+            const int k = kRQ + var[r];
+            const bool scalar = kSA && !on[r];
+            at[r] = scalar ? 8 * kSlots : (k >> 1) * 2 * kSlots + (k & 1);
+            stride[r] = scalar ? 1 : 2;
+            q0[r] = sq[at[r] + stride[r] * cell];
+        }
+        for (int q = 0; 4 * q < cnt; ++q) {
             const SlotChunk ch = cur;
             cur = nxt;
-            if (q + 2 * kLanes < nchn) nxt = chn[(q + 2 * kLanes) * nt];
-            for (int e = 0; e < 4 && 4 * q + e < cnt; ++e) {
-                const int slot = chunk_slot(ch, e);
-                const LdsSlot<kSlots> rn{sq, slot};
-                const double dx = rn[kRC] - x0, dy = rn[kRC + 1] - y0, dz = rn[kRC + 2] - z0;
-                const double r2 = dx * dx + dy * dy + dz * dz;
-                const double wgt = 1.0 / dmax(r2, 1.0e-30);
-                const double rx = wgt * dx, ry = wgt * dy, rz = wgt * dz;
-                const double cx = i0 * rx + i1 * ry + i2 * rz;
-                const double cy = i1 * rx + i4 * ry + i5 * rz;
-                const double cz = i2 * rx + i5 * ry + i8 * rz;
-                for (int v = 0; v < 5; ++v) {
-                    const double d = rn[kRQ + v] - qc[v];
-                    g[v][0] += cx * d;
-                    g[v][1] += cy * d;
-                    g[v][2] += cz * d;
-                }
-                if constexpr (kSA) {
-                    const double d = sq[8 * kSlots + slot] - sc0;
-                    gs[0] += cx * d;
-                    gs[1] += cy * d;
-                    gs[2] += cz * d;
+            if (q + 2 < nchn) nxt = chn[(q + 2) * nt];
+            for (int e = 0; e < 4 && 4 * q + e < cnt; e += 2) {  // the lanes of a cell together
+                const bool both = 4 * q + e + 1 < cnt;
+                double mine[3], theirs[3];
+                coefficients(chunk_slot(ch, both ? e + h : e), mine);
+#pragma unroll
+                for (int d = 0; d < 3; ++d) theirs[d] = other_lane(mine[d]);
+                for (int u = 0; u < (both ? 2 : 1); ++u) {
+                    const int slot = chunk_slot(ch, e + u);
+#pragma unroll
+                    for (int r = 0; r < kRounds; ++r) {
+                        const double dq = sq[at[r] + stride[r] * slot] - q0[r];
+#pragma unroll
+                        for (int d = 0; d < 3; ++d) gv[r][d] += (u == h ? mine[d] : theirs[d]) * dq;
+                    }
                 }
             }
         }
-    }
-    // the lanes' sums added (every lane takes part)
-#pragma unroll
-    for (int x = 1; x < kLanes; x <<= 1) {
-        for (int v = 0; v < 5; ++v)
-            for (int d = 0; d < 3; ++d) g[v][d] += __shfl_xor(g[v][d], x, 64);
         if constexpr (kSA)
-            for (int d = 0; d < 3; ++d) gs[d] += __shfl_xor(gs[d], x, 64);
+            for (int d = 0; d < 3; ++d) gs[d] = gv[kRounds - 1][d];
+    } else {
+        double g[5][3], qc[5];
+        for (int v = 0; v < 5; ++v) {
+            g[v][0] = g[v][1] = g[v][2] = 0.0;
+            qc[v] = self[kRQ + v];
+        }
+        for (int q = h; 4 * q < cnt; q += kStep) {
+            const SlotChunk ch = cur;
+            cur = nxt;
+            if (q + 2 * kStep < nchn) nxt = chn[(q + 2 * kStep) * nt];
+            for (int e = 0; e < 4 && 4 * q + e < cnt; ++e) {
+                const int slot = chunk_slot(ch, e);
+                const LdsSlot<kSlots> rn{sq, slot};
+                double k[3];
+                coefficients(slot, k);
+                for (int v = 0; v < 5; ++v) {
+                    const double d = rn[kRQ + v] - qc[v];
+                    for (int x = 0; x < 3; ++x) g[v][x] += k[x] * d;
+                }
+                if constexpr (kSA) {
+                    const double d = sq[8 * kSlots + slot] - sc0;
+                    for (int x = 0; x < 3; ++x) gs[x] += k[x] * d;
+                }
+            }
+        }
+        // the lanes' sums added (every lane takes part)
+        for (int v = 0; v < 5; ++v)
+            for (int d = 0; d < 3; ++d) g[v][d] += other_lane(g[v][d]);
+        if constexpr (kSA)
+            for (int d = 0; d < 3; ++d) gs[d] += other_lane(gs[d]);
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r)
+            for (int d = 0; d < 3; ++d) {
+                gv[r][d] = g[0][d];
+                for (int w = 1; w < 5; ++w) gv[r][d] = (var[r] == w) ? g[w][d] : gv[r][d];
+            }
     }
     if (!live) return;
     if constexpr (kSA) {
         const long long nc = m.nc;
-        if (h == 0) {
+        if (h == 1) {
             sa.g[c] = gs[0];
             sa.g[nc + c] = gs[1];
             sa.g[2 * nc + c] = gs[2];
@@ -628,7 +690,7 @@ __global__ void __launch_bounds__(2 * kTileCells) k_gradient_limiter_lanes(MeshA
         ey = fvp[(vw + k) * nt];
         ez = fvp[(2 * vw + k) * nt];
     };
-    store_and_limit_split<kLanes>(m, f, nm, c, h, self, g, nbf, fvec);
+    store_and_limit_split(m, f, nm, c, self, var, on, gv, nbf, fvec);
 }
 
 __device__ __forceinline__ void grad_dirichlet(double* g, const double* gi, double qin, double qfix, double nx,
@@ -1281,9 +1343,8 @@ static void launch_staged_gradient(const MeshArgs& m, const FieldArgs& f, const 
     const dim3 g(static_cast<unsigned>(m.ngtiles));
     // Two lanes per cell in the wide form, whose LDS leaves room for two workgroups per
     // CU, and where there is no second workgroup for a CU anyway.  The narrow form with
-    // one / two lanes: 12 tiles 17.2 / 14.5 us, 106 tiles 21.8 / 18.7, 384 tiles 27.8 /
-    // 28.2, 1,024 tiles 44.8 / 52.4, 8,192 tiles 330 / 432 (four lanes are slower from
-    // the start: 17.6, 21.1, 41).
+    // one / two lanes: 12 tiles 14.6 / 13.6 us, 106 tiles 19.4 / 18.1, 256 tiles 20.0 / 18.8,
+    // 320 tiles 23.5 / 25.9, 1,024 tiles 40 / 48.
     if (m.gslots > kGradSlots)
         hipLaunchKernelGGL((k_gradient_limiter_lanes<kSA, kGradSlotsBig>), g, dim3(2 * cells), 0, s, m, f, nm, sa);
     else if (m.ngtiles <= kFewTiles)
