@@ -1142,7 +1142,7 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
     c.dots.alloc(8);
     c.norms.alloc(5);
     c.norms.zero(s);
-    c.stamp.alloc(cfdg::kStampCount);
+    c.stamp.alloc(2 * static_cast<std::size_t>(cfdg::kStampCount));
     c.stamp.zero(s);
     c.singular.zero(s);
     c.ks.alloc(2 * cfdg::kKsCount);
@@ -1863,7 +1863,8 @@ int cfdg_time_flux_kernel(cfdg_ctx* c, int32_t reps, double* ms_per_launch) {
         if (reps < 1 || !ms_per_launch) throw CfdgError(CFDG_ERR_ARG, "reps >= 1 and an output are required");
         if (!c->have_residual) throw CfdgError(CFDG_ERR_STATE, "time_flux_kernel needs an evaluated residual");
         const auto m = c->margs();
-        const auto f = c->fargs();
+        auto f = c->fargs();
+        f.stamp += cfdg::kStampCount;  // not the stage times of the last residual
         hip_check(hipEventRecord(c->ev[0], c->stream), "event");
         for (int i = 0; i < reps; ++i) cfdg::launch_flux(m, f, c->nargs, c->stream);
         hip_check(hipEventRecord(c->ev[1], c->stream), "event");

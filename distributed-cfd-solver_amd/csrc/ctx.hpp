@@ -223,7 +223,7 @@ struct cfdg_ctx {
     }
     // timing
     hipEvent_t ev[2] = {};
-    DBuf<unsigned long long> stamp;  // kStamp...
+    DBuf<unsigned long long> stamp;  // kStamp..., and as many again for launches that are no stage
     bool timed_residual = false, timed_gradients = false, timed_jacobian = false, timed_linear = false;
 
     cfdg::MeshArgs margs() const {

@@ -37,3 +37,16 @@ def test_stage_times(order, recon):
     wall = 1e3 * (time.perf_counter() - t0)
     t = np.asarray(s.stage_times())
     assert t[4] > 0.0 and t[5] > 0.0 and t.sum() <= wall
+
+
+@pytest.mark.parametrize("recon", [cfdg.FIRST_ORDER, cfdg.MUSCL])
+def test_timing_the_flux_kernel_leaves_the_stage_times(recon):
+    case = cases.ramp(ni=24, nj=16, nk=8)
+    case.numerics.reconstruction = recon
+    s = cfdg.Solver(cfdg.Mesh.generate(**case.mesh), case.numerics, case.bcs)
+    s.set_state(perturbed_state(s, case))
+    s.implicit_step(cases.default_linparams())
+    s.eval_residual()
+    before = np.asarray(s.stage_times()).copy()
+    assert s.time_flux_kernel(3) > 0.0
+    assert np.array_equal(s.stage_times(), before)
