@@ -1374,7 +1374,10 @@ void launch_lsq_setup(const MeshArgs& m, const FieldArgs& f, hipStream_t s) {
 void launch_ghost_gradients(const MeshArgs& m, const FieldArgs& f, const NumArgs& nm, const BcTable& bcs,
                             hipStream_t s) {
     const int nbf = m.nf - m.ninner;
-    if (nbf > 0) hipLaunchKernelGGL(k_ghost_gradients, grid_for(nbf), dim3(kBlock), 0, s, m, f, nm, bcs);
+    if (nbf > 0)
+        hipLaunchKernelGGL(k_ghost_gradients, grid_for(nbf), dim3(kBlock), 0, s, m, f, nm, bcs);
+    else
+        launch_stamp(f.stamp, kStampGhostGradients, -1, s);  // the stage has no kernel on a closed mesh
 }
 
 template <int kThreads>

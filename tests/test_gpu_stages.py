@@ -50,3 +50,24 @@ def test_timing_the_flux_kernel_leaves_the_stage_times(recon):
     before = np.asarray(s.stage_times()).copy()
     assert s.time_flux_kernel(3) > 0.0
     assert np.array_equal(s.stage_times(), before)
+
+
+def test_stage_times_of_a_mesh_without_boundary():
+    """No ghost cells, so no kernel for their gradients: the stages around it keep
+    their times."""
+    case = cases.ramp(ni=24, nj=16, nk=8)
+    m = cfdg.Mesh.generate(**case.mesh)
+    a, n = m.arrays(), m.n_inner_faces
+    a["face_nodes"] = a["face_nodes"][:a["face_nodes_off"][n]]
+    a["face_nodes_off"] = a["face_nodes_off"][:n + 1]
+    for k in a:
+        if k.startswith("face_") and not k.startswith("face_nodes"):
+            a[k] = a[k][:n]
+    s = cfdg.Solver(cfdg.Mesh.from_arrays(a, 0), case.numerics, [])
+    s.set_state(perturbed_state(s, case))
+    s.eval_residual()
+    t0 = time.perf_counter()
+    s.eval_residual()
+    wall = 1e3 * (time.perf_counter() - t0)
+    t = np.asarray(s.stage_times())
+    assert (t[:2] > 0.0).all() and t[3] > 0.0 and t.sum() <= wall
