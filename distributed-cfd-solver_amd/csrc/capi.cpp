@@ -1188,8 +1188,11 @@ void implicit_step(cfdg_ctx& c, const cfdg_linparams& lp, cfdg_step_result* out)
 // (0.8 GB of staging): out != null reads them, in != null sets them.
 void transfer_blocks(cfdg_ctx& c, double* out, const double* in) {
     const std::size_t nnzb = c.h_cols.size();
-    if (c.block_code.size() != nnzb) c.block_code.upload(mesh_block_codes(c), c.stream);
-    c.sync();
+    if (c.block_code.size() != nnzb) {
+        const std::vector<i32> code = mesh_block_codes(c);
+        c.block_code.upload(code, c.stream);
+        c.sync();  // code is released here
+    }
     const std::size_t piece = std::min<std::size_t>(nnzb, 1u << 22);
     DBuf<double> stage;
     stage.alloc(piece * 25);
@@ -1716,7 +1719,8 @@ int cfdg_set_turbulence(cfdg_ctx* c, const cfdg_mesh* mesh, const cfdg_turbulenc
         c->sa_rho_nu_inf = t->rho_inf * c->sa_nu_inf;
         c->sa_kind.upload(kind, c->stream);
         c->sa_dist.upload(dist_dev, c->stream);
-        c->sa_rnu.upload(std::vector<double>(z(c->ntot), c->sa_rho_nu_inf), c->stream);
+        const std::vector<double> rnu_inf(z(c->ntot), c->sa_rho_nu_inf);
+        c->sa_rnu.upload(rnu_inf, c->stream);
         c->sa_nu.alloc(z(c->ntot));
         c->sa_rho.alloc(z(c->ntot));
         c->sa_mut.alloc(z(c->ntot));

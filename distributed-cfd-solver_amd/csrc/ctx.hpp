@@ -39,6 +39,8 @@ class DBuf {
         n_ = n;
         if (n > 0) hip_check(hipMalloc(reinterpret_cast<void**>(&p_), n * sizeof(T)), "hipMalloc");
     }
+    // h stays as it is until the copy has been waited for, so it cannot be a temporary.
+    void upload(const std::vector<T>&& h, hipStream_t s) = delete;
     void upload(const std::vector<T>& h, hipStream_t s) {
         alloc(h.size());
         if (n_ > 0) hip_check(hipMemcpyAsync(p_, h.data(), n_ * sizeof(T), hipMemcpyHostToDevice, s), "upload");
