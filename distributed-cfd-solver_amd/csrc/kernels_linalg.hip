@@ -824,20 +824,20 @@ template void launch_sgs_group<float>(const int*, int, const BsrArgs&, const voi
                                       const std::uint8_t*, const std::uint8_t*, const float*, float*, hipStream_t,
                                       const double*);
 
-int sgs_levels_capacity(int lu_f32) { return (160 * 1024) / (5 * static_cast<int>(lu_f32 ? sizeof(float) : sizeof(double))); }
+constexpr int kLevelLds = 160 * 1024;
+int sgs_levels_capacity(int lu_f32) { return kLevelLds / (5 * static_cast<int>(lu_f32 ? sizeof(float) : sizeof(double))); }
 
 template <class TS, class TL, class TV>
 static void launch_sgs_levels_as(int n, const SgsLevels& lv, const int* cols, const void* values, const void* lu,
                                  const std::uint8_t* piv, const TV* r, TV* z, hipStream_t s, const double* gate) {
-    const std::size_t lds = static_cast<std::size_t>(n) * 5 * sizeof(TV);
     const auto kernel = k_sgs_levels<TS, TL, TV>;
-    if (lds > 64 * 1024) {
-        const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
-                                                 hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(lds));
-        if (e != hipSuccess) throw std::runtime_error(std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
-    }
-    hipLaunchKernelGGL(kernel, dim3(1), dim3(kLevelThreads), lds, s, n, lv, cols, static_cast<const TS*>(values),
-                       static_cast<const TL*>(lu), piv, r, z, gate);
+    // the limit is the kernel's, for all threads and systems: always the whole LDS, so that
+    // one system's limit never falls below another's launch
+    const hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void*>(kernel),
+                                             hipFuncAttributeMaxDynamicSharedMemorySize, kLevelLds);
+    if (e != hipSuccess) throw std::runtime_error(std::string("hipFuncSetAttribute: ") + hipGetErrorString(e));
+    hipLaunchKernelGGL(kernel, dim3(1), dim3(kLevelThreads), static_cast<std::size_t>(n) * 5 * sizeof(TV), s, n, lv,
+                       cols, static_cast<const TS*>(values), static_cast<const TL*>(lu), piv, r, z, gate);
 }
 
 template <class TV>

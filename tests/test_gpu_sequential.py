@@ -6,6 +6,8 @@ multiple of twelve, and rows with more blocks than are requested ahead
 
 Tolerances: test_gpu_sliced.py.
 """
+from concurrent.futures import ThreadPoolExecutor
+
 import numpy as np
 import pytest
 
@@ -44,3 +46,19 @@ def test_sweeps_match_numpy(kind, size, form):
     if mesh.n_cells > 1:  # one block: s vanishes or not with the rounding of alpha
         assert res.status == cfdg.CONVERGED
         assert np.linalg.norm(b - _spmv(rp, cols, B, x)) <= 1.05e-6 * np.linalg.norm(b)
+
+
+@pytest.mark.parametrize("form", ["fp64", "bf16"])
+def test_threads_with_systems_of_different_size(form):
+    """The kernel's LDS limit is one for the process: a small system's call between
+    another thread's large ones changes nothing."""
+    sizes = [(16, 16, 16), (48, 8, 6), (13, 11, 12)] if form == "fp64" else [(32, 16, 16), (48, 8, 12), (13, 23, 12)]
+    solvers = [_solver("hex", n, form)[1] for n in sizes]
+    r = [np.random.default_rng(k).standard_normal(5 * s.n_cells) for k, s in enumerate(solvers)]
+    alone = [s.sgs_apply(cfdg.SGS_SEQUENTIAL, x) for s, x in zip(solvers, r)]
+
+    def work(k):
+        return all(np.array_equal(solvers[k].sgs_apply(cfdg.SGS_SEQUENTIAL, r[k]), alone[k]) for _ in range(20))
+
+    with ThreadPoolExecutor(len(sizes)) as pool:
+        assert all(pool.map(work, range(len(sizes))))
