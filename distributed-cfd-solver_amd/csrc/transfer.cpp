@@ -3,8 +3,8 @@
 
 #include <algorithm>
 #include <cstring>
+#include <exception>
 #include <string>
-#include <system_error>
 #include <thread>
 #include <vector>
 
@@ -54,7 +54,7 @@ void HostPipe::run(std::size_t bytes, F&& worker) {
     };
     try {
         for (; started + 1 < want; ++started) th.emplace_back(body, started + 1);
-    } catch (const std::system_error&) {
+    } catch (const std::exception&) {  // no thread, or no memory for one
     }
     body(0);
     for (int w = started + 1; w < want; ++w) body(w);
