@@ -867,14 +867,13 @@ void check_numerics(const cfdg_numerics* num) {
         throw CfdgError(CFDG_ERR_CONFIG, "viscous flow needs prandtl > 0 and prandtl_turb > 0");
 }
 
-// Block arrays and LU factors of the sliced layout.
+// Block arrays and LU factors of the sliced layout.  Neither they nor the vectors are
+// cleared: nothing reads what is past a slice's rows or a row's blocks.
 void alloc_blocks(cfdg_ctx& c, int storage) {
     c.sell_off.alloc(0);
     c.sell_diag.alloc(0);
     c.sell_off.alloc(z(c.sell.n_slots) * cfdg::sell_slot_bytes(storage));
     c.sell_diag.alloc(z(c.n_slices()) * cfdg::sell_slot_bytes(storage));
-    c.sell_off.zero(c.stream);
-    c.sell_diag.zero(c.stream);
     c.have_csr = false;
     c.values.alloc(0);
 }
@@ -1136,7 +1135,6 @@ void setup_context(cfdg_ctx& c, const cfdg::Mesh& m, const cfdg::MeshConnectivit
     c.singular.alloc(1);
     for (DBuf<double>* v : {&c.r, &c.r0, &c.p, &c.v, &c.s, &c.t, &c.ph, &c.sh, &c.bs, &c.xs, &c.b, &c.x}) {
         v->alloc(v == &c.b || v == &c.x ? 5 * ncs : c.vector_alloc());
-        v->zero(s);
     }
     c.partial.alloc(cfdg::kNormPartials + 5 * static_cast<std::size_t>(cfdg::kReduceBlocks));
     c.dots.alloc(8);
@@ -1232,7 +1230,6 @@ void set_precision(cfdg_ctx& c, const cfdg_precision& p) {
         auto& f = c.f32;
         for (DBuf<float>* v : {&f.b, &f.x, &f.r, &f.r0, &f.p, &f.v, &f.s, &f.t, &f.ph, &f.sh}) {
             if (v->size() != c.vector_alloc()) v->alloc(c.vector_alloc());
-            v->zero(c.stream);
         }
     } else {
         auto& f = c.f32;

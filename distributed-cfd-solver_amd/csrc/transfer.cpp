@@ -66,7 +66,6 @@ void HostPipe::to_device(void* dst, const void* src, std::size_t bytes, hipStrea
     if (bytes == 0) return;
     if (!piped(bytes)) {
         check(hipMemcpyAsync(dst, src, bytes, hipMemcpyHostToDevice, s), "H2D");
-        check(hipStreamSynchronize(s), "hipStreamSynchronize");
         return;
     }
     run(bytes, [&](int w, int workers) -> hipError_t {

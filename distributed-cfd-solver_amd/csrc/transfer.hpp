@@ -23,8 +23,9 @@ class HostPipe {
     // Pinned slots for arrays of up to this many bytes on the current device;
     // none are made when all are small.
     void reserve(std::size_t bytes);
-    // Both return with the host array read or written; the copies run on s after
-    // the work already enqueued there.
+    // The copies run on s after the work already enqueued there.  to_device's source stays
+    // as it is until s is waited for (small arrays are read by then, others on return);
+    // to_host returns with the array written.
     void to_device(void* dst, const void* src, std::size_t bytes, hipStream_t s);
     void to_host(void* dst, const void* src, std::size_t bytes, hipStream_t s);
 
