@@ -34,7 +34,10 @@ void HostPipe::reserve(std::size_t bytes) {
     check(hipGetDevice(&device_), "hipGetDevice");
     for (hipEvent_t& e : ev_)
         if (!e) check(hipEventCreateWithFlags(&e, hipEventDisableTiming), "hipEventCreate");
-    check(hipHostMalloc(reinterpret_cast<void**>(&pinned_), kSlots * kPiece), "hipHostMalloc");
+    if (hipHostMalloc(reinterpret_cast<void**>(&pinned_), kSlots * kPiece) != hipSuccess) {
+        pinned_ = nullptr;
+        (void)hipGetLastError();  // the runtime's own copies do without
+    }
 }
 
 // worker(w, workers) on every thread; the first error is thrown when all have

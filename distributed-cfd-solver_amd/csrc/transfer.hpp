@@ -21,7 +21,8 @@ class HostPipe {
     HostPipe& operator=(const HostPipe&) = delete;
     ~HostPipe();
     // Pinned slots for arrays of up to this many bytes on the current device;
-    // none are made when all are small.
+    // none are made when all are small, and without pinned memory for them every array
+    // goes through the runtime's copy.
     void reserve(std::size_t bytes);
     // The copies run on s after the work already enqueued there.  to_device's source stays
     // as it is until s is waited for (small arrays are read by then, others on return);

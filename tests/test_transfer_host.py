@@ -28,7 +28,14 @@ inline hipError_t hipEventSynchronize(hipEvent_t) { return 0; }
 inline hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return 0; }
 inline hipError_t hipGetDevice(int* d) { *d = 0; return 0; }
 inline hipError_t hipSetDevice(int) { return 0; }
-inline hipError_t hipHostMalloc(void** p, std::size_t n) { *p = std::malloc(n); return 0; }
+inline bool no_pinned = false;
+inline int last_error = 0;
+inline hipError_t hipHostMalloc(void** p, std::size_t n) {
+    if (no_pinned) return last_error = 2;
+    *p = std::malloc(n);
+    return 0;
+}
+inline hipError_t hipGetLastError() { const int e = last_error; last_error = 0; return e; }
 inline hipError_t hipHostFree(void* p) { std::free(p); return 0; }
 inline hipError_t hipStreamSynchronize(hipStream_t) { return 0; }
 inline hipError_t hipMemcpyAsync(void* d, const void* s, std::size_t n, int, hipStream_t) { std::memcpy(d, s, n); return 0; }
@@ -56,8 +63,11 @@ int main() {
     const std::size_t mib = 1u << 20;
     int failed = 0;
     for (std::size_t bytes : {mib / 2, 2 * mib, 5 * mib + 8, 16 * mib, 37 * mib + 123}) {
+      for (const bool pinned : {true, false}) {
+        no_pinned = !pinned;
         cfdg::HostPipe pipe;
         pipe.reserve(bytes);
+        if (last_error != 0) failed = 1;
         std::vector<char> src(bytes), dev(bytes), back(bytes);
         for (std::size_t i = 0; i < bytes; ++i) src[i] = static_cast<char>(i * 2654435761u >> 13);
         // the first allocation of a copy is its list of threads, the others one per thread
@@ -74,6 +84,7 @@ int main() {
                 failed = 1;
             }
         }
+      }
     }
     return failed;
 }
