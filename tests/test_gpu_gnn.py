@@ -169,3 +169,30 @@ def test_learned_warm_start_effect_on_a_steady_run():
     print(f"plain: {rp.steps} steps, {rp.linear_iterations} linear iterations; learned: {rw.steps} steps, "
           f"{rw.linear_iterations} linear iterations, kept {used}, rejected {rejected}; state difference {err:.2e}")
     assert err <= 1e-8
+
+
+@pytest.mark.parametrize("order", [cfdg.SGS_MULTICOLOUR, cfdg.SGS_SEQUENTIAL])
+@pytest.mark.parametrize("krylov", [cfdg.PREC_FP64, cfdg.PREC_FP32])
+@pytest.mark.parametrize("flow", ["plate", "bump"])  # two colours, and more
+def test_rejected_guess_leaves_the_solve_from_zero(flow, krylov, order):
+    """A network whose output bias makes every guess worse than zero: each solve
+    restarts from zero, with the bits of a solve that never had a guess."""
+    case = {"plate": lambda: cases.plate(ni=13, nj=11, nk=5), "bump": lambda: cases.bump(ni=6, nj=5, nk=4)}[flow]()
+    mesh = cfdg.Mesh.generate(**case.mesh)
+    g = cfdg.Gnn(seed=0)
+    p = np.zeros(g.num_params, np.float32)
+    p[-5:] = 1e6  # the output biases are the last five parameters
+    g.set_params(p)
+    lp = cases.default_linparams(order=order)
+    outs = []
+    for gnn in (None, g):
+        s = cfdg.Solver(mesh, case.numerics, case.bcs)
+        s.set_precision(cfdg.Precision.make(krylov, krylov))
+        s.set_state(perturbed_state(s, case))
+        if gnn is not None:
+            s.set_warm_start(gnn)
+        steps = [s.implicit_step(lp) for _ in range(3)]
+        outs.append((s.get_state(), [(r.linear.iterations, r.linear.status, tuple(r.l2)) for r in steps]))
+    assert s.warm_start_stats() == (0, 3)
+    assert outs[0][1] == outs[1][1]
+    assert np.array_equal(outs[0][0], outs[1][0])
