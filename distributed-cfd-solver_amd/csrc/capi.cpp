@@ -6,7 +6,7 @@
 // crossing the ABI is in mesh order.  States, block values and the multicolour
 // solve's vectors are permuted on the device from and to a staging buffer (2.1M
 // cells: set_state and get_state 2.8 ms each, where a permutation on the host and
-// a pageable copy took about 40 ms each); the rest is permuted here, on the host.
+// a pageable copy took 15 and 29 ms); the rest is permuted here, on the host.
 #include "cfdg.h"
 
 #include <hip/hip_runtime.h>

@@ -19,8 +19,8 @@
 // y + sum_{j<c} A_cj d_j with the backward sweep's corrections d, and A z = y in the first
 // colour.  They halve the bytes again, but put y where the product has D z, so that the
 // error of the 5x5 solve, large where a block's rows differ by orders of magnitude as at
-// low Mach number, no longer enters the residual and is never corrected: the update
-// lost a factor of 10 to 20 of accuracy on this solver's own matrices.
+// low Mach number, no longer enters the residual and is never corrected: the update was
+// 3 times (plate, one iteration) to 22 times (SA bump, two) further from 80-bit floats.
 //
 // Bound: HBM.  2.1M-cell plate (256 x 64 x 128) in FP64, per preconditioned product:
 // k_sell_sweep 320 us, k_first_colour 354 us, k_sell_spmv over the other colour 302 us
