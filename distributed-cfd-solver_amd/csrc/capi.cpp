@@ -867,13 +867,16 @@ void check_numerics(const cfdg_numerics* num) {
         throw CfdgError(CFDG_ERR_CONFIG, "viscous flow needs prandtl > 0 and prandtl_turb > 0");
 }
 
-// Block arrays and LU factors of the sliced layout.  Neither they nor the vectors are
-// cleared: nothing reads what is past a slice's rows or a row's blocks.
+// Block arrays and LU factors of the sliced layout.  The solver reads nothing past a
+// slice's rows or a row's blocks, so its vectors and factors are not cleared; the blocks
+// are, because cfdg_get_bsr_values gives zeros until they are set.
 void alloc_blocks(cfdg_ctx& c, int storage) {
     c.sell_off.alloc(0);
     c.sell_diag.alloc(0);
     c.sell_off.alloc(z(c.sell.n_slots) * cfdg::sell_slot_bytes(storage));
     c.sell_diag.alloc(z(c.n_slices()) * cfdg::sell_slot_bytes(storage));
+    c.sell_off.zero(c.stream);
+    c.sell_diag.zero(c.stream);
     c.have_csr = false;
     c.values.alloc(0);
 }

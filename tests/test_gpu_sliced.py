@@ -112,3 +112,23 @@ def test_orders_share_a_context(kind, size, form):
     s.set_bsr_values(2.0 * v)  # the copy follows the blocks
     for lp, x0 in zip(lps, fresh):
         assert np.allclose(s.linear_solve(lp, b=2.0 * b)[0], x0, rtol=0.0, atol=1e-6 * np.max(np.abs(x0)))
+
+
+@pytest.mark.parametrize("form", sorted(FORMS))
+def test_blocks_are_zero_until_set(form):
+    """In a new context and after a change of the storage, also where the memory held
+    another system's blocks before."""
+    for size in ((41, 40, 31), (41, 40, 31), (13, 11, 3)):
+        mesh, s, rp, cols, dg, v = _solver("hex", size, form)
+        assert s.bsr_values().any()
+        s.close()
+        case = _case("hex", size)
+        s = cfdg.Solver(mesh, case.numerics, case.bcs)
+        assert not s.bsr_values().any()
+        s.set_bsr_values(v)
+        s.set_precision(cfdg.Precision.make(cfdg.PREC_BF16, cfdg.PREC_FP32))
+        assert not s.bsr_values().any()
+        s.set_precision(FORMS[form])
+        if FORMS[form].block_storage != cfdg.PREC_BF16:
+            assert not s.bsr_values().any()
+        s.close()
